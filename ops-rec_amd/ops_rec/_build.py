@@ -5,6 +5,7 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
@@ -12,6 +13,7 @@ _PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(_PKG), "csrc")
 LIB_DIR = os.path.join(_PKG, "_lib")
 LIB_PATH = os.path.join(LIB_DIR, "libhstu_mi355.so")
+BINDING_PATH = os.path.join(LIB_DIR, "_torch_binding.so")
 
 # the host side, and the kernels by input type and direction: one translation unit each, compiled side by side
 SOURCES = [
@@ -48,11 +50,28 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}): {' '.join(cmd)}\n{res.stdout}")
+        raise RuntimeError(f"build failed ({res.returncode}): {' '.join(cmd)}\n{res.stdout}")
+
+
+def _binding_command(output: str) -> list[str]:
+    """The dispatcher kernels (``csrc/torch_binding.cpp``): host code only, against torch's headers and the HIP library next to it."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc_path())))
+    includes = (os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                os.path.join(rocm, "include"), sysconfig.get_paths()["include"])  # fmt: skip
+    return [
+        os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(a for i in includes for a in ("-isystem", i)),
+        os.path.join(CSRC, "torch_binding.cpp"), "-o", output, f"-L{os.path.join(root, 'lib')}", "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+        "-ltorch_hip", "-ltorch_python", f"-L{LIB_DIR}", f"-l:{os.path.basename(LIB_PATH)}", "-Wl,-rpath,$ORIGIN",
+    ]  # fmt: skip
 
 
 def build(verbose: bool = False, jobs: int | None = None, extra_flags: tuple = (), lib_path: str | None = None) -> str:
-    """Compile ``csrc/*.hip`` into ``ops_rec/_lib/libhstu_mi355.so`` (always recompiles every source).
+    """Compile ``csrc/*.hip`` into ``ops_rec/_lib/libhstu_mi355.so`` (always recompiles every source), and the dispatcher kernels
+    into ``_torch_binding.so`` beside it.
     ``extra_flags`` / ``lib_path`` build a variant elsewhere (the timeline example builds one with ``-DHSTU_TIMELINE``)."""
     target = lib_path or LIB_PATH
     os.makedirs(os.path.dirname(target), exist_ok=True)
@@ -70,4 +89,8 @@ def build(verbose: bool = False, jobs: int | None = None, extra_flags: tuple = (
         tmp = target + ".tmp"
         _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objects], verbose)
     os.replace(tmp, target)
+    if target == LIB_PATH:
+        tmp = BINDING_PATH + ".tmp"
+        _run(_binding_command(tmp), verbose)
+        os.replace(tmp, BINDING_PATH)
     return target

@@ -7,7 +7,9 @@ Mirrors the reference adapter for this path
 * ``_forward_impl`` does the argument normalisation and checks of
   ``hstu_deltaq_forward_impl_npu`` (``:22-67``) and then calls the C ABI of the HIP library
   where the reference calls ``aclnnHstuJaggedForward`` (``:63-65``);
-* device tensors dispatch on the ``CUDA`` key (PyTorch-ROCm's key for HIP tensors), shape
+* device tensors dispatch on the ``CUDA`` key (PyTorch-ROCm's key for HIP tensors): to the native kernels of
+  ``csrc/torch_binding.cpp`` where a call needs no check to fail and no conversion, and from there to the functions
+  of this module otherwise (``_dispatch.py``); shape
   inference for ``torch.compile`` on ``Meta`` (``:269-351``); autograd is attached from Python
   (``ops_rec/autograd/hstu_v1_autograd.py``), not here (``:258-263``).
 
@@ -58,7 +60,8 @@ _SCHEMAS = (
 _lib_def = torch.library.Library("ops_rec", "DEF")
 for _s in _SCHEMAS:
     _lib_def.define(_s)
-_lib_cuda = torch.library.Library("ops_rec", "IMPL", "CUDA")
+_lib_cuda = torch.library.Library("ops_rec", "IMPL", "CUDA")  # what ``_dispatch`` replaces by native kernels
+_lib_cuda_dense = torch.library.Library("ops_rec", "IMPL", "CUDA")
 _lib_meta = torch.library.Library("ops_rec", "IMPL", "Meta")
 
 _DTYPE_CODE = {
@@ -344,6 +347,9 @@ def _forward_impl(q, k, v, mask, attn_bias, mask_type, max_seq_len_q, max_seq_le
         return prepared.launch()
 
 
+_fp8_native = None  # the native form of the function below, once ``_dispatch`` has attached it
+
+
 def hstu_jagged_fp8(q, k, v, q_descale=None, k_descale=None, v_descale=None, *, mask=None, attn_bias=None, mask_type=0,
                     max_seq_len=0, max_seq_len_k=None, silu_scale=0.0, seq_offset=None, seq_offset_k=None,
                     num_context=None, num_target=None, target_group_size=0, alpha=1.0, out_dtype=torch.bfloat16):  # fmt: skip
@@ -357,6 +363,11 @@ def hstu_jagged_fp8(q, k, v, q_descale=None, k_descale=None, v_descale=None, *, 
     _check(q.dtype == torch.float8_e4m3fn, "hstu_jagged_fp8 takes float8_e4m3fn tensors")
     offs_k = seq_offset if seq_offset_k is None else seq_offset_k
     max_k = max_seq_len if max_seq_len_k is None else max_seq_len_k
+    if _fp8_native is not None and out_dtype in (torch.bfloat16, torch.float16) and seq_offset is not None:
+        out = _fp8_native(q, k, v, q_descale, k_descale, v_descale, mask, attn_bias, mask_type, max_seq_len, max_k, silu_scale,
+                          seq_offset, offs_k, num_context, num_target, target_group_size, alpha, out_dtype == torch.float16)  # fmt: skip
+        if out is not None:
+            return out
     prepared = prepare_forward(q, k, v, mask, attn_bias, mask_type, max_seq_len, max_k, silu_scale, seq_offset, offs_k,
                                num_context, num_target, target_group_size, alpha, False, out_dtype=out_dtype,
                                q_descale=q_descale, k_descale=k_descale, v_descale=v_descale)  # fmt: skip
@@ -607,9 +618,9 @@ def hstu_dense(q, k, v, mask=None, attn_bias=None, mask_type=0, max_seq_len=0, s
     offs_k = offs_q if s_k == s_q else _dense_offsets(batch, s_k, dev)
     if batch == 0 or s_q == 0:
         return torch.empty((batch, s_q, q.size(2), v.size(3)), dtype=_out_dtype(qc), device=dev)
-    out = _forward_impl(qc.view(batch * s_q, q.size(2), q.size(3)), kc.view(batch * s_k, k.size(2), k.size(3)),
-                        vc.view(batch * s_k, v.size(2), v.size(3)), mask, attn_bias, mask_type, max(s_q, 1), max(s_k, 1),
-                        real_scale, offs_q, offs_k, None, None, 0, 1.0)  # fmt: skip
+    out = torch.ops.ops_rec.hstu_jagged.delta(
+        qc.view(batch * s_q, q.size(2), q.size(3)), kc.view(batch * s_k, k.size(2), k.size(3)), vc.view(batch * s_k, v.size(2), v.size(3)),
+        mask, attn_bias, mask_type, max(s_q, 1), max(s_k, 1), real_scale, offs_q, offs_k, None, None, 0, 1.0)  # fmt: skip
     return out.view(batch, s_q, q.size(2), v.size(3))
 
 
@@ -713,8 +724,8 @@ def hstu_dense_backward(grad, q, k, v, mask, attn_bias, mask_type=0, max_seq_len
     dev = grad.device
     offs = _dense_offsets(batch, s_len, dev)
     flat = lambda t: t.contiguous().view(batch * s_len, heads, dim)  # noqa: E731
-    dq, dk, dv, dbias = _backward_impl(flat(grad), flat(q), flat(k), flat(v), mask, attn_bias, mask_type, s_len, s_len,
-                                       silu_scale, offs, offs, None, None, 0, 1.0)  # fmt: skip
+    dq, dk, dv, dbias = torch.ops.ops_rec.hstu_jagged_backward.delta(
+        flat(grad), flat(q), flat(k), flat(v), mask, attn_bias, mask_type, s_len, s_len, silu_scale, offs, offs, None, None, 0, 1.0)  # fmt: skip
     if dbias is None:
         padded = (s_len + 255) // 256 * 256
         dbias = torch.zeros((batch, heads, padded, padded), dtype=grad.dtype, device=dev)
@@ -731,11 +742,11 @@ def hstu_dense_backward_meta(grad, q, k, v, mask, attn_bias, mask_type=0, max_se
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), dbias
 
 
-_lib_cuda.impl("hstu_dense_backward", hstu_dense_backward)
+_lib_cuda_dense.impl("hstu_dense_backward", hstu_dense_backward)
 _lib_meta.impl("hstu_dense_backward", hstu_dense_backward_meta)
 _lib_cuda.impl("hstu_paged", hstu_paged)
 _lib_meta.impl("hstu_paged", hstu_paged_meta)
-_lib_cuda.impl("hstu_dense", hstu_dense)
+_lib_cuda_dense.impl("hstu_dense", hstu_dense)
 _lib_meta.impl("hstu_dense", hstu_dense_meta)
 _lib_cuda.impl("hstu_jagged.equal", hstu_jagged_equal)
 _lib_cuda.impl("hstu_jagged.delta", hstu_jagged_delta)
@@ -745,3 +756,23 @@ _lib_meta.impl("hstu_jagged.equal", hstu_jagged_equal_meta)
 _lib_meta.impl("hstu_jagged.delta", hstu_jagged_delta_meta)
 _lib_meta.impl("hstu_jagged_backward.equal", hstu_jagged_backward_equal_meta)
 _lib_meta.impl("hstu_jagged_backward.delta", hstu_jagged_backward_delta_meta)
+
+
+def _pick_overload_by_argument(packet, position: int) -> None:
+    """A call of the packet itself tries its overloads in turn, and each that does not fit costs an exception with its text (12 us
+    for ``delta``, the second).  The two differ in what stands at ``position``: the offsets (``equal``) or ``silu_scale``."""
+    resolve, equal, delta = packet._op, packet.equal._op, packet.delta._op
+
+    def call(*args, **kwargs):
+        if len(args) > position:
+            if isinstance(args[position], torch.Tensor):
+                return equal(*args, **kwargs)
+            if isinstance(args[position], (float, int)):
+                return delta(*args, **kwargs)
+        return resolve(*args, **kwargs)
+
+    packet._op = call
+
+
+_pick_overload_by_argument(torch.ops.ops_rec.hstu_jagged, 8)
+_pick_overload_by_argument(torch.ops.ops_rec.hstu_jagged_backward, 9)
