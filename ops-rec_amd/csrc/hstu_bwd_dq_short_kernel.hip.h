@@ -275,7 +275,7 @@ __global__ __launch_bounds__(kDqShortThreads, kDqShortWavesPerSimd) void hstu_bw
             ds[e] = score_ds(sv, dv, sconst);
             pv[e] = WANT_P ? score_p(sv, sconst) : 0.f;
         }
-        const bool full = (c0 + 32 <= wb.lim_min) && !(wb.any_hole && c0 + 32 > sq_info.hist_k && c0 < wb.hole_hi_max);
+        const bool full = (c0 + 32 <= wb.lim_min) & !(wb.any_hole & (c0 + 32 > sq_info.hist_k) & (c0 < wb.hole_hi_max));
         if (!full) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {

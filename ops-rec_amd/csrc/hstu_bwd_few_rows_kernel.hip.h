@@ -240,7 +240,7 @@ __global__ __launch_bounds__(kFewRowsThreads, 2) void hstu_bwd_few_rows_kernel(c
             ds[e] = score_ds(sv, dv, sconst);
             pv[e] = score_p(sv, sconst);
         }
-        const bool full = (c0 + 32 <= wb.lim_min) && !(wb.any_hole && c0 + 32 > si.hist_k && c0 < wb.hole_hi_max);
+        const bool full = (c0 + 32 <= wb.lim_min) & !(wb.any_hole & (c0 + 32 > si.hist_k) & (c0 < wb.hole_hi_max));
         if (!full) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {

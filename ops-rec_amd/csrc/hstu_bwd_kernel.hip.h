@@ -698,7 +698,7 @@ __global__ __launch_bounds__(256, bwd_dq_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void 
         // visibility, applied to the packed values and only when the sub-tile is not fully visible to this
         // wavefront's rows (as in the forward): key c0 + 8 (e / 4) + 4 lh + e % 4 of element e is hidden at or past
         // lim and inside the hole
-        const bool full = (c0 + 32 <= wb.lim_min) && !(wb.any_hole && c0 + 32 > sq_info.hist_k && c0 < wb.hole_hi_max);
+        const bool full = (c0 + 32 <= wb.lim_min) & !(wb.any_hole & (c0 + 32 > sq_info.hist_k) & (c0 < wb.hole_hi_max));
         if (!full && c0 >= row_only_lo && c0 + 32 <= row_only_hi) {
             const uint32_t keep = lim > c0 ? 0xffffffffu : 0u;  // (a context row's limit is at or past c0 + 32, any other row's at or before c0)
 #pragma unroll

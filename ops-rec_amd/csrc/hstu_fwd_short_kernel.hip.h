@@ -428,7 +428,9 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
                     tt = __builtin_amdgcn_rcpf(1.0f + tt);
                     p[e] = s * tt;
                 }
-                const bool full = (c0 + 32 <= wb.lim_min) && !(wb.any_hole && c0 + 32 > hist_k && c0 < wb.hole_hi_max);
+                // (combined without branches: where a branch stands between the last MFMA and the first read of its result, this compiler counts
+                // the instructions of the longer way round as wait states, and the shorter way may read too early)
+                const bool full = (c0 + 32 <= wb.lim_min) & !(wb.any_hole & (c0 + 32 > hist_k) & (c0 < wb.hole_hi_max));
                 if (!full) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
