@@ -27,6 +27,9 @@ constexpr int fwd_wgs_per_cu(int d, bool rab, bool mask)
 // channels.  With max_seq_len_k 8192 the plain count, 256 lines = 32 KiB, put them all on one (measured on MI355X, 2
 // sequences x 4 heads of 4096 .. 8192 rows: query-tile kernel 445 us, 298 us with the odd pitch).
 constexpr int64_t pair_full_pitch_lines(int64_t max_k) { return ((max_k + 31) / 32) | 1; }
+// wavefronts of a workgroup of the fp32 forward kernel (16 query rows or a share of their keys each): eight, four at the slot
+// 256, whose wavefronts need more than 128 registers and whose partial outputs fill 64 KiB of LDS already
+constexpr int f32_waves(int d) { return d <= 128 ? 8 : 4; }
 constexpr int kShortThreads = 512;  // threads of a workgroup of the forward kernel for short lists (eight wavefronts of 16 query rows)
 constexpr int kTinyThreads = 128;   // threads of a workgroup of the backward kernel for tiny sequences (two wavefronts of 16 query rows)
 constexpr int kTinyRows = 32;       // the longest sequence (rows and keys) that kernel takes; the forward one: 32 or 64, four threads per row
@@ -75,6 +78,7 @@ struct FwdArgs {
     const float* q_descale;  // fp8 inputs only; per head, nullptr = 1
     const float* k_descale;
     const float* v_descale;
+    int f32_splits;          // fp32 inputs only: wavefronts that share the keys of one row group (a power of two up to f32_waves)
     unsigned int* counters;  // kCounterBlockBytes at the head of the workspace, cleared ahead of the launch; null for the plain list
     float* ws;           // split variant: room for ws_parts partial outputs of kBlockM x D floats each (may be null)
     uint32_t ws_parts;

@@ -31,6 +31,15 @@ namespace hstu {
 
 typedef __attribute__((ext_vector_type(4))) float bwd_f32x4_t;
 
+// 16-byte chunks of a row are XOR-swizzled by the row number so that "32 lanes = 32 rows, same
+// column" reads (the A operand of S^T = K.Q^T) spread over the banks.
+template <int D>
+__device__ __forceinline__ int f32_chunk_swizzle(int row, int chunk)
+{
+    constexpr int CPR = D / 4;  // 16-byte chunks per row
+    return chunk ^ (row & (CPR - 1) & 31);
+}
+
 // the 16 values of a [max_q, max_k] fp32 plane at row `row`, keys c0 + 8 g + 4 half + 0..3 (g = 0..3): the elements of
 // a lane in the S^T layout (lane = query row)
 __device__ __forceinline__ void f32_load_row_keys(__amdgpu_buffer_rsrc_t rsrc, uint32_t row_off, int c0, int half, int max_k,

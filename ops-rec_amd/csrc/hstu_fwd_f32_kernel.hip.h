@@ -1,51 +1,65 @@
 // HSTU jagged attention forward for gfx950: fp32 inputs, fp32 output.
 //
-// Same algorithm and work split as the 16-bit kernel (one workgroup per 128-row query tile, four
-// wavefronts of 32 rows, K/V tiles staged in LDS by buffer loads that write LDS directly, S^T = K.Q^T
-// so that P^T feeds the second product from registers), but both products run on the fp32 matrix
-// instruction v_mfma_f32_32x32x2_f32 and P is not rounded.  This variant exists for dtype coverage
-// (the reference accepts fp32 q/k/v: op_host/atlas950/op_def_arch.h:23); it is not the tuned path.
+// A wavefront owns 16 query rows and works alone: both products run on v_mfma_f32_16x16x4_f32, whose operand layouts let it
+// read K and V from memory straight into the registers the instruction takes, 16 keys a block, the next block on its way
+// while the products of this one run; no LDS and no barrier in the sweep.  The fp32 matrix instruction is slow (32 cycles for
+// 2048 flops, 154 TFLOP/s of the card), so the sweep is bound by the matrix pipe, and a small launch by how long ONE
+// wavefront sweeps: a workgroup's wavefronts therefore stand for row groups x key shares, a.f32_splits of them dealing the
+// key blocks of one row group and adding their outputs through LDS in a fixed order.  The host takes as many shares as
+// it needs to fill the machine (f32_splits() there).
 //
-// Operand layouts of v_mfma_f32_32x32x2_f32 (A is 32x2, B is 2x32): lane l supplies A[l % 32][l / 32]
-// and B[l / 32][l % 32]; the accumulator layout is that of the 32x32 bf16 instruction.
+// Layouts (lane l, i = l % 16, g = l / 16): A[i][g], B[g][i], accumulator rows 4 g + r, column i.  The contraction order of
+// S^T = K Q^T is free: step (j, e) contracts the head dims 16 j + 4 g + e, so a lane holds 16-byte pieces of its row.
+// S^T leaves a lane with keys 4 g + r of query i, which is the B operand of step r of O^T += V^T P^T; there the M index of
+// tile (h, t) is mapped to head dim 64 h + 4 i + t, so that a lane's A operands of four tiles are 16 bytes of one V row
+// and its outputs 16-byte pieces of one output row.
+//
+// Measured (MI355X), the kernel this one replaced (one 128-row tile per workgroup, K and V through one LDS buffer without
+// overlap) against it: see the dispatch rule in hstu_mi355.hip.
 #pragma once
 #include "hstu_fwd_kernel.hip.h"
 
 namespace hstu {
 
-// 16-byte chunks of a row are XOR-swizzled by the row number so that "32 lanes = 32 rows, same
-// column" reads (the A operand of S^T = K.Q^T) spread over the banks.
-template <int D>
-__device__ __forceinline__ int f32_chunk_swizzle(int row, int chunk)
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+// one 16-byte piece at off + base (base uniform and inside the descriptor); outside the descriptor it reads zeros
+__device__ __forceinline__ f32x4_t buffer_f32x4(__amdgpu_buffer_rsrc_t rsrc, uint32_t off, uint32_t base = 0)
 {
-    constexpr int CPR = D / 4;  // 16-byte chunks per row
-    return chunk ^ (row & (CPR - 1) & 31);
+    return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(off), static_cast<int>(base), 0));
 }
 
 template <int D, bool HAS_RAB, bool HAS_MASK>
-__global__ __launch_bounds__(256, 1) void hstu_fwd_f32_kernel(const FwdArgs a)
+__global__ __launch_bounds__(f32_waves(D) * 64) void hstu_fwd_f32_kernel(const FwdArgs a)
 {
-    constexpr int kThreads = 256;
-    constexpr int BN = 32;                       // keys per LDS tile = one 32-key sub-tile
-    constexpr int CPR = D / 4;                   // 16-byte chunks per row
-    constexpr int TILE_FLOATS = BN * D;
-    constexpr int LOADS = TILE_FLOATS / 256 / 4;  // 1 KiB load instructions per wavefront per tile
-    static_assert(TILE_FLOATS % 1024 == 0, "tile must split evenly over four wavefronts");
-    constexpr int QCHUNKS = D / 8;               // float4 chunks of Q held per lane
-    constexpr int MTILES = D / 32;
+    constexpr int W = f32_waves(D);
+    constexpr int KCH = D / 16;                 // 16-byte pieces of a Q or K row per lane
+    constexpr int H = D >= 64 ? D / 64 : 1;     // spans of 64 output dims
+    constexpr int T = D >= 64 ? 4 : D / 16;     // tiles per span; a lane's V piece holds one element of each
+    constexpr bool kTurns = D <= 64 && !(D == 64 && (HAS_RAB || HAS_MASK));  // registers for two blocks side by side
+    static_assert(D == 32 || D % 64 == 0, "head-dim slots 32, 64, 128, 256");
 
-    __shared__ __attribute__((aligned(1024))) float s_k[TILE_FLOATS];
-    __shared__ __attribute__((aligned(1024))) float s_v[TILE_FLOATS];
+    __shared__ __attribute__((aligned(16))) float s_part[W * H * T * 4 * 64];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = uniform(tid >> 6);
-    const int ln = lane & 31;
-    const int lh = lane >> 5;
+    const int i = lane & 15;
+    const int g = lane >> 4;
+    const int splits = a.f32_splits;
+    const int group = wave / splits;
+    const int share = wave - group * splits;
+    const int rows_per_wg = 16 * (W / splits);
 
-    const int lvl = blockIdx.x / a.bh;
-    const int bhid = blockIdx.x - lvl * a.bh;
-    const int qt = a.n_qtiles - 1 - lvl;
+    // slots: tile levels from the last (longest key ranges) down, pairs padded to a multiple of 8 so that the tiles of a
+    // pair run on one XCD
+    const int bh_pad = (a.bh + 7) & ~7;
+    const int lvl = blockIdx.x / bh_pad;
+    const int bhid = blockIdx.x - lvl * bh_pad;
+    if (bhid >= a.bh) {
+        return;
+    }
+    const int qt = (a.max_q + rows_per_wg - 1) / rows_per_wg - 1 - lvl;
     const int b = bhid / a.n_heads_q;
     const int h = bhid - b * a.n_heads_q;
     const int hk = h / a.head_ratio;
@@ -54,6 +68,8 @@ __global__ __launch_bounds__(256, 1) void hstu_fwd_f32_kernel(const FwdArgs a)
     int64_t q1 = load_index(a.offs_q, b + 1, a.idx64);
     int64_t k0 = load_index(a.offs_k, b, a.idx64);
     int64_t k1 = load_index(a.offs_k, b + 1, a.idx64);
+    int n_ctx = (a.mask_type == 0 && a.num_ctx) ? static_cast<int>(load_index(a.num_ctx, b, a.idx64)) : 0;
+    int n_tgt = (a.mask_type == 0 && a.num_tgt) ? static_cast<int>(load_index(a.num_tgt, b, a.idx64)) : 0;
     q1 = q1 < a.total_q ? q1 : a.total_q;
     k1 = k1 < a.total_k ? k1 : a.total_k;
     q0 = q0 < 0 ? 0 : q0;
@@ -70,70 +86,37 @@ __global__ __launch_bounds__(256, 1) void hstu_fwd_f32_kernel(const FwdArgs a)
         const int64_t row_elems = static_cast<int64_t>(a.n_heads_q) * a.d_v;
         const int64_t n_tail = (a.total_q > first_tail ? a.total_q - first_tail : 0) * row_elems;
         float* tail = out32 + first_tail * row_elems;
-        for (int64_t e = static_cast<int64_t>(bhid) * kThreads + tid; e < n_tail;
-             e += static_cast<int64_t>(a.bh) * kThreads) {
+        for (int64_t e = static_cast<int64_t>(bhid) * (W * 64) + tid; e < n_tail; e += static_cast<int64_t>(a.bh) * (W * 64)) {
             tail[e] = 0.f;
         }
     }
-
-    const int r0 = qt * kBlockM;
-    if (r0 >= sq) {
+    if (qt * rows_per_wg >= sq) {
         return;
     }
-    const int wr0 = r0 + wave * kWaveM;
+    const int wr0 = qt * rows_per_wg + group * 16;
     const bool wave_active = wr0 < sq;
-
-    int n_ctx = 0;
-    int n_tgt = 0;
-    if (a.mask_type == 0) {
-        if (a.num_ctx) {
-            n_ctx = static_cast<int>(load_index(a.num_ctx, b, a.idx64));
-        }
-        if (a.num_tgt) {
-            n_tgt = static_cast<int>(load_index(a.num_tgt, b, a.idx64));
-        }
-        n_ctx = uniform(n_ctx < 0 ? 0 : n_ctx);
-        n_tgt = uniform(n_tgt < 0 ? 0 : (n_tgt > sk ? sk : n_tgt));
-    }
-    const int delta = sk - sq;
+    n_ctx = uniform(n_ctx < 0 ? 0 : n_ctx);
+    n_tgt = uniform(n_tgt < 0 ? 0 : (n_tgt > sk ? sk : n_tgt));
     const int hist_k = sk - n_tgt;
 
-    // per-row visibility: visible(j) = j < lim && !(hole_lo <= j < hole_hi)
-    int row = wr0 + ln;
+    // visibility of the lane's row: visible(j) = j < lim && !(hist_k <= j < hole_hi)
+    int row = wr0 + i;
     row = row < sq - 1 ? row : sq - 1;
-    int lim;
-    int hole_lo = 0;
+    int lim = sk;
     int hole_hi = 0;
     if (a.mask_type == 0) {
-        lim = row + delta + 1;
+        lim = row + (sk - sq) + 1;
         if (row < n_ctx) {
             lim = lim > hist_k ? lim : hist_k;
         }
         lim = lim < 0 ? 0 : (lim > sk ? sk : lim);
-        if (n_tgt > 0 && a.target_group > 0) {
-            const int ti = row - (sq - n_tgt);
-            if (ti >= 0) {
-                hole_lo = hist_k;
-                hole_hi = hist_k + (ti / a.target_group) * a.target_group;
-            }
+        const int ti = row - (sq - n_tgt);
+        if (n_tgt > 0 && a.target_group > 0 && ti >= 0) {
+            hole_hi = hist_k + (ti / a.target_group) * a.target_group;
         }
-    } else {
-        lim = sk;
     }
-    const WaveBounds wb = wave_bounds(a.mask_type, wr0, sq, sk, n_ctx, n_tgt, a.target_group, wave_active);
-
-    int kmax;
-    if (a.mask_type == 0) {
-        const int r1 = (r0 + kBlockM < sq) ? r0 + kBlockM : sq;
-        kmax = r1 + delta;
-        if (r0 < n_ctx) {
-            kmax = kmax > hist_k ? kmax : hist_k;
-        }
-        kmax = kmax < 0 ? 0 : (kmax > sk ? sk : kmax);
-    } else {
-        kmax = sk;
-    }
-    const int n_kt = uniform((kmax + BN - 1) / BN);
+    const WaveBounds wb = wave_bounds(a.mask_type, wr0, sq, sk, n_ctx, n_tgt, a.target_group, wave_active, 16);
+    const int n_blocks = uniform((wb.lim_max + 15) / 16);
 
     const uint32_t q_stride = static_cast<uint32_t>(a.n_heads_q) * a.d_qk * 4u;
     const uint32_t k_stride = static_cast<uint32_t>(a.n_heads_k) * a.d_qk * 4u;
@@ -150,172 +133,221 @@ __global__ __launch_bounds__(256, 1) void hstu_fwd_f32_kernel(const FwdArgs a)
                   sk > 0 ? static_cast<uint32_t>(sk - 1) * v_stride + a.d_v * 4u : 0u);
     const __amdgpu_buffer_rsrc_t o_rsrc = make_rsrc(out32 + (q0 * a.n_heads_q + h) * static_cast<int64_t>(a.d_v),
                                                     static_cast<uint32_t>(sq - 1) * o_stride + a.d_v * 4u);
-
-    // Q fragment: MFMA step 4*j + e of the QK product contracts head-dim element 4*(2j + lh) + e, so a
-    // lane holds the float4 chunks 2j + lh of its row (the contraction order is free, K follows it)
-    typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-    f32x4_t qf[QCHUNKS];
-    {
-        const uint32_t row_off = static_cast<uint32_t>(wr0 + ln) * q_stride;
-#pragma unroll
-        for (int j = 0; j < QCHUNKS; ++j) {
-            const int d0 = 4 * (2 * j + lh);
-            const uint32_t off = (d0 < a.d_qk) ? row_off + d0 * 4u : kOutOfRange;
-            qf[j] = __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, static_cast<int>(off), 0, 0));
-        }
-    }
-
-    uint32_t k_src[LOADS];
-    uint32_t v_src[LOADS];
-#pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int slot = (wave * LOADS + i) * 64 + lane;
-        const int r = slot / CPR;
-        const int pc = slot - r * CPR;
-        const int c = f32_chunk_swizzle<D>(r, pc);
-        k_src[i] = (c * 4 < a.d_qk) ? static_cast<uint32_t>(r) * k_stride + c * 16u : kOutOfRange;
-        v_src[i] = (c * 4 < a.d_v) ? static_cast<uint32_t>(r) * v_stride + c * 16u : kOutOfRange;
-    }
-
     const uint32_t bias_bytes = static_cast<uint32_t>(a.max_q) * static_cast<uint32_t>(a.max_k) * 4u;
     const int64_t bias_plane = (static_cast<int64_t>(b) * a.n_heads_q + h) * a.max_q * static_cast<int64_t>(a.max_k);
     const __amdgpu_buffer_rsrc_t rab_rsrc =
         make_rsrc(HAS_RAB ? static_cast<const float*>(a.rab) + bias_plane : nullptr, HAS_RAB ? bias_bytes : 0u);
     const __amdgpu_buffer_rsrc_t mask_rsrc =
         make_rsrc(HAS_MASK ? static_cast<const float*>(a.mask) + bias_plane : nullptr, HAS_MASK ? bias_bytes : 0u);
-    const uint32_t bias_row_off = static_cast<uint32_t>(wr0 + ln) * static_cast<uint32_t>(a.max_k) * 4u;
-    const bool bias_vec = a.bias_vec_ok != 0;
-    auto load_bias = [&](__amdgpu_buffer_rsrc_t rsrc, int c0, f32x16_t& w) {
+    const uint32_t bias_row_off = static_cast<uint32_t>(wr0 + i) * static_cast<uint32_t>(a.max_k) * 4u;
+
+    uint32_t k_off[KCH];  // of the lane's pieces of key i of a block
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t off = bias_row_off + static_cast<uint32_t>(c0 + 8 * g + 4 * lh) * 4u;
-            if (bias_vec) {
-                // (the result is reinterpreted as a float vector before its elements are taken: taking
-                // integer elements straight from this builtin's result is narrowed to a one-element load
-                // by the optimiser of this toolchain)
-                const f32x4_t t = __builtin_bit_cast(
-                    f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, static_cast<int>(off), 0, 0));
+    for (int j = 0; j < KCH; ++j) {
+        const int d0 = 16 * j + 4 * g;
+        k_off[j] = d0 < a.d_qk ? static_cast<uint32_t>(i) * k_stride + d0 * 4u : kOutOfRange;
+    }
+    // of the lane's pieces of keys 4 g + r of a block (one offset and three additions where registers are short)
+    constexpr int VR = kTurns ? 4 : 1;
+    uint32_t v_off[H][VR];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    w[4 * g + e] = t[e];
-                }
-            } else {
-                // the offset is laundered through an empty asm so that the optimiser cannot relate these
-                // element loads to the vector load of the other branch (it otherwise folds the two and
-                // replicates the first element)
-                uint32_t eoff = off;
-                asm volatile("" : "+v"(eoff));
+    for (int s = 0; s < H; ++s) {
+        const int d0 = 64 * s + T * i;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    w[4 * g + e] = __builtin_bit_cast(
-                        float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, static_cast<int>(eoff + 4u * e), 0, 0));
+        for (int r = 0; r < VR; ++r) {
+            v_off[s][r] = d0 < a.d_v ? static_cast<uint32_t>(4 * g + r) * v_stride + d0 * 4u : kOutOfRange;
+        }
+    }
+
+    struct Block {
+        f32x4_t k[KCH];
+        f32x4_t v[H][4];
+        f32x4_t rab;
+        f32x4_t mask;
+    };
+    // four values of a [max_q][max_k] row at keys c0 + 4 g ..; rows that are not 16-byte aligned element by element
+    auto load_plane = [&](__amdgpu_buffer_rsrc_t rsrc, int c0) {
+        const uint32_t off = bias_row_off + static_cast<uint32_t>(c0 + 4 * g) * 4u;
+        if (a.bias_vec_ok != 0) {
+            return buffer_f32x4(rsrc, off);
+        }
+        // (laundered so that the optimiser does not fold these loads with the vector load of the other branch)
+        uint32_t eoff = off;
+        asm volatile("" : "+v"(eoff));
+        f32x4_t w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, static_cast<int>(eoff + 4u * e), 0, 0));
+            w[e] = x;
+        }
+        return w;
+    };
+    // (a block past the last, which is asked for and never used, is the last one again: the bases stay inside the sequence)
+    auto load_block = [&](int block, Block& x) {
+        const int c0 = uniform((block < n_blocks ? block : n_blocks - 1) * 16);
+        const uint32_t kb = static_cast<uint32_t>(c0) * k_stride;
+        const uint32_t vb = static_cast<uint32_t>(c0) * v_stride;
+#pragma unroll
+        for (int j = 0; j < KCH; ++j) {
+            x.k[j] = buffer_f32x4(k_rsrc, k_off[j], kb);
+        }
+        if constexpr (HAS_RAB) {
+            x.rab = load_plane(rab_rsrc, c0);
+        }
+        if constexpr (HAS_MASK) {
+            x.mask = load_plane(mask_rsrc, c0);
+        }
+#pragma unroll
+        for (int s = 0; s < H; ++s) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t off = VR == 4 ? v_off[s][r % VR] : v_off[s][0] + static_cast<uint32_t>(r) * v_stride;
+                if constexpr (T == 4) {
+                    x.v[s][r] = buffer_f32x4(v_rsrc, off, vb);
+                } else {
+                    typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+                    const f32x2_t w = __builtin_bit_cast(f32x2_t, __builtin_amdgcn_raw_buffer_load_b64(v_rsrc, static_cast<int>(off), static_cast<int>(vb), 0));
+                    x.v[s][r] = f32x4_t{w[0], w[1], 0.f, 0.f};
                 }
             }
         }
     };
 
-    f32x16_t o_acc[MTILES];
+    f32x4_t acc[H][T];
 #pragma unroll
-    for (int mt = 0; mt < MTILES; ++mt) {
+    for (int s = 0; s < H; ++s) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            o_acc[mt][i] = 0.f;
+        for (int t = 0; t < T; ++t) {
+            acc[s][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
     }
-    const float c_exp = a.c_exp;
-
-    for (int kt = 0; kt < n_kt; ++kt) {
-        const uint32_t kb = static_cast<uint32_t>(kt * BN) * k_stride;
-        const uint32_t vb = static_cast<uint32_t>(kt * BN) * v_stride;
+    if (share < n_blocks) {
+        f32x4_t qf[KCH];
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(k_rsrc, (__attribute__((address_space(3))) void*)(s_k + (wave * LOADS + i) * 256),
-                                                     16, static_cast<int>(k_src[i] + kb), 0, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (__attribute__((address_space(3))) void*)(s_v + (wave * LOADS + i) * 256),
-                                                     16, static_cast<int>(v_src[i] + vb), 0, 0, 0);
+        for (int j = 0; j < KCH; ++j) {
+            const int d0 = 16 * j + 4 * g;
+            qf[j] = buffer_f32x4(q_rsrc, d0 < a.d_qk ? static_cast<uint32_t>(wr0 + i) * q_stride + d0 * 4u : kOutOfRange);
         }
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-
-        const int c0 = kt * BN;
-        if (c0 < wb.lim_max) {
-            f32x16_t s;
-            if constexpr (HAS_RAB) {
-                load_bias(rab_rsrc, c0, s);
-            } else {
+        const float c_exp = a.c_exp;
+        auto products = [&](int block, const Block& cur) {
+            const int c0 = block * 16;
+            f32x4_t s = HAS_RAB ? cur.rab : f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[i] = 0.f;
-                }
-            }
-            f32x16_t mw;
-            if constexpr (HAS_MASK) {
-                load_bias(mask_rsrc, c0, mw);
-            }
-            // S^T = K . Q^T
-#pragma unroll
-            for (int j = 0; j < QCHUNKS; ++j) {
-                const f32x4_t kc =
-                    *reinterpret_cast<const f32x4_t*>(s_k + ln * D + f32_chunk_swizzle<D>(ln, 2 * j + lh) * 4);
+            for (int j = 0; j < KCH; ++j) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kc[e], qf[j][e], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.k[j][e], qf[j][e], s, 0, 0, 0);
                 }
             }
             // P^T = S^T * sigmoid(alpha * S^T), masked
-            const bool full = !HAS_MASK && (c0 + 32 <= wb.lim_min) &&
-                              !(wb.any_hole && c0 + 32 > hist_k && c0 < wb.hole_hi_max);
+            // (the conditions are combined without branches: where a branch stands between the last MFMA and the first read of its
+            // result, this compiler counts the instructions of the longer way round as wait states, and the read came too early)
+            const bool hole = wb.any_hole & (c0 + 16 > hist_k) & (c0 < wb.hole_hi_max);
+            const bool full = !HAS_MASK & (c0 + 16 <= wb.lim_min) & !hole;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const float sv = s[i];
-                const float ex = __builtin_amdgcn_exp2f(sv * c_exp);
-                s[i] = sv * __builtin_amdgcn_rcpf(1.0f + ex);
+            for (int r = 0; r < 4; ++r) {
+                s[r] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s[r] * c_exp));
             }
             if (!full) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const int jj = c0 + 8 * (i / 4) + 4 * lh + (i % 4);
-                    const bool vis = (jj < lim) && !(jj >= hole_lo && jj < hole_hi);
-                    float p = s[i];
-                    if constexpr (HAS_MASK) {
-                        p *= mw[i];
-                    }
-                    s[i] = vis ? p : 0.f;
+                for (int r = 0; r < 4; ++r) {
+                    const int key = c0 + 4 * g + r;
+                    const bool visible = key < lim && !(key >= hist_k && key < hole_hi);
+                    const float p = HAS_MASK ? s[r] * cur.mask[r] : s[r];
+                    s[r] = visible ? p : 0.f;
                 }
             }
-            // O^T += V^T . P^T : step i contracts the key pair {8 (i/4) + i % 4, same + 4}, one per lane half
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int vr = 8 * (i / 4) + 4 * lh + (i % 4);
+            for (int r = 0; r < 4; ++r) {
 #pragma unroll
-                for (int mt = 0; mt < MTILES; ++mt) {
-                    const int col = 32 * mt + ln;
-                    const float va = s_v[vr * D + f32_chunk_swizzle<D>(vr, col >> 2) * 4 + (col & 3)];
-                    o_acc[mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, s[i], o_acc[mt], 0, 0, 0);
+                for (int sp = 0; sp < H; ++sp) {
+#pragma unroll
+                    for (int t = 0; t < T; ++t) {
+                        acc[sp][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[sp][r][t], s[r], acc[sp][t], 0, 0, 0);
+                    }
                 }
+            }
+        };
+        // two blocks in turn, each asked for while the products of the other run (with wide heads through copies, which
+        // the compiler keeps without spilling)
+        Block even;
+        Block odd;
+        load_block(share, even);
+        if constexpr (kTurns) {
+            for (int block = share; block < n_blocks; block += 2 * splits) {
+                load_block(block + splits, odd);
+                products(block, even);
+                if (block + splits >= n_blocks) {
+                    break;
+                }
+                load_block(block + 2 * splits, even);
+                products(block + splits, odd);
+            }
+        } else {
+            for (int block = share; block < n_blocks; block += splits) {
+                load_block(block + splits, odd);
+                products(block, even);
+                even = odd;
             }
         }
-        __syncthreads();
     }
 
-    // store O: lane holds query row (wr0 + ln), dims 32 mt + 8 g + 4 lh + 0..3
-    {
-        const float c_out = a.c_out;
-        const uint32_t row_off = static_cast<uint32_t>(wr0 + ln) * o_stride;
+    // a lane's accumulators are dims 64 sp + T (4 g + r) + t of row wr0 + i: units (sp, r) of T values each
+    const float c_out = a.c_out;
+    const uint32_t row_off = static_cast<uint32_t>(wr0 + i) * o_stride;
+    auto store_unit = [&](int sp, int r, const float* value) {
+        const int d0 = 64 * sp + T * (4 * g + r);
+        const uint32_t off = (wave_active && d0 < a.d_v) ? row_off + d0 * 4u : kOutOfRange;
+        if constexpr (T == 4) {
+            const f32x4_t w = {value[0] * c_out, value[1] * c_out, value[2] * c_out, value[3] * c_out};
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, w), o_rsrc, static_cast<int>(off), 0, 0);
+        } else {
+            typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+            const f32x2_t w = {value[0] * c_out, value[1] * c_out};
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2_t, w), o_rsrc, static_cast<int>(off), 0, 0);
+        }
+    };
+    if (splits == 1) {
 #pragma unroll
-        for (int mt = 0; mt < MTILES; ++mt) {
+        for (int sp = 0; sp < H; ++sp) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d0 = 32 * mt + 8 * g + 4 * lh;
-                const uint32_t off = (d0 < a.d_v) ? row_off + d0 * 4u : kOutOfRange;
-                u32x4_t w;
+            for (int r = 0; r < 4; ++r) {
+                float value[T];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    w[e] = __builtin_bit_cast(uint32_t, o_acc[mt][4 * g + e] * c_out);
+                for (int t = 0; t < T; ++t) {
+                    value[t] = acc[sp][t][r];
                 }
-                __builtin_amdgcn_raw_buffer_store_b128(w, o_rsrc, static_cast<int>(off), 0, 0);
+                store_unit(sp, r, value);
             }
         }
+        return;
+    }
+    float* const mine = s_part + wave * (H * T * 4 * 64);
+#pragma unroll
+    for (int sp = 0; sp < H; ++sp) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                mine[((sp * 4 + r) * T + t) * 64 + lane] = acc[sp][t][r];
+            }
+        }
+    }
+    __syncthreads();
+    const float* const parts = s_part + (wave - share) * (H * T * 4 * 64);
+    for (int u = share; u < H * 4; u += splits) {
+        float value[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            value[t] = parts[(u * T + t) * 64 + lane];
+        }
+        for (int p = 1; p < splits; ++p) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                value[t] += parts[p * (H * T * 4 * 64) + (u * T + t) * 64 + lane];
+            }
+        }
+        store_unit(u / 4, u % 4, value);
     }
 }
 

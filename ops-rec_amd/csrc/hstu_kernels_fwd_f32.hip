@@ -10,7 +10,7 @@
 
 #define HSTU_F32_VARIANT(D, RAB, MASK)                                                                              \
     {"hstu_fwd_f32_d" #D "_rab" #RAB "_mask" #MASK, nullptr, nullptr, hstu::hstu_fwd_f32_kernel<D, RAB, MASK>, nullptr, \
-     nullptr, nullptr, D, 256, 0}
+     nullptr, nullptr, D, hstu::f32_waves(D) * 64, 0}
 #define HSTU_F32_DIMS(RAB, MASK) \
     {HSTU_F32_VARIANT(32, RAB, MASK), HSTU_F32_VARIANT(64, RAB, MASK), HSTU_F32_VARIANT(128, RAB, MASK), \
      HSTU_F32_VARIANT(256, RAB, MASK)}

@@ -473,6 +473,26 @@ uint64_t forward_workspace_bytes(const Variant* var, const hstu_jagged_fwd_param
     return split_workspace_bytes(var, p);
 }
 
+// fp32 inputs: how many wavefronts share the keys of one 16-row group (hstu_fwd_f32_kernel.hip.h).  As many as it takes to put
+// two wavefronts on every SIMD, at most those of a workgroup and one 16-key block each; and on long key ranges (512 keys a
+// share) more, so that the workgroups, which then own fewer rows, are many enough to even out the causal ranges -- up to
+// slots 64 until there are eight of them per CU, above (two wavefronts per SIMD as it is) two.  Measured against the kernel of
+// 128-row tiles before: 4 x 2 heads, d 64, 16..128 rows 15.6 -> 5 us (kernel time), 3 x 8 heads, d 64, 1662..1971 rows 180 -> 105 us
+// (167 without the second clause), 1 x 8, d 128, 4065 rows 603 -> 336, 2 x 4, d 32, 8113 rows 450 -> 356 (492 without), 48 x 2,
+// d 128, 1196..1350 rows 500 -> 415, 16 x 4, d 256, 170..1023 rows 368 -> 242.
+int f32_splits(const Variant* var, const hstu_jagged_fwd_params* p, int cus)
+{
+    const int64_t groups = (p->n_offsets - 1) * p->num_heads_q * ((p->max_seq_len_q + 15) / 16);
+    const int64_t fill = 8 * static_cast<int64_t>(cus);
+    const int64_t even_out = (var->d_pad <= 64 ? 64 : 16) * static_cast<int64_t>(cus);
+    int splits = 1;
+    while (switches().split != 0 && splits < hstu::f32_waves(var->d_pad) && splits * 16 < p->max_seq_len_k &&
+           (groups * splits < fill || (groups * splits < even_out && splits * 512 <= p->max_seq_len_k))) {
+        splits *= 2;
+    }
+    return splits;
+}
+
 bool usable_workspace(const void* workspace, uint64_t bytes, uint64_t need)
 {
     return workspace != nullptr && bytes >= need && reinterpret_cast<uintptr_t>(workspace) % 16 == 0;
@@ -1526,6 +1546,20 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         }
         if (a.counters != nullptr) {
             launch_clear(a.counters, static_cast<int64_t>(kCounterBytes), stream);
+        }
+    }
+    const Variant* const f32 = &hstu::fwd_variants_f32()[0][0][0];
+    if (var >= f32 && var < f32 + 16) {
+        int cus = 0;
+        const int rc_cu = compute_units(&cus);
+        if (rc_cu != HSTU_OK) {
+            return rc_cu;
+        }
+        a.f32_splits = f32_splits(var, p, cus);
+        const int64_t rows = 16 * (hstu::f32_waves(var->d_pad) / a.f32_splits);
+        n_blocks = (a.max_q + rows - 1) / rows * ((a.bh + 7) & ~7);
+        if (n_blocks > 0x7fffffffLL) {
+            return fail(HSTU_ERR_INVALID, "grid of %lld workgroups is out of range", (long long)n_blocks);
         }
     }
     // (the kernel for head dims above 256 takes a workgroup per window of 256 output dims)
