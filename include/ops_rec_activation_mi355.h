@@ -89,8 +89,8 @@ HSTU_API const char* in_linear_silu_fwd_kernel_name(const in_linear_silu_params*
  * aclnnInLinearSiluBackward, ascendc/activation/in_linear_silu/in_linear_silu_backward/docs/aclnn_in_linear_silu_backward.md;
  * its adapter: torch_extension/in_linear_silu_backward_plugin.cpp:112-153):
  *   d_mixed = cat(user_grad, value_grad, query_grad, key_grad) * silu'(linear_output),  bias_grad = column sums.
- * The two products that follow (d x = d_mixed @ weight, d weight = d_mixed^T @ x) are plain matrix products and are left
- * to the caller's BLAS.
+ * Of the two products that follow, d x = d_mixed @ weight is a plain matrix product left to the caller's BLAS; for
+ * d weight = d_mixed^T @ x see in_linear_silu_bwd_weight below.
  */
 typedef struct in_linear_silu_bwd_params {
     uint32_t struct_size; /* sizeof(in_linear_silu_bwd_params), checked */
@@ -116,6 +116,26 @@ HSTU_API int in_linear_silu_bwd_dmixed_workspace_size(const in_linear_silu_bwd_p
 /* Launches on `stream` and returns without waiting.  HSTU_OK, or HSTU_ERR_NULLPTR / HSTU_ERR_INVALID /
  * HSTU_ERR_WORKSPACE (nothing launched) / HSTU_ERR_RUNTIME. */
 HSTU_API int in_linear_silu_bwd_dmixed(const in_linear_silu_bwd_params* params, void* workspace, uint64_t workspace_bytes,
+                                       void* stream);
+
+/*
+ * The whole backward but d x: the stage above together with d weight = d_mixed^T @ x, whose contraction over the m rows is cut
+ * into chunks that run side by side (partial outputs in the workspace, added in a fixed order).
+ */
+typedef struct in_linear_silu_bwd_weight_params {
+    uint32_t struct_size; /* sizeof(in_linear_silu_bwd_weight_params), checked */
+    uint32_t reserved0;
+    in_linear_silu_bwd_params stage; /* as above (stage.struct_size is checked too) */
+    const void* x;                   /* [m, k], type of linear_output, 16-byte aligned */
+    void* weight_grad;               /* [n, k], same type; every element is written */
+    int64_t k;                       /* a multiple of 16 in [16, 8192] */
+} in_linear_silu_bwd_weight_params;
+
+/* bytes of device scratch in_linear_silu_bwd_weight needs (one fp32 partial output per chunk of rows; never 0) */
+HSTU_API int in_linear_silu_bwd_weight_workspace_size(const in_linear_silu_bwd_weight_params* params, uint64_t* workspace_bytes);
+
+/* Launches on `stream` and returns without waiting; codes as above. */
+HSTU_API int in_linear_silu_bwd_weight(const in_linear_silu_bwd_weight_params* params, void* workspace, uint64_t workspace_bytes,
                                        void* stream);
 
 #ifdef __cplusplus

@@ -212,4 +212,25 @@ struct InLinearSiluBwdArgs {
     int split_end[3];
 };
 
+// in_linear_silu's backward with the weight gradient (in_linear_silu_wgrad_kernel.hip.h)
+struct InLinearSiluWgradArgs {
+    const void* linear_output;  // [m, n], 16-bit
+    const void* user_grad;      // [m, split_end[0]]
+    const void* value_grad;     // [m, split_end[1] - split_end[0]]
+    const void* query_grad;     // [m, split_end[2] - split_end[1]]
+    const void* key_grad;       // [m, n - split_end[2]]
+    const void* x;              // [m, k]
+    void* d_mixed;              // [m, n]
+    void* weight_grad;          // [n, k]
+    float* bias_grad;           // [n], or nullptr
+    float* partial;             // [chunks, n, k]
+    float* partial_sums;        // [chunks, n], or nullptr when no bias gradient is wanted
+    int64_t m;
+    int64_t chunk_rows;  // rows per chunk, a multiple of the step
+    int chunks;
+    int n;
+    int k;
+    int split_end[3];
+};
+
 }  // namespace hstu

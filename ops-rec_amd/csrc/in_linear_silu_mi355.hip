@@ -8,6 +8,7 @@
 #include "hstu_error.h"
 #include "in_linear_silu_bwd_kernel.hip.h"
 #include "in_linear_silu_kernel.hip.h"
+#include "in_linear_silu_wgrad_kernel.hip.h"
 
 namespace {
 
@@ -172,9 +173,149 @@ uint64_t bwd_workspace_bytes(const in_linear_silu_bwd_params* p)
     return p->bias_grad == nullptr ? 0 : static_cast<uint64_t>(bwd_row_blocks(p)) * static_cast<uint64_t>(p->n) * sizeof(float);
 }
 
+int validate_weight(const in_linear_silu_bwd_weight_params* p)
+{
+    if (p == nullptr) {
+        return hstu::set_error(HSTU_ERR_NULLPTR, "params is NULL");
+    }
+    if (p->struct_size != sizeof(in_linear_silu_bwd_weight_params)) {
+        return hstu::set_error(HSTU_ERR_INVALID, "struct_size %u does not match this library (%zu)", p->struct_size,
+                               sizeof(in_linear_silu_bwd_weight_params));
+    }
+    const int rc = validate_bwd(&p->stage);
+    if (rc != HSTU_OK) {
+        return rc;
+    }
+    if (p->x == nullptr || p->weight_grad == nullptr) {
+        return hstu::set_error(HSTU_ERR_NULLPTR, "x and weight_grad must be given");
+    }
+    if (p->k < kMinDim || p->k > kMaxDim || p->k % kMinDim != 0) {
+        return hstu::set_error(HSTU_ERR_INVALID, "x dim[1] must in range[16, 8192] and multiples of 16.");
+    }
+    if (!aligned16(p->x) || !aligned16(p->weight_grad) || !aligned16(p->stage.bias_grad)) {
+        return hstu::set_error(HSTU_ERR_INVALID, "every tensor must start at a multiple of 16 bytes");
+    }
+    return HSTU_OK;
+}
+
+// How the weight gradient is cut: tiles of 128 x tile_k (the narrowest of the three widths that spans k, 512 above), and the
+// number of chunks of rows, each of eight 32-row steps at least, that an estimate of the time puts first -- rounds of
+// workgroups over the CUs (two of the narrowest tile each, one of the others) times a chunk's steps, and the partial outputs, which
+// are written and read back once.  Chunks beyond eight come in whole groups of 8, one per XCD.  Measured, element-wise stage +
+// column sums + library product -> the two kernels: m 20480, n 2048, k 512 187 -> 92 us (340 MB of operands, d_mixed and partial
+// outputs: 3.7 TB/s); m 95697, n 512, k 128 338 -> 76 us.
+struct WeightPlan {
+    int tile_k;
+    int tiles;
+    int chunks;
+    int64_t chunk_rows;
+};
+WeightPlan plan_weight(const in_linear_silu_bwd_weight_params* p)
+{
+    WeightPlan w;
+    w.tile_k = p->k <= 128 ? 128 : (p->k <= 256 ? 256 : 512);
+    w.tiles = static_cast<int>((p->stage.n + hstu::kWgradCols - 1) / hstu::kWgradCols * ((p->k + w.tile_k - 1) / w.tile_k));
+    constexpr int kCus = 256;
+    const int64_t slots = w.tile_k == 128 ? 2 * kCus : kCus;  // resident workgroups
+    const int64_t steps = (p->stage.m + hstu::kWgradRows - 1) / hstu::kWgradRows;
+    // (a chunk stays behind 32-bit descriptors)
+    const int64_t widest = p->stage.n > p->k ? p->stage.n : p->k;
+    const int64_t least = (steps * hstu::kWgradRows * widest * 2) / (int64_t{1} << 30) + 1;
+    const int64_t most = steps / 8 < 64 ? steps / 8 : 64;
+    const double step_us = w.tile_k == 512 ? 1.2 : 0.8;  // (measured where the machine is full of workgroups: 1.0 .. 1.9, bytes included)
+    const double partial_us = static_cast<double>(p->stage.n) * static_cast<double>(p->k) * 8.0 / 6e6;  // written and read back once
+    int64_t chunks = least;
+    double best = 0.0;
+    for (int64_t c = least; c <= most || c == least; ++c) {
+        if (c > 8 && c % 8 != 0) {
+            continue;
+        }
+        const double rounds = static_cast<double>((w.tiles * c + slots - 1) / slots);
+        const double cost = rounds * (static_cast<double>((steps + c - 1) / c) * step_us + 3.0) + static_cast<double>(c) * partial_us;
+        if (c == least || cost < best) {
+            best = cost;
+            chunks = c;
+        }
+    }
+    w.chunk_rows = (steps + chunks - 1) / chunks * hstu::kWgradRows;
+    w.chunks = static_cast<int>(chunks);
+    return w;
+}
+
+uint64_t weight_workspace_bytes(const in_linear_silu_bwd_weight_params* p)
+{
+    const WeightPlan w = plan_weight(p);
+    const uint64_t per_chunk = static_cast<uint64_t>(p->stage.n) * static_cast<uint64_t>(p->k + (p->stage.bias_grad != nullptr ? 1 : 0));
+    return static_cast<uint64_t>(w.chunks) * per_chunk * sizeof(float);
+}
+
 }  // namespace
 
 extern "C" {
+
+HSTU_API int in_linear_silu_bwd_weight_workspace_size(const in_linear_silu_bwd_weight_params* p, uint64_t* workspace_bytes)
+{
+    if (workspace_bytes == nullptr) {
+        return hstu::set_error(HSTU_ERR_NULLPTR, "workspace_bytes is NULL");
+    }
+    *workspace_bytes = 0;
+    const int rc = validate_weight(p);
+    if (rc != HSTU_OK) {
+        return rc;
+    }
+    *workspace_bytes = weight_workspace_bytes(p);
+    return HSTU_OK;
+}
+
+HSTU_API int in_linear_silu_bwd_weight(const in_linear_silu_bwd_weight_params* p, void* workspace, uint64_t workspace_bytes, void* stream)
+{
+    const int rc = validate_weight(p);
+    if (rc != HSTU_OK) {
+        return rc;
+    }
+    const uint64_t need = weight_workspace_bytes(p);
+    if (workspace == nullptr || workspace_bytes < need || !aligned16(workspace)) {
+        return hstu::set_error(HSTU_ERR_WORKSPACE, "workspace of %llu bytes (16-byte aligned) needed for the weight gradient, got %llu",
+                               static_cast<unsigned long long>(need), static_cast<unsigned long long>(workspace_bytes));
+    }
+    const WeightPlan w = plan_weight(p);
+    const in_linear_silu_bwd_params& s = p->stage;
+    hstu::InLinearSiluWgradArgs a;
+    a.linear_output = s.linear_output;
+    a.user_grad = s.user_grad;
+    a.value_grad = s.value_grad;
+    a.query_grad = s.query_grad;
+    a.key_grad = s.key_grad;
+    a.x = p->x;
+    a.d_mixed = s.d_mixed;
+    a.weight_grad = p->weight_grad;
+    a.bias_grad = s.bias_grad;
+    a.m = s.m;
+    a.n = static_cast<int>(s.n);
+    a.k = static_cast<int>(p->k);
+    a.chunks = w.chunks;
+    a.chunk_rows = w.chunk_rows;
+    a.partial = static_cast<float*>(workspace);
+    a.partial_sums = s.bias_grad != nullptr ? a.partial + static_cast<int64_t>(w.chunks) * a.n * a.k : nullptr;
+    a.split_end[0] = static_cast<int>(s.split[0]);
+    a.split_end[1] = a.split_end[0] + static_cast<int>(s.split[1]);
+    a.split_end[2] = a.split_end[1] + static_cast<int>(s.split[2]);
+    const bool bf16 = s.dtype == HSTU_DT_BF16;
+    void (*const kernel)(const hstu::InLinearSiluWgradArgs) =
+        w.tile_k == 128   ? (bf16 ? hstu::in_linear_silu_wgrad_kernel<hstu::bf16_tag, 128> : hstu::in_linear_silu_wgrad_kernel<hstu::f16_tag, 128>)
+        : w.tile_k == 256 ? (bf16 ? hstu::in_linear_silu_wgrad_kernel<hstu::bf16_tag, 256> : hstu::in_linear_silu_wgrad_kernel<hstu::f16_tag, 256>)
+                          : (bf16 ? hstu::in_linear_silu_wgrad_kernel<hstu::bf16_tag, 512> : hstu::in_linear_silu_wgrad_kernel<hstu::f16_tag, 512>);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(w.tiles * w.chunks)), dim3(hstu::kWgradThreads), 0, static_cast<hipStream_t>(stream), a);
+    const int64_t quads = (static_cast<int64_t>(a.n) * a.k + a.n) / 4;
+    const unsigned sum_grid = static_cast<unsigned>((quads + 255) / 256 < 8192 ? (quads + 255) / 256 : 8192);
+    hipLaunchKernelGGL(bf16 ? hstu::in_linear_silu_wgrad_sum_kernel<hstu::bf16_tag> : hstu::in_linear_silu_wgrad_sum_kernel<hstu::f16_tag>,
+                       dim3(sum_grid), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) {
+        return hstu::set_error(HSTU_ERR_RUNTIME, "launch of in_linear_silu_wgrad failed: %s", hipGetErrorString(err));
+    }
+    return HSTU_OK;
+}
 
 HSTU_API int in_linear_silu_bwd_dmixed_workspace_size(const in_linear_silu_bwd_params* p, uint64_t* workspace_bytes)
 {

@@ -464,37 +464,49 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
         const c10::DeviceGuard guard(x.device());
         const int64_t m = x.size(0), n = weight.size(0);
         const Tensor g[4] = {contiguous(user_grad), contiguous(value_grad), contiguous(query_grad), contiguous(key_grad)};
-        Tensor d_mixed = empty({m, n}, x.scalar_type(), x.device()), bias_grad;
+        Tensor d_mixed = empty({m, n}, x.scalar_type(), x.device()), weight_grad, bias_grad;
         if (is_set(bias)) {
             bias_grad = empty({n}, at::kFloat, x.device());
         }
-        in_linear_silu_bwd_params p;
+        // A weight of that size gives a library product a tile for every CU, and the rows enough work per tile: the element-wise
+        // stage in a kernel of its own and d_mixed^T @ x from the library (m = 9600, n = 8192, k = 2048: level at 12 M
+        // elements, 6144 x 1536, and 2 % ahead here).
+        const bool library = n * x.size(1) >= (int64_t{12} << 20) && m >= 4096;
+        if (!library) {
+            weight_grad = empty({n, x.size(1)}, x.scalar_type(), x.device());
+        }
+        in_linear_silu_bwd_weight_params p;
         std::memset(&p, 0, sizeof p);
         p.struct_size = sizeof p;
-        p.linear_output = linear_output.data_ptr();
-        p.user_grad = g[0].data_ptr();
-        p.value_grad = g[1].data_ptr();
-        p.query_grad = g[2].data_ptr();
-        p.key_grad = g[3].data_ptr();
-        p.d_mixed = d_mixed.data_ptr();
-        p.bias_grad = static_cast<decltype(p.bias_grad)>(ptr(bias_grad));
-        p.m = m;
-        p.n = n;
+        p.x = x.data_ptr();
+        p.weight_grad = ptr(weight_grad);
+        p.k = x.size(1);
+        in_linear_silu_bwd_params& s = p.stage;
+        s.struct_size = sizeof s;
+        s.linear_output = linear_output.data_ptr();
+        s.user_grad = g[0].data_ptr();
+        s.value_grad = g[1].data_ptr();
+        s.query_grad = g[2].data_ptr();
+        s.key_grad = g[3].data_ptr();
+        s.d_mixed = d_mixed.data_ptr();
+        s.bias_grad = static_cast<float*>(ptr(bias_grad));
+        s.m = m;
+        s.n = n;
         for (int i = 0; i < 4; ++i) {
-            p.split[i] = split[i];
+            s.split[i] = split[i];
         }
-        p.dtype = dtype_code(x.scalar_type());
+        s.dtype = dtype_code(x.scalar_type());
         uint64_t ws_bytes = 0;
-        int rc = in_linear_silu_bwd_dmixed_workspace_size(&p, &ws_bytes);
-        Tensor ws;
+        int rc = library ? in_linear_silu_bwd_dmixed_workspace_size(&s, &ws_bytes) : in_linear_silu_bwd_weight_workspace_size(&p, &ws_bytes);
         if (rc == HSTU_OK) {
-            if (ws_bytes != 0) {
-                ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, x.device());
-            }
-            rc = in_linear_silu_bwd_dmixed(&p, ptr(ws), ws_bytes, stream_of(x));
+            const Tensor ws = ws_bytes != 0 ? empty({static_cast<int64_t>(ws_bytes)}, at::kByte, x.device()) : Tensor();
+            rc = library ? in_linear_silu_bwd_dmixed(&s, ptr(ws), ws_bytes, stream_of(x)) : in_linear_silu_bwd_weight(&p, ptr(ws), ws_bytes, stream_of(x));
         }
         TORCH_CHECK(rc == HSTU_OK, "in_linear_silu_backward failed (", rc, "): ", hstu_last_error());
-        return {at::mm(d_mixed, weight), at::mm(d_mixed.t(), x), bias_grad, Tensor()};
+        if (library) {
+            weight_grad = at::mm(d_mixed.t(), x);
+        }
+        return {at::mm(d_mixed, weight), weight_grad, bias_grad, Tensor()};
     }
     py::gil_scoped_acquire gil;
     const auto r = in_python<std::tuple<Tensor, Tensor, OptTensor, OptTensor>>(fallbacks.in_linear_silu_backward, x, weight, bias, user_grad,

@@ -35,6 +35,8 @@ EXPORTED_SYMBOLS = (
     "in_linear_silu_fwd_kernel_name",
     "in_linear_silu_bwd_dmixed_workspace_size",
     "in_linear_silu_bwd_dmixed",
+    "in_linear_silu_bwd_weight_workspace_size",
+    "in_linear_silu_bwd_weight",
 )
 
 
@@ -174,6 +176,19 @@ class InLinearSiluBwdParams(ctypes.Structure):
     ]
 
 
+class InLinearSiluBwdWeightParams(ctypes.Structure):
+    """Mirror of ``in_linear_silu_bwd_weight_params`` (include/ops_rec_activation_mi355.h)."""
+
+    _fields_ = [
+        ("struct_size", ctypes.c_uint32),
+        ("reserved0", ctypes.c_uint32),
+        ("stage", InLinearSiluBwdParams),
+        ("x", ctypes.c_void_p),
+        ("weight_grad", ctypes.c_void_p),
+        ("k", ctypes.c_int64),
+    ]
+
+
 _lib: Optional[ctypes.CDLL] = None
 
 
@@ -239,6 +254,12 @@ def load() -> ctypes.CDLL:
                                                              ctypes.POINTER(ctypes.c_uint64)]  # fmt: skip
     lib.in_linear_silu_bwd_dmixed.restype = ctypes.c_int
     lib.in_linear_silu_bwd_dmixed.argtypes = [ctypes.POINTER(InLinearSiluBwdParams), ctypes.c_void_p, ctypes.c_uint64,
+                                              ctypes.c_void_p]  # fmt: skip
+    lib.in_linear_silu_bwd_weight_workspace_size.restype = ctypes.c_int
+    lib.in_linear_silu_bwd_weight_workspace_size.argtypes = [ctypes.POINTER(InLinearSiluBwdWeightParams),
+                                                             ctypes.POINTER(ctypes.c_uint64)]  # fmt: skip
+    lib.in_linear_silu_bwd_weight.restype = ctypes.c_int
+    lib.in_linear_silu_bwd_weight.argtypes = [ctypes.POINTER(InLinearSiluBwdWeightParams), ctypes.c_void_p, ctypes.c_uint64,
                                               ctypes.c_void_p]  # fmt: skip
     _lib = lib
     return lib
