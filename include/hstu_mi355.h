@@ -132,8 +132,8 @@ typedef struct hstu_jagged_fwd_params {
  * shorter than the machine (few, long sequences) cuts the key range of long items into parts that run on different
  * workgroups and adds their fp32 partial outputs, in a fixed order: 16 KiB of counters plus room for one partial
  * output per resident workgroup.  Lists in between run on a fixed schedule and need nothing.  The workspace is 16-byte
- * aligned; its contents are undefined before and after the call (the library clears the counters on the launch
- * stream ahead of its kernel) and it belongs to the call until the launch has completed: launches that overlap
+ * aligned; its contents are undefined before and after the call (the queues' counters are cleared on the launch
+ * stream ahead of the kernel, the others tell their launch by its number) and it belongs to the call until the launch has completed: launches that overlap
  * on a GPU -- several streams, captured graphs replayed side by side -- are independent of each other as long as
  * each has a workspace (and an output) of its own.  The library keeps no device state between calls.
  * A caller that passes less than asked for, or nothing, gets the same results from the fixed schedule.  Because a
@@ -153,7 +153,7 @@ HSTU_API int hstu_jagged_fwd(const hstu_jagged_fwd_params* params, void* workspa
  * workspace request exceeds that array (hstu_jagged_fwd_noalloc_max_workspace) is refused with HSTU_ERR_WORKSPACE
  * and nothing is launched.  All calls on one GPU share the one array: two calls that overlap there (different
  * streams, replays of two graphs side by side) race on it and are the caller's to serialise; calls that follow each
- * other on a stream are safe, whatever their sizes (the counters are cleared ahead of every launch). */
+ * other on a stream are safe, whatever their sizes (no launch depends on what the array holds). */
 HSTU_API int hstu_jagged_fwd_noalloc(const hstu_jagged_fwd_params* params, void* stream);
 HSTU_API uint64_t hstu_jagged_fwd_noalloc_max_workspace(void);
 

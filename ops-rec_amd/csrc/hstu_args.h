@@ -39,6 +39,7 @@ constexpr int kFewRowsThreads = 256;  // threads of a workgroup of the backward 
 constexpr int kFewRows = 64;          // the most query rows of a sequence that kernel takes
 constexpr int kFwdFewRowsThreads = 512;  // threads of a workgroup of the forward kernel for few query rows (eight wavefronts over row groups and keys)
 constexpr int kCounterBlockBytes = 16384;  // head of the workspace: device-side work counters (see the forward kernel)
+constexpr int kQueueCounterBytes = 1024;   // of which the work counters of the per-XCD queues, the part that has to be cleared
 constexpr int kDkvThreads = 256;   // threads of a workgroup of the key-tile backward kernel
 constexpr int kGatherThreads = 128;
 
@@ -79,7 +80,8 @@ struct FwdArgs {
     const float* k_descale;
     const float* v_descale;
     int f32_splits;          // fp32 inputs only: wavefronts that share the keys of one row group (a power of two up to f32_waves)
-    unsigned int* counters;  // kCounterBlockBytes at the head of the workspace, cleared ahead of the launch; null for the plain list
+    unsigned int* counters;  // kCounterBlockBytes at the head of the workspace, the queues' part cleared ahead of the launch; null for the plain list
+    uint64_t launch_id;      // split variant: the launch's number, 1 .. 2^48 - 1, above the counts of its arrival counters
     float* ws;           // split variant: room for ws_parts partial outputs of kBlockM x D floats each (may be null)
     uint32_t ws_parts;
     // paged variant: the first (key count - num_target) key rows of a sequence live in pages of kv_cache

@@ -313,17 +313,20 @@ __device__ __forceinline__ void load_to_lds_b128(__amdgpu_buffer_rsrc_t rsrc, ui
 }
 
 // ---- device-side work counters ---------------------------------------------------------------
-// The variants that pull items from counters (per-XCD queues, split items, paged keys) keep them in a block at the
-// head of the caller's workspace (FwdArgs::counters, kCounterBlockBytes): one work counter per queue, each in a
-// 128-byte line of its own, then one arrival counter per split item.  The host clears the block on the launch
-// stream ahead of every launch, so the library holds no device state of its own: launches that overlap on one
-// GPU, on streams or as replays of captured graphs, are independent as long as their workspaces are.
+// Two kinds live in a block at the head of the caller's workspace (FwdArgs::counters, kCounterBlockBytes): the work counters
+// of the per-XCD queues, each in a 128-byte line of its own, and the arrival counters of split items, 64 bits each.  The
+// library holds no device state of its own: launches that overlap on one GPU, on streams or as replays of captured graphs,
+// are independent as long as their workspaces are.  The queues' counters are cleared by a kernel ahead of the launch.  That
+// costs a short launch 3 - 5 us with the gap behind it, so the arrival counters do without: a counter that does not carry
+// the launch's number (FwdArgs::launch_id, 48 bits) above its count reads as zero, whatever the workspace held before, and
+// the part that completes an item puts its counter back to zero, so that a replay under the same number finds none of its own.
 constexpr int kQueues = 8;          // one work queue per XCD (MI355X: 8 XCDs; workgroup w runs on XCD w mod 8)
 constexpr int kCounterStride = 32;  // counters of different queues sit in different 128-byte lines
-constexpr int kMaxSplitItems = 2048;
+constexpr int kMaxSplitItems = 1024;  // (an item is only split when there are fewer items than resident workgroups)
 constexpr int kMaxParts = 8;
 constexpr int kSplitCounterBase = kQueues * kCounterStride;  // first arrival counter, in 32-bit words
-static_assert((kSplitCounterBase + kMaxSplitItems) * 4 <= kCounterBlockBytes, "the counter block holds all counters");
+static_assert(kSplitCounterBase * 4 == kQueueCounterBytes, "the queues come first");
+static_assert((kSplitCounterBase + 2 * kMaxSplitItems) * 4 <= kCounterBlockBytes, "the counter block holds all counters");
 
 constexpr int kInteriorMinSteps = 20;  // sweeps shorter than this take the general time step throughout
 constexpr int kMaxBatchSlots = 2048;  // sequences per call (the reference's limit)
@@ -457,10 +460,11 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     __shared__ uint32_t s_rank_start[kMaxLevels + 2];     // [nt]: number of sequences with more than nt query tiles
     __shared__ uint32_t s_queue_start[QUEUES ? kQueues : 1][kMaxLevels + 2];  // per queue: first item of each level / bucket
     __shared__ uint32_t s_item[12];  // [0..3]: the item handed to the workgroup (valid, query tile, sequence, head); [4]: queue order
-                                     // [7]: part | parts << 8, [8]: arrival counter, [9]: first partial buffer, [10]: arrivals before
+                                     // [10]: arrivals before (split items)
     // plain list: the next item of the workgroup, decoded one item ahead ([parity][valid, query tile, sequence, head,
     // K/V head, q0 lo/hi, q1 lo/hi, k0 lo/hi, k1 lo/hi, context count, target count])
-    __shared__ uint32_t s_next[(!QUEUES && !SPLIT) ? 2 : 1][16];
+    // and, with SPLIT, the part word, the arrival counter and the first partial buffer
+    __shared__ uint32_t s_next[!QUEUES ? 2 : 1][20];
     __shared__ uint8_t s_parts[SPLIT ? kMaxLevels + 2 : 1];         // parts per item of each level
     __shared__ uint32_t s_split_first[SPLIT ? kMaxLevels + 2 : 1];  // first arrival counter of each split level
     __shared__ uint32_t s_ws_first[SPLIT ? kMaxLevels + 2 : 1];     // first partial buffer of each split level
@@ -563,27 +567,41 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     // workgroup of 1024 or 512 rows).
     // "By tile" runs as ONE queue shared by all workgroups (the order that matters there is global), "by pair" as
     // one queue per XCD.
-    if ((QUEUES || SPLIT) && tid < (QUEUES ? kQueues : 1)) {
-        bool by_pair = false;
-        if constexpr (QUEUES) {
-            // total tiles = sum over nt of nt * (sequences with nt tiles); sequences with nt tiles =
-            // s_rank_start[nt-1] - s_rank_start[nt]  (every builder thread works the order out for itself)
-            uint32_t tiles = 0, seqs = 0;
-            int nt_max = 0;
-            for (int nt = 1; nt <= n_levels; ++nt) {
-                const uint32_t c = s_rank_start[nt - 1] - s_rank_start[nt];
-                tiles += c * static_cast<uint32_t>(nt);
-                seqs += c;
-                nt_max = c != 0 ? nt : nt_max;
-            }
-            const uint32_t items = tiles * static_cast<uint32_t>(n_heads);
-            by_pair = (items >= 4u * gridDim.x && 10u * tiles <= 7u * seqs * static_cast<uint32_t>(nt_max)) || items >= 6u * gridDim.x;
+    if (QUEUES && tid < kQueues) {
+        // total tiles = sum over nt of nt * (sequences with nt tiles); sequences with nt tiles =
+        // s_rank_start[nt-1] - s_rank_start[nt]  (every builder thread works the order out for itself)
+        uint32_t tiles = 0, seqs = 0;
+        int nt_max = 0;
+        for (int nt = 1; nt <= n_levels; ++nt) {
+            const uint32_t c = s_rank_start[nt - 1] - s_rank_start[nt];
+            tiles += c * static_cast<uint32_t>(nt);
+            seqs += c;
+            nt_max = c != 0 ? nt : nt_max;
         }
+        const uint32_t items = tiles * static_cast<uint32_t>(n_heads);
+        const bool by_pair = (items >= 4u * gridDim.x && 10u * tiles <= 7u * seqs * static_cast<uint32_t>(nt_max)) || items >= 6u * gridDim.x;
         if (tid == 0) {
             s_item[4] = by_pair ? 1u : 0u;
         }
         const int ratio = a.head_ratio;
         const int n_heads_k = a.n_heads_k;
+        uint32_t acc = 0;
+        for (int l = 0; l < n_levels; ++l) {
+            s_queue_start[tid][l] = acc;
+            if (by_pair) {
+                const int nt = n_levels - l;
+                const uint32_t p0 = s_rank_start[nt] * static_cast<uint32_t>(n_heads_k);
+                const uint32_t p1 = s_rank_start[nt - 1] * static_cast<uint32_t>(n_heads_k);
+                // pairs p in [p0, p1) with p mod 8 == tid
+                const uint32_t mine = (p1 + kQueues - 1 - tid) / kQueues - (p0 + kQueues - 1 - tid) / kQueues;
+                acc += mine * static_cast<uint32_t>(nt * ratio);
+            } else if (tid == 0) {
+                acc += s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);  // every pair that has this tile
+            }
+        }
+        s_queue_start[tid][n_levels] = acc;
+    }
+    if constexpr (SPLIT) {
         // Splitting long items.  Level l holds the items of query tile qt = tile_of_level(l); under the built-in
         // mask such an item sweeps about 4 (qt + 1) sub-tiles (tile 0 with context rows: all), otherwise all of
         // max_seq_len_k.  With `target` = the
@@ -601,79 +619,104 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         // For the same reason the target is raised until the list with its parts still has at most one entry per
         // workgroup: a second round of entries costs more than shorter parts gain (12 x 4 items of 1024 rows:
         // 42.5 us with the mean as the target, 35.2 us with this rule, 33.5 us unsplit).
-        uint32_t split_target = 0;
-        uint32_t split_items = 0, split_bufs = 0;
-        auto nominal_steps = [&](int qt) -> uint32_t {
-            const int all = (a.max_k + 31) / 32;
-            if (a.mask_type != 0 || (ctx_first && qt == 0)) {
-                return static_cast<uint32_t>(all);
-            }
-            const int causal = 4 * (qt + 1) + (a.max_k > a.max_q ? (a.max_k - a.max_q) / 32 : 0);
-            return static_cast<uint32_t>(causal < all ? causal : all);
-        };
-        if constexpr (SPLIT) {
+        // Wavefront 0 works it out, a lane per level (64 levels a trip): one thread walking the levels would wait an LDS
+        // round trip for each, three times over.
+        if (wave == 0) {
+            constexpr int kTrips = (kMaxLevels + 63) / 64;
+            auto nominal_steps = [&](int qt) -> uint32_t {
+                const int all = (a.max_k + 31) / 32;
+                if (a.mask_type != 0 || (ctx_first && qt == 0)) {
+                    return static_cast<uint32_t>(all);
+                }
+                const int causal = 4 * (qt + 1) + (a.max_k > a.max_q ? (a.max_k - a.max_q) / 32 : 0);
+                return static_cast<uint32_t>(causal < all ? causal : all);
+            };
+            auto lane_sum = [&](uint32_t v) -> uint32_t {
+#pragma unroll
+                for (int s = 1; s < 64; s *= 2) {
+                    v += static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), s));
+                }
+                return static_cast<uint32_t>(uniform(static_cast<int>(v)));
+            };
+            auto lanes_before = [&](uint32_t v) -> uint32_t {  // sum over the lanes below this one
+                uint32_t x = v;
+#pragma unroll
+                for (int s = 1; s < 64; s *= 2) {
+                    const uint32_t up = static_cast<uint32_t>(__shfl_up(static_cast<int>(x), s));
+                    x += lane >= s ? up : 0u;
+                }
+                return x - v;
+            };
+            uint32_t cnt[kTrips], nom[kTrips];
             uint32_t steps = 0, items = 0;
-            for (int l = 0; l < n_levels; ++l) {
-                const uint32_t cnt = s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);
-                steps += cnt * (nominal_steps(tile_of_level(l)) + 3u);
-                items += cnt;
+#pragma unroll
+            for (int i = 0; i < kTrips; ++i) {
+                const int l = 64 * i + lane;
+                cnt[i] = l < n_levels ? s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads) : 0u;
+                nom[i] = l < n_levels ? nominal_steps(tile_of_level(l)) : 0u;
+                steps += cnt[i] * (nom[i] + 3u);
+                items += cnt[i];
             }
-            split_target = steps / gridDim.x;
-            split_target = split_target < 8u ? 8u : split_target;
+            steps = lane_sum(steps);
+            items = lane_sum(items);
+            uint32_t target = steps / gridDim.x;
+            target = target < 8u ? 8u : target;
+            auto parts_of = [&](int i) -> uint32_t {
+                const uint32_t m = (nom[i] + target - 1u) / target;
+                return m > static_cast<uint32_t>(kMaxParts) ? static_cast<uint32_t>(kMaxParts) : (m < 1u ? 1u : m);
+            };
+            auto entries_of = [&]() -> uint32_t {
+                uint32_t n = 0;
+#pragma unroll
+                for (int i = 0; i < kTrips; ++i) {
+                    n += cnt[i] * parts_of(i);
+                }
+                return lane_sum(n);
+            };
             if (a.ws == nullptr || items >= gridDim.x) {
-                split_target = 0x7fffffffu;  // nothing is split
-            } else {
+                target = 0x3fffffffu;  // nothing is split
+            } else if (entries_of() > gridDim.x) {
                 // one round: if the list cut at the mean has more entries than there are workgroups, the target
                 // is raised so that the entries splitting adds (at most nominal / target per item) go to the
                 // workgroups that would have had no item
-                // (counted in floating point: one thread does this for up to 160 levels, and the count only picks
-                // the rule, so a part more or less at an exact multiple does not matter)
-                uint32_t entries = 0;
-                const float inv_target = 1.0f / static_cast<float>(split_target);
-                for (int l = 0; l < n_levels; ++l) {
-                    const uint32_t cnt = s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);
-                    const uint32_t m = static_cast<uint32_t>(static_cast<float>(nominal_steps(tile_of_level(l))) * inv_target + 0.999f);
-                    entries += cnt * (m > static_cast<uint32_t>(kMaxParts) ? static_cast<uint32_t>(kMaxParts) : (m < 1u ? 1u : m));
+                const uint32_t spare = gridDim.x - items;
+                const uint32_t fit = (steps - 3u * items + spare - 1u) / spare;
+                target = target < fit ? fit : target;
+            }
+            // a caller may bring room for fewer partial outputs than the split would use: coarser parts until they fit (none at
+            // last: a target beyond every item splits nothing)
+            for (;;) {
+                uint32_t bufs = 0;
+#pragma unroll
+                for (int i = 0; i < kTrips; ++i) {
+                    const uint32_t m = parts_of(i);
+                    bufs += m > 1u ? cnt[i] * m : 0u;
                 }
-                if (entries > gridDim.x) {
-                    const uint32_t spare = gridDim.x - items;
-                    const uint32_t fit = (steps - 3u * items + spare - 1u) / spare;
-                    split_target = split_target < fit ? fit : split_target;
+                if (lane_sum(bufs) <= a.ws_parts || target >= 0x3fffffffu) {
+                    break;
                 }
+                target = target < 0x10000u ? target * 2u : 0x3fffffffu;
+            }
+            uint32_t first = 0, first_item = 0, first_buf = 0;
+#pragma unroll
+            for (int i = 0; i < kTrips; ++i) {
+                const int l = 64 * i + lane;
+                const uint32_t m = parts_of(i);
+                const uint32_t split = m > 1u ? cnt[i] : 0u;
+                const uint32_t at = first + lanes_before(cnt[i] * m);
+                const uint32_t item_at = first_item + lanes_before(split);
+                const uint32_t buf_at = first_buf + lanes_before(split * m);
+                if (l <= n_levels) {  // (past the last level every count is zero: its start is the end of the list)
+                    s_queue_start[0][l] = at;
+                    s_parts[l] = static_cast<uint8_t>(m);
+                    s_split_first[l] = item_at;
+                    s_ws_first[l] = buf_at;
+                }
+                first += lane_sum(cnt[i] * m);
+                first_item += lane_sum(split);
+                first_buf += lane_sum(split * m);
             }
         }
-        uint32_t acc = 0;
-        for (int l = 0; l < n_levels; ++l) {
-            s_queue_start[tid][l] = acc;
-            if constexpr (SPLIT) {
-                const uint32_t cnt = s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);
-                uint32_t m = (nominal_steps(tile_of_level(l)) + split_target - 1u) / split_target;
-                m = m > static_cast<uint32_t>(kMaxParts) ? static_cast<uint32_t>(kMaxParts) : m;
-                if (m > 1u && (split_items + cnt > static_cast<uint32_t>(kMaxSplitItems) || split_bufs + cnt * m > a.ws_parts)) {
-                    m = 1u;
-                }
-                s_parts[l] = static_cast<uint8_t>(m);
-                s_split_first[l] = split_items;
-                s_ws_first[l] = split_bufs;
-                if (m > 1u) {
-                    split_items += cnt;
-                    split_bufs += cnt * m;
-                }
-                acc += cnt * m;
-                continue;
-            }
-            if (by_pair) {
-                const int nt = n_levels - l;
-                const uint32_t p0 = s_rank_start[nt] * static_cast<uint32_t>(n_heads_k);
-                const uint32_t p1 = s_rank_start[nt - 1] * static_cast<uint32_t>(n_heads_k);
-                // pairs p in [p0, p1) with p mod 8 == tid
-                const uint32_t mine = (p1 + kQueues - 1 - tid) / kQueues - (p0 + kQueues - 1 - tid) / kQueues;
-                acc += mine * static_cast<uint32_t>(nt * ratio);
-            } else if (tid == 0) {
-                acc += s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);  // every pair that has this tile
-            }
-        }
-        s_queue_start[tid][n_levels] = acc;
     }
     __syncthreads();
     // Stable scatter (sequences of one bucket stay in index order) by wavefront 0 alone: every workgroup
@@ -910,7 +953,6 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         lvl = lvl < n_levels - 1 ? lvl : n_levels - 1;
         const int j_item = static_cast<int>(fq_idx - s_queue_start[fq_queue][lvl]);
         int qt, p_item, r_item;
-        uint32_t part_word = 0, split_counter = 0, split_buffer = 0;
         if (by_pair) {
             // item j of bucket lvl (pairs with nt tiles) = pair j / (nt * ratio) of this queue there, query tile
             // nt - 1 - (j % (nt * ratio)) / ratio, query head (kv head) * ratio + j % ratio
@@ -931,17 +973,8 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         } else {
             // item j of level lvl (query tile qt) = pair j / ratio, query head (kv head) * ratio + j % ratio
             qt = tile_of_level(lvl);
-            int j_whole = j_item;
-            if constexpr (SPLIT) {
-                // entry j of a split level = part j % m of item j / m
-                const int m = s_parts[lvl];
-                j_whole = div_small(j_item, m);
-                part_word = static_cast<uint32_t>(j_item - j_whole * m) | (static_cast<uint32_t>(m) << 8);
-                split_counter = s_split_first[lvl] + static_cast<uint32_t>(j_whole);
-                split_buffer = s_ws_first[lvl] + static_cast<uint32_t>(j_whole * m);
-            }
-            p_item = div_small(j_whole, ratio);
-            r_item = j_whole - p_item * ratio;
+            p_item = div_small(j_item, ratio);
+            r_item = j_item - p_item * ratio;
         }
         const int rank = div_small(p_item, n_heads_k);
         const int hk_item = p_item - rank * n_heads_k;
@@ -953,22 +986,17 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             s_item[3] = static_cast<uint32_t>(hk_item * ratio + r_item);
             s_item[5] = (static_cast<uint32_t>(fq_queue) << 28) | fq_idx;  // (for the development item log)
             s_item[6] = static_cast<uint32_t>(hk_item);
-            if constexpr (SPLIT) {
-                s_item[7] = part_word;
-                s_item[8] = split_counter;
-                s_item[9] = split_buffer;
-            }
         }
     };
-    // Plain list (one queue, by tile, nothing split): no counter at all.  The items of workgroup w are fixed by the
+    // Plain and split lists (one queue, by tile): no work counter at all.  The items of workgroup w are fixed by the
     // list alone: in round r it takes item r * grid + w (r even) or r * grid + grid - 1 - w (r odd), so that the
     // workgroups whose item of one round was heaviest get the lightest of the next -- what pulling from a counter
     // gives such a short list as well (measured equal on MI355X), without the counter's round trip, without device
     // state shared between launches, and with the next item known in advance: wavefront 0 decodes it, offsets
     // included, while the tile requests of the current item are under way, and leaves it in LDS for the others.
-    constexpr bool kStaticList = !QUEUES && !SPLIT;
+    constexpr bool kStaticList = !QUEUES;
     auto decode_ahead = [&](int round) {  // executed by wavefront 0; fills s_next[round & 1]
-        uint32_t(&rec)[16] = s_next[kStaticList ? (round & 1) : 0];
+        uint32_t(&rec)[20] = s_next[kStaticList ? (round & 1) : 0];
         const uint32_t g = gridDim.x;
         const uint32_t idx = static_cast<uint32_t>(round) * g + ((round & 1) ? g - 1u - blockIdx.x : blockIdx.x);
         if (idx >= s_queue_start[0][n_levels]) {
@@ -984,7 +1012,18 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             lvl += __builtin_popcountll(__builtin_amdgcn_ballot_w64(ends_before));
         }
         lvl = lvl < n_levels - 1 ? lvl : n_levels - 1;
-        const int j_item = static_cast<int>(idx - s_queue_start[0][lvl]);
+        int j_item = static_cast<int>(idx - s_queue_start[0][lvl]);
+        if constexpr (SPLIT) {
+            // entry j of a split level = part j % m of item j / m
+            const int m = s_parts[lvl];
+            const int whole = div_small(j_item, m);
+            if (lane == 0) {
+                rec[15] = static_cast<uint32_t>(j_item - whole * m) | (static_cast<uint32_t>(m) << 8);
+                rec[16] = s_split_first[lvl] + static_cast<uint32_t>(whole);
+                rec[17] = s_ws_first[lvl] + static_cast<uint32_t>(whole * m);
+            }
+            j_item = whole;
+        }
         const int p_item = div_small(j_item, a.head_ratio);
         const int r_item = j_item - p_item * a.head_ratio;
         const int rank = div_small(p_item, a.n_heads_k);
@@ -1034,7 +1073,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         int n_ctx = 0;
         int n_tgt = 0;
         if constexpr (kStaticList) {
-            const uint32_t(&rec)[16] = s_next[kStaticList ? (round & 1) : 0];
+            const uint32_t(&rec)[20] = s_next[kStaticList ? (round & 1) : 0];
             if (rec[0] == 0) {
                 break;
             }
@@ -1187,8 +1226,9 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         int part = 0;
         int n_parts = 1;
         if constexpr (SPLIT) {
-            part = uniform(static_cast<int>(s_item[7] & 0xffu));
-            n_parts = uniform(static_cast<int>(s_item[7] >> 8));
+            const uint32_t part_word = s_next[round & 1][15];
+            part = uniform(static_cast<int>(part_word & 0xffu));
+            n_parts = uniform(static_cast<int>(part_word >> 8));
             if (n_parts > 1) {
                 const int len = ((n_sub + n_parts - 1) / n_parts + 3) & ~3;
                 x_begin = part * len;
@@ -1995,7 +2035,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 constexpr int kDeviceScope = 1 | 16;  // cache policy bits sc0 | sc1 of gfx94x / gfx950 buffer accesses
                 constexpr int kQuads = MTILES * 4;                       // 16-byte pieces of a lane's accumulators
                 constexpr uint32_t kPartBytes = kBlockM * D * 4u;        // one partial output
-                const int ws_index = uniform(static_cast<int>(s_item[9]));
+                const int ws_index = uniform(static_cast<int>(s_next[round & 1][17]));
                 const __amdgpu_buffer_rsrc_t ws_rsrc =
                     make_rsrc(reinterpret_cast<const uint8_t*>(a.ws) + static_cast<int64_t>(ws_index) * kPartBytes,
                               static_cast<uint32_t>(n_parts) * kPartBytes);
@@ -2015,9 +2055,19 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 }
                 __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();  // every wavefront's stores have completed
-                unsigned int* const arrived = a.counters + kSplitCounterBase + s_item[8];
+                uint64_t* const arrived = reinterpret_cast<uint64_t*>(a.counters + kSplitCounterBase) + s_next[round & 1][16];
                 if (tid == 0) {
-                    s_item[10] = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    const uint64_t none = a.launch_id << 16;  // no part has arrived in this launch
+                    uint64_t seen = __hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    uint64_t before;
+                    do {
+                        before = (seen >> 16) == a.launch_id ? seen : none;
+                    } while (!__hip_atomic_compare_exchange_strong(arrived, &seen, before + 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                                   __HIP_MEMORY_SCOPE_AGENT));
+                    s_item[10] = static_cast<uint32_t>(before & 0xffffu);
+                    if (s_item[10] == static_cast<uint32_t>(n_parts - 1)) {
+                        __hip_atomic_store(arrived, uint64_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
                 }
                 __syncthreads();
                 store_rows = s_item[10] == static_cast<uint32_t>(n_parts - 1);
@@ -2049,7 +2099,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                         }
                     }
                 }
-                __syncthreads();  // s_item[10] has been read before the next fetch writes the item
+                __syncthreads();  // s_item[10] has been read before the next item's is written
             }
         }
 

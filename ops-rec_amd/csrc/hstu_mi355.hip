@@ -14,6 +14,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <atomic>
+#include <chrono>
 #include <mutex>
 
 #include "hstu_clear.hip.h"
@@ -1409,6 +1411,15 @@ HSTU_API const char* hstu_jagged_fwd_kernel_name(const hstu_jagged_fwd_params* p
 
 namespace {
 
+// A number that no other launch whose counters may still lie in some workspace has carried: counted up from a start of its
+// own in every process (48 bits: a launch a microsecond wraps after nine years).
+uint64_t next_launch_id()
+{
+    static std::atomic<uint64_t> last{static_cast<uint64_t>(std::chrono::steady_clock::now().time_since_epoch().count()) << 16};
+    const uint64_t id = (last.fetch_add(1, std::memory_order_relaxed) + 1) & ((uint64_t{1} << 48) - 1);
+    return id != 0 ? id : next_launch_id();
+}
+
 // the forward launch; `paged` (optional) makes it the paged variant, which the caller has checked to exist
 int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params* paged, void* workspace,
                    uint64_t workspace_bytes, void* stream)
@@ -1544,8 +1555,10 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
             kernel = var->kernel_paged;  // (splits when it was given room above, otherwise not; the caller checked the block)
             a.counters = static_cast<unsigned int*>(workspace);
         }
-        if (a.counters != nullptr) {
-            launch_clear(a.counters, static_cast<int64_t>(kCounterBytes), stream);
+        if (kernel == var->kernel_queues) {
+            launch_clear(a.counters, hstu::kQueueCounterBytes, stream);
+        } else if (a.counters != nullptr) {
+            a.launch_id = next_launch_id();
         }
     }
     const Variant* const f32 = &hstu::fwd_variants_f32()[0][0][0];
