@@ -631,22 +631,18 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 const int causal = 4 * (qt + 1) + (a.max_k > a.max_q ? (a.max_k - a.max_q) / 32 : 0);
                 return static_cast<uint32_t>(causal < all ? causal : all);
             };
-            auto lane_sum = [&](uint32_t v) -> uint32_t {
-#pragma unroll
-                for (int s = 1; s < 64; s *= 2) {
-                    v += static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), s));
-                }
-                return static_cast<uint32_t>(uniform(static_cast<int>(v)));
+            auto up_to_lane = [&](uint32_t v) -> uint32_t {  // sum over this lane and those below it (row shifts, row broadcasts)
+                int x = static_cast<int>(v);
+                x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+                x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+                x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+                x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+                x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+                x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+                return static_cast<uint32_t>(x);
             };
-            auto lanes_before = [&](uint32_t v) -> uint32_t {  // sum over the lanes below this one
-                uint32_t x = v;
-#pragma unroll
-                for (int s = 1; s < 64; s *= 2) {
-                    const uint32_t up = static_cast<uint32_t>(__shfl_up(static_cast<int>(x), s));
-                    x += lane >= s ? up : 0u;
-                }
-                return x - v;
-            };
+            auto last_lane = [&](uint32_t v) -> uint32_t { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63)); };
+            auto lane_sum = [&](uint32_t v) -> uint32_t { return last_lane(up_to_lane(v)); };
             uint32_t cnt[kTrips], nom[kTrips];
             uint32_t steps = 0, items = 0;
 #pragma unroll
@@ -701,20 +697,23 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
 #pragma unroll
             for (int i = 0; i < kTrips; ++i) {
                 const int l = 64 * i + lane;
+                if (64 * i > n_levels) {
+                    break;
+                }
                 const uint32_t m = parts_of(i);
                 const uint32_t split = m > 1u ? cnt[i] : 0u;
-                const uint32_t at = first + lanes_before(cnt[i] * m);
-                const uint32_t item_at = first_item + lanes_before(split);
-                const uint32_t buf_at = first_buf + lanes_before(split * m);
+                const uint32_t at = up_to_lane(cnt[i] * m);
+                const uint32_t item_at = up_to_lane(split);
+                const uint32_t buf_at = up_to_lane(split * m);
                 if (l <= n_levels) {  // (past the last level every count is zero: its start is the end of the list)
-                    s_queue_start[0][l] = at;
+                    s_queue_start[0][l] = first + at - cnt[i] * m;
                     s_parts[l] = static_cast<uint8_t>(m);
-                    s_split_first[l] = item_at;
-                    s_ws_first[l] = buf_at;
+                    s_split_first[l] = first_item + item_at - split;
+                    s_ws_first[l] = first_buf + buf_at - split * m;
                 }
-                first += lane_sum(cnt[i] * m);
-                first_item += lane_sum(split);
-                first_buf += lane_sum(split * m);
+                first += last_lane(at);
+                first_item += last_lane(item_at);
+                first_buf += last_lane(buf_at);
             }
         }
     }
