@@ -408,8 +408,14 @@ struct U32Quad {
 //
 // PAGED: K / V rows come from a paged cache plus the tail of the k / v inputs (see "Paged keys" below); built on top
 // of the SPLIT variant, because its callers (inference: few query rows against a long cache) have short lists.
+//
+// DIRECT: short lists do without a list: a workgroup per (level, pair, query head of the pair) slot, pairs padded to a
+// multiple of 8 so that a pair's tiles meet on one XCD, levels in list order so that the longest items start first; slots
+// past the end of their sequence leave at once.  That spares every workgroup the histogram, the list and the hand-over of
+// its item through LDS, 1.5 .. 4 us ahead of its first request.  (A variant of its own: as a branch of the plain one it cost
+// that 1 us.)
 template <typename Tag, typename OutTag, int D, bool HAS_RAB, bool HAS_MASK, bool QUEUES = false, bool SPLIT = false,
-          bool PAGED = false>
+          bool PAGED = false, bool DIRECT = false>
 __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hstu_fwd_kernel(const FwdArgs a)
 {
     constexpr int kThreads = 256;
@@ -421,6 +427,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     static_assert(!F8 || !(HAS_RAB || HAS_MASK) || !SPLIT, "fp8 with rab / custom mask: whole items only");
     static_assert(!F8 || D >= 64, "fp8 rows are at least 64 bytes");
     static_assert(!(QUEUES && SPLIT), "one list policy per variant");
+    static_assert(!DIRECT || !(QUEUES || SPLIT || PAGED), "no list, no list policy");
     static_assert(!PAGED || (SPLIT && !F8), "the paged variant builds on the split variant, 16-bit inputs");
     constexpr int CPR = D * ES / 16;             // 16-byte chunks per row
     constexpr int EPC16 = 16 / ES;               // elements per 16-byte chunk
@@ -454,11 +461,13 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     __shared__ __attribute__((aligned(1024))) uint16_t s_v2[SUB_ELEMS];
     __shared__ __attribute__((aligned(1024))) uint16_t s_v3[SUB_ELEMS];
     // work list
-    __shared__ uint8_t s_ntiles[kMaxBatchSlots];          // query tiles of each sequence
-    __shared__ uint16_t s_order[kMaxBatchSlots];          // sequences, most query tiles first
-    __shared__ uint32_t s_bucket[kMaxLevels + 2];         // histogram, then scatter cursors
-    __shared__ uint32_t s_rank_start[kMaxLevels + 2];     // [nt]: number of sequences with more than nt query tiles
-    __shared__ uint32_t s_queue_start[QUEUES ? kQueues : 1][kMaxLevels + 2];  // per queue: first item of each level / bucket
+    constexpr int kListSlots = DIRECT ? 1 : kMaxBatchSlots;
+    constexpr int kListLevels = DIRECT ? 1 : kMaxLevels + 2;
+    __shared__ uint8_t s_ntiles[kListSlots];          // query tiles of each sequence
+    __shared__ uint16_t s_order[kListSlots];          // sequences, most query tiles first
+    __shared__ uint32_t s_bucket[kListLevels];         // histogram, then scatter cursors
+    __shared__ uint32_t s_rank_start[kListLevels];     // [nt]: number of sequences with more than nt query tiles
+    __shared__ uint32_t s_queue_start[QUEUES ? kQueues : 1][kListLevels];  // per queue: first item of each level / bucket
     __shared__ uint32_t s_item[12];  // [0..3]: the item handed to the workgroup (valid, query tile, sequence, head); [4]: queue order
                                      // [10]: arrivals before (split items)
     // plain list: the next item of the workgroup, decoded one item ahead ([parity][valid, query tile, sequence, head,
@@ -488,268 +497,271 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     // share the job); the offset is requested here, so that nothing waits for it
     const int64_t last_offset = load_index_uniform(a.offs_q, a.n_batch, a.idx64);
 
-    // ---- work list: bucket the sequences by their number of query tiles ----
-    for (int i = tid; i <= n_levels; i += kThreads) {
-        s_bucket[i] = 0;
-    }
-    __syncthreads();
-    for (int b = tid; b < a.n_batch; b += kThreads) {
-        int64_t q0 = load_index(a.offs_q, b, a.idx64);
-        int64_t q1 = load_index(a.offs_q, b + 1, a.idx64);
-        q1 = q1 < a.total_q ? q1 : a.total_q;
-        q0 = q0 < 0 ? 0 : q0;
-        int sq = static_cast<int>(q1 > q0 ? q1 - q0 : 0);
-        sq = sq < a.max_q ? sq : a.max_q;
-        const int nt = (sq + kBlockM - 1) / kBlockM;  // 0 .. n_levels
-        s_ntiles[b] = static_cast<uint8_t>(nt);
-        atomicAdd(&s_bucket[nt], 1u);
-    }
-    __syncthreads();
-    // Bucket starts in "most tiles first" order: s_rank_start[nt] = number of sequences with more than nt tiles.
-    // Thread nt sums the counts above its own level by itself: its reads are independent, so they stream through
-    // the LDS back to back, where a prefix walk by one thread waits a full LDS round trip per level (with at most
-    // 161 levels the extra additions cost nothing).  In the same pass it gets the first item of list level l = nt
-    // of the plain list (one queue, by tile, nothing split): level l' holds the items of query tile
-    // n_levels - 1 - l', i.e. n_heads per sequence with more tiles than that, so the levels before l hold
-    // n_heads * sum over nt' of count[nt'] * max(0, nt' - (n_levels - l)) items.  (With tile 0 in level 0, level
-    // l >= 1 starts after all sequences that have a tile at all plus what stood before level l - 1.)
-    static_assert(kMaxLevels + 2 <= kThreads, "one thread per level");
-    {
-        uint32_t above = 0;
-        uint32_t items_before = 0;
-        if (tid <= n_levels) {
-            const int floor_tiles = n_levels - tid + (ctx_first ? 1 : 0);
-            uint32_t with_tiles = 0;
-            for (int nt = n_levels; nt >= 1; --nt) {
-                const uint32_t c = s_bucket[nt];
-                above += nt > tid ? c : 0u;
-                with_tiles += c;
-                items_before += nt > floor_tiles ? c * static_cast<uint32_t>(nt - floor_tiles) : 0u;
-            }
-            if (ctx_first) {
-                items_before = tid == 0 ? 0u : items_before + with_tiles;
-            }
+    if constexpr (!DIRECT) {
+        // ---- work list: bucket the sequences by their number of query tiles ----
+        for (int i = tid; i <= n_levels; i += kThreads) {
+            s_bucket[i] = 0;
         }
-        __syncthreads();  // the counts have been read by everybody
-        if (tid <= n_levels) {
-            s_rank_start[tid] = above;
-            s_bucket[tid] = above;  // from here on: scatter cursors
+        __syncthreads();
+        for (int b = tid; b < a.n_batch; b += kThreads) {
+            int64_t q0 = load_index(a.offs_q, b, a.idx64);
+            int64_t q1 = load_index(a.offs_q, b + 1, a.idx64);
+            q1 = q1 < a.total_q ? q1 : a.total_q;
+            q0 = q0 < 0 ? 0 : q0;
+            int sq = static_cast<int>(q1 > q0 ? q1 - q0 : 0);
+            sq = sq < a.max_q ? sq : a.max_q;
+            const int nt = (sq + kBlockM - 1) / kBlockM;  // 0 .. n_levels
+            s_ntiles[b] = static_cast<uint8_t>(nt);
+            atomicAdd(&s_bucket[nt], 1u);
+        }
+        __syncthreads();
+        // Bucket starts in "most tiles first" order: s_rank_start[nt] = number of sequences with more than nt tiles.
+        // Thread nt sums the counts above its own level by itself: its reads are independent, so they stream through
+        // the LDS back to back, where a prefix walk by one thread waits a full LDS round trip per level (with at most
+        // 161 levels the extra additions cost nothing).  In the same pass it gets the first item of list level l = nt
+        // of the plain list (one queue, by tile, nothing split): level l' holds the items of query tile
+        // n_levels - 1 - l', i.e. n_heads per sequence with more tiles than that, so the levels before l hold
+        // n_heads * sum over nt' of count[nt'] * max(0, nt' - (n_levels - l)) items.  (With tile 0 in level 0, level
+        // l >= 1 starts after all sequences that have a tile at all plus what stood before level l - 1.)
+        static_assert(kMaxLevels + 2 <= kThreads, "one thread per level");
+        {
+            uint32_t above = 0;
+            uint32_t items_before = 0;
+            if (tid <= n_levels) {
+                const int floor_tiles = n_levels - tid + (ctx_first ? 1 : 0);
+                uint32_t with_tiles = 0;
+                for (int nt = n_levels; nt >= 1; --nt) {
+                    const uint32_t c = s_bucket[nt];
+                    above += nt > tid ? c : 0u;
+                    with_tiles += c;
+                    items_before += nt > floor_tiles ? c * static_cast<uint32_t>(nt - floor_tiles) : 0u;
+                }
+                if (ctx_first) {
+                    items_before = tid == 0 ? 0u : items_before + with_tiles;
+                }
+            }
+            __syncthreads();  // the counts have been read by everybody
+            if (tid <= n_levels) {
+                s_rank_start[tid] = above;
+                s_bucket[tid] = above;  // from here on: scatter cursors
+                if constexpr (!QUEUES && !SPLIT) {
+                    s_queue_start[0][tid] = items_before * static_cast<uint32_t>(n_heads);
+                }
+            }
             if constexpr (!QUEUES && !SPLIT) {
-                s_queue_start[0][tid] = items_before * static_cast<uint32_t>(n_heads);
+                if (tid == 0) {
+                    s_item[4] = 0u;  // by tile
+                }
             }
         }
-        if constexpr (!QUEUES && !SPLIT) {
+        __syncthreads();
+        // Work queues.  A "pair" is one (sequence, K/V head): its K / V rows are read by every query tile of every
+        // query head that shares the K/V head.  Pairs are numbered p = sorted position * n_heads_k + kv head; pair p
+        // belongs to queue p mod 8, and a queue is served first by the workgroups of one XCD, so that the rows of a
+        // pair are fetched into one L2 instead of eight.  Two orders inside a queue:
+        //   by tile  - the heaviest (highest) query tile of all its pairs first, then the next tile down, ...: longest
+        //              items first.  With a handful of items per workgroup and item lengths between 1 and
+        //              max_seq_len / 32 steps this is what keeps the end of the launch short.  Level l of the queue =
+        //              query tile tile_of_level(l) of its pairs that have it (the sequences at sorted positions
+        //              [0, s_rank_start[qt]) have more than qt tiles).
+        //   by pair  - pair after pair (most tiles first), the tiles of a pair together, heaviest first: the
+        //              workgroups of the XCD sweep the K / V rows of few pairs at a time, and each row is fetched
+        //              from HBM about once instead of once per query tile.  Bucket l of the queue = its pairs with
+        //              nt = n_levels - l tiles (sorted positions [s_rank_start[nt], s_rank_start[nt - 1])).
+        // "By pair" starts the heavy tiles of late pairs late; that is harmless when there are many items per
+        // workgroup and the late pairs are short (a jagged batch), and costly when all sequences are equally long.
+        // It is chosen when the list has at least 4 items per workgroup and the mean tile count of the sequences is
+        // at most 0.7 of the largest, and whatever the lengths from 6 items per workgroup on: by tile, the resident workgroups
+        // of a long list all work on different pairs, and every item streams its keys from memory (128 x 4 heads of 7621
+        // rows, d 128: 61 GB in 11.05 ms by tile, 7.21 ms by pair; 64 x 4 of 4096 rows 1.39 -> 1.14 ms; level at 8 items per
+        // workgroup of 1024 or 512 rows).
+        // "By tile" runs as ONE queue shared by all workgroups (the order that matters there is global), "by pair" as
+        // one queue per XCD.
+        if (QUEUES && tid < kQueues) {
+            // total tiles = sum over nt of nt * (sequences with nt tiles); sequences with nt tiles =
+            // s_rank_start[nt-1] - s_rank_start[nt]  (every builder thread works the order out for itself)
+            uint32_t tiles = 0, seqs = 0;
+            int nt_max = 0;
+            for (int nt = 1; nt <= n_levels; ++nt) {
+                const uint32_t c = s_rank_start[nt - 1] - s_rank_start[nt];
+                tiles += c * static_cast<uint32_t>(nt);
+                seqs += c;
+                nt_max = c != 0 ? nt : nt_max;
+            }
+            const uint32_t items = tiles * static_cast<uint32_t>(n_heads);
+            const bool by_pair = (items >= 4u * gridDim.x && 10u * tiles <= 7u * seqs * static_cast<uint32_t>(nt_max)) || items >= 6u * gridDim.x;
             if (tid == 0) {
-                s_item[4] = 0u;  // by tile
+                s_item[4] = by_pair ? 1u : 0u;
             }
-        }
-    }
-    __syncthreads();
-    // Work queues.  A "pair" is one (sequence, K/V head): its K / V rows are read by every query tile of every
-    // query head that shares the K/V head.  Pairs are numbered p = sorted position * n_heads_k + kv head; pair p
-    // belongs to queue p mod 8, and a queue is served first by the workgroups of one XCD, so that the rows of a
-    // pair are fetched into one L2 instead of eight.  Two orders inside a queue:
-    //   by tile  - the heaviest (highest) query tile of all its pairs first, then the next tile down, ...: longest
-    //              items first.  With a handful of items per workgroup and item lengths between 1 and
-    //              max_seq_len / 32 steps this is what keeps the end of the launch short.  Level l of the queue =
-    //              query tile tile_of_level(l) of its pairs that have it (the sequences at sorted positions
-    //              [0, s_rank_start[qt]) have more than qt tiles).
-    //   by pair  - pair after pair (most tiles first), the tiles of a pair together, heaviest first: the
-    //              workgroups of the XCD sweep the K / V rows of few pairs at a time, and each row is fetched
-    //              from HBM about once instead of once per query tile.  Bucket l of the queue = its pairs with
-    //              nt = n_levels - l tiles (sorted positions [s_rank_start[nt], s_rank_start[nt - 1])).
-    // "By pair" starts the heavy tiles of late pairs late; that is harmless when there are many items per
-    // workgroup and the late pairs are short (a jagged batch), and costly when all sequences are equally long.
-    // It is chosen when the list has at least 4 items per workgroup and the mean tile count of the sequences is
-    // at most 0.7 of the largest, and whatever the lengths from 6 items per workgroup on: by tile, the resident workgroups
-    // of a long list all work on different pairs, and every item streams its keys from memory (128 x 4 heads of 7621
-    // rows, d 128: 61 GB in 11.05 ms by tile, 7.21 ms by pair; 64 x 4 of 4096 rows 1.39 -> 1.14 ms; level at 8 items per
-    // workgroup of 1024 or 512 rows).
-    // "By tile" runs as ONE queue shared by all workgroups (the order that matters there is global), "by pair" as
-    // one queue per XCD.
-    if (QUEUES && tid < kQueues) {
-        // total tiles = sum over nt of nt * (sequences with nt tiles); sequences with nt tiles =
-        // s_rank_start[nt-1] - s_rank_start[nt]  (every builder thread works the order out for itself)
-        uint32_t tiles = 0, seqs = 0;
-        int nt_max = 0;
-        for (int nt = 1; nt <= n_levels; ++nt) {
-            const uint32_t c = s_rank_start[nt - 1] - s_rank_start[nt];
-            tiles += c * static_cast<uint32_t>(nt);
-            seqs += c;
-            nt_max = c != 0 ? nt : nt_max;
-        }
-        const uint32_t items = tiles * static_cast<uint32_t>(n_heads);
-        const bool by_pair = (items >= 4u * gridDim.x && 10u * tiles <= 7u * seqs * static_cast<uint32_t>(nt_max)) || items >= 6u * gridDim.x;
-        if (tid == 0) {
-            s_item[4] = by_pair ? 1u : 0u;
-        }
-        const int ratio = a.head_ratio;
-        const int n_heads_k = a.n_heads_k;
-        uint32_t acc = 0;
-        for (int l = 0; l < n_levels; ++l) {
-            s_queue_start[tid][l] = acc;
-            if (by_pair) {
-                const int nt = n_levels - l;
-                const uint32_t p0 = s_rank_start[nt] * static_cast<uint32_t>(n_heads_k);
-                const uint32_t p1 = s_rank_start[nt - 1] * static_cast<uint32_t>(n_heads_k);
-                // pairs p in [p0, p1) with p mod 8 == tid
-                const uint32_t mine = (p1 + kQueues - 1 - tid) / kQueues - (p0 + kQueues - 1 - tid) / kQueues;
-                acc += mine * static_cast<uint32_t>(nt * ratio);
-            } else if (tid == 0) {
-                acc += s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);  // every pair that has this tile
-            }
-        }
-        s_queue_start[tid][n_levels] = acc;
-    }
-    if constexpr (SPLIT) {
-        // Splitting long items.  Level l holds the items of query tile qt = tile_of_level(l); under the built-in
-        // mask such an item sweeps about 4 (qt + 1) sub-tiles (tile 0 with context rows: all), otherwise all of
-        // max_seq_len_k.  With `target` = the
-        // mean number of time steps per workgroup (3 steps of start-up per item included, never below 8), the items
-        // of a level whose nominal length exceeds it are listed as m = ceil(nominal / target) entries (at most
-        // kMaxParts), one per part of the key range, next to each other in the list.  Part i sweeps the sub-tiles
-        // [i * len, (i + 1) * len) of the item's real range, len a multiple of 4; it writes its fp32 accumulators
-        // to its own buffer in the workspace and counts itself in; the part that finds all others counted in adds
-        // the m buffers in part order (so the sum does not depend on who came last) and stores the rows.
-        // A level is split only while arrival counters and workspace buffers last, and nothing is split when the
-        // list has an item for every workgroup anyway: measured on MI355X, an entry of the list costs 4 - 6 us on
-        // top of its sweep (its own start-up, the hand-over of its accumulators), which a list of 1.4 items per
-        // workgroup (batch 32 x 4 heads, lengths 256..1024) no longer earns back, while a list that leaves workgroups
-        // idle (one 20480-row sequence, or 4 sequences x 2 heads up to 3000 rows) finishes in 0.5 - 0.65 of the time.
-        // For the same reason the target is raised until the list with its parts still has at most one entry per
-        // workgroup: a second round of entries costs more than shorter parts gain (12 x 4 items of 1024 rows:
-        // 42.5 us with the mean as the target, 35.2 us with this rule, 33.5 us unsplit).
-        // Wavefront 0 works it out, a lane per level (64 levels a trip): one thread walking the levels would wait an LDS
-        // round trip for each, three times over.
-        if (wave == 0) {
-            constexpr int kTrips = (kMaxLevels + 63) / 64;
-            auto nominal_steps = [&](int qt) -> uint32_t {
-                const int all = (a.max_k + 31) / 32;
-                if (a.mask_type != 0 || (ctx_first && qt == 0)) {
-                    return static_cast<uint32_t>(all);
+            const int ratio = a.head_ratio;
+            const int n_heads_k = a.n_heads_k;
+            uint32_t acc = 0;
+            for (int l = 0; l < n_levels; ++l) {
+                s_queue_start[tid][l] = acc;
+                if (by_pair) {
+                    const int nt = n_levels - l;
+                    const uint32_t p0 = s_rank_start[nt] * static_cast<uint32_t>(n_heads_k);
+                    const uint32_t p1 = s_rank_start[nt - 1] * static_cast<uint32_t>(n_heads_k);
+                    // pairs p in [p0, p1) with p mod 8 == tid
+                    const uint32_t mine = (p1 + kQueues - 1 - tid) / kQueues - (p0 + kQueues - 1 - tid) / kQueues;
+                    acc += mine * static_cast<uint32_t>(nt * ratio);
+                } else if (tid == 0) {
+                    acc += s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads);  // every pair that has this tile
                 }
-                const int causal = 4 * (qt + 1) + (a.max_k > a.max_q ? (a.max_k - a.max_q) / 32 : 0);
-                return static_cast<uint32_t>(causal < all ? causal : all);
-            };
-            auto up_to_lane = [&](uint32_t v) -> uint32_t {  // sum over this lane and those below it (row shifts, row broadcasts)
-                int x = static_cast<int>(v);
-                x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
-                x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
-                x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
-                x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
-                x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
-                x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
-                return static_cast<uint32_t>(x);
-            };
-            auto last_lane = [&](uint32_t v) -> uint32_t { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63)); };
-            auto lane_sum = [&](uint32_t v) -> uint32_t { return last_lane(up_to_lane(v)); };
-            uint32_t cnt[kTrips], nom[kTrips];
-            uint32_t steps = 0, items = 0;
-#pragma unroll
-            for (int i = 0; i < kTrips; ++i) {
-                const int l = 64 * i + lane;
-                cnt[i] = l < n_levels ? s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads) : 0u;
-                nom[i] = l < n_levels ? nominal_steps(tile_of_level(l)) : 0u;
-                steps += cnt[i] * (nom[i] + 3u);
-                items += cnt[i];
             }
-            steps = lane_sum(steps);
-            items = lane_sum(items);
-            uint32_t target = steps / gridDim.x;
-            target = target < 8u ? 8u : target;
-            auto parts_of = [&](int i) -> uint32_t {
-                const uint32_t m = (nom[i] + target - 1u) / target;
-                return m > static_cast<uint32_t>(kMaxParts) ? static_cast<uint32_t>(kMaxParts) : (m < 1u ? 1u : m);
-            };
-            auto entries_of = [&]() -> uint32_t {
-                uint32_t n = 0;
+            s_queue_start[tid][n_levels] = acc;
+        }
+        if constexpr (SPLIT) {
+            // Splitting long items.  Level l holds the items of query tile qt = tile_of_level(l); under the built-in
+            // mask such an item sweeps about 4 (qt + 1) sub-tiles (tile 0 with context rows: all), otherwise all of
+            // max_seq_len_k.  With `target` = the
+            // mean number of time steps per workgroup (3 steps of start-up per item included, never below 8), the items
+            // of a level whose nominal length exceeds it are listed as m = ceil(nominal / target) entries (at most
+            // kMaxParts), one per part of the key range, next to each other in the list.  Part i sweeps the sub-tiles
+            // [i * len, (i + 1) * len) of the item's real range, len a multiple of 4; it writes its fp32 accumulators
+            // to its own buffer in the workspace and counts itself in; the part that finds all others counted in adds
+            // the m buffers in part order (so the sum does not depend on who came last) and stores the rows.
+            // A level is split only while arrival counters and workspace buffers last, and nothing is split when the
+            // list has an item for every workgroup anyway: measured on MI355X, an entry of the list costs 4 - 6 us on
+            // top of its sweep (its own start-up, the hand-over of its accumulators), which a list of 1.4 items per
+            // workgroup (batch 32 x 4 heads, lengths 256..1024) no longer earns back, while a list that leaves workgroups
+            // idle (one 20480-row sequence, or 4 sequences x 2 heads up to 3000 rows) finishes in 0.5 - 0.65 of the time.
+            // For the same reason the target is raised until the list with its parts still has at most one entry per
+            // workgroup: a second round of entries costs more than shorter parts gain (12 x 4 items of 1024 rows:
+            // 42.5 us with the mean as the target, 35.2 us with this rule, 33.5 us unsplit).
+            // Wavefront 0 works it out, a lane per level (64 levels a trip): one thread walking the levels would wait an LDS
+            // round trip for each, three times over.
+            if (wave == 0) {
+                constexpr int kTrips = (kMaxLevels + 63) / 64;
+                auto nominal_steps = [&](int qt) -> uint32_t {
+                    const int all = (a.max_k + 31) / 32;
+                    if (a.mask_type != 0 || (ctx_first && qt == 0)) {
+                        return static_cast<uint32_t>(all);
+                    }
+                    const int causal = 4 * (qt + 1) + (a.max_k > a.max_q ? (a.max_k - a.max_q) / 32 : 0);
+                    return static_cast<uint32_t>(causal < all ? causal : all);
+                };
+                auto up_to_lane = [&](uint32_t v) -> uint32_t {  // sum over this lane and those below it (row shifts, row broadcasts)
+                    int x = static_cast<int>(v);
+                    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+                    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+                    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+                    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+                    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+                    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+                    return static_cast<uint32_t>(x);
+                };
+                auto last_lane = [&](uint32_t v) -> uint32_t { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63)); };
+                auto lane_sum = [&](uint32_t v) -> uint32_t { return last_lane(up_to_lane(v)); };
+                uint32_t cnt[kTrips], nom[kTrips];
+                uint32_t steps = 0, items = 0;
 #pragma unroll
                 for (int i = 0; i < kTrips; ++i) {
-                    n += cnt[i] * parts_of(i);
+                    const int l = 64 * i + lane;
+                    cnt[i] = l < n_levels ? s_rank_start[tile_of_level(l)] * static_cast<uint32_t>(n_heads) : 0u;
+                    nom[i] = l < n_levels ? nominal_steps(tile_of_level(l)) : 0u;
+                    steps += cnt[i] * (nom[i] + 3u);
+                    items += cnt[i];
                 }
-                return lane_sum(n);
-            };
-            if (a.ws == nullptr || items >= gridDim.x) {
-                target = 0x3fffffffu;  // nothing is split
-            } else if (entries_of() > gridDim.x) {
-                // one round: if the list cut at the mean has more entries than there are workgroups, the target
-                // is raised so that the entries splitting adds (at most nominal / target per item) go to the
-                // workgroups that would have had no item
-                const uint32_t spare = gridDim.x - items;
-                const uint32_t fit = (steps - 3u * items + spare - 1u) / spare;
-                target = target < fit ? fit : target;
-            }
-            // a caller may bring room for fewer partial outputs than the split would use: coarser parts until they fit (none at
-            // last: a target beyond every item splits nothing)
-            for (;;) {
-                uint32_t bufs = 0;
+                steps = lane_sum(steps);
+                items = lane_sum(items);
+                uint32_t target = steps / gridDim.x;
+                target = target < 8u ? 8u : target;
+                auto parts_of = [&](int i) -> uint32_t {
+                    const uint32_t m = (nom[i] + target - 1u) / target;
+                    return m > static_cast<uint32_t>(kMaxParts) ? static_cast<uint32_t>(kMaxParts) : (m < 1u ? 1u : m);
+                };
+                auto entries_of = [&]() -> uint32_t {
+                    uint32_t n = 0;
+#pragma unroll
+                    for (int i = 0; i < kTrips; ++i) {
+                        n += cnt[i] * parts_of(i);
+                    }
+                    return lane_sum(n);
+                };
+                if (a.ws == nullptr || items >= gridDim.x) {
+                    target = 0x3fffffffu;  // nothing is split
+                } else if (entries_of() > gridDim.x) {
+                    // one round: if the list cut at the mean has more entries than there are workgroups, the target
+                    // is raised so that the entries splitting adds (at most nominal / target per item) go to the
+                    // workgroups that would have had no item
+                    const uint32_t spare = gridDim.x - items;
+                    const uint32_t fit = (steps - 3u * items + spare - 1u) / spare;
+                    target = target < fit ? fit : target;
+                }
+                // a caller may bring room for fewer partial outputs than the split would use: coarser parts until they fit (none at
+                // last: a target beyond every item splits nothing)
+                for (;;) {
+                    uint32_t bufs = 0;
+#pragma unroll
+                    for (int i = 0; i < kTrips; ++i) {
+                        const uint32_t m = parts_of(i);
+                        bufs += m > 1u ? cnt[i] * m : 0u;
+                    }
+                    if (lane_sum(bufs) <= a.ws_parts || target >= 0x3fffffffu) {
+                        break;
+                    }
+                    target = target < 0x10000u ? target * 2u : 0x3fffffffu;
+                }
+                uint32_t first = 0, first_item = 0, first_buf = 0;
 #pragma unroll
                 for (int i = 0; i < kTrips; ++i) {
+                    const int l = 64 * i + lane;
+                    if (64 * i > n_levels) {
+                        break;
+                    }
                     const uint32_t m = parts_of(i);
-                    bufs += m > 1u ? cnt[i] * m : 0u;
+                    const uint32_t split = m > 1u ? cnt[i] : 0u;
+                    const uint32_t at = up_to_lane(cnt[i] * m);
+                    const uint32_t item_at = up_to_lane(split);
+                    const uint32_t buf_at = up_to_lane(split * m);
+                    if (l <= n_levels) {  // (past the last level every count is zero: its start is the end of the list)
+                        s_queue_start[0][l] = first + at - cnt[i] * m;
+                        s_parts[l] = static_cast<uint8_t>(m);
+                        s_split_first[l] = first_item + item_at - split;
+                        s_ws_first[l] = first_buf + buf_at - split * m;
+                    }
+                    first += last_lane(at);
+                    first_item += last_lane(item_at);
+                    first_buf += last_lane(buf_at);
                 }
-                if (lane_sum(bufs) <= a.ws_parts || target >= 0x3fffffffu) {
-                    break;
-                }
-                target = target < 0x10000u ? target * 2u : 0x3fffffffu;
-            }
-            uint32_t first = 0, first_item = 0, first_buf = 0;
-#pragma unroll
-            for (int i = 0; i < kTrips; ++i) {
-                const int l = 64 * i + lane;
-                if (64 * i > n_levels) {
-                    break;
-                }
-                const uint32_t m = parts_of(i);
-                const uint32_t split = m > 1u ? cnt[i] : 0u;
-                const uint32_t at = up_to_lane(cnt[i] * m);
-                const uint32_t item_at = up_to_lane(split);
-                const uint32_t buf_at = up_to_lane(split * m);
-                if (l <= n_levels) {  // (past the last level every count is zero: its start is the end of the list)
-                    s_queue_start[0][l] = first + at - cnt[i] * m;
-                    s_parts[l] = static_cast<uint8_t>(m);
-                    s_split_first[l] = first_item + item_at - split;
-                    s_ws_first[l] = first_buf + buf_at - split * m;
-                }
-                first += last_lane(at);
-                first_item += last_lane(item_at);
-                first_buf += last_lane(buf_at);
             }
         }
-    }
-    __syncthreads();
-    // Stable scatter (sequences of one bucket stay in index order) by wavefront 0 alone: every workgroup
-    // must arrive at the very same list, which an order-of-arrival scatter over four wavefronts would
-    // not give.  64 sequences per trip; lanes holding the same tile count are ranked with a ballot.
-    // (the cursors of all 64 sequences of a trip are read in one go before the loop over the distinct tile counts
-    // among them, which then runs on ballots alone: no LDS round trip per distinct count)
-    if (wave == 0) {
-        for (int base = 0; base < a.n_batch; base += 64) {
-            const int b = base + lane;
-            const bool valid = b < a.n_batch;
-            const int key = valid ? static_cast<int>(s_ntiles[valid ? b : 0]) : -1;
-            const uint32_t start = s_bucket[valid ? key : 0];
-            uint32_t before = 0;
-            uint64_t todo = __builtin_amdgcn_ballot_w64(valid);
-            while (todo != 0) {
-                const int leader = __builtin_ctzll(todo);
-                const int k0 = __builtin_amdgcn_readlane(key, leader);
-                const bool mine = valid && key == k0;
-                const uint64_t same = __builtin_amdgcn_ballot_w64(mine);
-                if (mine) {
-                    before = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+        __syncthreads();
+        // Stable scatter (sequences of one bucket stay in index order) by wavefront 0 alone: every workgroup
+        // must arrive at the very same list, which an order-of-arrival scatter over four wavefronts would
+        // not give.  64 sequences per trip; lanes holding the same tile count are ranked with a ballot.
+        // (the cursors of all 64 sequences of a trip are read in one go before the loop over the distinct tile counts
+        // among them, which then runs on ballots alone: no LDS round trip per distinct count)
+        if (wave == 0) {
+            for (int base = 0; base < a.n_batch; base += 64) {
+                const int b = base + lane;
+                const bool valid = b < a.n_batch;
+                const int key = valid ? static_cast<int>(s_ntiles[valid ? b : 0]) : -1;
+                const uint32_t start = s_bucket[valid ? key : 0];
+                uint32_t before = 0;
+                uint64_t todo = __builtin_amdgcn_ballot_w64(valid);
+                while (todo != 0) {
+                    const int leader = __builtin_ctzll(todo);
+                    const int k0 = __builtin_amdgcn_readlane(key, leader);
+                    const bool mine = valid && key == k0;
+                    const uint64_t same = __builtin_amdgcn_ballot_w64(mine);
+                    if (mine) {
+                        before = __builtin_popcountll(same & ((1ull << lane) - 1ull));
+                    }
+                    if (lane == leader) {
+                        s_bucket[k0] = start + static_cast<uint32_t>(__builtin_popcountll(same));
+                    }
+                    todo &= ~same;
                 }
-                if (lane == leader) {
-                    s_bucket[k0] = start + static_cast<uint32_t>(__builtin_popcountll(same));
+                if (valid) {
+                    s_order[start + before] = static_cast<uint16_t>(b);
                 }
-                todo &= ~same;
-            }
-            if (valid) {
-                s_order[start + before] = static_cast<uint16_t>(b);
             }
         }
+        __syncthreads();
+
     }
-    __syncthreads();
 
     // ---- per-lane constants that do not depend on the item ----
     const uint32_t q_stride = static_cast<uint32_t>(a.n_heads_q) * a.d_qk * ES;  // bytes per row
@@ -993,7 +1005,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     // gives such a short list as well (measured equal on MI355X), without the counter's round trip, without device
     // state shared between launches, and with the next item known in advance: wavefront 0 decodes it, offsets
     // included, while the tile requests of the current item are under way, and leaves it in LDS for the others.
-    constexpr bool kStaticList = !QUEUES;
+    constexpr bool kStaticList = !QUEUES && !DIRECT;
     auto decode_ahead = [&](int round) {  // executed by wavefront 0; fills s_next[round & 1]
         uint32_t(&rec)[20] = s_next[kStaticList ? (round & 1) : 0];
         const uint32_t g = gridDim.x;
@@ -1071,7 +1083,33 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         int64_t q0, q1, k0, k1;
         int n_ctx = 0;
         int n_tgt = 0;
-        if constexpr (kStaticList) {
+        if constexpr (DIRECT) {
+            const int pairs_pad = (a.n_batch * a.n_heads_k + 7) & ~7;
+            const int per_level = pairs_pad * a.head_ratio;
+            const int lvl = static_cast<int>(blockIdx.x) / per_level;
+            const int rest = static_cast<int>(blockIdx.x) - lvl * per_level;
+            const int in_group = rest / pairs_pad;
+            const int pair = rest - in_group * pairs_pad;
+            if (pair >= a.n_batch * a.n_heads_k) {
+                break;
+            }
+            qt = tile_of_level(lvl);
+            b = pair / a.n_heads_k;
+            hk = pair - b * a.n_heads_k;
+            h = hk * a.head_ratio + in_group;
+            q0 = load_index_uniform(a.offs_q, b, a.idx64);
+            q1 = load_index_uniform(a.offs_q, b + 1, a.idx64);
+            k0 = load_index_uniform(a.offs_k, b, a.idx64);
+            k1 = load_index_uniform(a.offs_k, b + 1, a.idx64);
+            if (a.mask_type == 0) {
+                if (a.num_ctx) {
+                    n_ctx = static_cast<int>(load_index_uniform(a.num_ctx, b, a.idx64));
+                }
+                if (a.num_tgt) {
+                    n_tgt = static_cast<int>(load_index_uniform(a.num_tgt, b, a.idx64));
+                }
+            }
+        } else if constexpr (kStaticList) {
             const uint32_t(&rec)[20] = s_next[kStaticList ? (round & 1) : 0];
             if (rec[0] == 0) {
                 break;
@@ -1124,6 +1162,11 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         sk = sk < a.max_k ? sk : a.max_k;
 
         const int r0 = qt * kBlockM;  // < sq by construction of the work list
+        if constexpr (DIRECT) {
+            if (r0 >= sq) {
+                break;
+            }
+        }
         const int wr0 = r0 + wave * kWaveM;
         const bool wave_active = wr0 < sq;  // inactive wavefronts still take part in loads and barriers
 
@@ -2175,6 +2218,9 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         if constexpr (kStaticList) {
             ++round;
             __syncthreads();  // every wavefront has read its staged rows back before the next requests write the slots
+        }
+        if constexpr (DIRECT) {
+            break;
         }
     }
 

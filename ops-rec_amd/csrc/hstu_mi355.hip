@@ -398,6 +398,27 @@ int wgs_per_cu(const Variant* var, const hstu_jagged_fwd_params* p)
     return var->persistent_wgs_per_cu;
 }
 
+// slots of a launch without a list: pairs padded to a multiple of 8 (hstu_fwd_kernel.hip.h)
+int64_t direct_slots(const hstu_jagged_fwd_params* p)
+{
+    const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
+    const int64_t pairs_pad = ((p->n_offsets - 1) * p->num_heads_k + 7) & ~int64_t{7};
+    return n_qtiles * pairs_pad * (p->num_heads_q / p->num_heads_k);
+}
+
+// Whether a plain launch does without a list, a workgroup per slot: when every slot is resident at once, and, up to the head-dim
+// slot 128, on sweeps of at most 384 keys (a list long enough for the queues takes those).  Measured, list -> slots: one slot
+// per resident workgroup at most -- 7 x 2 heads, d 64, 148 rows 10.8 -> 9.3 us, 4 x 8, d 192, 96 x 121 15.9 -> 14.2, 43 x 1, d 192,
+// 456 rows 26.8 -> 24.7, 10 x 1, d 32, 1487..2975 rows 43.1 -> 38.7; more of them on short sweeps -- 103 x 4, d 64, 142 rows 23.1 ->
+// 17.9, fp8 248 x 4, 27..64 rows 21.0 -> 19.9, 150 x 4, d 64, 100..384 rows 33.0 -> 30.2, with a bias 300 x 2, d 64, 231..299 rows 77.7 ->
+// 71.0; but 16 x 4 with a bias of 512..2048 rows 77 -> 88, d 256: 16 x 4 of 200..1000 42.5 -> 47.6 and 150 x 2 of 100..384 55 -> 67, and
+// lists of four slots per workgroup and more lose to the queues from 200 rows on (600 x 4 of 50..380 90.9 -> 97.5).
+bool takes_direct_list(const Variant* var, const hstu_jagged_fwd_params* p, int64_t resident)
+{
+    const int64_t slots = direct_slots(p);
+    return slots <= resident || (var->d_pad <= 128 && p->max_seq_len_k <= 384 && slots < 4 * resident);
+}
+
 // whether the launch described by p takes the variant with per-XCD work queues: only when the list may hold
 // several items per resident workgroup.  *resident_out (optional) receives the resident grid.
 bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, int64_t* resident_out)
@@ -1554,6 +1575,10 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         if (paged != nullptr) {
             kernel = var->kernel_paged;  // (splits when it was given room above, otherwise not; the caller checked the block)
             a.counters = static_cast<unsigned int*>(workspace);
+        }
+        if (a.counters == nullptr && takes_direct_list(var, p, static_cast<int64_t>(cus) * wgs_per_cu(var, p))) {
+            kernel = var->kernel_direct;
+            n_blocks = direct_slots(p);
         }
         if (kernel == var->kernel_queues) {
             launch_clear(a.counters, hstu::kQueueCounterBytes, stream);

@@ -20,6 +20,7 @@ struct Variant {
     int d_pad;
     int threads;
     int persistent_wgs_per_cu;  // > 0: persistent kernel, this many workgroups per CU; 0: one workgroup per tile
+    void (*kernel_direct)(const FwdArgs);  // the persistent kernel without a list, a workgroup per slot, for the shortest lists
 };
 
 // the forward kernel for short work lists (hstu_fwd_short_kernel.hip.h): one workgroup of `threads` per
