@@ -575,15 +575,15 @@ struct JaggedFunction : torch::autograd::Function<JaggedFunction<DELTA>> {
 template <bool DELTA>
 Tensor with_autograd(const Call& c, bool deterministic)
 {
-    if (needs_grad(c.mask)) {
-        TORCH_CHECK_NOT_IMPLEMENTED(false, DELTA ? "hstu_jagged.delta" : "hstu_jagged.equal",
-                                    ": mask is a non-differentiable input (the backward op returns no mask gradient); "
-                                    "do not pass a mask with requires_grad=True");
-    }
-    if (!at::GradMode::is_enabled() || !(needs_grad(c.q) || needs_grad(c.k) || needs_grad(c.v) || needs_grad(c.bias))) {
+    if (!at::GradMode::is_enabled() ||
+        !(needs_grad(c.q) || needs_grad(c.k) || needs_grad(c.v) || needs_grad(c.bias) || needs_grad(c.mask))) {
         const at::AutoDispatchBelowADInplaceOrView below;
         return call_forward<DELTA>(c, deterministic);
     }
+    // (only a call that records a gradient is refused: under no_grad the mask is an input like any other)
+    TORCH_CHECK_NOT_IMPLEMENTED(!needs_grad(c.mask), DELTA ? "hstu_jagged.delta" : "hstu_jagged.equal",
+                                ": mask is a non-differentiable input (the backward op returns no mask gradient); "
+                                "do not pass a mask with requires_grad=True");
     return JaggedFunction<DELTA>::apply(c.q, c.k, c.v, c.bias, &c, deterministic);
 }
 
