@@ -240,8 +240,8 @@ __global__ __launch_bounds__(f32_waves(D) * 64) void hstu_fwd_f32_kernel(const F
                 }
             }
             // P^T = S^T * sigmoid(alpha * S^T), masked
-            // (the conditions are combined without branches: where a branch stands between the last MFMA and the first read of its
-            // result, this compiler counts the instructions of the longer way round as wait states, and the read came too early)
+            // (the conditions are combined without branches: the products and the first use of S stay one basic block, in which the
+            // element-wise stage can be scheduled; the compiler's wait states are right either way)
             const bool hole = wb.any_hole & (c0 + 16 > hist_k) & (c0 < wb.hole_hi_max);
             const bool full = !HAS_MASK & (c0 + 16 <= wb.lim_min) & !hole;
 #pragma unroll

@@ -428,8 +428,7 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
                     tt = __builtin_amdgcn_rcpf(1.0f + tt);
                     p[e] = s * tt;
                 }
-                // (combined without branches: where a branch stands between the last MFMA and the first read of its result, this compiler counts
-                // the instructions of the longer way round as wait states, and the shorter way may read too early)
+                // (combined without branches: the block's class costs a few scalar instructions instead of a chain of jumps)
                 const bool full = (c0 + 32 <= wb.lim_min) & !(wb.any_hole & (c0 + 32 > hist_k) & (c0 < wb.hole_hi_max));
                 if (!full) {
 #pragma unroll

@@ -264,8 +264,7 @@ __global__ __launch_bounds__(256, 1) void hstu_fwd_wide_kernel(const FwdArgs a)
                 }
             }
             // P^T = S^T * sigmoid(alpha * S^T), masked
-            // (combined without branches: where a branch stands between the last MFMA and the first read of its result, this compiler counts
-            // the instructions of the longer way round as wait states, and the shorter way may read too early)
+            // (combined without branches: the block's class costs a few scalar instructions instead of a chain of jumps)
             const bool full = !HAS_MASK & (c0 + 32 <= wb.lim_min) & !(wb.any_hole & (c0 + 32 > hist_k) & (c0 < wb.hole_hi_max));
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
