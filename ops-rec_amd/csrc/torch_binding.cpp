@@ -7,7 +7,9 @@
 // Every other call (something to convert, an argument to refuse, an empty output) goes to the Python implementation, which
 // holds the checks, their messages and the conversions; so nothing is accepted or refused here that is not there.
 
+#include <ATen/Context.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/native/TensorFactories.h>
 #include <ATen/ops/mm.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/DeviceGuard.h>
@@ -65,9 +67,16 @@ int dtype_code(at::ScalarType t)
     }
 }
 
+// torch.empty without its way through the dispatcher: memory nobody has written yet holds NaN (all ones) when the program has asked
+// for that (torch.use_deterministic_algorithms with torch.utils.deterministic.fill_uninitialized_memory)
 Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const at::Device& device)
 {
-    return Tensor(at::detail::empty_cuda(size, dtype, device, std::nullopt));
+    Tensor t(at::detail::empty_cuda(size, dtype, device, std::nullopt));
+    const at::Context& context = at::globalContext();
+    if (context.deterministicAlgorithms() && context.deterministicFillUninitializedMemory()) {
+        at::native::fill_empty_deterministic_(t);
+    }
+    return t;
 }
 
 void* ptr(const Tensor& t) { return t.defined() && t.numel() != 0 ? t.data_ptr() : nullptr; }

@@ -89,3 +89,20 @@ def test_ln_mul(python_only):
     step = lambda: (torch.ops.ops_rec.ln_mul(x, u, g, b), torch.ops.ops_rec.ln_mul(x.t().contiguous().t(), u, g, b))  # noqa: E731
     same(step(), python_only(step))
     same(step()[:1], (_activation.ln_mul(x, u, g, b),))
+
+
+def test_memory_that_nobody_writes_is_filled_when_the_program_asks_for_it():
+    """``torch.use_deterministic_algorithms`` has torch hand out new tensors full of NaN; what the native side allocates is no
+    exception.  (Rows ahead of a non-zero first offset belong to no work item.)"""
+    w = small_case(seed=4, batch=2, dim=64, lo=20, hi=60, dtype=torch.bfloat16).to(DEV)
+    q, k, v = (torch.cat([torch.ones_like(t[:3]), t]) for t in (w.q, w.k, w.v))
+    offs = w.seq_offset + 3
+    call = lambda: torch.ops.ops_rec.hstu_jagged.equal(q, k, v, None, None, 0, w.max_seq_len, 0.0, offs)  # noqa: E731
+    want = call()
+    torch.zeros_like(want)  # (what the allocator hands out next holds zeros)
+    torch.use_deterministic_algorithms(True, warn_only=True)
+    try:
+        out = call()
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert out[:3].isnan().all() and torch.equal(out[3:], want[3:])
