@@ -18,7 +18,6 @@
 #include <torch/csrc/utils/pybind.h>
 #include <torch/library.h>
 
-#include <atomic>
 #include <cstring>
 #include <optional>
 #include <tuple>
@@ -44,9 +43,6 @@ struct Fallbacks {
     PyObject* in_linear_silu = nullptr;   // _activation.distance_in_linear_silu
     PyObject* in_linear_silu_backward = nullptr;
 } fallbacks;
-
-// false: every call goes to Python (something there has been replaced: its allocators are seams)
-std::atomic<bool> native_enabled{true};
 
 template <typename R, typename... A>
 R in_python(PyObject* fn, const A&... args)
@@ -203,16 +199,14 @@ Tensor launch_forward(hstu_jagged_fwd_params& p, const Tensor& q, at::ScalarType
 
 Tensor forward(const Call& c, bool deterministic)
 {
-    if (native_enabled.load(std::memory_order_relaxed)) {
-        hstu_jagged_fwd_params p;
-        if (describe(c, p)) {
-            const bool fp8 = p.dtype == HSTU_DT_FP8_E4M3;
-            p.deterministic = deterministic ? 1 : 0;
-            p.fp8_scaled_p = fp8 ? 1 : 0;  // e4m3 tensors through the reference's entry point: its rounding point of P
-            Tensor out = launch_forward(p, c.q, fp8 ? at::kHalf : c.q.scalar_type());
-            if (out.defined()) {
-                return out;
-            }
+    hstu_jagged_fwd_params p;
+    if (describe(c, p)) {
+        const bool fp8 = p.dtype == HSTU_DT_FP8_E4M3;
+        p.deterministic = deterministic ? 1 : 0;
+        p.fp8_scaled_p = fp8 ? 1 : 0;  // e4m3 tensors through the reference's entry point: its rounding point of P
+        Tensor out = launch_forward(p, c.q, fp8 ? at::kHalf : c.q.scalar_type());
+        if (out.defined()) {
+            return out;
         }
     }
     return in_python<Tensor>(fallbacks.forward, c.q, c.k, c.v, c.mask, c.bias, c.mask_type, c.max_q, c.max_k, c.silu_scale, c.offs_q, c.offs_k,
@@ -228,7 +222,7 @@ Gradients backward(const Tensor& grad_in, const Call& c)
     // (a gradient may come as an expanded view: from a sum, for instance)
     const Tensor grad = grad_in.defined() && !grad_in.is_contiguous() ? grad_in.contiguous() : grad_in;
     hstu_jagged_bwd_params p;
-    if (native_enabled.load(std::memory_order_relaxed) && dtype != at::kFloat8_e4m3fn && is_set(c.ctx) == is_set(c.tgt) && grad.defined() &&
+    if (dtype != at::kFloat8_e4m3fn && is_set(c.ctx) == is_set(c.tgt) && grad.defined() &&
         describe(c, p.fwd) && grad.dim() == 3 && grad.scalar_type() == dtype && grad.device() == q.device() && grad.size(0) == q.size(0) &&
         grad.size(1) == q.size(1) && grad.size(2) == c.v.size(2) && (q.numel() != 0 || c.k.numel() != 0)) {
         const c10::DeviceGuard guard(q.device());
@@ -307,8 +301,7 @@ OptTensor fp8_forward(const Tensor& q, const Tensor& k, const Tensor& v, const O
                       const OptTensor& tgt, std::optional<int64_t> group, std::optional<double> alpha, bool half_out)
 {
     hstu_jagged_fwd_params p;
-    if (!native_enabled.load(std::memory_order_relaxed) ||
-        !describe({q, k, v, mask, bias, mask_type, max_seq_len, max_seq_len_k, silu_scale, offs, offs_k, ctx, tgt, group, alpha}, p) ||
+    if (!describe({q, k, v, mask, bias, mask_type, max_seq_len, max_seq_len_k, silu_scale, offs, offs_k, ctx, tgt, group, alpha}, p) ||
         p.dtype != HSTU_DT_FP8_E4M3 || !absent_or_vector(q_descale, at::kFloat, q.size(1), q.device()) ||
         !absent_or_vector(k_descale, at::kFloat, k.size(1), q.device()) || !absent_or_vector(v_descale, at::kFloat, k.size(1), q.device())) {
         return std::nullopt;
@@ -328,7 +321,7 @@ Tensor paged(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& ca
 {
     hstu_paged_fwd_params p;
     const OptTensor tgt = num_target.defined() ? OptTensor(num_target) : std::nullopt;
-    if (native_enabled.load(std::memory_order_relaxed) && cache.defined() && page_ids.defined() && last_page_len.defined() && offs_t.defined() &&
+    if (cache.defined() && page_ids.defined() && last_page_len.defined() && offs_t.defined() &&
         page_offsets.defined() && describe({q, k, v, mask, bias, mask_type, max_seq_len, max_seq_len_k, silu_scale, offs, offs_k, std::nullopt, tgt, group, alpha}, p.fwd)) {
         const at::ScalarType index = offs.scalar_type();
         const auto vector = [&](const Tensor& t) {
@@ -375,7 +368,7 @@ Tensor ln_mul(const Tensor& x, const Tensor& u, const Tensor& gamma, const Tenso
 {
     const at::ScalarType dtype = x.scalar_type(), affine = gamma.scalar_type();
     const at::Device device = x.device();
-    if (native_enabled.load(std::memory_order_relaxed) && device.is_cuda() && x.dim() == 2 && u.dim() == 2 && gamma.dim() == 1 && beta.dim() == 1 &&
+    if (device.is_cuda() && x.dim() == 2 && u.dim() == 2 && gamma.dim() == 1 && beta.dim() == 1 &&
         x.numel() != 0 && x.sizes() == u.sizes() && (dtype == at::kFloat || dtype == at::kBFloat16 || dtype == at::kHalf) && u.scalar_type() == dtype &&
         beta.scalar_type() == affine && (affine == at::kFloat || affine == dtype) && gamma.size(0) == x.size(1) && beta.size(0) == x.size(1) &&
         u.device() == device && gamma.device() == device && beta.device() == device && x.is_contiguous() && u.is_contiguous() &&
@@ -428,7 +421,7 @@ using Projection = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>;
 Projection in_linear_silu(const Tensor& x, const Tensor& weight, const Tensor& bias_in, at::IntArrayRef split)
 {
     const OptTensor bias = bias_in.defined() ? OptTensor(bias_in) : std::nullopt;
-    if (native_enabled.load(std::memory_order_relaxed) && in_linear_silu_canonical(x, weight, bias, split)) {
+    if (in_linear_silu_canonical(x, weight, bias, split)) {
         const c10::DeviceGuard guard(x.device());
         const int64_t m = x.size(0), n = weight.size(0);
         const auto rows = [&](int64_t cols) { return empty({m, cols}, x.scalar_type(), x.device()); };
@@ -462,7 +455,7 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
                                   const Tensor& query_grad, const Tensor& key_grad, const Tensor& linear_output, at::IntArrayRef split)
 {
     const Tensor* const grads[4] = {&user_grad, &value_grad, &query_grad, &key_grad};
-    bool ok = native_enabled.load(std::memory_order_relaxed) && in_linear_silu_canonical(x, weight, bias, split) && linear_output.dim() == 2 &&
+    bool ok = in_linear_silu_canonical(x, weight, bias, split) && linear_output.dim() == 2 &&
               linear_output.size(0) == x.size(0) && linear_output.size(1) == weight.size(0) && linear_output.scalar_type() == x.scalar_type() &&
               linear_output.device() == x.device() && linear_output.is_contiguous();
     for (int i = 0; ok && i < 4; ++i) {
@@ -690,6 +683,5 @@ PYBIND11_MODULE(_torch_binding, m)
         fallbacks.in_linear_silu = projection.release().ptr();
         fallbacks.in_linear_silu_backward = projection_backward.release().ptr();
     });
-    m.def("set_native", [](bool on) { native_enabled.store(on, std::memory_order_relaxed); });
     m.def("fp8_forward", &fp8_forward, py::call_guard<py::gil_scoped_release>());
 }

@@ -23,7 +23,7 @@ import torch
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), ".."))
 import ops_rec  # noqa: E402
-from ops_rec import _native, _ops, workloads  # noqa: E402
+from ops_rec import _native, workloads  # noqa: E402
 
 # the shapes the rule's constants were fitted on
 FIT = [
@@ -75,6 +75,15 @@ def time_us(fn, launches):
     return best
 
 
+def workspace_bytes(fn):
+    """What a call asks torch's allocator for at its peak beside what it returns."""
+    torch.cuda.reset_peak_memory_stats()
+    out = fn()
+    stats = torch.cuda.memory_stats()
+    del out
+    return stats["requested_bytes.all.peak"] - stats["requested_bytes.all.current"]
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--set", default="heldout", choices=["heldout", "fit", "bias"])
@@ -85,9 +94,6 @@ def main():
     ap.add_argument("--only", choices=sorted(NAMES.values()), help="run this launch order only and print its time")
     args = ap.parse_args()
     bwd = ops_rec.ascendc.attention.hstu_jagged_backward
-    asked = []
-    new_workspace = _ops._new_workspace
-    _ops._new_workspace = lambda n, dev: (asked.append(n), new_workspace(n, dev))[1]
     print("| batch, heads (K/V), head dim, lengths, mask | two us | three us | planes us | rule | rule / best |")
     print("|---|---|---|---|---|---|")
     worst, within = 0.0, 0
@@ -116,14 +122,14 @@ def main():
             else:
                 os.environ["HSTU_MI355_BWD_HANDOFF"] = order
             _native.reload_switches()
-            del asked[:]
             times[order] = time_us(lambda: bwd(*call), args.launches)
             if order is None:
+                asked = workspace_bytes(lambda: bwd(*call))
                 dense = batch * heads * max_len * max_len * 2
                 if rab is None:
-                    pick = "two" if asked[-1] == 0 else ("three" if asked[-1] == dense else "planes")
+                    pick = "two" if asked == 0 else ("three" if asked == dense else "planes")
                 else:  # (two and three both run without a workspace: told apart by their times below)
-                    pick = "planes" if asked[-1] else None
+                    pick = "planes" if asked else None
         # (a forced order falls back to another when its workspace is over the limit: its time is then that order's)
         best = min(times[o] for o in ("0", "1", "2"))
         if pick is None:

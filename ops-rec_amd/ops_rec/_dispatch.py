@@ -10,22 +10,10 @@ from __future__ import annotations
 import importlib.machinery
 import importlib.util
 import os
-import sys
-import types
 
 from . import _activation, _build, _ops
 
 binding = None
-# the allocators of the Python implementations: replacing one of them (to look at, or to spoil, what a call allocates) sends every
-# call through Python until it is put back
-_SEAMS = {name: getattr(_ops, name) for name in ("_new_workspace", "_new_grad")}
-
-
-class _OpsModule(types.ModuleType):
-    def __setattr__(self, name, value):
-        super().__setattr__(name, value)
-        if name in _SEAMS and binding is not None:
-            binding.set_native(all(getattr(self, n) is f for n, f in _SEAMS.items()))
 
 
 def attach() -> None:
@@ -43,7 +31,6 @@ def attach() -> None:
                          _activation.distance_in_linear_silu, _activation.in_linear_silu_backward)  # fmt: skip
     _ops._fp8_native = module.fp8_forward
     binding = module
-    sys.modules[_ops.__name__].__class__ = _OpsModule
 
 
 attach()

@@ -36,7 +36,11 @@ def _switches_follow_the_environment():
     holding that value; once the test's environment has been put back (this fixture is set up first, so it is torn
     down last) the library reads its switches again."""
     yield
+    import torch
+
     from ops_rec import _native
+
+    torch.use_deterministic_algorithms(False)  # (helpers.poison_workspace)
 
     if _native._lib is not None:
         _native.reload_switches()

@@ -22,29 +22,61 @@ def set_switch(monkeypatch, name, value):
 
 
 def poison_workspace(monkeypatch):
-    """The backward's workspace is handed out holding NaN in every element, so that a read of something never
-    written shows in the gradients.  Returns the list to which the sizes asked for are appended."""
+    """Everything the operators allocate from here on -- the backward's workspace, outputs, gradients -- is handed out holding
+    NaN in every element, so that a read of something never written, or an element of a result that nobody wrote, shows: torch's
+    own setting, which the native kernels follow.  (``tests/conftest.py`` switches it off again.)"""
+    monkeypatch.setattr(torch.utils.deterministic, "fill_uninitialized_memory", True)
+    torch.use_deterministic_algorithms(True, warn_only=True)
+
+
+def allocated_beside(call):
+    """``call()``, and how many bytes it had asked torch's allocator for at its peak beside what it returned: the workspace of an
+    operator whose arguments are taken as they are."""
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    out = call()
+    stats = torch.cuda.memory_stats()
+    return out, stats["requested_bytes.all.peak"] - stats["requested_bytes.all.current"]
+
+
+def with_room_for(call, n_bytes, like):
+    """``call()`` while torch's allocator may take no more than ``n_bytes`` from the device beyond free blocks of the sizes in
+    ``like`` (its results), and how many requests it refused."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    blocks = [torch.empty_like(t) for t in like if t is not None]
+    del blocks
+    total = torch.cuda.get_device_properties(0).total_memory
+    before = torch.cuda.memory_stats()["num_ooms"]
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + n_bytes) / total)
+    try:
+        out = call()
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    return out, torch.cuda.memory_stats()["num_ooms"] - before
+
+
+def backward_args(w, grad):
+    """The arguments of ``hstu_jagged_backward`` (its longer form) for a workload."""
+    k_offs = w.seq_offset if w.seq_offset_k is None else w.seq_offset_k
+    max_k = w.max_seq_len if w.max_seq_len_k is None else w.max_seq_len_k
+    ctx, tgt = w.num_context, w.num_target
+    if (ctx is None) != (tgt is None):  # the backward op wants both or neither (hstu_jagged_plugin.cpp:81-84)
+        zeros = torch.zeros_like(ctx if tgt is None else tgt)
+        ctx, tgt = (zeros if ctx is None else ctx), (zeros if tgt is None else tgt)
+    return (grad, w.q, w.k, w.v, w.mask, w.attn_bias, w.mask_type, w.max_seq_len, max_k, w.silu_scale, w.seq_offset, k_offs, ctx, tgt,
+            w.target_group_size, w.alpha)  # fmt: skip
+
+
+def backward_without_workspace(monkeypatch, w, grad):
+    """The gradients from a caller that brings no workspace, whatever the library asks for: through the Python implementation,
+    whose allocations can be replaced."""
     from ops_rec import _ops
 
-    plain = _ops._new_workspace
-    asked = []
-
-    def poisoned(n_bytes, device):
-        asked.append(n_bytes)
-        ws = plain(n_bytes, device)
-        if ws is not None:
-            ws.fill_(0xFF)
-        return ws
-
-    monkeypatch.setattr(_ops, "_new_workspace", poisoned)
-    return asked
-
-
-def withhold_workspace(monkeypatch):
-    """The backward gets no workspace, as when the device has no room for it: the call must work without."""
-    from ops_rec import _ops
-
-    monkeypatch.setattr(_ops, "_new_workspace", lambda n_bytes, device: None)
+    with monkeypatch.context() as patch:
+        patch.setattr(_ops, "_new_workspace", lambda n_bytes, device: None)
+        return _ops.hstu_jagged_backward_delta(*backward_args(w, grad))
 
 
 def small_case(seed=0, batch=3, heads=2, dim=32, lo=1, hi=40, dtype=torch.float32, std=1.0, rab=False, custom_mask=False,

@@ -38,15 +38,7 @@ def oracle_grads(w, grad_out):
 
 
 def device_grads(w, grad_out):
-    k_offs = w.seq_offset if w.seq_offset_k is None else w.seq_offset_k
-    max_k = w.max_seq_len if w.max_seq_len_k is None else w.max_seq_len_k
-    ctx, tgt = w.num_context, w.num_target
-    if (ctx is None) != (tgt is None):  # the backward op wants both or neither (hstu_jagged_plugin.cpp:81-84)
-        zeros = torch.zeros_like(ctx if tgt is None else tgt)
-        ctx, tgt = (zeros if ctx is None else ctx), (zeros if tgt is None else tgt)
-    got = ops_rec.ascendc.attention.hstu_jagged_backward(
-        grad_out, w.q, w.k, w.v, w.mask, w.attn_bias, w.mask_type, w.max_seq_len, max_k, w.silu_scale, w.seq_offset,
-        k_offs, ctx, tgt, w.target_group_size, w.alpha)  # fmt: skip
+    got = ops_rec.ascendc.attention.hstu_jagged_backward(*helpers.backward_args(w, grad_out))
     torch.cuda.synchronize()
     return got
 
@@ -188,8 +180,7 @@ def test_ds_handed_to_the_dk_workgroups_through_a_workspace(kw, mask, monkeypatc
             scale = two[i].float().abs().max().item()
             torch.testing.assert_close(other[i].float(), two[i].float(), atol=tol * scale, rtol=tol)
         # a caller that does not bring the workspace the library asked for gets the two-launch order
-        helpers.withhold_workspace(monkeypatch)
-        without = device_grads(w, grad_out)
+        without = helpers.backward_without_workspace(monkeypatch, w, grad_out)
         assert all(torch.equal(x, y) for x, y in zip(two[:3], without[:3]))
 
 
@@ -205,19 +196,13 @@ def test_planes_with_a_max_seq_len_that_is_not_a_multiple_of_8(kw, mask_type, mo
     workspace, and the gradients come out right with it full of NaN.  (Rows of [max_q][max_k] tensors start at multiples
     of 16 bytes only when max_seq_len_k is a multiple of 8: with such a tensor in the call the same shapes run in two
     launches, or on the generic kernels.)"""
-    from ops_rec import _ops
-
     kw = dict(kw)
     w = dataclasses.replace(make(batch=3, heads=kw.pop("heads", 2), seed=77, **kw), mask_type=mask_type)
-    asked = []
-    plain = _ops._new_workspace
-    monkeypatch.setattr(_ops, "_new_workspace", lambda n, dev: (asked.append(n), plain(n, dev))[1])
     helpers.set_switch(monkeypatch, "HSTU_MI355_GENERIC_BACKWARD", "0")
     helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "2")
     g = torch.Generator(device=DEV).manual_seed(6)
     grad_out = torch.randn(w.q.shape[0], w.q.shape[1], w.v.shape[2], generator=g, device=DEV).to(w.q.dtype)
-    device_grads(w, grad_out)
-    assert asked and asked[-1] > 0  # the planes (and, for the windows, the partial scores)
+    assert helpers.allocated_beside(lambda: device_grads(w, grad_out))[1] > 0  # the planes (and, for the windows, the partial scores)
     check(w, monkeypatch)  # with the workspace full of NaN, against the oracle and the generic kernels
 
 

@@ -25,13 +25,7 @@ DEV = "cuda:0"
 
 
 def backward(w, grad_out):
-    ctx, tgt = w.num_context, w.num_target
-    if (ctx is None) != (tgt is None):  # the backward op wants both or neither (hstu_jagged_plugin.cpp:81-84)
-        zeros = torch.zeros_like(ctx if tgt is None else tgt)
-        ctx, tgt = (zeros if ctx is None else ctx), (zeros if tgt is None else tgt)
-    got = ops_rec.ascendc.attention.hstu_jagged_backward(
-        grad_out, w.q, w.k, w.v, w.mask, w.attn_bias, w.mask_type, w.max_seq_len, w.max_seq_len, w.silu_scale,
-        w.seq_offset, w.seq_offset, ctx, tgt, w.target_group_size, w.alpha)  # fmt: skip
+    got = ops_rec.ascendc.attention.hstu_jagged_backward(*helpers.backward_args(w, grad_out))
     torch.cuda.synchronize()
     return got
 
@@ -114,10 +108,10 @@ def test_planes_beyond_4_gib_agree_with_the_two_launch_order(monkeypatch):
     grad_out = torch.randn(w.q.shape, generator=g, device=DEV).to(torch.bfloat16)
     helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "0")
     two = backward(w, grad_out)
-    asked = helpers.poison_workspace(monkeypatch)
+    helpers.poison_workspace(monkeypatch)
     helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "2")
-    planes = backward(w, grad_out)
-    assert asked and asked[-1] > (4 << 30), asked
+    planes, workspace = helpers.allocated_beside(lambda: backward(w, grad_out))
+    assert workspace > (4 << 30), workspace
     assert torch.equal(two[0], planes[0])
     for i in (1, 2):
         assert torch.isfinite(planes[i].float()).all()

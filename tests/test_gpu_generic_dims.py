@@ -95,8 +95,16 @@ def test_rows_past_the_last_offset_are_zero_and_empty_sequences_cost_nothing():
     assert torch.count_nonzero(out[-2:]) == 0
 
 
-def check_backward(w, seed=3):
-    """dq, dk, dv (and the attn_bias gradient) of the generic backward kernels, through loss.backward(), against
+def backward_workspace(w):
+    """The bytes of workspace the backward takes on these inputs."""
+    d = w.to(DEV)
+    args = helpers.backward_args(d, torch.randn(d.q.shape[0], d.q.shape[1], d.v.shape[2], device=DEV).to(d.q.dtype))
+    return helpers.allocated_beside(lambda: ops_rec.ascendc.attention.hstu_jagged_backward(*args))[1]
+
+
+def check_backward(w, seed=3, backward=None):
+    """dq, dk, dv (and the attn_bias gradient) of the generic backward kernels, through loss.backward() (or ``backward``, a
+    function of the workload and the output's gradient), against
     autograd on the fp32 oracle: fp32 inputs within 2e-4 of the largest reference value, 16-bit inputs within 1e-2
     (their gradients are rounded to the input type)."""
     d = w.to(DEV)
@@ -107,7 +115,11 @@ def check_backward(w, seed=3):
     out = ops_rec.ascendc.attention.hstu_jagged(*args)
     g = torch.Generator().manual_seed(seed)
     grad_out = torch.randn(out.shape, generator=g).to(out.dtype)
-    out.backward(grad_out.to(DEV))
+    if backward is None:
+        out.backward(grad_out.to(DEV))
+        got = (q.grad, k.grad, v.grad, bias.grad if bias is not None else None)
+    else:
+        got = backward(d, grad_out.to(DEV))
     qc, kc, vc = (t.float().clone().requires_grad_() for t in (w.q, w.k, w.v))
     kw = w.oracle_kwargs()
     bc = None
@@ -116,9 +128,9 @@ def check_backward(w, seed=3):
         kw["attn_bias"] = bc
     O.hstu_jagged_forward(qc, kc, vc, out_dtype=torch.float32, **kw).backward(grad_out.float())
     tol = 2e-4 if w.q.dtype == torch.float32 else 1e-2
-    pairs = [("dq", q.grad, qc.grad), ("dk", k.grad, kc.grad), ("dv", v.grad, vc.grad)]
+    pairs = [("dq", got[0], qc.grad), ("dk", got[1], kc.grad), ("dv", got[2], vc.grad)]
     if bias is not None:
-        pairs.append(("dbias", bias.grad, bc.grad))
+        pairs.append(("dbias", got[3], bc.grad))
     for name, got, ref in pairs:
         assert got.dtype == w.q.dtype and got.shape == ref.shape, name
         assert torch.isfinite(got).all(), name
@@ -217,7 +229,7 @@ def test_backward_above_head_dim_256_as_two_windows(name, mask, dtype, monkeypat
     the library asks for -- the pair plane of the planes order plus 256 bytes per (query row, 32-key block, head) of
     fp32 partial scores -- full of NaN.  Without the workspace, and with HSTU_MI355_GENERIC_BACKWARD=1, the generic
     kernels take the call."""
-    from ops_rec import _ops, workloads
+    from ops_rec import workloads
 
     kw = dict(WINDOW_CASES[name])
     w = workloads.make("win", dtype=dtype, std=0.4, seed=len(name), **kw)
@@ -227,46 +239,33 @@ def test_backward_above_head_dim_256_as_two_windows(name, mask, dtype, monkeypat
         w = dataclasses.replace(w, mask=(torch.rand(shape, generator=g) < 0.7).to(dtype), mask_type=3)
     elif mask == "none":
         w = dataclasses.replace(w, mask_type=2)
-    asked = []
-    plain = _ops._new_workspace
-
-    def poisoned(n_bytes, device):
-        asked.append(n_bytes)
-        ws = plain(n_bytes, device)
-        if ws is not None:
-            ws.fill_(0xFF)
-        return ws
-
-    monkeypatch.setattr(_ops, "_new_workspace", poisoned)
+    helpers.poison_workspace(monkeypatch)
     helpers.set_switch(monkeypatch, "HSTU_MI355_GENERIC_BACKWARD", None)
     check_backward(w)
     rows, heads, blocks = w.q.shape[0], w.q.shape[1], (w.max_seq_len + 31) // 32
     partial = heads * rows * blocks * 256
-    assert asked and asked[-1] > partial and (asked[-1] - partial) % (128 * heads) == 0, (asked, partial)
+    asked = backward_workspace(w)
+    assert asked > partial and (asked - partial) % (128 * heads) == 0, (asked, partial)
     # the generic kernels on the same inputs: no workspace
     helpers.set_switch(monkeypatch, "HSTU_MI355_GENERIC_BACKWARD", "1")
     check_backward(w)
-    assert asked[-1] == 0
+    assert backward_workspace(w) == 0
     helpers.set_switch(monkeypatch, "HSTU_MI355_GENERIC_BACKWARD", None)
-    helpers.withhold_workspace(monkeypatch)
-    check_backward(w)
+    check_backward(w, backward=lambda d, grad: helpers.backward_without_workspace(monkeypatch, d, grad))
 
 
-def test_backward_windows_and_rows_that_are_not_16_byte_pieces(monkeypatch):
+def test_backward_windows_and_rows_that_are_not_16_byte_pieces():
     """Rows of [max_q][max_k] tensors are 16-byte pieces only when max_seq_len_k is a multiple of 8: a call with an
     attn_bias at another max_seq_len_k stays on the generic kernels (no workspace), one without such tensors takes the
     windows all the same; a head dim that is not a multiple of 16 stays on the generic kernels either way."""
-    from ops_rec import _ops, workloads
+    from ops_rec import workloads
 
-    asked = []
-    plain = _ops._new_workspace
-    monkeypatch.setattr(_ops, "_new_workspace", lambda n, dev: (asked.append(n), plain(n, dev))[1])
     w = workloads.make("win", dtype=torch.bfloat16, std=0.4, batch=2, heads=2, dim=512, lo=1, hi=90, max_seq_len=90, rab_std=0.5)
     check_backward(w)
-    assert asked[-1] == 0
+    assert backward_workspace(w) == 0
     w = workloads.make("win", dtype=torch.bfloat16, std=0.4, batch=2, heads=2, dim=512, lo=1, hi=90, max_seq_len=90)
     check_backward(w)
-    assert asked[-1] > 0
+    assert backward_workspace(w) > 0
     w = workloads.make("win", dtype=torch.bfloat16, std=0.4, batch=2, heads=2, dim=264, dim_v=272, lo=1, hi=88, max_seq_len=88)
     check_backward(w)  # a head dim that is not a multiple of 16
-    assert asked[-1] == 0
+    assert backward_workspace(w) == 0

@@ -1,29 +1,18 @@
 """The native dispatcher kernels (csrc/torch_binding.cpp) against the Python implementations they stand in for: the same bits
 from both, for calls in canonical form and for calls that the native side hands over (views, index types that differ)."""
 
+import dataclasses
+
 import pytest
 import torch
 
 import ops_rec
+import helpers
 from helpers import small_case
-from ops_rec import _activation, _dispatch, _ops
+from ops_rec import _activation, _ops, workloads
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-
-
-@pytest.fixture
-def python_only():
-    """Switches the native side off for one call, as replacing an allocator of ``_ops`` does."""
-
-    def call(fn, *args):
-        _dispatch.binding.set_native(False)
-        try:
-            return fn(*args)
-        finally:
-            _dispatch.binding.set_native(True)
-
-    return call
 
 
 def same(a, b):
@@ -36,7 +25,7 @@ def same(a, b):
 @pytest.mark.parametrize("kw", [dict(), dict(delta=True), dict(rab=True, ctx=3, max_target=5, group=2), dict(heads=4, heads_k=2)],
                          ids=["equal", "delta", "bias", "grouped"])  # fmt: skip
 @pytest.mark.parametrize("form", ["canonical", "view", "int64 targets"])
-def test_attention_forward_and_gradients(kw, form, python_only):
+def test_attention_forward_and_gradients(kw, form):
     w = small_case(seed=9, batch=3, dim=64, lo=1, hi=150, dtype=torch.bfloat16, std=0.5, **kw).to(DEV)
     args = list(w.op_args())
     leaves = [t.clone().requires_grad_() for t in (w.q, w.k, w.v)] + ([w.attn_bias.clone().requires_grad_()] if w.attn_bias is not None else [])
@@ -49,49 +38,41 @@ def test_attention_forward_and_gradients(kw, form, python_only):
         args[-3] = torch.zeros(3, dtype=torch.int64, device=DEV) if args[-3] is None else args[-3].long()
         args[-4] = torch.zeros(3, dtype=torch.int64, device=DEV) if args[-4] is None else args[-4].long()
 
-    def step():
-        out = ops_rec.ascendc.attention.hstu_jagged(*args)
-        return (out, *torch.autograd.grad(out.float().square().sum(), leaves))
-
-    same(step(), python_only(step))
-
-
-def test_a_replaced_allocator_sends_calls_through_python(monkeypatch):
-    w = small_case(seed=2, batch=2, dim=64, lo=20, hi=90, dtype=torch.float16).to(DEV)
-    made, plain = [], _ops._new_grad
-    monkeypatch.setattr(_ops, "_new_grad", lambda like: (made.append(like.shape), plain(like))[1])
-    grad = torch.randn_like(w.q)
-    op = torch.ops.ops_rec.hstu_jagged_backward.equal
-    op(grad, w.q, w.k, w.v, None, None, 0, w.max_seq_len, w.silu_scale, w.seq_offset)
-    assert len(made) == 3
-    monkeypatch.undo()
-    op(grad, w.q, w.k, w.v, None, None, 0, w.max_seq_len, w.silu_scale, w.seq_offset)
-    assert len(made) == 3
+    out = ops_rec.ascendc.attention.hstu_jagged(*args)
+    grad = torch.randn_like(out)
+    got = (out, *torch.autograd.grad(out, leaves, grad))
+    # the same through the Python implementations
+    with torch.no_grad():
+        want = (_ops.hstu_jagged_delta if w.seq_offset_k is not None else _ops.hstu_jagged_equal)(*args)
+        d = dataclasses.replace(w, q=args[0], num_target=args[-3], num_context=args[-4])
+        grads = _ops.hstu_jagged_backward_delta(*helpers.backward_args(d, grad))
+    same(got, (want, *grads[: len(leaves)]))
 
 
 @pytest.mark.parametrize("m,split,with_bias", [(1, [16] * 4, True), (130, [64, 192, 128, 128], True), (77, [128] * 4, False)])
-def test_projection_and_gradients_with_outputs_left_out(m, split, with_bias, python_only):
+def test_projection_and_gradients_with_outputs_left_out(m, split, with_bias):
     n = sum(split)
     x, w, b = (torch.randn(s, device=DEV).to(d).requires_grad_() for s, d in (((m, 16), torch.bfloat16), ((n, 16), torch.bfloat16), ((n,), torch.float32)))
     bias = b if with_bias else None
+    leaves = (x, w, b) if with_bias else (x, w)
+    outs = torch.ops.ops_rec.distance_in_linear_silu(x, w, bias, split)
+    gu, gk = torch.randn_like(outs[0]), torch.randn_like(outs[3])
+    got = (*outs, *torch.autograd.grad((outs[0], outs[3]), leaves, (gu, gk)))  # no gradient of v, q, lin
+    with torch.no_grad():
+        want = _activation.distance_in_linear_silu(x, w, bias, split)
+        grads = _activation.in_linear_silu_backward(x, w, bias, gu, torch.zeros_like(outs[1]), torch.zeros_like(outs[2]), gk, want[4], split)
+    same(got, (*want, *grads[: len(leaves)]))
 
-    def step():
-        u, v, q, k, lin = torch.ops.ops_rec.distance_in_linear_silu(x, w, bias, split)
-        leaves = (x, w, b) if with_bias else (x, w)
-        return (u, v, q, k, lin, *torch.autograd.grad((u.float().sum() + k.float().square().sum()), leaves))  # no gradient of v, q, lin
 
-    same(step(), python_only(step))
-
-
-def test_ln_mul(python_only):
+def test_ln_mul():
     x, u = torch.randn(33, 96, device=DEV).half(), torch.randn(33, 96, device=DEV).half()
     g, b = torch.randn(96, device=DEV), torch.randn(96, device=DEV)
-    step = lambda: (torch.ops.ops_rec.ln_mul(x, u, g, b), torch.ops.ops_rec.ln_mul(x.t().contiguous().t(), u, g, b))  # noqa: E731
-    same(step(), python_only(step))
-    same(step()[:1], (_activation.ln_mul(x, u, g, b),))
+    view = x.t().contiguous().t()
+    op = torch.ops.ops_rec.ln_mul
+    same((op(x, u, g, b), op(view, u, g, b)), (_activation.ln_mul(x, u, g, b), _activation.ln_mul(view, u, g, b)))
 
 
-def test_memory_that_nobody_writes_is_filled_when_the_program_asks_for_it():
+def test_memory_that_nobody_writes_is_filled_when_the_program_asks_for_it(monkeypatch):
     """``torch.use_deterministic_algorithms`` has torch hand out new tensors full of NaN; what the native side allocates is no
     exception.  (Rows ahead of a non-zero first offset belong to no work item.)"""
     w = small_case(seed=4, batch=2, dim=64, lo=20, hi=60, dtype=torch.bfloat16).to(DEV)
@@ -100,9 +81,19 @@ def test_memory_that_nobody_writes_is_filled_when_the_program_asks_for_it():
     call = lambda: torch.ops.ops_rec.hstu_jagged.equal(q, k, v, None, None, 0, w.max_seq_len, 0.0, offs)  # noqa: E731
     want = call()
     torch.zeros_like(want)  # (what the allocator hands out next holds zeros)
-    torch.use_deterministic_algorithms(True, warn_only=True)
-    try:
-        out = call()
-    finally:
-        torch.use_deterministic_algorithms(False)
+    helpers.poison_workspace(monkeypatch)
+    out = call()
     assert out[:3].isnan().all() and torch.equal(out[3:], want[3:])
+
+
+def test_a_backward_whose_workspace_does_not_fit(monkeypatch):
+    """The native kernel's answer to an allocator that has no room for the workspace is the launch order that needs none."""
+    w = workloads.make("oom", dtype=torch.bfloat16, device=DEV, seed=3, batch=8, heads=4, dim=128, lo=1500, hi=2048, max_seq_len=2048)
+    args = helpers.backward_args(w, torch.randn_like(w.q))
+    call = lambda: ops_rec.ascendc.attention.hstu_jagged_backward(*args)  # noqa: E731
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "0")
+    want = call()
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "2")
+    assert helpers.allocated_beside(call)[1] > 64 << 20
+    got, refused = helpers.with_room_for(call, 32 << 20, like=want)
+    assert refused == 1 and all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, want))
