@@ -138,7 +138,9 @@ typedef struct hstu_jagged_fwd_params {
  * each has a workspace (and an output) of its own.  The library keeps no device state between calls.
  * A caller that passes less than asked for, or nothing, gets the same results from the fixed schedule.  Because a
  * split changes the order of the fp32 sums, the last bit of an output element may then depend on what else is in
- * the batch; HSTU_MI355_SPLIT=0 in the environment turns the split off. */
+ * the batch; HSTU_MI355_SPLIT=0 in the environment turns the split off.  The same holds for fp32 inputs, whose kernel
+ * needs no workspace: it deals the keys of a row over as many wavefronts as it takes to fill the machine, which
+ * depends on the batch, the heads and max_seq_len; with HSTU_MI355_SPLIT=0 one wavefront takes them all. */
 HSTU_API int hstu_jagged_fwd_workspace_size(const hstu_jagged_fwd_params* params, uint64_t* workspace_bytes);
 
 /* replaces aclnnHstuJaggedForward: enqueues the forward on `stream` (a hipStream_t passed as void*;

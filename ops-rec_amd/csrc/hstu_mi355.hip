@@ -78,8 +78,8 @@ int compute_units(int* out)
 // Process-wide switches.  They are read from the environment once, at the first call that looks at one, and again
 // only when hstu_reload_switches() is called (a test that changes the environment calls it); a launch reads no
 // environment variable.  A value of -1 means "not set: the library's own rule applies".
-//   HSTU_MI355_SPLIT=0             forward: never cut long items into parts (the rows of a sequence are then the same bits
-//                                  whatever else is in the batch)
+//   HSTU_MI355_SPLIT=0             forward: never cut long items into parts, nor deal the keys of an fp32 row over wavefronts (the
+//                                  rows of a sequence are then the same bits whatever else is in the batch, where both take one kernel)
 //   HSTU_MI355_SHORT=0 / 1         forward: never / whenever possible the kernel for short lists
 //   HSTU_MI355_GENERIC_BACKWARD=1  backward: the generic kernels also where tuned ones exist (for comparisons)
 //   HSTU_MI355_BWD_HANDOFF=0/1/2   backward: force the launch order (two launches / three / planes)
@@ -502,7 +502,8 @@ uint64_t forward_workspace_bytes(const Variant* var, const hstu_jagged_fwd_param
 // slots 64 until there are eight of them per CU, above (two wavefronts per SIMD as it is) two.  Measured against the kernel of
 // 128-row tiles before: 4 x 2 heads, d 64, 16..128 rows 15.6 -> 5 us (kernel time), 3 x 8 heads, d 64, 1662..1971 rows 180 -> 105 us
 // (167 without the second clause), 1 x 8, d 128, 4065 rows 603 -> 336, 2 x 4, d 32, 8113 rows 450 -> 356 (492 without), 48 x 2,
-// d 128, 1196..1350 rows 500 -> 415, 16 x 4, d 256, 170..1023 rows 368 -> 242.
+// d 128, 1196..1350 rows 500 -> 415, 16 x 4, d 256, 170..1023 rows 368 -> 242.  The order of a row's sums depends on it, and
+// with that the last bits on the size of the batch; HSTU_MI355_SPLIT=0 keeps one share.
 int f32_splits(const Variant* var, const hstu_jagged_fwd_params* p, int cus)
 {
     const int64_t groups = (p->n_offsets - 1) * p->num_heads_q * ((p->max_seq_len_q + 15) / 16);
