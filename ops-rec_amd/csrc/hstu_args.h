@@ -40,6 +40,14 @@ constexpr int kFewRows = 64;          // the most query rows of a sequence that 
 constexpr int kFwdFewRowsThreads = 512;  // threads of a workgroup of the forward kernel for few query rows (eight wavefronts over row groups and keys)
 constexpr int kCounterBlockBytes = 16384;  // head of the workspace: device-side work counters (see the forward kernel)
 constexpr int kQueueCounterBytes = 1024;   // of which the work counters of the per-XCD queues, the part that has to be cleared
+// Arrival counters of split items in that block.  An item is split only where there are fewer items than workgroups, so the
+// grid of a launch that may split is what bounds them: at most this many workgroups (split_grid).
+constexpr int kMaxSplitItems = 1024;
+constexpr int64_t split_grid(int64_t resident) { return resident < kMaxSplitItems ? resident : kMaxSplitItems; }
+// (on the 256 CUs of an MI355X that is every resident workgroup of the variants that split, the slots 64 and 128)
+static_assert(split_grid(256 * fwd_wgs_per_cu(64, false, false)) == 256 * 3 && split_grid(256 * fwd_wgs_per_cu(128, false, false)) == 256 * 2,
+              "no resident workgroup is left out");
+static_assert(split_grid(int64_t{2048} * 3) == kMaxSplitItems, "and no launch has more items to split than there are counters");
 constexpr int kDkvThreads = 256;   // threads of a workgroup of the key-tile backward kernel
 constexpr int kGatherThreads = 128;
 

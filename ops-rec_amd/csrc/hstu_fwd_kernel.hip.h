@@ -322,7 +322,6 @@ __device__ __forceinline__ void load_to_lds_b128(__amdgpu_buffer_rsrc_t rsrc, ui
 // the part that completes an item puts its counter back to zero, so that a replay under the same number finds none of its own.
 constexpr int kQueues = 8;          // one work queue per XCD (MI355X: 8 XCDs; workgroup w runs on XCD w mod 8)
 constexpr int kCounterStride = 32;  // counters of different queues sit in different 128-byte lines
-constexpr int kMaxSplitItems = 1024;  // (an item is only split when there are fewer items than resident workgroups)
 constexpr int kMaxParts = 8;
 constexpr int kSplitCounterBase = kQueues * kCounterStride;  // first arrival counter, in 32-bit words
 static_assert(kSplitCounterBase * 4 == kQueueCounterBytes, "the queues come first");

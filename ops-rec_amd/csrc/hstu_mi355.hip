@@ -1571,7 +1571,7 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
             a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
             const uint64_t parts = (workspace_bytes - kCounterBytes) / part_bytes;
             a.ws_parts = static_cast<uint32_t>(parts < 0x7fffffffull ? parts : 0x7fffffffull);
-            n_blocks = resident;  // the list may have more entries than items: all resident workgroups take part
+            n_blocks = hstu::split_grid(resident);  // the list may have more entries than items: all resident workgroups take part
         }
         if (paged != nullptr) {
             kernel = var->kernel_paged;  // (splits when it was given room above, otherwise not; the caller checked the block)
