@@ -21,7 +21,7 @@ from typing import List, Optional
 import torch
 
 from . import _native
-from ._ops import _DTYPE_CODE, _check, _lib_cuda, _lib_def, _lib_meta
+from ._ops import _DTYPE_CODE, _PYTHON_KERNELS, _check, _lib_def, _lib_meta
 
 LN_MUL_EPSILON = 1e-5
 
@@ -114,7 +114,7 @@ def ln_mul_meta(x, u, gamma, beta):
     return torch.empty_like(x)
 
 
-_lib_cuda.impl("ln_mul", ln_mul)
+_PYTHON_KERNELS["ln_mul"] = ln_mul
 _lib_meta.impl("ln_mul", ln_mul_meta)
 
 
@@ -292,9 +292,9 @@ def in_linear_silu_backward_meta(x, weight, bias, user_grad, value_grad, query_g
     return torch.empty_like(x), torch.empty_like(weight), (torch.empty_like(bias) if bias is not None else None), None
 
 
-_lib_cuda.impl("distance_in_linear_silu", distance_in_linear_silu)
+_PYTHON_KERNELS["distance_in_linear_silu"] = distance_in_linear_silu
 _lib_meta.impl("distance_in_linear_silu", distance_in_linear_silu_meta)
-_lib_cuda.impl("in_linear_silu_backward", in_linear_silu_backward)
+_PYTHON_KERNELS["in_linear_silu_backward"] = in_linear_silu_backward
 _lib_meta.impl("in_linear_silu_backward", in_linear_silu_backward_meta)
 
 

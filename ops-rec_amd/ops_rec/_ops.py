@@ -60,9 +60,10 @@ _SCHEMAS = (
 _lib_def = torch.library.Library("ops_rec", "DEF")
 for _s in _SCHEMAS:
     _lib_def.define(_s)
-_lib_cuda = torch.library.Library("ops_rec", "IMPL", "CUDA")  # what ``_dispatch`` replaces by native kernels
 _lib_cuda_dense = torch.library.Library("ops_rec", "IMPL", "CUDA")
 _lib_meta = torch.library.Library("ops_rec", "IMPL", "Meta")
+
+_PYTHON_KERNELS: dict = {}  # by operator: what ``_dispatch`` registers for device tensors where it has no native kernel
 
 _DTYPE_CODE = {
     torch.bfloat16: _native.DT_BF16,
@@ -744,14 +745,14 @@ def hstu_dense_backward_meta(grad, q, k, v, mask, attn_bias, mask_type=0, max_se
 
 _lib_cuda_dense.impl("hstu_dense_backward", hstu_dense_backward)
 _lib_meta.impl("hstu_dense_backward", hstu_dense_backward_meta)
-_lib_cuda.impl("hstu_paged", hstu_paged)
+_PYTHON_KERNELS["hstu_paged"] = hstu_paged
 _lib_meta.impl("hstu_paged", hstu_paged_meta)
 _lib_cuda_dense.impl("hstu_dense", hstu_dense)
 _lib_meta.impl("hstu_dense", hstu_dense_meta)
-_lib_cuda.impl("hstu_jagged.equal", hstu_jagged_equal)
-_lib_cuda.impl("hstu_jagged.delta", hstu_jagged_delta)
-_lib_cuda.impl("hstu_jagged_backward.equal", hstu_jagged_backward_equal)
-_lib_cuda.impl("hstu_jagged_backward.delta", hstu_jagged_backward_delta)
+_PYTHON_KERNELS["hstu_jagged.equal"] = hstu_jagged_equal
+_PYTHON_KERNELS["hstu_jagged.delta"] = hstu_jagged_delta
+_PYTHON_KERNELS["hstu_jagged_backward.equal"] = hstu_jagged_backward_equal
+_PYTHON_KERNELS["hstu_jagged_backward.delta"] = hstu_jagged_backward_delta
 _lib_meta.impl("hstu_jagged.equal", hstu_jagged_equal_meta)
 _lib_meta.impl("hstu_jagged.delta", hstu_jagged_delta_meta)
 _lib_meta.impl("hstu_jagged_backward.equal", hstu_jagged_backward_equal_meta)
@@ -760,8 +761,12 @@ _lib_meta.impl("hstu_jagged_backward.delta", hstu_jagged_backward_delta_meta)
 
 def _pick_overload_by_argument(packet, position: int) -> None:
     """A call of the packet itself tries its overloads in turn, and each that does not fit costs an exception with its text (12 us
-    for ``delta``, the second).  The two differ in what stands at ``position``: the offsets (``equal``) or ``silu_scale``."""
-    resolve, equal, delta = packet._op, packet.equal._op, packet.delta._op
+    for ``delta``, the second).  The two differ in what stands at ``position``: the offsets (``equal``) or ``silu_scale``.  (Where a
+    torch keeps its packets another way they stay as they are.)"""
+    try:
+        resolve, equal, delta = packet._op, packet.equal._op, packet.delta._op
+    except AttributeError:
+        return
 
     def call(*args, **kwargs):
         if len(args) > position:
