@@ -75,6 +75,18 @@ Tensor empty(at::IntArrayRef size, at::ScalarType dtype, const at::Device& devic
     return t;
 }
 
+// A workspace a call can do without: none (undefined) when the allocator has no room for it.
+Tensor empty_or_none(uint64_t bytes, const at::Device& device)
+{
+    if (bytes != 0) {
+        try {
+            return empty({static_cast<int64_t>(bytes)}, at::kByte, device);
+        } catch (const c10::OutOfMemoryError&) {
+        }
+    }
+    return Tensor();
+}
+
 void* ptr(const Tensor& t) { return t.defined() && t.numel() != 0 ? t.data_ptr() : nullptr; }
 void* ptr(const OptTensor& t) { return t.has_value() ? ptr(*t) : nullptr; }
 
@@ -240,13 +252,7 @@ Gradients backward(const Tensor& grad_in, const Call& c)
         p.grad_attn_bias = ptr(dbias);
         uint64_t ws_bytes = 0;
         if (hstu_jagged_bwd_workspace_size(&p, &ws_bytes) == HSTU_OK) {
-            Tensor ws;
-            if (ws_bytes != 0) {
-                try {
-                    ws = empty({static_cast<int64_t>(ws_bytes)}, at::kByte, q.device());
-                } catch (const c10::OutOfMemoryError&) {  // the library then runs the launch order that needs none
-                }
-            }
+            const Tensor ws = empty_or_none(ws_bytes, q.device());  // (without one the library runs the launch order that needs none)
             const int rc = hstu_jagged_bwd(&p, ptr(ws), ws.defined() ? ws_bytes : 0, stream_of(q));
             TORCH_CHECK(rc == HSTU_OK, "hstu_jagged_bwd failed (", rc, "): ", hstu_last_error());
             return {dq, dk, dv, dbias};
@@ -473,15 +479,11 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
         // A weight of that size gives a library product a tile for every CU, and the rows enough work per tile: the element-wise
         // stage in a kernel of its own and d_mixed^T @ x from the library (m = 9600, n = 8192, k = 2048: level at 12 M
         // elements, 6144 x 1536, and 2 % ahead here).
-        const bool library = n * x.size(1) >= (int64_t{12} << 20) && m >= 4096;
-        if (!library) {
-            weight_grad = empty({n, x.size(1)}, x.scalar_type(), x.device());
-        }
+        bool library = n * x.size(1) >= (int64_t{12} << 20) && m >= 4096;
         in_linear_silu_bwd_weight_params p;
         std::memset(&p, 0, sizeof p);
         p.struct_size = sizeof p;
         p.x = x.data_ptr();
-        p.weight_grad = ptr(weight_grad);
         p.k = x.size(1);
         in_linear_silu_bwd_params& s = p.stage;
         s.struct_size = sizeof s;
@@ -499,10 +501,25 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
         }
         s.dtype = dtype_code(x.scalar_type());
         uint64_t ws_bytes = 0;
-        int rc = library ? in_linear_silu_bwd_dmixed_workspace_size(&s, &ws_bytes) : in_linear_silu_bwd_weight_workspace_size(&p, &ws_bytes);
-        if (rc == HSTU_OK) {
-            const Tensor ws = ws_bytes != 0 ? empty({static_cast<int64_t>(ws_bytes)}, at::kByte, x.device()) : Tensor();
-            rc = library ? in_linear_silu_bwd_dmixed(&s, ptr(ws), ws_bytes, stream_of(x)) : in_linear_silu_bwd_weight(&p, ptr(ws), ws_bytes, stream_of(x));
+        int rc = HSTU_OK;
+        if (!library) {
+            weight_grad = empty({n, x.size(1)}, x.scalar_type(), x.device());
+            p.weight_grad = weight_grad.data_ptr();
+            rc = in_linear_silu_bwd_weight_workspace_size(&p, &ws_bytes);
+            if (rc == HSTU_OK) {
+                if (const Tensor ws = empty_or_none(ws_bytes, x.device()); ws.defined()) {
+                    rc = in_linear_silu_bwd_weight(&p, ws.data_ptr(), ws_bytes, stream_of(x));
+                } else {  // no room for the partial weight gradients (up to 1 GiB): the library product needs none
+                    library = true;
+                }
+            }
+        }
+        if (library) {
+            rc = in_linear_silu_bwd_dmixed_workspace_size(&s, &ws_bytes);
+            if (rc == HSTU_OK) {
+                const Tensor ws = ws_bytes != 0 ? empty({static_cast<int64_t>(ws_bytes)}, at::kByte, x.device()) : Tensor();
+                rc = in_linear_silu_bwd_dmixed(&s, ptr(ws), ws_bytes, stream_of(x));
+            }
         }
         TORCH_CHECK(rc == HSTU_OK, "in_linear_silu_backward failed (", rc, "): ", hstu_last_error());
         if (library) {

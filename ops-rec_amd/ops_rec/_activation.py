@@ -278,11 +278,15 @@ def in_linear_silu_backward(x, weight, bias: Optional[torch.Tensor], user_grad, 
            "weight, linear_output and the gradients must have the dtype of x")  # fmt: skip
     _check(all(t.is_cuda and t.device == x.device for t in (weight, linear_output, *grads)),
            "all tensors must be on the GPU of x")  # fmt: skip
-    if weight.numel() >= 12 << 20 and x.size(0) >= 4096:  # (the rule of the native kernel, csrc/torch_binding.cpp)
+    weight_grad = None
+    if weight.numel() < 12 << 20 or x.size(0) < 4096:  # (the rule of the native kernel, csrc/torch_binding.cpp)
+        try:
+            d_mixed, weight_grad, bias_sums = silu_backward_with_weight(linear_output, grads, split, x, want_bias_grad=bias is not None)
+        except torch.cuda.OutOfMemoryError:  # no room for the partial weight gradients: the library product needs none
+            pass
+    if weight_grad is None:
         d_mixed, bias_sums = silu_backward_stage(linear_output, grads, split, want_bias_grad=bias is not None)
         weight_grad = d_mixed.t() @ x
-    else:
-        d_mixed, weight_grad, bias_sums = silu_backward_with_weight(linear_output, grads, split, x, want_bias_grad=bias is not None)
     x_grad = d_mixed @ weight
     bias_grad = bias_sums.to(bias.dtype) if bias is not None else None
     return x_grad, weight_grad, bias_grad, None

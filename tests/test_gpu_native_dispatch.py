@@ -9,7 +9,7 @@ import torch
 import ops_rec
 import helpers
 from helpers import small_case
-from ops_rec import _activation, _ops, workloads
+from ops_rec import _activation, _dispatch, _ops, workloads
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -97,3 +97,20 @@ def test_a_backward_whose_workspace_does_not_fit(monkeypatch):
     assert helpers.allocated_beside(call)[1] > 64 << 20
     got, refused = helpers.with_room_for(call, 32 << 20, like=want)
     assert refused == 1 and all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("python", [False, True], ids=["native", "python"])
+def test_a_projection_backward_whose_workspace_does_not_fit(python):
+    """Without room for the partial weight gradients the weight gradient is a product of what the element-wise stage left."""
+    m, k, split = 3000, 1024, [1024] * 4
+    x, w, b = torch.randn(m, k, device=DEV).bfloat16(), torch.randn(4096, k, device=DEV).bfloat16() / 32, torch.randn(4096, device=DEV)
+    lin = torch.ops.ops_rec.distance_in_linear_silu(x, w, b, split)[4]
+    grads = [torch.randn(m, 1024, device=DEV).bfloat16() for _ in range(4)]
+    op = _activation.in_linear_silu_backward if python else torch.ops.ops_rec.in_linear_silu_backward
+    call = lambda: op(x, w, b, *grads, lin, split)  # noqa: E731
+    want, workspace = helpers.allocated_beside(call)
+    assert _dispatch.binding is not None and workspace > 60 << 20
+    got, refused = helpers.with_room_for(call, 40 << 20, like=(*want, lin))
+    assert refused == 1
+    for a, e in zip(got[:3], want[:3]):
+        assert a.dtype == e.dtype and (a.double() - e.double()).norm() <= 5e-3 * e.double().norm()
