@@ -1423,10 +1423,14 @@ HSTU_API const char* hstu_jagged_fwd_kernel_name(const hstu_jagged_fwd_params* p
     if (const hstu::ShortVariant* const sv = short_variant(v, params)) {
         return sv->name;
     }
-    if (takes_queue_variant(v, params, nullptr)) {
+    int64_t resident = 0;
+    if (takes_queue_variant(v, params, &resident)) {
         return v->name_queues;
     }
-    return may_take_split_variant(v, params, nullptr) ? v->name_split : v->name;
+    if (may_take_split_variant(v, params, nullptr)) {
+        return v->name_split;
+    }
+    return takes_direct_list(v, params, resident) ? v->name_direct : v->name;
 }
 
 }  // extern "C"

@@ -50,7 +50,8 @@ constexpr auto paged_kernel() -> void (*)(const FwdArgs)
      hstu::queues_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(),                                     \
      hstu::split_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(),                                      \
      hstu::paged_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(), D, 256, hstu::fwd_wgs_per_cu(D, RAB, MASK),  \
-     hstu::hstu_fwd_kernel<hstu::tag, hstu::tag, D, RAB, MASK, false, false, false, true>}
+     hstu::hstu_fwd_kernel<hstu::tag, hstu::tag, D, RAB, MASK, false, false, false, true>,          \
+     "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_direct"}
 #define HSTU_DIMS(tag, tagname, RAB, MASK)                                                           \
     {HSTU_VARIANT(tag, tagname, 32, RAB, MASK), HSTU_VARIANT(tag, tagname, 64, RAB, MASK), \
      HSTU_VARIANT(tag, tagname, 128, RAB, MASK), HSTU_VARIANT(tag, tagname, 256, RAB, MASK)}

@@ -7,8 +7,8 @@
 
 namespace hstu {
 
-// kernel variants with the per-XCD work queues and with split items exist for the head-dim slots 64 and 128, the one
-// with paged keys for 64, 128 and 256 (nullptr elsewhere)
+// the persistent kernel's variants (hstu_variant_tables.h): with split items for the head-dim slots 64 and 128, with paged keys for
+// 64, 128 and 256 (nullptr elsewhere)
 struct Variant {
     const char* name;
     const char* name_queues;
@@ -21,6 +21,7 @@ struct Variant {
     int threads;
     int persistent_wgs_per_cu;  // > 0: persistent kernel, this many workgroups per CU; 0: one workgroup per tile
     void (*kernel_direct)(const FwdArgs);  // the persistent kernel without a list, a workgroup per slot, for the shortest lists
+    const char* name_direct;
 };
 
 // the forward kernel for short work lists (hstu_fwd_short_kernel.hip.h): one workgroup of `threads` per
