@@ -31,12 +31,14 @@ def cases():
         "split": lambda s: mk("s", dtype=bf, device=DEV, seed=s, batch=2, heads=2, dim=128, lo=2500, hi=3000),
         # a list in between: the plain variant, no counters (with the kernel for short lists switched off), and the
         # same list on that kernel
-        "plain": lambda s: mk("p", dtype=bf, device=DEV, seed=s, batch=24, heads=4, dim=128, lo=100, hi=900),
-        "short": lambda s: mk("p", dtype=bf, device=DEV, seed=s, batch=24, heads=4, dim=128, lo=100, hi=900),
+        "plain": lambda s: mk("p", dtype=bf, device=DEV, seed=s, batch=48, heads=4, dim=128, lo=100, hi=500, max_seq_len=500),
+        "short": lambda s: mk("p", dtype=bf, device=DEV, seed=s, batch=48, heads=4, dim=128, lo=100, hi=500, max_seq_len=500),
+        # a workgroup per slot, no list at all
+        "direct": lambda s: mk("d", dtype=bf, device=DEV, seed=s, batch=24, heads=4, dim=128, lo=100, hi=380),
     }
 
 
-@pytest.mark.parametrize("name", ["queues", "split", "plain", "short"])
+@pytest.mark.parametrize("name", ["queues", "split", "plain", "short", "direct"])
 def test_many_launches_in_flight_on_several_streams(name, monkeypatch):
     helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", None if name == "short" else "0")
     make = cases()[name]
@@ -46,7 +48,7 @@ def test_many_launches_in_flight_on_several_streams(name, monkeypatch):
     for w in inputs:
         p = prepared(w)
         assert name in ("plain",) or name in p.kernel_name()
-        assert name != "plain" or not p.kernel_name().endswith(("_queues", "_short"))
+        assert name != "plain" or not p.kernel_name().endswith(("_queues", "_short", "_split", "_direct"))
         serial.append(p.launch().clone())
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream(device=DEV) for _ in range(n_streams)]
