@@ -131,6 +131,10 @@ typedef struct in_linear_silu_bwd_weight_params {
     int64_t k;                       /* a multiple of 16 in [16, 8192] */
 } in_linear_silu_bwd_weight_params;
 
+/* 1 where the call below is the faster one, 0 where in_linear_silu_bwd_dmixed and a product of the caller's BLAS are (k above 1024);
+ * either way is right for every shape */
+HSTU_API int in_linear_silu_bwd_weight_pays(const in_linear_silu_bwd_weight_params* params);
+
 /* bytes of device scratch in_linear_silu_bwd_weight needs (one fp32 partial output per chunk of rows; never 0) */
 HSTU_API int in_linear_silu_bwd_weight_workspace_size(const in_linear_silu_bwd_weight_params* params, uint64_t* workspace_bytes);
 

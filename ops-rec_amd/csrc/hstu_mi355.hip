@@ -42,37 +42,36 @@ int hstu::set_error(int code, const char* fmt, ...)
     return code;
 }
 
-namespace {
-
-using hstu::BwdVariant;
-using hstu::Variant;
-
-#define fail(...) hstu::set_error(__VA_ARGS__)
-
-
-// compute units of each device, looked up once
-int compute_units(int* out)
+int hstu::compute_units(int* out)
 {
-    static int cached[64] = {0};
+    static std::atomic<int> cached[64];
     int dev = 0;
     hipError_t err = hipGetDevice(&dev);
     if (err != hipSuccess) {
-        return fail(HSTU_ERR_RUNTIME, "hipGetDevice failed: %s", hipGetErrorString(err));
+        return set_error(HSTU_ERR_RUNTIME, "hipGetDevice failed: %s", hipGetErrorString(err));
     }
     if (dev < 0 || dev >= 64) {
         dev = 0;
     }
-    if (cached[dev] == 0) {
-        int n = 0;
+    int n = cached[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
         err = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
         if (err != hipSuccess || n <= 0) {
-            return fail(HSTU_ERR_RUNTIME, "cannot read the number of compute units: %s", hipGetErrorString(err));
+            return set_error(HSTU_ERR_RUNTIME, "cannot read the number of compute units: %s", hipGetErrorString(err));
         }
-        cached[dev] = n;
+        cached[dev].store(n, std::memory_order_relaxed);
     }
-    *out = cached[dev];
+    *out = n;
     return HSTU_OK;
 }
+
+namespace {
+
+using hstu::BwdVariant;
+using hstu::compute_units;
+using hstu::Variant;
+
+#define fail(...) hstu::set_error(__VA_ARGS__)
 
 
 // Process-wide switches.  They are read from the environment once, at the first call that looks at one, and again

@@ -201,9 +201,11 @@ int validate_weight(const in_linear_silu_bwd_weight_params* p)
 // How the weight gradient is cut: tiles of 128 x tile_k (the narrowest of the three widths that spans k, 512 above), and the
 // number of chunks of rows, each of eight 32-row steps at least, that an estimate of the time puts first -- rounds of
 // workgroups over the CUs (two of the narrowest tile each, one of the others) times a chunk's steps, and the partial outputs, which
-// are written and read back once.  Chunks beyond eight come in whole groups of 8, one per XCD.  Measured, element-wise stage +
-// column sums + library product -> the two kernels: m 20480, n 2048, k 512 187 -> 92 us (340 MB of operands, d_mixed and partial
-// outputs: 3.7 TB/s); m 95697, n 512, k 128 338 -> 76 us.
+// are written and read back once.  Chunks beyond eight come in whole groups of 8, one per XCD.  The estimate only has to rank
+// chunk counts: over 14 shapes of 1000 .. 300000 rows, n 256 .. 8192, k 64 .. 1024 its choice took 0.97 .. 1.12 of the best of thirteen
+// counts (worst 20000 x 1024 x 128: 33.2 against 29.7 us); below 1000 rows the eight steps bind (700 x 512 x 128: 14.3 against 9.4 us).
+// Measured, element-wise stage + column sums + library product -> the two kernels: m 20480, n 2048, k 512 187 -> 92 us (340 MB of
+// operands, d_mixed and partial outputs: 3.7 TB/s); m 95697, n 512, k 128 338 -> 76 us.
 struct WeightPlan {
     int tile_k;
     int tiles;
@@ -215,14 +217,17 @@ WeightPlan plan_weight(const in_linear_silu_bwd_weight_params* p)
     WeightPlan w;
     w.tile_k = p->k <= 128 ? 128 : (p->k <= 256 ? 256 : 512);
     w.tiles = static_cast<int>((p->stage.n + hstu::kWgradCols - 1) / hstu::kWgradCols * ((p->k + w.tile_k - 1) / w.tile_k));
-    constexpr int kCus = 256;
-    const int64_t slots = w.tile_k == 128 ? 2 * kCus : kCus;  // resident workgroups
+    int cus = 0;
+    if (hstu::compute_units(&cus) != HSTU_OK) {
+        cus = 256;  // (a size asked for where there is no device)
+    }
+    const int64_t slots = w.tile_k == 128 ? 2 * cus : cus;  // resident workgroups
     const int64_t steps = (p->stage.m + hstu::kWgradRows - 1) / hstu::kWgradRows;
     // (a chunk stays behind 32-bit descriptors)
     const int64_t widest = p->stage.n > p->k ? p->stage.n : p->k;
     const int64_t least = (steps * hstu::kWgradRows * widest * 2) / (int64_t{1} << 30) + 1;
     const int64_t most = steps / 8 < 64 ? steps / 8 : 64;
-    const double step_us = w.tile_k == 512 ? 1.2 : 0.8;  // (measured where the machine is full of workgroups: 1.0 .. 1.9, bytes included)
+    const double step_us = w.tile_k == 512 ? 1.2 : 0.8;
     const double partial_us = static_cast<double>(p->stage.n) * static_cast<double>(p->k) * 8.0 / 6e6;  // written and read back once
     int64_t chunks = least;
     double best = 0.0;
@@ -252,6 +257,13 @@ uint64_t weight_workspace_bytes(const in_linear_silu_bwd_weight_params* p)
 }  // namespace
 
 extern "C" {
+
+// Up to two tiles of 512 columns span k.  From the third on the element-wise stage, which each of them runs for itself, and the
+// narrower tiles of a plain product decide: stage + library product against the kernels of in_linear_silu_bwd_weight (GPU time, bf16),
+// k 256 .. 768: 1.05 .. 4.3 of their time from m = 512 on; k 1024: 0.93 .. 1.31 (n 4096 .. 28672; level from n 8192 on); k 1152: 0.85 ..
+// 1.04; 1280: 0.91 .. 1.04; 1408: 0.68 .. 1.04 (1.31 at m 100000); 1536: 0.70 .. 1.04 (1.18 at n 12288, m 100000); 2048: 0.81 .. 0.91;
+// 3072: 0.59 .. 0.80.  (n and m hardly matter: 32768 x 512, as large a weight as 8192 x 2048, 1.14 .. 1.21.)
+HSTU_API int in_linear_silu_bwd_weight_pays(const in_linear_silu_bwd_weight_params* p) { return p != nullptr && p->k <= 1024 ? 1 : 0; }
 
 HSTU_API int in_linear_silu_bwd_weight_workspace_size(const in_linear_silu_bwd_weight_params* p, uint64_t* workspace_bytes)
 {

@@ -476,10 +476,6 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
         if (is_set(bias)) {
             bias_grad = empty({n}, at::kFloat, x.device());
         }
-        // A weight of that size gives a library product a tile for every CU, and the rows enough work per tile: the element-wise
-        // stage in a kernel of its own and d_mixed^T @ x from the library (m = 9600, n = 8192, k = 2048: level at 12 M
-        // elements, 6144 x 1536, and 2 % ahead here).
-        bool library = n * x.size(1) >= (int64_t{12} << 20) && m >= 4096;
         in_linear_silu_bwd_weight_params p;
         std::memset(&p, 0, sizeof p);
         p.struct_size = sizeof p;
@@ -502,6 +498,7 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
         s.dtype = dtype_code(x.scalar_type());
         uint64_t ws_bytes = 0;
         int rc = HSTU_OK;
+        bool library = in_linear_silu_bwd_weight_pays(&p) == 0;
         if (!library) {
             weight_grad = empty({n, x.size(1)}, x.scalar_type(), x.device());
             p.weight_grad = weight_grad.data_ptr();

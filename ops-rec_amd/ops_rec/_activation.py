@@ -279,7 +279,7 @@ def in_linear_silu_backward(x, weight, bias: Optional[torch.Tensor], user_grad, 
     _check(all(t.is_cuda and t.device == x.device for t in (weight, linear_output, *grads)),
            "all tensors must be on the GPU of x")  # fmt: skip
     weight_grad = None
-    if weight.numel() < 12 << 20 or x.size(0) < 4096:  # (the rule of the native kernel, csrc/torch_binding.cpp)
+    if _native.load().in_linear_silu_bwd_weight_pays(_native.InLinearSiluBwdWeightParams(k=x.size(1))):
         try:
             d_mixed, weight_grad, bias_sums = silu_backward_with_weight(linear_output, grads, split, x, want_bias_grad=bias is not None)
         except torch.cuda.OutOfMemoryError:  # no room for the partial weight gradients: the library product needs none

@@ -35,6 +35,7 @@ EXPORTED_SYMBOLS = (
     "in_linear_silu_fwd_kernel_name",
     "in_linear_silu_bwd_dmixed_workspace_size",
     "in_linear_silu_bwd_dmixed",
+    "in_linear_silu_bwd_weight_pays",
     "in_linear_silu_bwd_weight_workspace_size",
     "in_linear_silu_bwd_weight",
 )
@@ -258,6 +259,8 @@ def load() -> ctypes.CDLL:
     lib.in_linear_silu_bwd_weight_workspace_size.restype = ctypes.c_int
     lib.in_linear_silu_bwd_weight_workspace_size.argtypes = [ctypes.POINTER(InLinearSiluBwdWeightParams),
                                                              ctypes.POINTER(ctypes.c_uint64)]  # fmt: skip
+    lib.in_linear_silu_bwd_weight_pays.restype = ctypes.c_int
+    lib.in_linear_silu_bwd_weight_pays.argtypes = [ctypes.POINTER(InLinearSiluBwdWeightParams)]
     lib.in_linear_silu_bwd_weight.restype = ctypes.c_int
     lib.in_linear_silu_bwd_weight.argtypes = [ctypes.POINTER(InLinearSiluBwdWeightParams), ctypes.c_void_p, ctypes.c_uint64,
                                               ctypes.c_void_p]  # fmt: skip

@@ -99,6 +99,22 @@ def test_a_backward_whose_workspace_does_not_fit(monkeypatch):
     assert refused == 1 and all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("k", [1024, 1040])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_projection_backward_on_both_sides_of_the_rule_for_its_weight_gradient(k, dtype):
+    m, split = 77, [k] * 4
+    x, w, b = torch.randn(m, k, device=DEV).to(dtype), (torch.randn(4 * k, k, device=DEV) / 32).to(dtype), torch.randn(4 * k, device=DEV)
+    lin = torch.ops.ops_rec.distance_in_linear_silu(x, w, b, split)[4]
+    grads = [torch.randn(m, k, device=DEV).to(dtype) for _ in range(4)]
+    call = lambda: torch.ops.ops_rec.in_linear_silu_backward(x, w, b, *grads, lin, split)  # noqa: E731
+    (dx, dw, db, _), workspace = helpers.allocated_beside(call)
+    assert (workspace >= 4 * dw.numel()) == (k <= 1024)  # fp32 partial outputs, or none
+    same((dx, dw, db), _activation.in_linear_silu_backward(x, w, b, *grads, lin, split)[:3])
+    d_mixed, own_dw, own_db = _activation.silu_backward_with_weight(lin, grads, split, x)
+    for got, other in ((dw, own_dw), (dw, d_mixed.double().t() @ x.double()), (db, own_db)):
+        assert (got.double() - other.double()).norm() <= 5e-3 * other.double().norm()
+
+
 @pytest.mark.parametrize("python", [False, True], ids=["native", "python"])
 def test_a_projection_backward_whose_workspace_does_not_fit(python):
     """Without room for the partial weight gradients the weight gradient is a product of what the element-wise stage left."""

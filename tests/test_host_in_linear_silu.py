@@ -166,3 +166,10 @@ def test_backward_stage_c_abi_validation_codes():
         got = lib.in_linear_silu_bwd_dmixed_workspace_size(ctypes.byref(p), ctypes.byref(ws))
         assert got == code, (name, got, _native.last_error())
         assert re.search(text, _native.last_error()), _native.last_error()
+
+
+def test_where_the_weight_gradient_has_a_kernel_of_its_own():
+    lib = _native.load()
+    pays = lambda k: lib.in_linear_silu_bwd_weight_pays(ctypes.byref(_native.InLinearSiluBwdWeightParams(k=k)))  # noqa: E731
+    assert [pays(k) for k in (16, 512, 1024, 1040, 8192)] == [1, 1, 1, 0, 0]
+    assert lib.in_linear_silu_bwd_weight_pays(None) == 0
