@@ -69,3 +69,15 @@ def test_the_native_kernels_are_the_ones_registered():
     assert ops_rec._dispatch.binding is not None and ops_rec._dispatch._lib is None
     for op in ("hstu_jagged.equal", "hstu_jagged_backward.delta", "hstu_paged", "ln_mul", "in_linear_silu_backward"):
         assert torch._C._dispatch_has_kernel_for_dispatch_key("ops_rec::" + op, "CUDA"), op
+
+
+def test_building_loads_no_library_that_it_replaces():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = (
+        "import sys, __graft_entry__ as g\n"
+        "b = g._builder()\n"
+        "assert b.BINDING_PATH.startswith(g._ROOT) and callable(b.build)\n"
+        "assert 'ops_rec' not in sys.modules\n"
+        "assert not [line for line in open('/proc/self/maps') if 'libhstu_mi355' in line]\n"
+    )
+    subprocess.run([sys.executable, "-c", code], cwd=root, check=True, timeout=120)
