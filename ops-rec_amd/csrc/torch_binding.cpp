@@ -567,7 +567,10 @@ struct JaggedFunction : torch::autograd::Function<JaggedFunction<DELTA>> {
     {
         const at::AutoDispatchBelowADInplaceOrView below;
         const Call& c = *call;
-        ctx->save_for_backward({q, k, v, unwrap(c.mask), unwrap(bias), c.offs_q, c.offs_k, unwrap(c.ctx), unwrap(c.tgt)});
+        // offsets that serve both sides are saved once: saved-tensor hooks (offloading, for one) hand back a tensor per saved one, and
+        // the library tells self-attention, whose pair plane takes half the room, by the two being the same
+        const Tensor offs_k = c.offs_k.is_same(c.offs_q) ? Tensor() : c.offs_k;
+        ctx->save_for_backward({q, k, v, unwrap(c.mask), unwrap(bias), c.offs_q, offs_k, unwrap(c.ctx), unwrap(c.tgt)});
         ctx->saved_data["ints"] = std::vector<int64_t>{c.mask_type, c.max_q, c.max_k, c.group.has_value() ? 1 : 0, c.group.value_or(0),
                                                        c.alpha.has_value() ? 1 : 0};
         ctx->saved_data["reals"] = std::vector<double>{c.silu_scale, c.alpha.value_or(1.0)};
@@ -582,8 +585,8 @@ struct JaggedFunction : torch::autograd::Function<JaggedFunction<DELTA>> {
         const auto reals = ctx->saved_data["reals"].toDoubleVector();
         const auto group = ints[3] != 0 ? std::optional<int64_t>(ints[4]) : std::nullopt;
         const auto alpha = ints[5] != 0 ? std::optional<double>(reals[1]) : std::nullopt;
-        const auto [dq, dk, dv, dbias] = op.call(grads[0], s[0], s[1], s[2], wrap(s[3]), wrap(s[4]), ints[0], ints[1], ints[2], reals[0], s[5], s[6],
-                                                 wrap(s[7]), wrap(s[8]), group, alpha);
+        const auto [dq, dk, dv, dbias] = op.call(grads[0], s[0], s[1], s[2], wrap(s[3]), wrap(s[4]), ints[0], ints[1], ints[2], reals[0], s[5],
+                                                 s[6].defined() ? s[6] : s[5], wrap(s[7]), wrap(s[8]), group, alpha);
         return {dq, dk, dv, dbias, Tensor(), Tensor()};
     }
 };

@@ -86,6 +86,29 @@ def test_memory_that_nobody_writes_is_filled_when_the_program_asks_for_it(monkey
     assert out[:3].isnan().all() and torch.equal(out[3:], want[3:])
 
 
+@pytest.mark.parametrize("delta", [False, True], ids=["equal", "delta"])
+def test_offsets_that_serve_both_sides_are_saved_once(delta, monkeypatch):
+    """Hooks that copy what is saved leave the backward with the workspace of self-attention (offsets that are one tensor)."""
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "2")
+    w = workloads.make("saved", dtype=torch.bfloat16, device=DEV, seed=5, batch=4, heads=2, dim=64, lo=500, hi=512, max_seq_len=512)
+    leaves = [t.requires_grad_() for t in (w.q, w.k, w.v)]
+    grad = torch.randn_like(w.q)
+    packed = []
+
+    def workspace(pack):
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+            if delta:
+                out = torch.ops.ops_rec.hstu_jagged.delta(*leaves, None, None, 0, 512, 512, 1.0, w.seq_offset, w.seq_offset, None, None, 0, w.alpha)
+            else:
+                out = torch.ops.ops_rec.hstu_jagged.equal(*leaves, None, None, 0, 512, 1.0, w.seq_offset, None, None, 0, w.alpha)
+        return helpers.allocated_beside(lambda: torch.autograd.grad(out, leaves, grad, retain_graph=True))
+
+    want, size = workspace(lambda t: t)
+    got, copied = workspace(lambda t: (packed.append(t), t.clone())[1])
+    assert len(packed) == 4 and copied == size > 0
+    same(got, want)
+
+
 def test_a_backward_whose_workspace_does_not_fit(monkeypatch):
     """The native kernel's answer to an allocator that has no room for the workspace is the launch order that needs none."""
     w = workloads.make("oom", dtype=torch.bfloat16, device=DEV, seed=3, batch=8, heads=4, dim=128, lo=1500, hi=2048, max_seq_len=2048)
