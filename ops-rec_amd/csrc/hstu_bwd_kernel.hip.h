@@ -126,8 +126,9 @@ __device__ __forceinline__ void slot_of(const BwdArgs& a, int slot, int n_levels
         // The workgroups of an XCD go to its shader engines in turn, whether or not they find work: with an even number of pairs
         // per XCD a pair would meet the same engines at every level, those of the short sequences (whose slots of the first
         // levels are empty) would stand idle, and the others, full, would hold up the dispatch -- so the pairs move on by one
-        // place per level, on their XCD.  8 x 8 heads, d 128, 4096..8000 rows: 320 of 512 workgroups resident through the
-        // first half of the query-tile launch -> 504, 1134 -> 939 us; key-tile launch 2274 -> 2089 us.
+        // place per level, on their XCD.  8 x 8 heads, d 128, 4096..8000 rows: 389 -> 474 of 512 workgroups resident on average over
+        // the query-tile launch, 1136 -> 989 us; key-tile launch 424 -> 432, 2219 -> 2183 us (wave-cycle counters and kernel trace);
+        // the backward 3277 -> 3102 us, 16 x 8 heads, d 256, 512..2048 rows 610 -> 518, 12 x 4, d 64, 1000..4000 rows 402 -> 391.
         if ((n_pairs & 15) == 0) {
             pair = (pair + 8 * lvl) % n_pairs;
         }

@@ -406,12 +406,13 @@ int64_t direct_slots(const hstu_jagged_fwd_params* p)
 }
 
 // Whether a plain launch does without a list, a workgroup per slot: when every slot is resident at once, and, up to the head-dim
-// slot 128, on sweeps of at most 384 keys (a list long enough for the queues takes those).  Measured, list -> slots: one slot
-// per resident workgroup at most -- 7 x 2 heads, d 64, 148 rows 10.8 -> 9.3 us, 4 x 8, d 192, 96 x 121 15.9 -> 14.2, 43 x 1, d 192,
-// 456 rows 26.8 -> 24.7, 10 x 1, d 32, 1487..2975 rows 43.1 -> 38.7; more of them on short sweeps -- 103 x 4, d 64, 142 rows 23.1 ->
-// 17.9, fp8 248 x 4, 27..64 rows 21.0 -> 19.9, 150 x 4, d 64, 100..384 rows 33.0 -> 30.2, with a bias 300 x 2, d 64, 231..299 rows 77.7 ->
-// 71.0; but 16 x 4 with a bias of 512..2048 rows 77 -> 88, d 256: 16 x 4 of 200..1000 42.5 -> 47.6 and 150 x 2 of 100..384 55 -> 67, and
-// lists of four slots per workgroup and more lose to the queues from 200 rows on (600 x 4 of 50..380 90.9 -> 97.5).
+// slot 128, on sweeps of at most 384 keys (a list long enough for the queues takes those).  Measured, launches queued back to back,
+// list -> slots: one slot per resident workgroup at most -- 7 x 2 heads, d 64, 148 rows 10.3 -> 8.1 us, 4 x 8, d 192, 96..121 rows 15.2 ->
+// 12.6, 43 x 1, d 192, 456 rows 26.6 -> 23.0, 10 x 1, d 32, 1487..2975 rows 41.5 -> 38.0; more of them on short sweeps -- 103 x 4, d 64,
+// 142 rows 22.1 -> 15.3, fp8 248 x 4, d 128, 27..64 rows 20.5 -> 16.3, 150 x 4, d 64, 100..384 rows 32.5 -> 26.8, with a bias 300 x 2,
+// d 64, 231..299 rows 72.4 -> 61.2; but 16 x 4 with a bias of 512..2048 rows 77 -> 88, d 256: 16 x 4 of 200..1000 42.5 -> 47.6 and
+// 150 x 2 of 100..384 55 -> 67, and lists of four slots per workgroup and more lose to the queues from 200 rows on (600 x 4 of 50..380
+// 90.9 -> 97.5).
 bool takes_direct_list(const Variant* var, const hstu_jagged_fwd_params* p, int64_t resident)
 {
     const int64_t slots = direct_slots(p);
@@ -498,10 +499,11 @@ uint64_t forward_workspace_bytes(const Variant* var, const hstu_jagged_fwd_param
 // fp32 inputs: how many wavefronts share the keys of one 16-row group (hstu_fwd_f32_kernel.hip.h).  As many as it takes to put
 // two wavefronts on every SIMD, at most those of a workgroup and one 16-key block each; and on long key ranges (512 keys a
 // share) more, so that the workgroups, which then own fewer rows, are many enough to even out the causal ranges -- up to
-// slots 64 until there are eight of them per CU, above (two wavefronts per SIMD as it is) two.  Measured against the kernel of
-// 128-row tiles before: 4 x 2 heads, d 64, 16..128 rows 15.6 -> 5 us (kernel time), 3 x 8 heads, d 64, 1662..1971 rows 180 -> 105 us
-// (167 without the second clause), 1 x 8, d 128, 4065 rows 603 -> 336, 2 x 4, d 32, 8113 rows 450 -> 356 (492 without), 48 x 2,
-// d 128, 1196..1350 rows 500 -> 415, 16 x 4, d 256, 170..1023 rows 368 -> 242.  The order of a row's sums depends on it, and
+// slots 64 until there are eight of them per CU, above (two wavefronts per SIMD as it is) two.  Measured, launches queued back to back,
+// against the kernel of 128-row tiles before: 4 x 2 heads, d 64, 16..128 rows 15.3 -> 6.0 us, 3 x 8 heads, d 64, 1662..1971 rows 186 ->
+// 119, 32 x 4, d 64, 256..1024 rows 123 -> 78, 115 x 1, d 128, 78 rows 20.4 -> 13.7, 1 x 8, d 128, 4065 rows 604 -> 319, 2 x 4, d 32,
+// 8113 rows 450 -> 358 (kernel time 492 without the second clause), 48 x 2, d 128, 1196..1350 rows 487 -> 426, 16 x 4, d 256,
+// 170..1023 rows 428 -> 330.  The order of a row's sums depends on it, and
 // with that the last bits on the size of the batch; HSTU_MI355_SPLIT=0 keeps one share.
 int f32_splits(const Variant* var, const hstu_jagged_fwd_params* p, int cus)
 {

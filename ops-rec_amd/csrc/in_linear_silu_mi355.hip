@@ -204,8 +204,9 @@ int validate_weight(const in_linear_silu_bwd_weight_params* p)
 // are written and read back once.  Chunks beyond eight come in whole groups of 8, one per XCD.  The estimate only has to rank
 // chunk counts: over 14 shapes of 1000 .. 300000 rows, n 256 .. 8192, k 64 .. 1024 its choice took 0.97 .. 1.12 of the best of thirteen
 // counts (worst 20000 x 1024 x 128: 33.2 against 29.7 us); below 1000 rows the eight steps bind (700 x 512 x 128: 14.3 against 9.4 us).
-// Measured, element-wise stage + column sums + library product -> the two kernels: m 20480, n 2048, k 512 187 -> 92 us (340 MB of
-// operands, d_mixed and partial outputs: 3.7 TB/s); m 95697, n 512, k 128 338 -> 76 us.
+// Measured, element-wise stage + column sums + library product -> the two kernels: m 20480, n 2048, k 512 187 -> 92 us (by the
+// counters 340 MB moved by the first kernel, 69 MB by the second, which adds the partial outputs: 84 + 14 us in a trace, 4.2 TB/s);
+// m 95697, n 512, k 128 338 -> 76 us.
 struct WeightPlan {
     int tile_k;
     int tiles;
