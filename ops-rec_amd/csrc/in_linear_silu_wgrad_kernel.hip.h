@@ -37,6 +37,7 @@ __global__ __launch_bounds__(kWgradThreads, KB >= 256 ? 2 : 4) void in_linear_si
     constexpr int kStage = R * (NB + KB);            // 16-bit elements of an LDS stage
     static_assert(XCH >= 1 && R * NB / 8 == kWgradThreads, "a step is dealt evenly over the threads");
     __shared__ __attribute__((aligned(1024))) uint16_t s_tiles[2 * kStage];
+    __shared__ __attribute__((aligned(16))) float s_sums[R * NB];  // [32 rows of a step][128 columns]
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -112,11 +113,24 @@ __global__ __launch_bounds__(kWgradThreads, KB >= 256 ? 2 : 4) void in_linear_si
         }
     };
 
+    // Column sums in two levels: a thread's sums of eight steps, then of the chunk, in LDS places of its own.  (In one chain of hundreds
+    // of additions the bias gradient came out twice as far from its 64-bit value as with the element-wise kernel's blocks of 64 rows,
+    // 3.5e-7 against 1.4e-7 at 20000 rows; in two levels 1.6e-7, at the same time per call.)
+    const bool want_sums = a.partial_sums != nullptr && first_k;
+    float* const my_sums = s_sums + erow * NB + 8 * (tid & 15);
     float sums[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         sums[e] = 0.0f;
+        my_sums[e] = 0.0f;
     }
+    auto flush_sums = [&]() {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            my_sums[e] += sums[e];
+            sums[e] = 0.0f;
+        }
+    };
     f32x16_t acc[AB][BB];
 #pragma unroll
     for (int i = 0; i < AB; ++i) {
@@ -238,6 +252,9 @@ __global__ __launch_bounds__(kWgradThreads, KB >= 256 ? 2 : 4) void in_linear_si
         if (row0 + 2 * R < rows) {
             load_step(row0 + 2 * R);
         }
+        if (want_sums && (row0 & (7 * R)) == 7 * R) {
+            flush_sums();
+        }
         __syncthreads();
         stage ^= 1;
     }
@@ -258,23 +275,18 @@ __global__ __launch_bounds__(kWgradThreads, KB >= 256 ? 2 : 4) void in_linear_si
             }
         }
     }
-    if (a.partial_sums == nullptr || !first_k) {
+    if (!want_sums) {
         return;
     }
-    __syncthreads();
-    float* const s_sums = reinterpret_cast<float*>(s_tiles);  // [32 rows][128 columns]
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        s_sums[erow * NB + 8 * (tid & 15) + e] = sums[e];
-    }
+    flush_sums();
     __syncthreads();
     if (tid < NB && n0 + tid < a.n) {
-        float total = 0.0f;
-#pragma unroll 8
+        float total[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
         for (int r = 0; r < R; ++r) {
-            total += s_sums[r * NB + tid];
+            total[r & 3] += s_sums[r * NB + tid];
         }
-        a.partial_sums[static_cast<int64_t>(chunk) * a.n + n0 + tid] = total;
+        a.partial_sums[static_cast<int64_t>(chunk) * a.n + n0 + tid] = (total[0] + total[1]) + (total[2] + total[3]);
     }
 }
 

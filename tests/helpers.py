@@ -44,17 +44,27 @@ def with_room_for(call, n_bytes, like):
     ``like`` (its results), and how many requests it refused."""
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    blocks = [torch.empty_like(t) for t in like if t is not None]
-    del blocks
     total = torch.cuda.get_device_properties(0).total_memory
-    before = torch.cuda.memory_stats()["num_ooms"]
-    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + n_bytes) / total)
+    limit = lambda n: torch.cuda.set_per_process_memory_fraction(n / total)  # noqa: E731
+    blocks = [torch.empty_like(t) for t in like if t is not None]
+    taken = []
     try:
+        limit(torch.cuda.memory_reserved())
+        for size in (1 << n for n in range(34, 19, -1)):  # (whatever is free inside blocks that live tensors keep from being given back)
+            try:
+                while True:
+                    taken.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+            except torch.cuda.OutOfMemoryError:
+                pass
+        del blocks
+        limit(torch.cuda.memory_reserved() + n_bytes)
+        before = torch.cuda.memory_stats()["num_ooms"]
         out = call()
         torch.cuda.synchronize()
+        return out, torch.cuda.memory_stats()["num_ooms"] - before
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
-    return out, torch.cuda.memory_stats()["num_ooms"] - before
+        del taken
 
 
 def backward_args(w, grad):

@@ -31,3 +31,18 @@ def test_against_the_stage_and_a_double_product(m, split, k, dtype):
     assert (weight_grad.double() - want).norm() <= 3e-3 * want.norm()
     again = _activation.silu_backward_with_weight(lin, grads, split, x, want_bias_grad=False)
     assert again[2] is None and torch.equal(again[1], weight_grad) and torch.equal(again[0], d_mixed)
+
+
+@pytest.mark.parametrize("m,n,k", [(20000, 1024, 16), (20000, 8192, 1024), (30001, 8192, 512), (4096, 16384, 1024)])
+def test_column_sums_are_as_close_to_64_bits_as_the_stage_alone(m, n, k):
+    """A chunk of a wide weight is thousands of rows long: its sums are taken in two levels, as close to the 64-bit sums as those of the
+    element-wise kernel, which adds blocks of 64 rows (within a quarter: the two round at other places)."""
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    split = [n // 4] * 4
+    lin = torch.randn(m, n, generator=g, device=DEV).bfloat16()
+    grads = [torch.randn(m, n // 4, generator=g, device=DEV).bfloat16() for _ in split]
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    sums, stage = _activation.silu_backward_with_weight(lin, grads, split, x)[2], _activation.silu_backward_stage(lin, grads, split)[1]
+    z, s = lin.double(), torch.sigmoid(lin.double())
+    want = (torch.cat(grads, 1).double() * s * (1 + z * (1 - s))).sum(0)
+    assert (sums.double() - want).norm() <= 1.25 * (stage.double() - want).norm()
