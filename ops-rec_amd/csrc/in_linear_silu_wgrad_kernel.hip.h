@@ -5,7 +5,7 @@
 //
 // The contraction runs over the m rows of the batch -- tens of thousands -- into an output of a few hundred tiles at most, so
 // the rows are cut into chunks and every (chunk, tile) has a workgroup; the fp32 partial outputs go through the workspace and
-// a second kernel adds them in chunk order (the same bits every launch).  As a library product with one workgroup per output
+// a second kernel adds them in a fixed order (the same bits every launch).  As a library product with one workgroup per output
 // tile this took 134 us at m = 20480, n = 2048, k = 512 (104 workgroups), behind 48 us for the element-wise stage and 5 us for
 // the column sums; here the three together: see the dispatch rule in in_linear_silu_mi355.hip.
 //
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kWgradThreads, KB >= 256 ? 2 : 4) void in_linear_si
     }
 }
 
-// weight_grad and bias_grad = the partial outputs added in chunk order.  A thread owns four consecutive elements (k is a
+// weight_grad and bias_grad = the partial outputs, added in one order whatever finished first: eight chunks pairwise at a time.  A thread owns four consecutive elements (k is a
 // multiple of 16); its loads of eight chunks are in flight together.
 template <typename Tag>
 __global__ __launch_bounds__(256) void in_linear_silu_wgrad_sum_kernel(const InLinearSiluWgradArgs a)
@@ -310,10 +310,7 @@ __global__ __launch_bounds__(256) void in_linear_silu_wgrad_sum_kernel(const InL
             for (int u = 0; u < 8; ++u) {
                 v[u] = from[(c + u) * stride];
             }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                total += v[u];
-            }
+            total += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
         }
         for (; c < a.chunks; ++c) {
             total += from[c * stride];
