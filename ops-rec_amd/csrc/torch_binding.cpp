@@ -506,7 +506,7 @@ Gradients in_linear_silu_backward(const Tensor& x, const Tensor& weight, const O
             if (rc == HSTU_OK) {
                 if (const Tensor ws = empty_or_none(ws_bytes, x.device()); ws.defined()) {
                     rc = in_linear_silu_bwd_weight(&p, ws.data_ptr(), ws_bytes, stream_of(x));
-                } else {  // no room for the partial weight gradients (up to 1 GiB): the library product needs none
+                } else {  // no room for the partial weight gradients: the library product needs none
                     library = true;
                 }
             }

@@ -81,3 +81,12 @@ def test_building_loads_no_library_that_it_replaces():
         "assert not [line for line in open('/proc/self/maps') if 'libhstu_mi355' in line]\n"
     )
     subprocess.run([sys.executable, "-c", code], cwd=root, check=True, timeout=120)
+
+
+def test_a_packet_of_unknown_layout_is_left_as_it_is():
+    from ops_rec import _ops
+
+    packet = type("Packet", (), {})()
+    _ops._pick_overload_by_argument(packet, 8)
+    assert not vars(packet)
+    assert torch.ops.ops_rec.hstu_jagged._op.__name__ == "call"  # (and this torch's layout is known)
