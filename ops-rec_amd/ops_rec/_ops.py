@@ -10,8 +10,8 @@ Mirrors the reference adapter for this path
 * device tensors dispatch on the ``CUDA`` key (PyTorch-ROCm's key for HIP tensors): to the native kernels of
   ``csrc/torch_binding.cpp`` where a call needs no check to fail and no conversion, and from there to the functions
   of this module otherwise (``_dispatch.py``); shape
-  inference for ``torch.compile`` on ``Meta`` (``:269-351``); autograd is attached from Python
-  (``ops_rec/autograd/hstu_v1_autograd.py``), not here (``:258-263``).
+  inference for ``torch.compile`` on ``Meta`` (``:269-351``); autograd is attached by the native kernels' file and, for
+  everything else, from Python (``ops_rec/autograd/hstu_v1_autograd.py``), not here (``:258-263``).
 
 There is no CPU implementation: calling the op on CPU tensors raises, as it does in the
 reference (which registers only the NPU and Meta keys).

@@ -2,7 +2,9 @@
 
 The forward operators carry no autograd kernel of their own; this module binds
 ``hstu_jagged_backward`` as their formula with ``torch.library.register_autograd`` so that
-``loss.backward()`` works in eager mode and under ``torch.compile``.  Behaviour follows the
+``loss.backward()`` works in eager mode and under ``torch.compile``.  For device tensors of the jagged forms a C++
+node with the same formula stands in front of it where the binding is built (``csrc/torch_binding.cpp``); ``hstu_dense`` runs
+on the one here.  Behaviour follows the
 reference wrapper (ascendc/attention/hstu_v1/torch_extension/hstu_v1_autograd.py:53-374):
 
 * what is saved: q, k, v, mask, attn_bias, the offsets, num_context, num_target + the scalars;
