@@ -14,6 +14,8 @@ constexpr int bwd_dkv_wgs_per_cu(int d, bool rab, bool mask) { return (!rab && !
 // the dK workgroups that read dS back from memory keep neither V nor dO nor the score blocks: 90 / 148 / 137 registers
 // and 16 / 32 / 64 KB of LDS at the head-dim slots 64 / 128 / 256
 constexpr int bwd_dk_from_ds_wgs_per_cu(int d) { return d <= 64 ? 4 : (d <= 128 ? 3 : 2); }
+constexpr int bwd_kv_fused_wgs_per_cu(int d) { return d <= 128 ? 2 : 1; }
+constexpr int bwd_dq_from_ds_wgs_per_cu(int d) { return d <= 64 ? 4 : (d <= 128 ? 3 : 2); }
 constexpr int bwd_dq_wgs_per_cu(int d, bool rab, bool mask) { return (!(rab && mask) && d <= 64) ? 3 : (d <= 128 ? 2 : 1); }
 // resident workgroups per CU of the forward kernel (registers and LDS): without bias or custom mask four for the
 // head-dim slot 32 (127 registers, 25 KB of LDS) and three for 64 (168 registers, 45 KB); three for the slot 32 with
@@ -128,6 +130,13 @@ struct BwdArgs {
     // Order of the (tile level, pair) slots in the grids of the tuned 16-bit kernels (hstu_bwd_kernel.hip.h, slot_of):
     // 0 = level after level (heaviest tiles of all pairs first), 1 = pair after pair, the pairs dealt to the 8 XCDs.
     int pair_major;
+    // dS handed from the key-tile kernel to the query-tile kernel (hstu_bwd_fused_kernel.hip.h): the tiles, how many per head, whether a
+    // row group holds those up to its diagonal only, and the query heads of this pair of launches
+    void* ds_tiles;
+    int64_t ds_head_tiles;
+    int ds_tri;
+    int head_first;
+    int head_count;
     float* partial;  // S and dP summed over the first window, fp32, for the launch that adds the second (or null)
     int64_t drab_clear_bytes;  // > 0: the key-tile kernel clears this many bytes at drab beside its work
     const void* offs_q;

@@ -349,6 +349,64 @@ __device__ __forceinline__ void store_tile_rows(uint16_t* stage, const f32x16_t 
     }
 }
 
+// 32 values of a row of an attn_bias-shaped tensor, packed in accumulator order (words 2 g, 2 g + 1 of lane (row, lh): the keys
+// c0 + 8 g + 4 lh + 0 .. 3), to memory, up to the sequence's last key.  `row_off` leaves the descriptor for rows past the sequence.
+__device__ __forceinline__ void store_bias_row_values(const __amdgpu_buffer_rsrc_t rsrc, const uint32_t (&pk)[8], uint32_t row_off, int c0,
+                                                      int lh, int sk, int vec_ok)
+{
+    if (vec_ok == 2) {
+        // 16-byte aligned rows: the two lanes of a row trade halves (v_permlane32_swap), so that each holds 8
+        // consecutive keys and a store instruction writes whole 32-byte sectors of 32 rows instead of 16-byte
+        // pieces.  Lane (row, 0) ends up with keys 16 h2 + 0..7, lane (row, 1) with keys 16 h2 + 8..15.
+        typedef __attribute__((ext_vector_type(2))) unsigned u2_t;
+#pragma unroll
+        for (int h2 = 0; h2 < 2; ++h2) {
+            const u2_t r0 = __builtin_amdgcn_permlane32_swap(pk[4 * h2 + 0], pk[4 * h2 + 2], false, false);
+            const u2_t r1 = __builtin_amdgcn_permlane32_swap(pk[4 * h2 + 1], pk[4 * h2 + 3], false, false);
+            const u32x4_t w4 = {r0[0], r1[0], r0[1], r1[1]};
+            const int key = c0 + 16 * h2 + 8 * lh;
+            const uint32_t off = row_off + static_cast<uint32_t>(key) * 2u;
+            __builtin_amdgcn_raw_buffer_store_b128(w4, rsrc, static_cast<int>(key < sk ? off : kOutOfRange), 0, 0);
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int key = c0 + 8 * g + 4 * lh;
+            const uint32_t off = row_off + static_cast<uint32_t>(key) * 2u;
+            if (vec_ok != 0) {
+                const u32x2_t w2 = {pk[2 * g], pk[2 * g + 1]};
+                __builtin_amdgcn_raw_buffer_store_b64(w2, rsrc, static_cast<int>(key < sk ? off : kOutOfRange), 0, 0);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t word = pk[2 * g + i / 2];
+                    const uint16_t val = static_cast<uint16_t>((i & 1) ? (word >> 16) : (word & 0xffffu));
+                    __builtin_amdgcn_raw_buffer_store_b16(val, rsrc, static_cast<int>(key + i < sk ? off + 2u * i : kOutOfRange), 0, 0);
+                }
+            }
+        }
+    }
+}
+
+// The same rows written as the accumulators hold them, 8 bytes at a time: for outputs that are not 16-byte aligned.
+template <typename Tag, int D>
+__device__ __forceinline__ void store_tile_pieces(const f32x16_t (&acc)[D / 32], const __amdgpu_buffer_rsrc_t rsrc, uint32_t first_row_off,
+                                                  uint32_t stride, int dim_limit, int lane)
+{
+    const uint32_t row_off = first_row_off + static_cast<uint32_t>(lane & 31) * stride;
+#pragma unroll
+    for (int mt = 0; mt < D / 32; ++mt) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int d0 = 32 * mt + 8 * g + 4 * (lane >> 5);
+            u32x2_t w;
+            w[0] = pack2<Tag>(acc[mt][4 * g + 0], acc[mt][4 * g + 1]);
+            w[1] = pack2<Tag>(acc[mt][4 * g + 2], acc[mt][4 * g + 3]);
+            __builtin_amdgcn_raw_buffer_store_b64(w, rsrc, static_cast<int>(d0 < dim_limit ? row_off + d0 * 2u : kOutOfRange), 0, 0);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // dQ (and d rab)
 // ---------------------------------------------------------------------------------------------------------
@@ -753,39 +811,7 @@ __global__ __launch_bounds__(256, bwd_dq_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void 
             }
         }
         if constexpr (WANT_DRAB && !WANT_P) {
-            if (vec16) {
-                // 16-byte aligned rows: the two lanes of a row trade halves (v_permlane32_swap), so that each holds 8
-                // consecutive keys and a store instruction writes whole 32-byte sectors of 32 rows instead of 16-byte
-                // pieces.  Lane (row, 0) ends up with keys 16 h2 + 0..7, lane (row, 1) with keys 16 h2 + 8..15.
-                typedef __attribute__((ext_vector_type(2))) unsigned u2_t;
-#pragma unroll
-                for (int h2 = 0; h2 < 2; ++h2) {
-                    const u2_t r0 = __builtin_amdgcn_permlane32_swap(pk[4 * h2 + 0], pk[4 * h2 + 2], false, false);
-                    const u2_t r1 = __builtin_amdgcn_permlane32_swap(pk[4 * h2 + 1], pk[4 * h2 + 3], false, false);
-                    const u32x4_t w4 = {r0[0], r1[0], r0[1], r1[1]};
-                    const int key = c0 + 16 * h2 + 8 * lh;
-                    const uint32_t off = bias_row_off + static_cast<uint32_t>(key) * 2u;
-                    __builtin_amdgcn_raw_buffer_store_b128(w4, drab_rsrc, static_cast<int>(key < sk ? off : kOutOfRange), 0, 0);
-                }
-            } else {
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int key = c0 + 8 * g + 4 * lh;
-                    const uint32_t off = bias_row_off + static_cast<uint32_t>(key) * 2u;
-                    if (vec) {
-                        const u32x2_t w2 = {pk[2 * g], pk[2 * g + 1]};
-                        __builtin_amdgcn_raw_buffer_store_b64(w2, drab_rsrc, static_cast<int>(key < sk ? off : kOutOfRange), 0, 0);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const uint32_t word = pk[2 * g + i / 2];
-                            const uint16_t val = static_cast<uint16_t>((i & 1) ? (word >> 16) : (word & 0xffffu));
-                            __builtin_amdgcn_raw_buffer_store_b16(val, drab_rsrc,
-                                                                  static_cast<int>(key + i < sk ? off + 2u * i : kOutOfRange), 0, 0);
-                        }
-                    }
-                }
-            }
+            store_bias_row_values(drab_rsrc, pk, bias_row_off, c0, lh, sk, a.bias_vec_ok);
         }
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
@@ -826,19 +852,7 @@ __global__ __launch_bounds__(256, bwd_dq_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void 
         uint16_t* const stage = wave == 0 ? s_k0 : (wave == 1 ? s_k1 : (wave == 2 ? s_k2 : s_v0));
         store_tile_rows<Tag, D>(stage, dq_acc, dq_rsrc, static_cast<uint32_t>(wr0) * q_stride, q_stride, a.d_qk, lane);
     } else {
-        const uint32_t row_off = static_cast<uint32_t>(wr0 + ln) * q_stride;
-#pragma unroll
-        for (int mt = 0; mt < MTILES; ++mt) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d0 = 32 * mt + 8 * g + 4 * lh;
-                const uint32_t off = (d0 < a.d_qk) ? row_off + d0 * 2u : kOutOfRange;
-                u32x2_t w;
-                w[0] = pack2<Tag>(dq_acc[mt][4 * g + 0], dq_acc[mt][4 * g + 1]);
-                w[1] = pack2<Tag>(dq_acc[mt][4 * g + 2], dq_acc[mt][4 * g + 3]);
-                __builtin_amdgcn_raw_buffer_store_b64(w, dq_rsrc, static_cast<int>(off), 0, 0);
-            }
-        }
+        store_tile_pieces<Tag, D>(dq_acc, dq_rsrc, static_cast<uint32_t>(wr0) * q_stride, q_stride, a.d_qk, lane);
     }
 }
 
@@ -1379,18 +1393,7 @@ __global__ __launch_bounds__(kDkvThreads, (MODE == 2 || MODE >= 4) ? bwd_dk_from
         uint16_t* const stage = wave == 0 ? s_st0 : (wave == 1 ? s_st1 : (wave == 2 ? s_st2 : s_st3));
         store_tile_rows<Tag, D>(stage, acc, out_rsrc, static_cast<uint32_t>(cw0) * out_stride, out_stride, out_dim, lane);
     } else {
-        const uint32_t row_off = static_cast<uint32_t>(key) * out_stride;
-#pragma unroll
-        for (int mt = 0; mt < MTILES; ++mt) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d0 = 32 * mt + 8 * g + 4 * lh;
-                u32x2_t w;
-                w[0] = pack2<Tag>(acc[mt][4 * g + 0], acc[mt][4 * g + 1]);
-                w[1] = pack2<Tag>(acc[mt][4 * g + 2], acc[mt][4 * g + 3]);
-                __builtin_amdgcn_raw_buffer_store_b64(w, out_rsrc, static_cast<int>(d0 < out_dim ? row_off + d0 * 2u : kOutOfRange), 0, 0);
-            }
-        }
+        store_tile_pieces<Tag, D>(acc, out_rsrc, static_cast<uint32_t>(cw0) * out_stride, out_stride, out_dim, lane);
     }
 }
 

@@ -108,7 +108,7 @@ void read_switches()
     g_switches.split = switch_digit("HSTU_MI355_SPLIT", 1);
     g_switches.short_lists = switch_digit("HSTU_MI355_SHORT", 1);
     g_switches.generic_backward = switch_digit("HSTU_MI355_GENERIC_BACKWARD", 1);
-    g_switches.bwd_handoff = switch_digit("HSTU_MI355_BWD_HANDOFF", 2);
+    g_switches.bwd_handoff = switch_digit("HSTU_MI355_BWD_HANDOFF", 3);
     const char* const mb = getenv("HSTU_MI355_BWD_WORKSPACE_MB");
     g_switches.bwd_workspace_mb = (mb != nullptr && mb[0] >= '0' && mb[0] <= '9') ? atoll(mb) : -1;
     g_switches.bwd_pair_major = switch_digit("HSTU_MI355_BWD_PAIR_MAJOR", 1);
@@ -128,6 +128,12 @@ int64_t workspace_cap_mb(bool large = false)
 {
     const long long set = switches().bwd_workspace_mb;
     return set >= 0 ? static_cast<int64_t>(set) : (large ? 16384 : 2048);
+}
+// The same for the order that hands dS alone over, whose tiles hold half as much: a call with more takes several pairs of launches.
+int64_t fused_cap_mb()
+{
+    const long long set = switches().bwd_workspace_mb;
+    return set >= 0 ? static_cast<int64_t>(set) : 4096;
 }
 
 
@@ -827,6 +833,64 @@ static PairPlane pair_plane(const hstu_jagged_fwd_params* f)
     return pp;
 }
 
+// The order with dS handed over (hstu_bwd_fused_kernel.hip.h): the size of its tiles, and how many query heads of the call a pair of
+// launches takes so that they fit the limit.
+struct DsTiles {
+    bool tri;
+    int64_t head_tiles;
+    int64_t heads;  // per pair of launches, whole K/V heads; 0: no room for one
+    int64_t bytes;
+};
+static DsTiles ds_tiles(const hstu_jagged_fwd_params* f, int64_t cap)
+{
+    DsTiles t;
+    const int64_t n_blk = (f->max_seq_len_k + 31) / 32;
+    t.tri = f->mask_type == HSTU_MASK_TRIL && f->num_context == nullptr && f->seq_offset_k == f->seq_offset_q &&
+            f->total_k == f->total_q && f->max_seq_len_q <= f->max_seq_len_k;
+    const int64_t groups = f->total_q / 32 + (f->n_offsets - 1);
+    t.head_tiles = t.tri ? (groups * (n_blk + 1) + 1) / 2 : groups * n_blk;
+    const int64_t ratio = f->num_heads_q / f->num_heads_k;
+    const int64_t group_bytes = ratio * t.head_tiles * 2048;  // of the query heads of a K/V head
+    const int64_t fit = std::min(f->num_heads_k, cap / std::max<int64_t>(group_bytes, 1));
+    const int64_t launches = fit > 0 ? (f->num_heads_k + fit - 1) / fit : 0;
+    t.heads = launches > 0 ? (f->num_heads_k + launches - 1) / launches * ratio : 0;
+    t.bytes = t.heads * t.head_tiles * 2048;
+    return t;
+}
+static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* p, const BwdVariant* var)
+{
+    const hstu_jagged_fwd_params* f = &p->fwd;
+    const int64_t dmax = f->head_dim_qk > f->head_dim_v ? f->head_dim_qk : f->head_dim_v;
+    if ((f->dtype != HSTU_DT_BF16 && f->dtype != HSTU_DT_FP16) || f->attn_bias != nullptr || p->grad_attn_bias != nullptr ||
+        f->mask_type == HSTU_MASK_CUSTOM || dmax > 256 || f->head_dim_qk % 8 != 0 || f->head_dim_v % 8 != 0 || is_generic_bwd(var) ||
+        var->dq_ds_p == nullptr) {
+        return nullptr;
+    }
+    return &hstu::bwd_variants_fused()[f->dtype == HSTU_DT_BF16 ? 0 : 1][dmax <= 64 ? 0 : (dmax <= 128 ? 1 : 2)];
+}
+
+// Calls whose key-tile launch is a few workgroups that one sweep of all query rows (times query heads per K/V head) keeps busy long after
+// the machine has emptied: there the planes order, whose long launch has a workgroup per query tile and head, is the shorter one.
+// Grouped heads, K/V tiles of 128 keys (us, planes / dS handed over): 16 x 8 heads on 2, 256..1024 rows, d 128, 160 tiles 131 / 158, d 64
+// 111 / 124; 16 x 8 on 1, 1024 rows, 128 tiles 276 / 301; 4 x 8 on 2, 2048..4096 rows, 192 tiles 631 / 575; 32 x 8 on 2, 256..1024 rows, 320
+// tiles 234 / 185; 8 x 8 on 4, 1024 rows, 256 tiles 102 / 100 -- the line is at three quarters of the compute units.  One query head per
+// K/V head: only short rows at the slot 128, where the planes order has its 64-row query tiles: 2 x 1, 300 rows 22.5 / 25.4; 8 x 2, 200..300
+// rows, 40 tiles 22.6 / 24.9; 4 x 4, 300..700 rows, 70 tiles 39.6 / 38.5; 1 x 4, 1000 rows, 32 tiles 55.6 / 52.9.
+static bool few_key_tiles(const hstu_jagged_fwd_params* f)
+{
+    int cus = 0;
+    if (compute_units(&cus) != HSTU_OK) {
+        cus = 256;
+    }
+    const int64_t batch = f->n_offsets - 1;
+    const int64_t dmax = f->head_dim_qk > f->head_dim_v ? f->head_dim_qk : f->head_dim_v;
+    const int64_t tiles = (f->total_k + 64 * batch) / 128 * f->num_heads_k;
+    if (f->num_heads_q > f->num_heads_k) {
+        return 4 * tiles < 3LL * cus;
+    }
+    return dmax > 64 && dmax <= 128 && tiles <= 64 && f->total_q <= 512 * batch;
+}
+
 // estimated microseconds of the three launch orders (see above)
 struct BwdCost {
     double two, three, planes;
@@ -934,7 +998,7 @@ static BwdPlan plan_bwd(const hstu_jagged_bwd_params* p, const BwdVariant* var)
     const bool planes_fit = pp.fits_32 && pp.bytes <= cap && (!bias_grad || var->dv_dk_from_planes_drab != nullptr);
     const BwdPlan three = {kThreeLaunches, static_cast<uint64_t>(ds_plane)};
     const BwdPlan planes = {kPlanes, static_cast<uint64_t>(pp.bytes)};
-    if (forced == 2) {
+    if (forced >= 2) {
         return planes_fit ? planes : (three_fits ? three : two);
     }
     if (forced == 1) {
@@ -960,6 +1024,36 @@ static BwdPlan plan_bwd(const hstu_jagged_bwd_params* p, const BwdVariant* var)
         return best_small;
     }
     return best;
+}
+
+// The tiles of the order that hands dS alone over, for a call that takes it when it has `room` bytes of workspace: none (heads == 0) where
+// another order is the faster one or is asked for.  5 products and 4 bytes of traffic per pair beside the operands, where the planes
+// order has 5 and 8: measured on 66 shapes (us, best other order -> this one) 32 x 4 heads of 256..1024 rows, d 128 100 -> 79, 16 x 4 of
+// 512..2048 210 -> 126, 8 x 8 of 4096..8000 2909 -> 2005, 32 x 8 of 1024 rows, d 64 244 -> 195, 16 x 4 of 501 rows and 1000 keys, d 64 62 -> 44,
+// 32 x 4 of 256..1024, d 256 191 -> 135, 256 x 4 of 40..200 88 -> 69; behind on few_key_tiles() only.
+static DsTiles fused_plan(const hstu_jagged_bwd_params* p, const BwdVariant* var, int64_t room)
+{
+    const hstu_jagged_fwd_params* f = &p->fwd;
+    const DsTiles none = {false, 0, 0, 0};
+    const int forced = switches().bwd_handoff;
+    if (fused_variant(p, var) == nullptr || (forced >= 0 && forced != 3) || f->total_q == 0 || f->total_k == 0) {
+        return none;
+    }
+    const DsTiles t = ds_tiles(f, room);
+    if (forced == 3 || t.heads == 0) {
+        return t;
+    }
+    // (a share of the heads that leaves the machine half empty costs more than the products it saves)
+    int cus = 0;
+    if (compute_units(&cus) != HSTU_OK) {
+        cus = 256;
+    }
+    const int64_t batch = f->n_offsets - 1;
+    const int64_t tiles = (f->total_k + 64 * batch) / 128 * (t.heads * f->num_heads_k / f->num_heads_q);
+    if ((t.heads < f->num_heads_q && tiles < 4LL * cus) || few_key_tiles(f)) {
+        return none;
+    }
+    return t;
 }
 
 // The query-tile kernel with 64-row tiles (hstu_bwd_dq_short_kernel.hip.h) where it is the faster one: 16-bit inputs at
@@ -1116,6 +1210,23 @@ HSTU_API int hstu_jagged_bwd_workspace_size(const hstu_jagged_bwd_params* params
     }
     const WindowPlan windows = plan_windows(params);
     *workspace_bytes = windows.var != nullptr ? windows.workspace_bytes : plan_bwd(params, var).workspace_bytes;
+    return HSTU_OK;
+}
+
+HSTU_API int hstu_jagged_bwd_best_workspace_size(const hstu_jagged_bwd_params* params, uint64_t* workspace_bytes)
+{
+    const int rc = hstu_jagged_bwd_workspace_size(params, workspace_bytes);
+    unsigned one_launch_threads = 0;
+    if (rc != HSTU_OK || bwd_one_launch_variant(params, &one_launch_threads) != nullptr) {
+        return rc;
+    }
+    const BwdVariant* const var = select_bwd(params);
+    if (plan_windows(params).var == nullptr) {
+        const DsTiles tiles = fused_plan(params, var, fused_cap_mb() * (1LL << 20));
+        if (tiles.heads > 0) {
+            *workspace_bytes = static_cast<uint64_t>(tiles.bytes);
+        }
+    }
     return HSTU_OK;
 }
 
@@ -1280,6 +1391,29 @@ HSTU_API int hstu_jagged_bwd(const hstu_jagged_bwd_params* p, void* workspace, u
     const int64_t grid_q = static_cast<int64_t>(a.n_qtiles) * (a.pair_major ? 8 * ((pairs_q + 7) / 8) : pairs_q);
     if (grid_kv > 0x7fffffffLL || grid_q > 0x7fffffffLL) {
         return fail(HSTU_ERR_INVALID, "grid out of range");
+    }
+    const DsTiles tiles = generic || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace == nullptr
+                              ? DsTiles{false, 0, 0, 0}
+                              : fused_plan(p, var, static_cast<int64_t>(std::min<uint64_t>(workspace_bytes, INT64_MAX)));
+    if (tiles.heads > 0 && grid_kv > 0 && grid_q > 0) {
+        const hstu::BwdFusedVariant* const fv = fused_variant(p, var);
+        a.ds_tiles = workspace;
+        a.ds_head_tiles = tiles.head_tiles;
+        a.ds_tri = tiles.tri ? 1 : 0;
+        for (int first = 0; first < a.n_heads_q; first += static_cast<int>(tiles.heads)) {
+            a.head_first = first;
+            a.head_count = std::min(static_cast<int>(tiles.heads), a.n_heads_q - first);
+            const int64_t pq = static_cast<int64_t>(a.n_batch) * a.head_count, pk = pq / a.head_ratio;
+            const int64_t kv_slots = static_cast<int64_t>(a.n_ktiles) * (a.pair_major ? 8 * ((pk + 7) / 8) : pk);
+            const int64_t q_slots = static_cast<int64_t>(a.n_qtiles) * (a.pair_major ? 8 * ((pq + 7) / 8) : pq);
+            hipLaunchKernelGGL(fv->kv, dim3(static_cast<unsigned>(kv_slots)), dim3(hstu::kDkvThreads), 0, static_cast<hipStream_t>(stream), a);
+            hipLaunchKernelGGL(fv->dq, dim3(static_cast<unsigned>(q_slots)), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+        }
+        const hipError_t err_f = hipGetLastError();
+        if (err_f != hipSuccess) {
+            return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", fv->name, hipGetErrorString(err_f));
+        }
+        return HSTU_OK;
     }
     if (generic) {
         // the generic kernels write what they compute and nothing else: every output starts from zero

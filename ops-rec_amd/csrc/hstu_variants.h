@@ -46,6 +46,14 @@ struct DqShortVariant {
     void (*dq_ds_p)(const BwdArgs);  // storing dS and P for the key-tile workgroups that read them back
 };
 
+// the five products in two launches with dS handed over (hstu_bwd_fused_kernel.hip.h)
+struct BwdFusedVariant {
+    const char* name;
+    void (*kv)(const BwdArgs);       // dK and dV, storing dS
+    void (*dq)(const BwdArgs);       // dQ from that dS
+    void (*dq_drab)(const BwdArgs);  // the same, dS also to the attn_bias gradient
+};
+
 struct BwdVariant {
     const char* name;
     void (*dkv)(const BwdArgs);
@@ -89,6 +97,8 @@ const Variant* fwd_variants_generic();
 // backward: [rab][custom mask][dim slot: 64, 128, 256]
 const BwdVariant (*bwd_variants_bf16())[2][3];
 const BwdVariant (*bwd_variants_f16())[2][3];
+// backward with dS handed over, 16-bit inputs without bias or custom mask: [bf16, fp16][head-dim slot 64, 128, 256]
+const BwdFusedVariant (*bwd_variants_fused())[3];
 // backward, query-tile kernel for short rows: [bf16, fp16]
 const DqShortVariant* bwd_variants_dq_short();
 // backward for batches of sequences of at most 32 rows and keys (one workgroup of kTinyThreads per (sequence, K/V head)),

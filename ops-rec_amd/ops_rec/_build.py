@@ -27,7 +27,11 @@ SOURCES = [
     "hstu_kernels_fwd_short.hip",
     "hstu_kernels_bwd_bf16.hip",
     "hstu_kernels_bwd_f16.hip",
+    "hstu_kernels_bwd_fused.hip",
 ]
+# These kernels name the accumulator registers they keep their sums in (hstu_pinned_acc.hip.h); every other matrix result belongs in
+# vector registers, where the compiler would otherwise keep it in accumulators as well and copy each element out.
+SOURCE_FLAGS = {"hstu_kernels_bwd_fused.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form=1")}
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -81,7 +85,7 @@ def build(verbose: bool = False, jobs: int | None = None, extra_flags: tuple = (
         objects = [os.path.join(obj_dir, os.path.splitext(s)[0] + ".o") for s in SOURCES]
         with ThreadPoolExecutor(max_workers=jobs) as pool:
             jobs_done = [
-                pool.submit(_run, [hipcc, *HIPCC_FLAGS, *extra_flags, "-c", os.path.join(CSRC, s), "-o", o], verbose)
+                pool.submit(_run, [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(s, ()), *extra_flags, "-c", os.path.join(CSRC, s), "-o", o], verbose)
                 for s, o in zip(SOURCES, objects)
             ]
             for j in jobs_done:

@@ -26,6 +26,7 @@ EXPORTED_SYMBOLS = (
     "hstu_version",
     "hstu_jagged_fwd_kernel_name",
     "hstu_jagged_bwd_workspace_size",
+    "hstu_jagged_bwd_best_workspace_size",
     "hstu_jagged_bwd",
     "hstu_paged_fwd_workspace_size",
     "hstu_paged_fwd",
@@ -234,8 +235,9 @@ def load() -> ctypes.CDLL:
     lib.hstu_version.argtypes = []
     lib.hstu_jagged_fwd_kernel_name.restype = ctypes.c_char_p
     lib.hstu_jagged_fwd_kernel_name.argtypes = [ctypes.POINTER(FwdParams)]
-    lib.hstu_jagged_bwd_workspace_size.restype = ctypes.c_int
-    lib.hstu_jagged_bwd_workspace_size.argtypes = [ctypes.POINTER(BwdParams), ctypes.POINTER(ctypes.c_uint64)]
+    for size in (lib.hstu_jagged_bwd_workspace_size, lib.hstu_jagged_bwd_best_workspace_size):
+        size.restype = ctypes.c_int
+        size.argtypes = [ctypes.POINTER(BwdParams), ctypes.POINTER(ctypes.c_uint64)]
     lib.hstu_jagged_bwd.restype = ctypes.c_int
     lib.hstu_jagged_bwd.argtypes = [ctypes.POINTER(BwdParams), ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
     lib.hstu_paged_fwd_workspace_size.restype = ctypes.c_int

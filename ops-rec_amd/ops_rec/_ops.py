@@ -522,9 +522,9 @@ def _backward_hip(grad, q, k, v, mask, attn_bias, mask_type, max_seq_len_q, max_
     p.grad, p.grad_q, p.grad_k, p.grad_v, p.grad_attn_bias = _ptr(g_c), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dbias)
     lib = _native.load()
     ws_bytes = ctypes.c_uint64(0)
-    rc = lib.hstu_jagged_bwd_workspace_size(ctypes.byref(p), ctypes.byref(ws_bytes))
+    rc = lib.hstu_jagged_bwd_best_workspace_size(ctypes.byref(p), ctypes.byref(ws_bytes))
     if rc != _native.HSTU_OK:
-        raise RuntimeError(f"hstu_jagged_bwd_workspace_size failed ({rc}): {_native.last_error()}")
+        raise RuntimeError(f"hstu_jagged_bwd_best_workspace_size failed ({rc}): {_native.last_error()}")
     _launch_backward(p, ws_bytes.value, q_c.device)
     # (cached when every tensor was taken as it came: the next call with this description only patches addresses in)
     same = (q_c is q and k_c is k and v_c is v and g_c is grad and offs_q is seq_offset and

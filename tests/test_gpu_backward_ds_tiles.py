@@ -1,0 +1,115 @@
+"""The backward's order that hands dS alone from the key-tile kernel to the query-tile kernel (hstu_bwd_fused_kernel.hip.h, forced with
+HSTU_MI355_BWD_HANDOFF=3): against torch autograd on the CPU oracle and the library's generic kernels (the bars of
+test_gpu_backward.py, the workspace full of NaN), and against the order that recomputes everything."""
+
+import dataclasses
+
+import pytest
+import torch
+
+import helpers
+from ops_rec import workloads
+from test_gpu_backward import DEV, check, device_grads, make
+
+pytestmark = pytest.mark.gpu
+
+
+def grad_for(w, seed=6):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return torch.randn(w.q.shape[0], w.q.shape[1], w.v.shape[2], generator=g, device=DEV).to(w.q.dtype)
+
+
+def against_recomputing(w, monkeypatch):
+    grad_out = grad_for(w)
+    helpers.set_switch(monkeypatch, "HSTU_MI355_GENERIC_BACKWARD", "0")
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "0")
+    two = device_grads(w, grad_out)
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+    got, beside = helpers.allocated_beside(lambda: device_grads(w, grad_out))
+    assert beside >= 2048  # the tiles
+    # S is formed with its operands the other way round and dS is rounded before dQ's product, as before dK's: one rounding of the
+    # input type in the terms of a sum
+    tol = 1e-2 if w.q.dtype == torch.bfloat16 else 2e-3
+    for a, b in zip(got[:3], two[:3]):
+        torch.testing.assert_close(a.float(), b.float(), atol=tol * b.float().abs().max().item(), rtol=tol)
+    return got
+
+
+CASES = {
+    "tile_edges": dict(batch=9, dim=128, lo=0, hi=0, lengths=[1, 31, 32, 33, 127, 128, 129, 257, 384], max_seq_len=384),
+    "tile_edges_64": dict(batch=9, dim=64, lo=0, hi=0, lengths=[1, 31, 32, 33, 127, 128, 129, 257, 384], max_seq_len=384),
+    "tile_edges_256": dict(batch=8, dim=256, lo=0, hi=0, lengths=[1, 31, 33, 95, 127, 129, 160, 257], max_seq_len=257),
+    "loose_bound": dict(batch=5, dim=128, lo=70, hi=300, max_seq_len=1000),
+    "empty_sequences": dict(batch=5, dim=64, lo=0, hi=0, lengths=[0, 200, 0, 0, 65], max_seq_len=200),
+    "grouped_heads": dict(batch=3, dim=128, heads=6, heads_k=2, lo=66, hi=300, max_seq_len=300),
+    "dims_40_48": dict(batch=3, dim=40, dim_v=48, heads=3, lo=66, hi=300, max_seq_len=300),
+    "dims_72_128": dict(batch=3, dim=72, dim_v=128, lo=66, hi=300, max_seq_len=301),
+    "dims_128_16": dict(batch=3, dim=128, dim_v=16, lo=66, hi=300, max_seq_len=300),
+    "dims_200_144": dict(batch=3, dim=200, dim_v=144, lo=66, hi=300, max_seq_len=300),
+    "context_targets_groups": dict(batch=4, dim=128, lo=150, hi=400, max_seq_len=400, num_context=37, max_target=50, target_group_size=3),
+    "context_in_the_first_block": dict(batch=4, dim=64, lo=150, hi=400, max_seq_len=400, num_context=5, max_target=1, target_group_size=1),
+    "targets": dict(batch=4, dim=256, lo=100, hi=260, max_seq_len=260, max_target=70, target_group_size=1),
+    "int64_offsets": dict(batch=4, dim=64, lo=70, hi=260, max_seq_len=260, index_dtype=torch.int64),
+}  # fmt: skip
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_causal(name, dtype, monkeypatch):
+    kw = dict(CASES[name])
+    w = make(heads=kw.pop("heads", 2), seed=len(name), dtype=dtype, **kw)
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", "0")
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+    check(w, monkeypatch)
+    against_recomputing(w, monkeypatch)
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("mask_type", [0, 2], ids=["causal", "none"])
+@pytest.mark.parametrize("lq,lk", [([70, 200, 1, 96], [370, 333, 129, 96]), ([300, 129, 40], [65, 200, 0])], ids=["more_keys", "fewer_keys"])
+def test_key_offsets_of_their_own(dim, mask_type, lq, lk, monkeypatch):
+    g = torch.Generator(device=DEV).manual_seed(dim)
+    mk = lambda n, d: (torch.randn(n, 2, d, generator=g, device=DEV) * 0.5).to(torch.bfloat16)  # noqa: E731
+    offs = lambda ls: torch.tensor([0] + list(torch.tensor(ls).cumsum(0)), dtype=torch.int64, device=DEV)  # noqa: E731
+    w = workloads.Workload(name="delta", q=mk(sum(lq), dim), k=mk(sum(lk), dim), v=mk(sum(lk), dim), seq_offset=offs(lq),
+                           max_seq_len=max(lq), silu_scale=1.0, alpha=dim**-0.5, seq_offset_k=offs(lk), max_seq_len_k=max(lk), lengths=lq,
+                           mask_type=mask_type)  # fmt: skip
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", "0")
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+    check(w, monkeypatch)
+    against_recomputing(w, monkeypatch)
+
+
+@pytest.mark.parametrize("heads_k", [4, 2], ids=["own", "grouped"])
+def test_heads_over_several_launches(heads_k, monkeypatch):
+    """With room for some of the heads the tiles are used by one share of them after the other: the same bits."""
+    w = make(batch=5, heads=4, heads_k=heads_k, dim=64, lo=100, hi=600, max_seq_len=600, seed=3)
+    grad_out = grad_for(w)
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_WORKSPACE_MB", None)
+    whole, room = helpers.allocated_beside(lambda: device_grads(w, grad_out))
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_WORKSPACE_MB", str(room // 2 // 2**20 + 1))
+    helpers.poison_workspace(monkeypatch)
+    shares, less = helpers.allocated_beside(lambda: device_grads(w, grad_out))
+    assert 0 < less <= 0.6 * room
+    assert all(torch.equal(a, b) for a, b in zip(whole[:3], shares[:3]))
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_rows_and_keys_that_belong_to_no_tile(dim, monkeypatch):
+    """Rows ahead of the first offset and past max_seq_len are not written, rows past the last offset are zero, and a row of dO that is
+    infinite reaches the keys it sees and no tile that it does not."""
+    w = make(batch=3, heads=2, dim=dim, lo=200, hi=260, max_seq_len=260, seed=4)
+    grad_out = grad_for(w)
+    row = int(w.seq_offset[1]) + 70  # a row of the second sequence: its keys 0 .. 70
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+    clean = device_grads(w, grad_out)
+    bad = grad_out.clone()
+    bad[row, 0] = float("inf")
+    dirty = device_grads(dataclasses.replace(w), bad)
+    first = int(w.seq_offset[1])
+    for a, b in zip(clean[1:3], dirty[1:3]):
+        assert not torch.isfinite(b[first : first + 64, 0]).all()
+        keep = torch.ones(a.shape[0], dtype=torch.bool, device=DEV)
+        keep[first : first + 96] = False  # (the 32-key blocks that the row's 32-row block touches)
+        assert torch.equal(a[keep], b[keep]) and torch.equal(a[:, 1], b[:, 1])

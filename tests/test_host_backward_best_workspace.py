@@ -1,0 +1,75 @@
+"""hstu_jagged_bwd_best_workspace_size (no GPU needed): 2 KiB per head and 32 x 32 block of dS where the call takes the order that hands
+dS alone over, and what hstu_jagged_bwd_workspace_size says elsewhere."""
+
+import ctypes
+
+import pytest
+
+import helpers
+from ops_rec import _native
+from test_host_boundary import _copy_fwd, _valid_params
+
+FAKE = 0x1000
+BATCH = dict(n_offsets=33, num_heads_q=4, num_heads_k=4, total_q=20292, total_k=20292, max_seq_len_q=1024, max_seq_len_k=1024)
+
+
+def sizes(grad_attn_bias=None, **fwd):
+    b = _native.new_bwd_params()
+    f = _valid_params()
+    for k, v in fwd.items():
+        setattr(f, k, v)
+    if grad_attn_bias is not None:
+        f.attn_bias = FAKE
+    _copy_fwd(b.fwd, f)
+    b.grad = b.grad_q = b.grad_k = b.grad_v = FAKE
+    b.grad_attn_bias = grad_attn_bias
+    ws = (ctypes.c_uint64 * 2)()
+    for i, size in enumerate((_native.load().hstu_jagged_bwd_workspace_size, _native.load().hstu_jagged_bwd_best_workspace_size)):
+        assert size(ctypes.byref(b), ctypes.cast(ctypes.byref(ws, 8 * i), ctypes.POINTER(ctypes.c_uint64))) == 0, _native.last_error()
+    return tuple(ws)
+
+
+def tiles(rows=20292, batch=32, heads=4, blocks=32, below_diagonal=True):
+    groups = rows // 32 + batch
+    return heads * 2048 * ((groups * (blocks + 1) + 1) // 2 if below_diagonal else groups * blocks)
+
+
+@pytest.fixture(autouse=True)
+def no_switches(monkeypatch):
+    for name in ("HSTU_MI355_BWD_HANDOFF", "HSTU_MI355_BWD_WORKSPACE_MB", "HSTU_MI355_SHORT", "HSTU_MI355_GENERIC_BACKWARD"):
+        helpers.set_switch(monkeypatch, name, None)
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_tiles(dim):
+    call = dict(BATCH, head_dim_qk=dim, head_dim_v=dim)
+    assert sizes(**call)[1] == tiles()
+    assert sizes(**dict(call, mask_type=2))[1] == tiles(below_diagonal=False)
+    assert sizes(**dict(call, num_context=FAKE))[1] == tiles(below_diagonal=False)
+    assert sizes(**dict(call, seq_offset_k=FAKE + 64))[1] == tiles(below_diagonal=False)
+    assert sizes(**dict(call, max_seq_len_k=900))[1] == tiles(blocks=29, below_diagonal=False)  # (more query rows than keys in a sequence)
+
+
+def test_as_the_other_orders_elsewhere():
+    for call in (dict(BATCH, head_dim_qk=512, head_dim_v=512), dict(BATCH, dtype=_native.DT_FP32, out_dtype=_native.DT_FP32),
+                 dict(BATCH, total_q=600, total_k=600, max_seq_len_q=32, max_seq_len_k=32),
+                 dict(BATCH, n_offsets=3, total_q=500, total_k=500, max_seq_len_q=300, max_seq_len_k=300),  # a few workgroups
+                 dict(BATCH, n_offsets=5, total_q=2000, total_k=2000, num_heads_k=1)):  # fmt: skip
+        size, best = sizes(**call)
+        assert size == best
+
+
+def test_limits_and_switches(monkeypatch):
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_WORKSPACE_MB", "60")
+    size, best = sizes(**BATCH)  # room for two of the four heads, whose share of the launch would leave the machine half empty
+    assert size == best
+    long = dict(BATCH, n_offsets=65, total_q=64 * 4096, total_k=64 * 4096, max_seq_len_q=4096, max_seq_len_k=4096)
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_WORKSPACE_MB", "3000")
+    assert sizes(**long)[1] == tiles(rows=64 * 4096, batch=64, blocks=128, heads=2)  # two pairs of launches of two heads
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_WORKSPACE_MB", None)
+    for order in ("0", "1", "2"):
+        helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", order)
+        size, best = sizes(**BATCH)
+        assert size == best
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+    assert sizes(**dict(BATCH, n_offsets=3, total_q=500, total_k=500))[1] == tiles(rows=500, batch=2)
