@@ -137,6 +137,8 @@ struct BwdArgs {
     int ds_tri;
     int head_first;
     int head_count;
+    int drab_lines;  // the query-tile launch writes the attn_bias gradient 128 bytes of a row at a time
+    int clear_wgs;  // leading workgroups of that key-tile launch that clear the attn_bias gradient, a multiple of 8
     float* partial;  // S and dP summed over the first window, fp32, for the launch that adds the second (or null)
     int64_t drab_clear_bytes;  // > 0: the key-tile kernel clears this many bytes at drab beside its work
     const void* offs_q;

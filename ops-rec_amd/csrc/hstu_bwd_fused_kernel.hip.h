@@ -19,6 +19,8 @@
 // 2.0 + 0.9 ms of the kernels that recompute.  Ordinary ones the vector unit and the longest workgroup: 32 x 4 heads, d 128, 256..1024
 // rows 62 + 21 us, where the query-tile kernel with dS and P took 61 and the kernels that read them 41.  A wavefront with 64 keys and
 // all 512 registers, one per SIMD, took as long as this one (1.39 ms at the large shape) and has half as many workgroups.
+// With attn_bias memory bounds the key-tile kernel: 16 x 4 heads, d 128, 512..2048 rows 890 MB (415 of zeros, 122 of dS, 306 fetched) in
+// 205 us = 4.3 TB/s; the call 364 -> 280 us, where dV, dQ storing dS and dK from it took 185 + 139 + 61.
 // The query-tile kernel moves dS once: 4.4 TB/s from memory at the large shape (0.64 ms), 0.35 of that from the cache.
 #pragma once
 #include "hstu_bwd_kernel.hip.h"
@@ -72,7 +74,47 @@ __device__ __forceinline__ bool row_sees(uint32_t visible, int e)
     return __builtin_amdgcn_inverse_ballot_w64((static_cast<uint64_t>(up) << 32) | lo);
 }
 
-template <typename Tag, int D>
+// 16 bytes of attn_bias per lane straight into registers, as assembly for the reason the tile requests are: the kernel waits for them by
+// count.  The registers pass through, so that whatever read them before has been issued, and hold the values once the wait is over.
+template <int OFFSET>
+__device__ __forceinline__ void request_bias(u32x4_t& dst, u32x4_t rsrc, uint32_t voffset)
+{
+    asm volatile("buffer_load_dwordx4 %0, %1, %2, 0 offen offset:%3" : "+v"(dst) : "v"(voffset), "s"(rsrc), "n"(OFFSET));
+}
+
+// Clears what hstu_bwd_dq_from_ds_kernel does not write of the attn_bias gradient: in the rows of a 32-row group, the keys past the blocks
+// that the group's tiles cover; rows past their sequence whole.  Workgroup `wg` of `n_wgs` takes its share of the groups, a wavefront a
+// row at a time.  (max_k a multiple of 8, the gradient on a 16-byte boundary.)
+__device__ __forceinline__ void clear_unswept(const BwdArgs& a, int wg, int n_wgs, int wave, int lane)
+{
+    typedef uint32_t piece_t __attribute__((ext_vector_type(4)));
+    const piece_t zero = {0u, 0u, 0u, 0u};
+    const int groups = (a.max_q + 31) / 32;
+    const int64_t n_items = static_cast<int64_t>(a.n_batch) * a.n_heads_q * groups;
+    const int row_pieces = a.max_k / 8;
+    for (int64_t item = static_cast<int64_t>(wg) * 4 + wave; item < n_items; item += static_cast<int64_t>(n_wgs) * 4) {
+        const int64_t plane = item / groups;
+        const int r0 = static_cast<int>(item - plane * groups) * 32;
+        const SeqInfo si = load_seq(a, uniform(static_cast<int>(plane / a.n_heads_q)));
+        int limit = r0 < si.sq ? (swept_key_limit(a, si, r0) + 31) & ~31 : 0;
+        limit = limit < si.sk ? limit : si.sk;
+        piece_t* const first = reinterpret_cast<piece_t*>(static_cast<uint16_t*>(a.drab) + (plane * a.max_q + r0) * a.max_k);
+        const int rows = a.max_q - r0 < 32 ? a.max_q - r0 : 32;
+        if (limit == 0) {  // whole rows: one run
+            for (int i = lane; i < rows * row_pieces; i += 64) {
+                __builtin_nontemporal_store(zero, first + i);
+            }
+            continue;
+        }
+        for (int r = 0; r < rows; ++r) {
+            for (int i = (r0 + r < si.sq ? limit / 8 : 0) + lane; i < row_pieces; i += 64) {
+                __builtin_nontemporal_store(zero, first + static_cast<int64_t>(r) * row_pieces + i);
+            }
+        }
+    }
+}
+
+template <typename Tag, int D, bool HAS_RAB = false>
 __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_bwd_kv_fused_kernel(const BwdArgs a)
 {
     typedef SubTile<D> T;
@@ -93,11 +135,21 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     const int grid_heads = a.head_count / a.head_ratio;
     const int per_level = a.n_batch * grid_heads;
     int kt_idx, rem;
-    slot_of(a, static_cast<int>(blockIdx.x), a.n_ktiles, per_level, kt_idx, rem);
+    slot_of(a, static_cast<int>(blockIdx.x) - (HAS_RAB ? a.clear_wgs : 0), a.n_ktiles, per_level, kt_idx, rem);
     const int b = rem / grid_heads;
     const int hk = a.head_first / a.head_ratio + rem - b * grid_heads;
     zero_tail_rows(a.dk, a.offs_k, a.n_batch, a.idx64, a.total_k, static_cast<int64_t>(a.n_heads_k) * a.d_qk, kDkvThreads);
     zero_tail_rows(a.dv, a.offs_k, a.n_batch, a.idx64, a.total_k, static_cast<int64_t>(a.n_heads_k) * a.d_v, kDkvThreads);
+    if constexpr (HAS_RAB) {
+        if (static_cast<int>(blockIdx.x) < a.clear_wgs) {
+            if (a.bias_vec_ok == 2) {
+                clear_unswept(a, static_cast<int>(blockIdx.x), a.clear_wgs, wave, lane);
+            } else {
+                clear_share(a.drab, a.drab_clear_bytes, blockIdx.x, static_cast<unsigned>(a.clear_wgs), tid, kDkvThreads);
+            }
+            return;
+        }
+    }
     if (rem >= per_level) {
         return;
     }
@@ -197,6 +249,31 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             }
         }
     };
+    // attn_bias of the next step's block: lane (ln, lh) has row ln, keys 8 lh .. + 7 and 16 + 8 lh .. + 7 (past the row's end the next row's,
+    // which no key of the sequence takes)
+    u32x4_t bias[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+    const uint32_t bias_pitch = static_cast<uint32_t>(a.max_k) * 2u;
+    const uint32_t bias_lane = (HAS_RAB && cw0 + 8 * lh < a.max_k) ? static_cast<uint32_t>(ln) * bias_pitch + (cw0 + 8 * lh) * 2u : kOutOfRange;
+    const uint8_t* bias_head = static_cast<const uint8_t*>(a.rab) + (HAS_RAB ? bias_plane_of(a, b, first_h) * 2 : 0);
+    int bias_left = n_iter, bias_x = x_first;
+    auto next_bias = [&]() {
+        const u32x4_t rsrc = make_rsrc_words(bias_head, static_cast<uint32_t>(a.max_q) * bias_pitch);
+        const uint32_t off = bias_lane + (bias_left > 0 ? static_cast<uint32_t>(bias_x * 32) * bias_pitch : kOutOfRange);
+        request_bias<0>(bias[0], rsrc, off);
+        request_bias<32>(bias[1], rsrc, off);
+        --bias_left;
+        if (++bias_x == x_skip_from) {
+            bias_x = x_skip_to;
+        }
+        if (bias_x >= n_qsub) {
+            bias_x = x_first;
+            bias_head += static_cast<int64_t>(a.max_q) * bias_pitch;
+        }
+    };
+    // The product with a 0/1 matrix that moves a lane's pieces to its keys (see hstu_bwd_dkv_kernel): the element of k-slot (lh, e) of
+    // product j that is 1 is e = ln - 16 j - 8 lh.  Eight registers for the whole sweep are not to be had: a block works it out.
+    const uint32_t one = (std::is_same<Tag, bf16_tag>::value ? 0x3f80u : 0x3c00u) << (16 * (ln & 1));  // 1.0 in the input type, in its half
+    const int one_word = (ln - 8 * lh) >> 1;  // (8 lh is even; words 0 .. 3 of product 0, 8 .. 11 of product 1)
     // The sub-tiles all of whose rows see all keys of this wavefront: from the first whose first row does, past the context rows, up to
     // those with target rows or without 32 rows.  The others take the general path.
     int full_from = n_qsub, full_to = 0;
@@ -220,6 +297,9 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     const ScoreConsts sconst = score_consts(a.alpha, a.scale);
     u32x4_t kf[KSTEPS];
     if (n_iter > 0) {
+        if constexpr (HAS_RAB) {
+            next_bias();
+        }
         request(0);
         request(1);
         const u32x4_t v_rsrc = make_rsrc_words(static_cast<const uint8_t*>(a.v) + v_first, v_bytes);
@@ -239,6 +319,9 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             kf[js] = __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, static_cast<int>(d0 < a.d_qk ? k_off + d0 * 2u : kOutOfRange), 0, 0);
         }
         __builtin_amdgcn_s_waitcnt(0);  // (everything, once: the compiler does not know of the requests in assembly)
+        if constexpr (HAS_RAB) {
+            asm volatile("" : "+v"(bias[0]), "+v"(bias[1]));
+        }
     }
 
     auto read_n = [&](const uint16_t* tile, int first_off, int js) -> u32x4_t {
@@ -258,20 +341,23 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     const uint32_t ds_lane = static_cast<uint32_t>(ln * 32 + lh * 16);
 #define HSTU_FENCE() __builtin_amdgcn_sched_barrier(0)
 
-    auto block = [&](auto masked, const uint16_t* q_tile, int rq0) {
+    auto block = [&](auto masked, const uint16_t* q_tile, int rq0, const f32x16_t& s_first) {
         constexpr bool kMasked = decltype(masked)::value;
         const uint16_t* const g_tile = q_tile + T::ELEMS;
         uint32_t pk[8], ds[8];
         f32x16_t s, dp;
         // The operands that come from LDS, kAhead slots of one MFMA ahead of their use across the phases: Q plain, dO plain, dO and Q
         // transposed; V, which only dP reads, kAheadV slots ahead.
-        constexpr int kAhead = 2, kAheadV = 2;
+        constexpr int kAhead = HAS_RAB ? 1 : 2, kAheadV = HAS_RAB ? 1 : 2;
         u32x4_t op[kAhead + 1], vo[kAheadV + 1];
         acc_fence<kAccRegs>();
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             s[i] = 0.f;
             dp[i] = 0.f;
+        }
+        if constexpr (HAS_RAB) {
+            s = s_first;
         }
         uint32_t visible = 0;  // (masked blocks) lane = row: its visible keys
         if constexpr (kMasked) {
@@ -427,16 +513,43 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     auto step = [&](const uint16_t* q_tile, int stage_o) {
         // this step's sub-tile has landed for everybody; the stage of the previous step is free
         HSTU_FENCE();
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW) : "memory");
+        if constexpr (HAS_RAB) {
+            asm volatile("s_waitcnt vmcnt(%2)" : "+v"(bias[0]), "+v"(bias[1]) : "n"(2 * LPW) : "memory");
+        } else {
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPW) : "memory");
+        }
         __builtin_amdgcn_s_barrier();
         HSTU_FENCE();
+        f32x16_t s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = 0.f;
+        }
+        if constexpr (HAS_RAB) {
+            // the matrix pipe transposes the bias into the scores' accumulators; its registers take the next block's at once
+            int word = one_word;
+            asm volatile("" : "+v"(word));
+            u32x4_t route[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    route[j][i] = word == 8 * j + i ? one : 0u;
+                }
+            }
+            s = mfma32<Tag>(bias[0], route[0], s);
+            s = mfma32<Tag>(bias[1], route[1], s);
+            asm volatile("" : "+v"(s));
+            HSTU_FENCE();
+            next_bias();
+        }
         request(stage_o);
         const int x = cur_x;
         HSTU_FENCE();
         if (x >= full_from && x < full_to) {
-            block(std::false_type{}, q_tile, x * 32);
+            block(std::false_type{}, q_tile, x * 32, s);
         } else if (cw0 < swept_key_limit(a, si, x * 32)) {  // (otherwise nothing is visible: the query-tile kernel does not read this tile)
-            block(std::true_type{}, q_tile, x * 32);
+            block(std::true_type{}, q_tile, x * 32, s);
         }
         if (++cur_x == x_skip_from) {
             cur_x = x_skip_to;
@@ -465,6 +578,9 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
         }
     }
 
+    if constexpr (HAS_RAB) {
+        asm volatile("s_waitcnt vmcnt(0)" : "+v"(bias[0]), "+v"(bias[1]) : : "memory");  // (the last request lands before its registers are used again)
+    }
     acc_settle();
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -570,8 +686,20 @@ __global__ __launch_bounds__(256, bwd_dq_from_ds_wgs_per_cu(D)) void hstu_bwd_dq
     const uint32_t bias_bytes = static_cast<uint32_t>(a.max_q) * static_cast<uint32_t>(a.max_k) * 2u;
     const __amdgpu_buffer_rsrc_t drab_rsrc =
         make_rsrc(WANT_DRAB ? static_cast<uint16_t*>(a.drab) + bias_plane_of(a, b, h) : nullptr, WANT_DRAB ? bias_bytes : 0u);
-    const uint32_t bias_row_off =
-        (wr0 + ln < sq) ? static_cast<uint32_t>(wr0 + ln) * static_cast<uint32_t>(a.max_k) * 2u : kOutOfRange;
+    // 8 keys of a row of the gradient, up to the sequence's last; `end`: the first key past those that the wavefront writes now
+    auto store_piece = [&](const u32x4_t& w, int row, int key, int end) {
+        const uint32_t off = (static_cast<uint32_t>(row) * static_cast<uint32_t>(a.max_k) + static_cast<uint32_t>(key)) * 2u;
+        const bool write = row < sq && key < sk;
+        __builtin_amdgcn_raw_buffer_store_b128(w, drab_rsrc, static_cast<int>(write && key + 8 <= a.max_k ? off : kOutOfRange), 0, 0);
+        if (end > a.max_k) {  // (a piece that would reach into the next row: its keys one by one)
+            const bool part = write && key + 8 > a.max_k;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint16_t value = static_cast<uint16_t>(e % 2 ? w[e / 2] >> 16 : w[e / 2] & 0xffffu);
+                __builtin_amdgcn_raw_buffer_store_b16(value, drab_rsrc, static_cast<int>(part && key + e < sk ? off + 2u * e : kOutOfRange), 0, 0);
+            }
+        }
+    };
 
     f32x16_t acc[MTILES];
 #pragma unroll
@@ -581,6 +709,7 @@ __global__ __launch_bounds__(256, bwd_dq_from_ds_wgs_per_cu(D)) void hstu_bwd_dq
             acc[mt][i] = 0.f;
         }
     }
+    u32x4_t even[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};  // (WANT_DRAB) the pieces of an even step, until the odd one's are there
     const uint32_t ring_lds = lds_address(s_ring);
     auto request = [&](int stage, int x) {
         const uint32_t base = ring_lds + static_cast<uint32_t>(stage) * (kStageElems * 2u);
@@ -627,7 +756,56 @@ __global__ __launch_bounds__(256, bwd_dq_from_ds_wgs_per_cu(D)) void hstu_bwd_dq
             acc[mt] = mfma32<Tag>(kt, pb, acc[mt]);
         }
         if constexpr (WANT_DRAB) {
-            store_bias_row_values(drab_rsrc, pk, bias_row_off, x * 32, lh, sk, a.bias_vec_ok);
+            // The two lanes of a row trade halves (see store_bias_row_values): 8 keys of a row per lane and piece.  Rows start at multiples
+            // of four bytes, which is what a 16-byte store needs.
+            typedef __attribute__((ext_vector_type(2))) unsigned u2_t;
+            u32x4_t now[2];
+#pragma unroll
+            for (int h2 = 0; h2 < 2; ++h2) {
+                const u2_t d0 = __builtin_amdgcn_permlane32_swap(pk[4 * h2 + 0], pk[4 * h2 + 2], false, false);
+                const u2_t d1 = __builtin_amdgcn_permlane32_swap(pk[4 * h2 + 1], pk[4 * h2 + 3], false, false);
+                now[h2] = u32x4_t{d0[0], d1[0], d0[1], d1[1]};
+            }
+            if (a.drab_lines == 0 || ((x & 1) == 0 && x + 1 >= nx_w)) {
+#pragma unroll
+                for (int h2 = 0; h2 < 2; ++h2) {
+                    store_piece(now[h2], wr0 + ln, x * 32 + 16 * h2 + 8 * lh, x * 32 + 32);
+                }
+            } else {
+                // Whole lines: the blocks of an even step and the odd one behind it leave together, 64 keys = 128 bytes of a row, eight
+                // rows an instruction.  The pieces go through the wavefront's own dS tile of this step, whose values are in registers
+                // by now, 16 rows at a time.
+                if ((x & 1) == 0) {
+                    even[0] = now[0];
+                    even[1] = now[1];
+                    return;
+                }
+                uint8_t* const stage = reinterpret_cast<uint8_t*>(const_cast<uint16_t*>(ds_tile));
+                const int c0 = (x - 1) * 32;
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    if ((ln >> 4) == half) {
+                        const int r = ln & 15;
+#pragma unroll
+                        for (int h2 = 0; h2 < 2; ++h2) {
+                            *reinterpret_cast<u32x4_t*>(stage + r * 128 + (((2 * h2 + lh) ^ (r & 7)) * 16)) = even[h2];
+                            *reinterpret_cast<u32x4_t*>(stage + r * 128 + (((4 + 2 * h2 + lh) ^ (r & 7)) * 16)) = now[h2];
+                        }
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int r = i * 8 + (lane >> 3);
+                        const u32x4_t piece = *reinterpret_cast<const u32x4_t*>(stage + r * 128 + (((lane & 7) ^ (r & 7)) * 16));
+                        store_piece(piece, wr0 + 16 * half + r, c0 + 8 * (lane & 7), c0 + 64);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                }
+            }
         }
     };
     if (n_sub > 0) {

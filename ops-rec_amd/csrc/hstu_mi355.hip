@@ -861,12 +861,25 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
 {
     const hstu_jagged_fwd_params* f = &p->fwd;
     const int64_t dmax = f->head_dim_qk > f->head_dim_v ? f->head_dim_qk : f->head_dim_v;
-    if ((f->dtype != HSTU_DT_BF16 && f->dtype != HSTU_DT_FP16) || f->attn_bias != nullptr || p->grad_attn_bias != nullptr ||
-        f->mask_type == HSTU_MASK_CUSTOM || dmax > 256 || f->head_dim_qk % 8 != 0 || f->head_dim_v % 8 != 0 || is_generic_bwd(var) ||
+    // (attn_bias: rows that start at multiples of four bytes, which 16-byte loads and stores need)
+    const bool bias_ok = f->attn_bias == nullptr || (reinterpret_cast<uintptr_t>(f->attn_bias) % 4 == 0 && f->max_seq_len_k % 2 == 0 &&
+                                                     reinterpret_cast<uintptr_t>(p->grad_attn_bias) % 4 == 0);
+    if ((f->dtype != HSTU_DT_BF16 && f->dtype != HSTU_DT_FP16) || !bias_ok || f->mask_type == HSTU_MASK_CUSTOM || dmax > 256 || f->head_dim_qk % 8 != 0 || f->head_dim_v % 8 != 0 || is_generic_bwd(var) ||
         var->dq_ds_p == nullptr) {
         return nullptr;
     }
     return &hstu::bwd_variants_fused()[f->dtype == HSTU_DT_BF16 ? 0 : 1][dmax <= 64 ? 0 : (dmax <= 128 ? 1 : 2)];
+}
+
+// Workgroups of the key-tile launch that do nothing but clear the attn_bias gradient: at the front of the grid, so that the zeros go out
+// beside the products from the start.  The fewer products a byte of the gradient comes with, the more of them (us of the backward with
+// 64 / 96 / 128): 16 x 4 heads, d 128, 512..2048 rows 287 / 290 / 296; 32 x 4 of
+// 256..1024 154 / 153 / 149; d 64 130 / - / 113; 64 x 4, d 64, 64..512 rows 82 / - / 68.  (Dealt over all workgroups ahead of their sweeps,
+// as the other orders have it, the zeros hold up every one of them: the dV launch alone takes 185 us at the first shape.)
+static int clear_workgroups(int64_t bytes, int64_t dmax, int cus)
+{
+    const int64_t most = dmax <= 64 ? cus / 2 : (dmax <= 128 ? 3 * cus / 8 : cus / 4);
+    return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, bytes >> 20) / 8 * 8));
 }
 
 // Calls whose key-tile launch is a few workgroups that one sweep of all query rows (times query heads per K/V head) keeps busy long after
@@ -885,6 +898,11 @@ static bool few_key_tiles(const hstu_jagged_fwd_params* f)
     const int64_t batch = f->n_offsets - 1;
     const int64_t dmax = f->head_dim_qk > f->head_dim_v ? f->head_dim_qk : f->head_dim_v;
     const int64_t tiles = (f->total_k + 64 * batch) / 128 * f->num_heads_k;
+    if (f->attn_bias != nullptr) {
+        // (its rows then go through two launches in every order: 16 x 8 on 2, 256..1024 rows, d 64 226 / 184; 3 x 2, 100..304 rows 32 / 28;
+        // 2 x 4 on 2, 60..136 rows, d 256 34 / 36)
+        return false;
+    }
     if (f->num_heads_q > f->num_heads_k) {
         return 4 * tiles < 3LL * cus;
     }
@@ -1400,14 +1418,28 @@ HSTU_API int hstu_jagged_bwd(const hstu_jagged_bwd_params* p, void* workspace, u
         a.ds_tiles = workspace;
         a.ds_head_tiles = tiles.head_tiles;
         a.ds_tri = tiles.tri ? 1 : 0;
+        int cus = 0;
+        if (compute_units(&cus) != HSTU_OK) {
+            return HSTU_ERR_RUNTIME;
+        }
+        // (rows of the gradient as whole lines from two query tiles per compute unit on: 16 x 4 heads of 512..2048 rows, query-tile kernel
+        // 105 -> 79 us; a launch as long as one workgroup waits for the way through LDS: 2 x 4 of 2000..4000 rows, the call 269 -> 281 us)
+        a.drab_lines = f->total_q / hstu::kBlockM * f->num_heads_q >= 2LL * cus ? 1 : 0;
         for (int first = 0; first < a.n_heads_q; first += static_cast<int>(tiles.heads)) {
             a.head_first = first;
             a.head_count = std::min(static_cast<int>(tiles.heads), a.n_heads_q - first);
             const int64_t pq = static_cast<int64_t>(a.n_batch) * a.head_count, pk = pq / a.head_ratio;
             const int64_t kv_slots = static_cast<int64_t>(a.n_ktiles) * (a.pair_major ? 8 * ((pk + 7) / 8) : pk);
             const int64_t q_slots = static_cast<int64_t>(a.n_qtiles) * (a.pair_major ? 8 * ((pq + 7) / 8) : pq);
-            hipLaunchKernelGGL(fv->kv, dim3(static_cast<unsigned>(kv_slots)), dim3(hstu::kDkvThreads), 0, static_cast<hipStream_t>(stream), a);
-            hipLaunchKernelGGL(fv->dq, dim3(static_cast<unsigned>(q_slots)), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+            a.drab_clear_bytes = drab_bytes;
+            a.clear_wgs = drab_bytes > 0 && first == 0 ? clear_workgroups(drab_bytes, std::max(f->head_dim_qk, f->head_dim_v), cus) : 0;
+            if (kv_slots + a.clear_wgs > 0x7fffffffLL || q_slots > 0x7fffffffLL) {
+                return fail(HSTU_ERR_INVALID, "grid out of range");
+            }
+            hipLaunchKernelGGL(f->attn_bias != nullptr ? fv->kv_rab : fv->kv, dim3(static_cast<unsigned>(kv_slots + a.clear_wgs)),
+                               dim3(hstu::kDkvThreads), 0, static_cast<hipStream_t>(stream), a);
+            hipLaunchKernelGGL(p->grad_attn_bias != nullptr ? fv->dq_drab : fv->dq, dim3(static_cast<unsigned>(q_slots)), dim3(256), 0,
+                               static_cast<hipStream_t>(stream), a);
         }
         const hipError_t err_f = hipGetLastError();
         if (err_f != hipSuccess) {

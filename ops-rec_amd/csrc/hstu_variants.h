@@ -50,6 +50,7 @@ struct DqShortVariant {
 struct BwdFusedVariant {
     const char* name;
     void (*kv)(const BwdArgs);       // dK and dV, storing dS
+    void (*kv_rab)(const BwdArgs);   // the same with attn_bias, clearing what dq_drab does not write of its gradient
     void (*dq)(const BwdArgs);       // dQ from that dS
     void (*dq_drab)(const BwdArgs);  // the same, dS also to the attn_bias gradient
 };
@@ -97,7 +98,7 @@ const Variant* fwd_variants_generic();
 // backward: [rab][custom mask][dim slot: 64, 128, 256]
 const BwdVariant (*bwd_variants_bf16())[2][3];
 const BwdVariant (*bwd_variants_f16())[2][3];
-// backward with dS handed over, 16-bit inputs without bias or custom mask: [bf16, fp16][head-dim slot 64, 128, 256]
+// backward with dS handed over, 16-bit inputs without custom mask: [bf16, fp16][head-dim slot 64, 128, 256]
 const BwdFusedVariant (*bwd_variants_fused())[3];
 // backward, query-tile kernel for short rows: [bf16, fp16]
 const DqShortVariant* bwd_variants_dq_short();
