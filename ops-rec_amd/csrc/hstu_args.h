@@ -89,6 +89,7 @@ struct FwdArgs {
     const float* q_descale;  // fp8 inputs only; per head, nullptr = 1
     const float* k_descale;
     const float* v_descale;
+    int pair_major;          // kernels of one workgroup per slot: the slots pair after pair (0: level after level)
     int f32_splits;          // fp32 inputs only: wavefronts that share the keys of one row group (a power of two up to f32_waves)
     unsigned int* counters;  // kCounterBlockBytes at the head of the workspace, the queues' part cleared ahead of the launch; null for the plain list
     uint64_t launch_id;      // split variant: the launch's number, 1 .. 2^48 - 1, above the counts of its arrival counters

@@ -445,6 +445,41 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
     return var->kernel_queues != nullptr && n_blocks >= 4 * resident;
 }
 
+// The kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): 16-bit inputs at the slot 256 without bias and custom mask, more
+// slots than a launch without a list takes.  It has no list that sorts the sequences, so it takes batches whose mean lengths are at least
+// half of the largest (a Zipf law of lengths up to 8192 with a mean of an eighth: 416 -> 761 us), and, where the sequences are long, only
+// those with little between them and pairs enough for all XCDs (6 x 2 heads, 3000..6000 rows: 209 -> 258 us; 32 x 2, 1000..4000 326 -> 340).
+// *pair_major: the tiles of a pair side by side on one XCD, once the K / V rows are about what the last-level cache holds (24 x 8 heads
+// of 512..2048 rows, 244 MB: 272 us before, 261 level after level, 227 pair after pair; 12 x 8 of 2048 rows, 201 MB: 290, 224, 247), or on
+// keys that are mostly history, where a pair's tiles are equally long and nothing is lost at the end (30 x 8, 300 rows on 600 keys: 87, 76, 60).
+// Measured list -> this kernel, launches queued back to back: 200 x 4 of 65..128 rows 57.8 -> 36.5 us, 48 x 4 of 129..512 rows 55.3 -> 37.2,
+// 16 x 4 of 512..2048 rows 95.2 -> 90.8, 32 x 2 of the same 98.0 -> 98.7, 24 x 8 of 1024 rows 187 -> 143, 64 x 4 of 1000..4000 rows 1192 -> 1029.
+const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool* pair_major)
+{
+    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || var->d_pad != 256 || var->persistent_wgs_per_cu <= 0 ||
+        p->attn_bias != nullptr || p->mask != nullptr || p->mask_type == HSTU_MASK_CUSTOM) {
+        return nullptr;
+    }
+    int cus = 0;
+    if (compute_units(&cus) != HSTU_OK) {
+        return nullptr;
+    }
+    const int64_t slots = direct_slots(p);
+    if (takes_direct_list(var, p, static_cast<int64_t>(cus) * wgs_per_cu(var, p)) || slots > (1LL << 22)) {
+        return nullptr;
+    }
+    const int64_t batch = p->n_offsets - 1;
+    if (2 * p->total_q < batch * p->max_seq_len_q || 2 * p->total_k < batch * p->max_seq_len_k) {
+        return nullptr;
+    }
+    const int64_t kv_bytes = p->total_k * p->num_heads_k * (p->head_dim_qk + p->head_dim_v) * 2;
+    *pair_major = kv_bytes >= (224LL << 20) || p->total_k >= 2 * p->total_q;
+    if (!*pair_major && p->max_seq_len_k > 2048 && (batch * p->num_heads_k < 24 || 4 * p->total_q < 3 * batch * p->max_seq_len_q)) {
+        return nullptr;
+    }
+    return &hstu::fwd_variants_pinned()[p->dtype == HSTU_DT_BF16 ? 0 : 1];
+}
+
 // Split items: a list that cannot have two items per resident workgroup takes the variant that may cut long items
 // into parts (it does so when there are fewer items than workgroups), if the caller brings a workspace.  Behind the
 // counter block the workspace holds the fp32 partial outputs, kBlockM x d_pad floats each; room for one per resident
@@ -493,7 +528,9 @@ uint64_t split_workspace_bytes(const Variant* var, const hstu_jagged_fwd_params*
 uint64_t forward_workspace_bytes(const Variant* var, const hstu_jagged_fwd_params* p)
 {
     unsigned one_item_threads = 0;
-    if (short_variant(var, p) != nullptr || one_item_variant(var, p, &one_item_threads) != nullptr) {
+    bool pair_major = false;
+    if (short_variant(var, p) != nullptr || one_item_variant(var, p, &one_item_threads) != nullptr ||
+        pinned_variant(var, p, &pair_major) != nullptr) {
         return 0;
     }
     if (takes_queue_variant(var, p, nullptr)) {
@@ -1591,6 +1628,10 @@ HSTU_API const char* hstu_jagged_fwd_kernel_name(const hstu_jagged_fwd_params* p
         return sv->name;
     }
     int64_t resident = 0;
+    bool pair_major = false;
+    if (const hstu::ShortVariant* const pv = pinned_variant(v, params, &pair_major)) {
+        return pv->name;
+    }
     if (takes_queue_variant(v, params, &resident)) {
         return v->name_queues;
     }
@@ -1715,6 +1756,16 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         const hipError_t err_short = hipGetLastError();
         if (err_short != hipSuccess) {
             return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", sv->name, hipGetErrorString(err_short));
+        }
+        return HSTU_OK;
+    }
+    bool pair_major = false;
+    if (const hstu::ShortVariant* const pv = (paged == nullptr) ? pinned_variant(var, p, &pair_major) : nullptr) {
+        a.pair_major = pair_major ? 1 : 0;
+        hipLaunchKernelGGL(pv->kernel, dim3(static_cast<unsigned>(direct_slots(p))), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+        const hipError_t err_pinned = hipGetLastError();
+        if (err_pinned != hipSuccess) {
+            return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", pv->name, hipGetErrorString(err_pinned));
         }
         return HSTU_OK;
     }

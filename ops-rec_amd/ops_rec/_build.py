@@ -28,10 +28,12 @@ SOURCES = [
     "hstu_kernels_bwd_bf16.hip",
     "hstu_kernels_bwd_f16.hip",
     "hstu_kernels_bwd_fused.hip",
+    "hstu_kernels_fwd_pinned.hip",
 ]
 # These kernels name the accumulator registers they keep their sums in (hstu_pinned_acc.hip.h); every other matrix result belongs in
 # vector registers, where the compiler would otherwise keep it in accumulators as well and copy each element out.
-SOURCE_FLAGS = {"hstu_kernels_bwd_fused.hip": ("-mllvm", "-amdgpu-mfma-vgpr-form=1")}
+_VGPR_FORM = ("-mllvm", "-amdgpu-mfma-vgpr-form=1")
+SOURCE_FLAGS = {"hstu_kernels_bwd_fused.hip": _VGPR_FORM, "hstu_kernels_fwd_pinned.hip": _VGPR_FORM}
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",

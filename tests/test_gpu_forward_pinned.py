@@ -1,0 +1,125 @@
+"""The forward at the head-dim slot 256 with the output sums in pinned accumulators (hstu_fwd_pinned_kernel.hip.h; host rule: 16-bit inputs,
+no bias, no custom mask, more slots than a launch without a list takes, mean lengths of at least half the largest).
+
+Every case is compared with the same sequences run in batches small enough for hstu_fwd_kernel without a list, and with the CPU oracle.  The
+two kernels add the same products in the same order: bf16 outputs are the same bits.  In fp16 one of them may round silu(s) once where the
+other rounds s * sigmoid to fp32 first: P differs by at most one unit, 2^-10 of it, in the elements near a rounding boundary, and the
+output by as much of the sum of |P V|, which stays below 8 times the largest output here.
+"""
+
+import pytest
+import torch
+
+import ops_rec  # noqa: F401
+from ops_rec import _ops, workloads
+from oracle import hstu_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF, FP = torch.bfloat16, torch.float16
+EDGES = [1, 31, 32, 33, 64, 127, 128, 129, 160, 255, 256, 257, 300, 0, 290, 298, 300]
+
+
+def prepared(w):
+    k_offs = w.seq_offset if w.seq_offset_k is None else w.seq_offset_k
+    max_k = w.max_seq_len if w.max_seq_len_k is None else w.max_seq_len_k
+    return _ops.prepare_forward(w.q, w.k, w.v, None, None, w.mask_type, w.max_seq_len, max_k, w.silu_scale, w.seq_offset, k_offs,
+                                w.num_context, w.num_target, w.target_group_size, w.alpha)  # fmt: skip
+
+
+def part_of(w, b0, b1):
+    """Sequences b0 .. b1 - 1 of workload w, and their query rows."""
+    ko = w.seq_offset if w.seq_offset_k is None else w.seq_offset_k
+    q0, q1, k0, k1 = int(w.seq_offset[b0]), int(w.seq_offset[b1]), int(ko[b0]), int(ko[b1])
+    pick = lambda t: None if t is None else t[b0:b1].contiguous()  # noqa: E731
+    p = workloads.Workload(name="part", q=w.q[q0:q1], k=w.k[k0:k1], v=w.v[k0:k1], seq_offset=(w.seq_offset[b0 : b1 + 1] - q0).contiguous(),
+                           max_seq_len=w.max_seq_len, silu_scale=w.silu_scale, alpha=w.alpha, mask_type=w.mask_type,
+                           num_context=pick(w.num_context), num_target=pick(w.num_target), target_group_size=w.target_group_size,
+                           lengths=[])  # fmt: skip
+    if w.seq_offset_k is not None:
+        p.seq_offset_k, p.max_seq_len_k = (ko[b0 : b1 + 1] - k0).contiguous(), w.max_seq_len_k
+    return p, (q0, q1)
+
+
+CASES = {
+    "edges": (dict(lengths=EDGES * 5, heads=2, dim=256), BF),
+    "edges, fp16": (dict(lengths=EDGES * 5, heads=2, dim=256), FP),
+    "grouped heads": (dict(lengths=EDGES * 3, heads=6, heads_k=2, dim=256), BF),
+    "odd number of pairs, dims between slots": (dict(lengths=EDGES * 6 + [300], heads=1, dim=200, dim_v=144), BF),
+    "wider values": (dict(lengths=EDGES * 5, heads=2, dim=72, dim_v=240), BF),
+    "context and targets": (dict(lengths=[n + 41 for n in EDGES] * 5, heads=2, dim=256, num_context=5, max_target=40, target_group_size=3), BF),
+    "long context": (dict(lengths=[300, 150, 280] * 16, heads=2, dim=256, num_context=130, max_target=9), FP),
+    "no mask": (dict(lengths=EDGES * 5, heads=2, dim=256, mask_type=2), BF),
+    "many short": (dict(lengths=[70, 128, 65, 100] * 70, heads=1, dim=256), FP),
+    "64-bit offsets": (dict(lengths=EDGES * 5, heads=2, dim=256, index_dtype=torch.int64), BF),
+    "history": (dict(lengths=[130, 129, 256, 200] * 18, heads=2, dim=256, history=500), BF),
+    "history, grouped": (dict(lengths=[130, 31, 256, 200] * 15, heads=4, heads_k=2, dim=256, history=450), FP),
+    "fewer keys than rows": (dict(lengths=[130, 129, 256, 200] * 18, heads=2, dim=256, history=-60), BF),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_against_the_kernel_without_a_list_and_the_oracle(name):
+    kw, dtype = CASES[name]
+    kw = dict(kw)
+    history, mask_type = kw.pop("history", 0), kw.pop("mask_type", 0)
+    w = workloads.make(name, batch=len(kw["lengths"]), lo=0, hi=0, dtype=dtype, std=0.5, seed=len(name), **kw)
+    w.mask_type = mask_type
+    gen = torch.Generator().manual_seed(3)
+    rand = lambda rows, heads, dim: (torch.randn(rows, heads, dim, generator=gen) * 0.5).to(dtype)  # noqa: E731
+    if history:
+        lk = [max(0, n + history) for n in kw["lengths"]]
+        w.seq_offset_k = torch.tensor([0] + lk).cumsum(0).to(w.seq_offset.dtype)
+        w.max_seq_len_k = max(lk)
+        w.k, w.v = (rand(sum(lk), w.k.shape[1], t.shape[2]) for t in (w.k, w.v))
+    d = w.to(DEV)
+    d.q = torch.cat([d.q, torch.randn(3, d.q.shape[1], d.q.shape[2], device=DEV).to(dtype)])  # rows past the last offset
+    p = prepared(d)
+    assert p.kernel_name().endswith("_pinned"), p.kernel_name()
+    out = p.launch()
+    assert not out[-3:].any()
+    ref = O.hstu_jagged_forward(w.q, w.k, w.v, out_dtype=torch.float32, **w.oracle_kwargs())
+    scale = float(ref.abs().max())
+    torch.testing.assert_close(out[:-3].float().cpu(), ref, atol=(2**-6 if dtype == BF else 2**-8) * scale, rtol=2**-7)
+    batch = len(kw["lengths"])
+    for b0 in range(0, batch, 12):
+        part, (q0, q1) = part_of(d, b0, min(b0 + 12, batch))
+        if q1 == q0:
+            continue
+        pp = prepared(part)
+        assert not pp.kernel_name().endswith("_pinned"), pp.kernel_name()
+        same = pp.launch()
+        if dtype == BF:
+            assert torch.equal(out[q0:q1], same)
+        else:
+            torch.testing.assert_close(out[q0:q1].float(), same.float(), atol=8 * 2**-10 * scale, rtol=2**-10)
+
+
+def test_every_replay_of_a_captured_launch_is_the_eager_result():
+    w = workloads.make("capture", batch=40, heads=4, dim=256, lo=200, hi=300, dtype=BF, device=DEV, seed=2)
+    p = prepared(w)
+    assert p.kernel_name().endswith("_pinned")
+    want = p.launch().clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = p.launch()
+    for _ in range(4):
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
+def test_batches_the_rule_leaves_to_the_lists():
+    def name(**kw):
+        w = workloads.make("route", batch=kw.pop("batch", 40), dtype=BF, device=DEV, seed=1, **kw)
+        d_bias = w.attn_bias
+        return _ops.prepare_forward(w.q, w.k, w.v, None, d_bias, 0, w.max_seq_len, w.max_seq_len, w.silu_scale, w.seq_offset, w.seq_offset,
+                                    None, None, 0, w.alpha).kernel_name()  # fmt: skip
+
+    assert name(heads=4, dim=256, lo=200, hi=300).endswith("_pinned")
+    assert name(heads=4, dim=128, lo=200, hi=1100).find("_pinned") < 0
+    assert name(heads=4, dim=256, lo=200, hi=300, rab_std=0.2).find("_pinned") < 0
+    assert name(heads=4, dim=256, lo=200, hi=300, max_seq_len=800).find("_pinned") < 0  # most slots would be empty
+    assert name(heads=4, dim=256, lo=200, hi=300, batch=8).endswith("_direct")
