@@ -78,7 +78,8 @@ using hstu::Variant;
 // only when hstu_reload_switches() is called (a test that changes the environment calls it); a launch reads no
 // environment variable.  A value of -1 means "not set: the library's own rule applies".
 //   HSTU_MI355_SPLIT=0             forward: never cut long items into parts, nor deal the keys of an fp32 row over wavefronts (the
-//                                  rows of a sequence are then the same bits whatever else is in the batch, where both take one kernel)
+//                                  rows of a sequence are then the same bits whatever else is in the batch, where both take one kernel);
+//                                  =1: cut them also on sweeps that are short for it
 //   HSTU_MI355_SHORT=0 / 1         forward: never / whenever possible the kernel for short lists
 //   HSTU_MI355_GENERIC_BACKWARD=1  backward: the generic kernels also where tuned ones exist (for comparisons)
 //   HSTU_MI355_BWD_HANDOFF=0/1/2   backward: force the launch order (two launches / three / planes)
@@ -488,7 +489,7 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
 constexpr uint64_t kMaxWorkspaceBytes = 128ull << 20;
 constexpr uint64_t kCounterBytes = hstu::kCounterBlockBytes;  // head of the workspace of the variants that pull from counters
 uint64_t split_part_bytes(const Variant* var) { return static_cast<uint64_t>(hstu::kBlockM) * var->d_pad * sizeof(float); }
-bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p, int64_t* resident_out)
+bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p, int64_t* resident_out, bool paged = false)
 {
     if (var->persistent_wgs_per_cu <= 0 || var->kernel_split == nullptr) {
         return false;
@@ -510,12 +511,29 @@ bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p,
     const int64_t n_blocks = n_qtiles * (p->n_offsets - 1) * p->num_heads_q;
     // (items of at most 16 sub-tiles: parts of 8, the kernel's shortest, do not earn back what a part costs --
     // 8 x 4 sequences of 512 rows: 23.0 us split, 20.7 us not)
-    return n_blocks < 2 * resident && p->max_seq_len_k > 16 * 32;
+    if (n_blocks >= 2 * resident || p->max_seq_len_k <= 16 * 32) {
+        return false;
+    }
+    // A launch without a list (which the paged variant does not have) needs no building of a list, no hand-over of parts through memory
+    // and no counters: on short sweeps that outweighs what idle compute units could add, unless there is next to nothing to do or a
+    // tile is much longer than the others.  Measured, split -> without a list: up to 1024 keys -- slot 64, 16 x 4 heads, 501 rows on 1000
+    // 30.6 -> 22.3 us, 8 x 4 of 512..1000 22.0 -> 18.9, slot 128 with a bias 26.6 <- 34.1; up to 2048 keys, the rows at most half of them --
+    // slot 64, 16 x 4, 200 rows on 1500 34.5 -> 25.2, slot 128 37.9 -> 33.3.  It loses below 64 slots (1 x 2 of 2000 24.4 -> 30.3), with a bias
+    // on longer keys (slot 64, 4 x 4 of 1000..2000 30.5 -> 34.2), on longer causal rows (slot 128, 1 x 8 of 2000 36.4 -> 38.9; slot 64 mixed),
+    // with context rows (4 x 8 of 600..2000 37.6 -> 46.9) and past 2048 keys (16 x 4, 128 rows on 1000..3000 33.6 -> 41.4).
+    // (HSTU_MI355_SPLIT=1: split all the same.)
+    if (paged || switches().split == 1 || p->mask_type == HSTU_MASK_CUSTOM || p->num_context != nullptr || direct_slots(p) > resident) {
+        return true;
+    }
+    if (p->attn_bias != nullptr) {
+        return n_blocks < 128 || p->max_seq_len_k > 1024;
+    }
+    return n_blocks < 64 || p->max_seq_len_k > (2 * p->max_seq_len_q <= p->max_seq_len_k ? 2048 : 1024);
 }
-uint64_t split_workspace_bytes(const Variant* var, const hstu_jagged_fwd_params* p)
+uint64_t split_workspace_bytes(const Variant* var, const hstu_jagged_fwd_params* p, bool paged = false)
 {
     int64_t resident = 0;
-    if (!may_take_split_variant(var, p, &resident)) {
+    if (!may_take_split_variant(var, p, &resident, paged)) {
         return 0;
     }
     const uint64_t bytes = kCounterBytes + static_cast<uint64_t>(resident) * split_part_bytes(var);
@@ -727,7 +745,7 @@ HSTU_API int hstu_paged_fwd_workspace_size(const hstu_paged_fwd_params* params, 
     if (var->kernel_paged != nullptr) {
         // the kernel reads the pages itself; the counter block (required: the variant pulls its items from a
         // counter) and, for short lists, room for the partial outputs of split items (optional)
-        const uint64_t split = split_workspace_bytes(var, &g);
+        const uint64_t split = split_workspace_bytes(var, &g, true);
         *workspace_bytes = split > kCounterBytes ? split : kCounterBytes;
         return HSTU_OK;
     }
@@ -1787,7 +1805,8 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         }
         n_blocks = n_blocks < resident ? n_blocks : resident;
         const uint64_t part_bytes = split_part_bytes(var);
-        if (usable_workspace(workspace, workspace_bytes, kCounterBytes + 2 * part_bytes) && may_take_split_variant(var, p, nullptr)) {
+        if (usable_workspace(workspace, workspace_bytes, kCounterBytes + 2 * part_bytes) &&
+            may_take_split_variant(var, p, nullptr, paged != nullptr)) {
             kernel = var->kernel_split;
             a.counters = static_cast<unsigned int*>(workspace);
             a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
