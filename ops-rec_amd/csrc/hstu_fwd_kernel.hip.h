@@ -448,6 +448,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     constexpr int kWaitEven64 = ((4 * LPW) & 15) | (7 << 4) | (15 << 8);  // after an even step: V, V, K of it and K of the step before
     constexpr int kWaitOdd64 = ((2 * LPW) & 15) | (7 << 4) | (15 << 8);   // after an odd step: its K and the K of the step before
     constexpr uint32_t kPastEnd = 0x40000000u;   // added to a source offset: leaves every descriptor
+    constexpr int kRabWords = F8 ? 8 : 9;        // registers of a sub-tile's rab words (load_rab)
 
     // eight separate arrays (not one block) so that the compiler can tell the slot being filled by the
     // asynchronous loads from the slot being read, and does not wait for the loads early
@@ -837,7 +838,8 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             }
         }
     }
-    const int bias_mode = a.bias_vec_ok;  // 0: element loads, 1: 8-byte loads, 2: 16-byte loads + lane exchange
+    const bool rab_words = a.max_k % 2 == 0 && reinterpret_cast<uintptr_t>(a.rab) % 4 == 0;  // (16-bit rab: rows start with a word)
+    const int bias_mode = a.bias_vec_ok;  // custom mask: 0: element loads, 1: 8-byte loads, 2: 16-byte loads + lane exchange
 
     auto k_slot = [&](auto ic) -> uint16_t* {
         constexpr int I = decltype(ic)::value & 3;
@@ -1424,11 +1426,15 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         const uint32_t bias_bytes = static_cast<uint32_t>(a.max_q) * static_cast<uint32_t>(a.max_k) * ES;
         const int64_t bias_plane =
             (static_cast<int64_t>(b) * a.n_heads_q + h) * a.max_q * static_cast<int64_t>(a.max_k);
+        // (16-bit rab: from the word that holds the plane's first value to the one that holds its last)
+        const uint8_t* const rab_plane = static_cast<const uint8_t*>(a.rab) + (HAS_RAB ? bias_plane * ES : 0);
+        const uint32_t rab_ahead = F8 ? 0u : static_cast<uint32_t>(reinterpret_cast<uintptr_t>(rab_plane)) & 2u;
         const __amdgpu_buffer_rsrc_t rab_rsrc =
-            make_rsrc(HAS_RAB ? static_cast<const uint8_t*>(a.rab) + bias_plane * ES : nullptr, HAS_RAB ? bias_bytes : 0u);
+            make_rsrc(HAS_RAB ? rab_plane - rab_ahead : nullptr, HAS_RAB ? (F8 ? bias_bytes : (bias_bytes + rab_ahead + 3u) & ~3u) : 0u);
         const __amdgpu_buffer_rsrc_t mask_rsrc = make_rsrc(
             HAS_MASK ? static_cast<const uint8_t*>(a.mask) + bias_plane * ES : nullptr, HAS_MASK ? bias_bytes : 0u);
         const uint32_t bias_row_off = static_cast<uint32_t>(wr0 + ln) * static_cast<uint32_t>(a.max_k) * ES;
+        const uint32_t rab_off = (rab_ahead + bias_row_off + 32u * lh) & ~3u;  // the word that holds the lane's first value
 
         // fp8 inputs: rab and the custom mask are e4m3 tensors like q.  The 16 values of a 32-key sub-tile a lane
         // needs -- keys c0 + 8 g + 4 lh + 0..3 for g = 0..3, the order of its score registers -- are four words of
@@ -1469,34 +1475,37 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             }
         };
 
-        // Requests the rab values of keys c0 + 16 lh .. + 15 of this lane's row, 8 packed words in memory order
-        // (what the routing MFMAs above take as their B operands).
-        auto load_rab = [&](int c0, uint32_t (&w)[8]) {
-            const uint32_t off = bias_row_off + static_cast<uint32_t>(c0 + 16 * lh) * 2u;
-            if (bias_mode == 2) {
-                const U32Quad t0 = __builtin_bit_cast(U32Quad, __builtin_amdgcn_raw_buffer_load_b128(rab_rsrc, static_cast<int>(off), 0, 0));
-                const U32Quad t1 = __builtin_bit_cast(U32Quad, __builtin_amdgcn_raw_buffer_load_b128(rab_rsrc, static_cast<int>(off + 16u), 0, 0));
+        // Requests the rab values of keys c0 + 16 lh .. + 15 of this lane's row, 8 packed words in memory order (what the routing MFMAs above
+        // take as their B operands).  A row may start on any even address: the words asked for are the aligned ones that hold the values,
+        // nine of them where some rows start in the middle of a word (!rab_words), and shift_rab() brings those into place.
+        // The words at the two ends of a plane may hold a neighbour's value, or two bytes in front of or behind the tensor; shift_rab() drops
+        // both.  16 x 4 heads of 512..2048 rows, d 128: max_seq_len_k 2049 143 -> 77 us and 2050 138 -> 72 (one value at a time before), 2052
+        // 67.4 -> 65.8 (8 bytes at a time), 2048 64 -> 61 (no branch left in the straight-line step).
+        auto load_rab = [&](int c0, uint32_t (&w)[kRabWords], bool words) {
+            const uint32_t off = rab_off + static_cast<uint32_t>(c0) * 2u;
+            const U32Quad t0 = __builtin_bit_cast(U32Quad, __builtin_amdgcn_raw_buffer_load_b128(rab_rsrc, static_cast<int>(off), 0, 0));
+            const U32Quad t1 = __builtin_bit_cast(U32Quad, __builtin_amdgcn_raw_buffer_load_b128(rab_rsrc, static_cast<int>(off + 16u), 0, 0));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    w[i] = t0.v[i];
-                    w[4 + i] = t1.v[i];
-                }
-            } else if (bias_mode == 1) {
+            for (int i = 0; i < 4; ++i) {
+                w[i] = t0.v[i];
+                w[4 + i] = t1.v[i];
+            }
+            if (!words) {
+                w[kRabWords - 1] = __builtin_amdgcn_raw_buffer_load_b32(rab_rsrc, static_cast<int>(off + 32u), 0, 0);
+            }
+        };
+        auto shift_rab = [&](int c0, uint32_t (&w)[kRabWords]) {
+            const uint32_t shift = 8u * ((rab_ahead + 2u * static_cast<uint32_t>((wr0 + ln) * a.max_k)) & 2u);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const U32Pair t = __builtin_bit_cast(
-                        U32Pair, __builtin_amdgcn_raw_buffer_load_b64(rab_rsrc, static_cast<int>(off + 8u * i), 0, 0));
-                    w[2 * i + 0] = t.v[0];
-                    w[2 * i + 1] = t.v[1];
-                }
-            } else {
-                uint32_t eoff = off;
-                asm volatile("" : "+v"(eoff));  // (keeps the optimiser from relating these to the vector loads above)
+            for (int i = 0; i < kRabWords - 1; ++i) {
+                w[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], shift);
+            }
+            if (c0 + 32 > a.max_k) {
+                // (what lies behind the row, which may be anything, must not meet the products: 0 x NaN)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint32_t e0 = __builtin_amdgcn_raw_buffer_load_b16(rab_rsrc, static_cast<int>(eoff + 4u * i), 0, 0);
-                    const uint32_t e1 = __builtin_amdgcn_raw_buffer_load_b16(rab_rsrc, static_cast<int>(eoff + 4u * i + 2u), 0, 0);
-                    w[i] = (e0 & 0xffffu) | (e1 << 16);
+                for (int i = 0; i < kRabWords - 1; ++i) {
+                    const int left = a.max_k - (c0 + 16 * lh + 2 * i);
+                    w[i] = left >= 2 ? w[i] : (left == 1 ? w[i] & 0xffffu : 0u);
                 }
             }
         };
@@ -1581,7 +1590,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         f32x16_t s_blk0, s_blk1;     // S^T
         uint32_t p_blk0[8], p_blk1[8];  // P^T, packed pairs
         uint32_t p_blk2[8], p_blk3[8];  // 64-deep PV only: sub-tile x uses P^T block x & 3 (a pair is consumed two and three steps on)
-        uint32_t rabw0[8], rabw1[8];  // rab words of sub-tile x in block x & 1
+        uint32_t rabw0[kRabWords], rabw1[kRabWords];  // rab words of sub-tile x in block x & 1
         uint32_t mw0[8], mw1[8];      // custom mask words of sub-tile x in block x & 1
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -1596,12 +1605,14 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             p_blk3[i] = 0;
             rabw0[i] = 0;
             rabw1[i] = 0;
+            rabw0[kRabWords - 1] = 0;
+            rabw1[kRabWords - 1] = 0;
             mw0[i] = 0;
             mw1[i] = 0;
         }
         if constexpr (HAS_RAB && !F8) {
             if (nx_w > x_begin) {
-                load_rab(x_begin * 32, rabw0);
+                load_rab(x_begin * 32, rabw0, rab_words);
             }
         }
 
@@ -1637,8 +1648,8 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             const int t0 = PAR ? t - 3 : t - 2;
             uint32_t(&mw_cur)[8] = PAR ? mw1 : mw0;               // custom mask words of sub-tile t
             uint32_t(&mw_nxt)[8] = PAR ? mw0 : mw1;
-            uint32_t(&rab_far)[8] = PAR ? rabw1 : rabw0;          // receives rab(t+2)
-            uint32_t(&rab_nxt)[8] = PAR ? rabw0 : rabw1;          // rab(t+1)
+            uint32_t(&rab_far)[kRabWords] = PAR ? rabw1 : rabw0;          // receives rab(t+2)
+            uint32_t(&rab_nxt)[kRabWords] = PAR ? rabw0 : rabw1;          // rab(t+1)
             const uint16_t* const kt = k_slot(std::integral_constant<int, (S + 1) & 3>{});  // K(t+1)
             const uint16_t* const vt = v_slot(std::integral_constant<int, (S + 3) & 3>{});  // V(t-1)
             const int c0 = t * 32;
@@ -1912,10 +1923,11 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 }
             }
             if constexpr (HAS_RAB && !F8) {
-                // the bias of sub-tile t + 2 (added to S^T(t + 2) at the end of the next step's QK block)
+                // the bias of sub-tile t + 2 (added to S^T(t + 2) at the end of the next step's QK block; in the straight-line step the branch,
+                // always taken, only keeps the two blocks apart: 16 x 8 heads of 1024..4096 rows 402 -> 399 us)
                 __builtin_amdgcn_sched_barrier(0);
-                if (INTERIOR || t + 2 < nx_w) {
-                    load_rab(c0 + 64, rab_far);
+                if (INTERIOR ? rab_words : t + 2 < nx_w) {
+                    load_rab(c0 + 64, rab_far, INTERIOR || rab_words);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -1948,6 +1960,9 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 }
                 if constexpr (HAS_RAB && !F8) {
                     // S^T(t+1) += rab^T, last so that the rab request has had the whole block to land
+                    if (!INTERIOR && !rab_words) {
+                        shift_rab(c0 + 32, rab_nxt);
+                    }
                     const u32x4_t r0 = {rab_nxt[0], rab_nxt[1], rab_nxt[2], rab_nxt[3]};
                     const u32x4_t r1 = {rab_nxt[4], rab_nxt[5], rab_nxt[6], rab_nxt[7]};
                     s_nxt = mfma32<Tag>(rab_route[0], r0, s_nxt);
@@ -2025,7 +2040,8 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             }
             // (short sweeps stay on the general step: measured on MI355X, sweeps under about twenty steps gain nothing
             // from the second copy of the step and lose a little to fetching its instructions)
-            if (x_end - x_begin < kInteriorMinSteps) {
+            // (rab rows that start in the middle of a word too: the straight-line step has no room for their shifts)
+            if (x_end - x_begin < kInteriorMinSteps || (HAS_RAB && !F8 && !rab_words)) {
                 t_interior = -1;
             }
             typedef std::false_type general_t;
