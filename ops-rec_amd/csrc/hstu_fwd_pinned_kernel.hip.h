@@ -1,4 +1,4 @@
-// HSTU jagged attention forward at the head-dim slot 256: two wavefronts per SIMD, the output sums in pinned accumulators.
+// HSTU jagged attention forward at the head-dim slots 256 and 128: two (at 128 three) wavefronts per SIMD, the output sums in pinned accumulators.
 //
 // hstu_fwd_kernel needs 400 registers and more at this slot, so one wavefront per SIMD, which copies every score out of the accumulators
 // (195 copies beside 32 MFMAs a step) and has nothing to run while it waits: 35 % of the time in MFMAs.  Here a wavefront (32 query
@@ -8,7 +8,8 @@
 // The sums are added in the order of hstu_fwd_kernel.
 //
 // LDS, 80 KiB, so that two workgroups share a CU: K in a ring of three slots, V of two.  At the start of a step the slots of the step
-// before are free: V(t) is requested (a step ahead of its use), then K(t + 2) (two steps ahead).
+// before are free: V(t) is requested (a step ahead of its use), then K(t + 2) (two steps ahead).  The slot 128 has half of everything
+// and with it room for three workgroups, and for a third V slot: V(t + 1) is requested.
 //
 // One workgroup per (query tile, K/V pair, query head of the pair) slot: no list, no counters, no workspace.  Slots go level after level
 // (heaviest tiles of all pairs first), or pair after pair (a.pair_major): see the host's rule.
@@ -22,15 +23,14 @@
 namespace hstu {
 
 template <typename Tag, int D>
-__global__ __launch_bounds__(256, 2) void hstu_fwd_pinned_kernel(const FwdArgs a)
+__global__ __launch_bounds__(256, D == 256 ? 2 : 3) void hstu_fwd_pinned_kernel(const FwdArgs a)
 {
-    static_assert(D == 256, "the counts and the split of the registers are this slot's");
     constexpr int CPR = D / 8;                  // 16-byte chunks per row
     constexpr int SUB_BYTES = 32 * D * 2;       // a 32-key sub-tile
     constexpr int LPW = SUB_BYTES / 4096;       // 1 KiB load instructions per sub-tile and wavefront
     constexpr int KSTEPS = D / 16, MTILES = D / 32, NCH = 2 * MTILES;
-    constexpr int KS = 3, VS = 2;               // ring slots
-    constexpr int kOpen = LPW;                  // what may be under way when a step starts: K, the last thing that the step before requested
+    constexpr int KS = 3, VS = D == 256 ? 2 : 3;               // ring slots
+    constexpr int kOpen = VS == 2 ? LPW : 2 * LPW;                  // what may be under way when a step starts: behind V(t - 1), VS - 1 steps ago, and K(t), two steps ago
     constexpr int kAccRegs = MTILES * 16;
     constexpr uint32_t kPastEnd = 0x40000000u;
     constexpr int kV0 = 0, kK0 = VS * SUB_BYTES;
@@ -212,6 +212,10 @@ __global__ __launch_bounds__(256, 2) void hstu_fwd_pinned_kernel(const FwdArgs a
             qf[js] = __builtin_amdgcn_raw_buffer_load_b128(q_rsrc, static_cast<int>(d0 < a.d_qk ? row_off + d0 * 2u : kOutOfRange), 0, 0);
         }
 #pragma unroll
+        for (int x = 0; x < VS - 2; ++x) {
+            request_v(x, x);
+        }
+#pragma unroll
         for (int x = 1; x < KS - 1; ++x) {
             request_k(x, x);
         }
@@ -306,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void hstu_fwd_pinned_kernel(const FwdArgs a
             pk[i] = pack2<Tag>(s[2 * i], s[2 * i + 1]);
             asm volatile("" : "+v"(pk[i]));
         };
-        constexpr int kFirst = 2;  // (the last score product has to end first)
+        constexpr int kFirst = NCH >= 16 ? 2 : 1;  // (the last score product has to end first)
         auto parts_done = [](int g) constexpr { return g < kFirst ? 0 : ((g - kFirst + 1) * 16 + NCH - kFirst - 1) / (NCH - kFirst); };
         static_for<NCH>([&](auto ci) {
             constexpr int c = ci;

@@ -4,8 +4,10 @@
 
 namespace hstu {
 namespace {
-const ShortVariant kPinned[2] = {{"hstu_fwd_bf16_d256_rabfalse_maskfalse_pinned", hstu_fwd_pinned_kernel<bf16_tag, 256>},
-                                 {"hstu_fwd_f16_d256_rabfalse_maskfalse_pinned", hstu_fwd_pinned_kernel<f16_tag, 256>}};
+#define HSTU_PINNED(tag, tagname)                                                                    \
+    {{"hstu_fwd_" tagname "_d128_rabfalse_maskfalse_pinned", hstu_fwd_pinned_kernel<tag, 128>},      \
+     {"hstu_fwd_" tagname "_d256_rabfalse_maskfalse_pinned", hstu_fwd_pinned_kernel<tag, 256>}}
+const ShortVariant kPinned[2][2] = {HSTU_PINNED(bf16_tag, "bf16"), HSTU_PINNED(f16_tag, "f16")};
 }  // namespace
-const ShortVariant* fwd_variants_pinned() { return kPinned; }
+const ShortVariant (*fwd_variants_pinned())[2] { return kPinned; }
 }  // namespace hstu

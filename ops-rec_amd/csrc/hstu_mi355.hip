@@ -446,8 +446,8 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
     return var->kernel_queues != nullptr && n_blocks >= 4 * resident;
 }
 
-// The kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): 16-bit inputs at the slot 256 without bias and custom mask, more
-// slots than a launch without a list takes.  It has no list that sorts the sequences, so it takes batches whose mean lengths are at least
+// The kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): 16-bit inputs without bias and custom mask, more slots than a launch
+// without a list takes.  At the slot 256:  It has no list that sorts the sequences, so it takes batches whose mean lengths are at least
 // half of the largest (a Zipf law of lengths up to 8192 with a mean of an eighth: 416 -> 761 us), and, where the sequences are long, only
 // those with little between them and pairs enough for all XCDs (6 x 2 heads, 3000..6000 rows: 209 -> 258 us; 32 x 2, 1000..4000 326 -> 340).
 // *pair_major: the tiles of a pair side by side on one XCD, once the K / V rows are about what the last-level cache holds (24 x 8 heads
@@ -455,9 +455,14 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
 // keys that are mostly history, where a pair's tiles are equally long and nothing is lost at the end (30 x 8, 300 rows on 600 keys: 87, 76, 60).
 // Measured list -> this kernel, launches queued back to back: 200 x 4 of 65..128 rows 57.8 -> 36.5 us, 48 x 4 of 129..512 rows 55.3 -> 37.2,
 // 16 x 4 of 512..2048 rows 95.2 -> 90.8, 32 x 2 of the same 98.0 -> 98.7, 24 x 8 of 1024 rows 187 -> 143, 64 x 4 of 1000..4000 rows 1192 -> 1029.
+// At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of two
+// tiles and more on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
+// keys (629 MB) 470 -> 335 us, 200 x 4, 200 rows 524 -> 367, 400 x 2, 400 rows on 800..1000 (369 MB) 269 -> 200, 24 x 8, 400 rows on 3072 (302 MB) 178 ->
+// 160, 100 x 8 over 4 K/V heads, 400 rows on 1500..3000 493 -> 465; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 147 -> 150, of one
+// tile 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.
 const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool* pair_major)
 {
-    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || var->d_pad != 256 || var->persistent_wgs_per_cu <= 0 ||
+    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || var->d_pad < 128 || var->d_pad > 256 || var->persistent_wgs_per_cu <= 0 ||
         p->attn_bias != nullptr || p->mask != nullptr || p->mask_type == HSTU_MASK_CUSTOM) {
         return nullptr;
     }
@@ -474,11 +479,17 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
         return nullptr;
     }
     const int64_t kv_bytes = p->total_k * p->num_heads_k * (p->head_dim_qk + p->head_dim_v) * 2;
+    const hstu::ShortVariant* const pv = hstu::fwd_variants_pinned()[p->dtype == HSTU_DT_BF16 ? 0 : 1];
+    if (var->d_pad == 128) {
+        *pair_major = true;
+        const bool shared_history = p->total_k >= 2 * p->total_q && p->max_seq_len_q > hstu::kBlockM;
+        return shared_history && kv_bytes >= (288LL << 20) && slots >= 3LL * cus && switches().short_lists != 1 ? &pv[0] : nullptr;
+    }
     *pair_major = kv_bytes >= (224LL << 20) || p->total_k >= 2 * p->total_q;
     if (!*pair_major && p->max_seq_len_k > 2048 && (batch * p->num_heads_k < 24 || 4 * p->total_q < 3 * batch * p->max_seq_len_q)) {
         return nullptr;
     }
-    return &hstu::fwd_variants_pinned()[p->dtype == HSTU_DT_BF16 ? 0 : 1];
+    return &pv[1];
 }
 
 // Split items: a list that cannot have two items per resident workgroup takes the variant that may cut long items
@@ -1642,14 +1653,14 @@ HSTU_API const char* hstu_jagged_fwd_kernel_name(const hstu_jagged_fwd_params* p
     if (const hstu::ShortVariant* const tv = one_item_variant(v, params, &one_item_threads)) {
         return tv->name;
     }
-    if (const hstu::ShortVariant* const sv = short_variant(v, params)) {
-        return sv->name;
-    }
-    int64_t resident = 0;
     bool pair_major = false;
     if (const hstu::ShortVariant* const pv = pinned_variant(v, params, &pair_major)) {
         return pv->name;
     }
+    if (const hstu::ShortVariant* const sv = short_variant(v, params)) {
+        return sv->name;
+    }
+    int64_t resident = 0;
     if (takes_queue_variant(v, params, &resident)) {
         return v->name_queues;
     }
@@ -1756,6 +1767,16 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         }
         return HSTU_OK;
     }
+    bool pair_major = false;
+    if (const hstu::ShortVariant* const pv = (paged == nullptr) ? pinned_variant(var, p, &pair_major) : nullptr) {
+        a.pair_major = pair_major ? 1 : 0;
+        hipLaunchKernelGGL(pv->kernel, dim3(static_cast<unsigned>(direct_slots(p))), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+        const hipError_t err_pinned = hipGetLastError();
+        if (err_pinned != hipSuccess) {
+            return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", pv->name, hipGetErrorString(err_pinned));
+        }
+        return HSTU_OK;
+    }
     if (const hstu::ShortVariant* const sv =
             (paged == nullptr) ? short_variant(var, p, usable_workspace(workspace, workspace_bytes, kCounterBytes)) : nullptr) {
         // one workgroup per (query tile, K/V pair padded to a multiple of 8, query head of the pair) slot
@@ -1774,16 +1795,6 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         const hipError_t err_short = hipGetLastError();
         if (err_short != hipSuccess) {
             return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", sv->name, hipGetErrorString(err_short));
-        }
-        return HSTU_OK;
-    }
-    bool pair_major = false;
-    if (const hstu::ShortVariant* const pv = (paged == nullptr) ? pinned_variant(var, p, &pair_major) : nullptr) {
-        a.pair_major = pair_major ? 1 : 0;
-        hipLaunchKernelGGL(pv->kernel, dim3(static_cast<unsigned>(direct_slots(p))), dim3(256), 0, static_cast<hipStream_t>(stream), a);
-        const hipError_t err_pinned = hipGetLastError();
-        if (err_pinned != hipSuccess) {
-            return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", pv->name, hipGetErrorString(err_pinned));
         }
         return HSTU_OK;
     }

@@ -87,8 +87,8 @@ const Variant (*fwd_variants_wide())[2][2];
 // forward for short work lists, 16-bit inputs at the head-dim slot 128 without custom mask: [bf16, fp16, bf16 with
 // attn_bias, fp16 with attn_bias]
 const ShortVariant* fwd_variants_short();
-// the forward kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h), slot 256: bf16, f16
-const ShortVariant* fwd_variants_pinned();
+// the forward kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): [bf16, f16][slots 128, 256]
+const ShortVariant (*fwd_variants_pinned())[2];
 // forward for batches of sequences of at most 32 or 64 rows and keys (hstu_fwd_tiny_kernel.hip.h; one workgroup of four
 // threads per row per (sequence, head)), no bias, no custom mask: [bf16, fp16][head-dim slot 64, 128, 256][32, 64 rows]
 const ShortVariant (*fwd_variants_tiny())[3][2];

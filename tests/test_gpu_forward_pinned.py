@@ -1,5 +1,5 @@
-"""The forward at the head-dim slot 256 with the output sums in pinned accumulators (hstu_fwd_pinned_kernel.hip.h; host rule: 16-bit inputs,
-no bias, no custom mask, more slots than a launch without a list takes, mean lengths of at least half the largest).
+"""The forward with the output sums in pinned accumulators (hstu_fwd_pinned_kernel.hip.h; host rule: 16-bit inputs, no bias, no custom mask, more
+slots than a launch without a list takes, mean lengths of at least half the largest; at the slot 128 long histories only).
 
 Every case is compared with the same sequences run in batches small enough for hstu_fwd_kernel without a list, and with the CPU oracle.  The
 two kernels add the same products in the same order: bf16 outputs are the same bits.  In fp16 one of them may round silu(s) once where the
@@ -10,6 +10,7 @@ output by as much of the sum of |P V|, which stays below 8 times the largest out
 import pytest
 import torch
 
+import helpers
 import ops_rec  # noqa: F401
 from ops_rec import _ops, workloads
 from oracle import hstu_oracle as O
@@ -86,6 +87,42 @@ def test_against_the_kernel_without_a_list_and_the_oracle(name):
         part, (q0, q1) = part_of(d, b0, min(b0 + 12, batch))
         if q1 == q0:
             continue
+        pp = prepared(part)
+        assert not pp.kernel_name().endswith("_pinned"), pp.kernel_name()
+        same = pp.launch()
+        if dtype == BF:
+            assert torch.equal(out[q0:q1], same)
+        else:
+            torch.testing.assert_close(out[q0:q1].float(), same.float(), atol=8 * 2**-10 * scale, rtol=2**-10)
+
+
+@pytest.mark.parametrize(
+    "heads,heads_k,dim,dim_v,dtype,extra",
+    [
+        (2, 2, 128, 128, BF, dict()),
+        (4, 2, 128, 128, BF, dict(num_context=3, max_target=40, target_group_size=3)),
+        (2, 2, 128, 128, FP, dict(index_dtype=torch.int64)),
+        (3, 3, 96, 80, BF, dict()),
+    ],
+    ids=str,
+)
+def test_histories_at_the_slot_128(heads, heads_k, dim, dim_v, dtype, extra, monkeypatch):
+    batch = 210
+    lengths = [129, 200, 161, 256, 255, 130, 200] * (batch // 7)
+    w = workloads.make("history", batch=batch, heads=heads, heads_k=heads_k, dim=dim, dim_v=dim_v, lo=0, hi=0, lengths=lengths, dtype=dtype,
+                       std=0.5, seed=dim, device=DEV, **extra)  # fmt: skip
+    lk = [1350 + 37 * (i % 9) for i in range(batch)]
+    w.seq_offset_k = torch.tensor([0] + lk, device=DEV).cumsum(0).to(w.seq_offset.dtype)
+    w.max_seq_len_k = max(lk)
+    w.k, w.v = (torch.randn(sum(lk), heads_k, t.shape[2], device=DEV).mul_(0.5).to(dtype) for t in (w.k, w.v))
+    out = prepared(w)
+    assert out.kernel_name().endswith("_d128_rabfalse_maskfalse_pinned"), out.kernel_name()
+    out = out.launch()
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", "0")
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SPLIT", "0")
+    scale = float(out.float().abs().max())
+    for b0 in range(0, batch, 30):
+        part, (q0, q1) = part_of(w, b0, b0 + 30)
         pp = prepared(part)
         assert not pp.kernel_name().endswith("_pinned"), pp.kernel_name()
         same = pp.launch()
