@@ -50,7 +50,7 @@ INFINITY_CACHE_BYTES = 256 << 20  # MI355X memory-side cache; a working set belo
 # the forward kernel's source at the time).  A figure whose hash no longer matches the source in the tree is stale
 # and is reported as null.
 MEASURED_TRAFFIC = {
-    "C2": (99_200_000, "profiles/hstu_fwd_bf16_d128_C2_trace_and_counters.md", "d1cc2020dd2b2df1"),
+    "C2": (99_000_000, "profiles/hstu_fwd_bf16_d128_C2_trace_and_counters.md", "455880c465305171"),
     "C3": (300_900_000, "profiles/hstu_fwd_bf16_d128_rab_C3_trace_and_counters.md", "0129a427493bf494"),
     "C4": (1_499_000_000, "profiles/hstu_fwd_bf16_d128_rab_C4_trace_and_counters.md", "0129a427493bf494"),
     "C5": (840_700_000, "profiles/hstu_fwd_f8e4m3_d128_C5_trace_and_counters.md", "0129a427493bf494"),
@@ -507,9 +507,8 @@ def main() -> int:
             "tflops": round(bwd_flops / (bwd_ms * 1e-3) / 1e12, 3),
             "pct_of_bf16_mfma_peak": round(100.0 * bwd_flops / (bwd_ms * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 2),
             "note": "through torch.ops.ops_rec.hstu_jagged_backward, in the order the library picks for the shape: on this "
-            "workload hstu_bwd_dq_kernel storing dS and P, then hstu_bwd_dkv_kernel with a dV and a dK workgroup per key "
-            "tile that read them back (the five products of the formula issued once each); with an attn_bias gradient, "
-            "head dims up to 64 or long rows two or three launches that recompute S (and dP)",
+            "workload hstu_bwd_kv_fused_kernel for dV and dK, storing dS, then hstu_bwd_dq_from_ds_kernel that reads it back "
+            "(the five products of the formula issued once each)",
         }
 
     if legs["backward"] and not fp8:

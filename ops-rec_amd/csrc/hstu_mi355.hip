@@ -82,7 +82,7 @@ using hstu::Variant;
 //                                  =1: cut them also on sweeps that are short for it
 //   HSTU_MI355_SHORT=0 / 1         forward: never / whenever possible the kernel for short lists
 //   HSTU_MI355_GENERIC_BACKWARD=1  backward: the generic kernels also where tuned ones exist (for comparisons)
-//   HSTU_MI355_BWD_HANDOFF=0/1/2   backward: force the launch order (two launches / three / planes)
+//   HSTU_MI355_BWD_HANDOFF=0/1/2/3 backward: force the launch order (two launches / three / planes / dS tiles)
 //   HSTU_MI355_BWD_WORKSPACE_MB=n  backward: the largest workspace the library asks for
 //   HSTU_MI355_BWD_PAIR_MAJOR=0/1  backward: the grids of the tuned 16-bit kernels level after level / pair after pair
 struct Switches {
@@ -867,7 +867,7 @@ HSTU_API int hstu_paged_fwd(const hstu_paged_fwd_params* p, void* workspace, uin
 // Also tried, not kept: the dV workgroups on a second stream beside the query-tile kernel (C2 143 -> 149 us), and the
 // query-tile kernel first with dV and dK-from-dS workgroups in one launch behind it (C2 160 us).
 // HSTU_MI355_BWD_HANDOFF in the environment overrides the rule: 0 = two launches, 1 = three wherever possible,
-// 2 = planes wherever possible.
+// 2 = planes wherever possible; 3 = dS tiles wherever their workspace is there (fused_plan).
 enum BwdOrder { kTwoLaunches, kThreeLaunches, kPlanes };
 struct BwdPlan {
     BwdOrder order;
