@@ -249,8 +249,8 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             }
         }
     };
-    // attn_bias of the next step's block: lane (ln, lh) has row ln, keys 8 lh .. + 7 and 16 + 8 lh .. + 7 (past the row's end the next row's,
-    // which no key of the sequence takes)
+    // attn_bias of the next step's block: lane (ln, lh) has row ln, keys 8 lh .. + 7 and 16 + 8 lh .. + 7 (past the row's end the next row's:
+    // a step drops what the row does not see)
     u32x4_t bias[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
     const uint32_t bias_pitch = static_cast<uint32_t>(a.max_k) * 2u;
     const uint32_t bias_lane = (HAS_RAB && cw0 + 8 * lh < a.max_k) ? static_cast<uint32_t>(ln) * bias_pitch + (cw0 + 8 * lh) * 2u : kOutOfRange;
@@ -341,6 +341,14 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     const uint32_t ds_lane = static_cast<uint32_t>(ln * 32 + lh * 16);
 #define HSTU_FENCE() __builtin_amdgcn_sched_barrier(0)
 
+    // (masked blocks) lane = row: its visible keys
+    auto rows_see = [&](int rq0) -> uint32_t {
+        int lim, hole_lo, hole_hi;
+        row_bounds(si, a.mask_type, a.target_group, rq0 + ln, lim, hole_lo, hole_hi);
+        lim = rq0 + ln < sq ? lim : 0;
+        return bits_below(lim - cw0) & ~(bits_below(hole_hi - cw0) & ~bits_below(hole_lo - cw0));
+    };
+
     auto block = [&](auto masked, const uint16_t* q_tile, int rq0, const f32x16_t& s_first) {
         constexpr bool kMasked = decltype(masked)::value;
         const uint16_t* const g_tile = q_tile + T::ELEMS;
@@ -359,12 +367,9 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
         if constexpr (HAS_RAB) {
             s = s_first;
         }
-        uint32_t visible = 0;  // (masked blocks) lane = row: its visible keys
+        uint32_t visible = 0;
         if constexpr (kMasked) {
-            int lim, hole_lo, hole_hi;
-            row_bounds(si, a.mask_type, a.target_group, rq0 + ln, lim, hole_lo, hole_hi);
-            lim = rq0 + ln < sq ? lim : 0;
-            visible = bits_below(lim - cw0) & ~(bits_below(hole_hi - cw0) & ~bits_below(hole_lo - cw0));
+            visible = rows_see(rq0);
         }
         int n_off = n_first_off;
         asm volatile("" : "+v"(n_off));  // (not to be worked out ahead of the sweep)
@@ -525,6 +530,8 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
         for (int i = 0; i < 16; ++i) {
             s[i] = 0.f;
         }
+        const int x = cur_x;
+        const bool masked = x < full_from || x >= full_to;
         if constexpr (HAS_RAB) {
             // the matrix pipe transposes the bias into the scores' accumulators; its registers take the next block's at once
             int word = one_word;
@@ -537,6 +544,20 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
                     route[j][i] = word == 8 * j + i ? one : 0u;
                 }
             }
+            if (masked) {
+                // (what a row does not see -- hidden keys, padding, the next row -- may be anything and must not meet the products: 0 x NaN.
+                // A lane holds its row's bias, so the row's bit mask is at hand: 4 instructions a word, in masked blocks alone)
+                const int seen = static_cast<int>(rows_see(x * 32) >> (8 * lh));
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 16 * j + 2 * i, 1));
+                        const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 16 * j + 2 * i + 1, 1));
+                        bias[j][i] &= (hi << 16) | (lo & 0xffffu);
+                    }
+                }
+            }
             s = mfma32<Tag>(bias[0], route[0], s);
             s = mfma32<Tag>(bias[1], route[1], s);
             asm volatile("" : "+v"(s));
@@ -544,9 +565,8 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             next_bias();
         }
         request(stage_o);
-        const int x = cur_x;
         HSTU_FENCE();
-        if (x >= full_from && x < full_to) {
+        if (!masked) {
             block(std::false_type{}, q_tile, x * 32, s);
         } else if (cw0 < swept_key_limit(a, si, x * 32)) {  // (otherwise nothing is visible: the query-tile kernel does not read this tile)
             block(std::true_type{}, q_tile, x * 32, s);
