@@ -19,9 +19,10 @@
 // 2.0 + 0.9 ms of the kernels that recompute.  Ordinary ones the vector unit and the longest workgroup: 32 x 4 heads, d 128, 256..1024
 // rows 62 + 21 us, where the query-tile kernel with dS and P took 61 and the kernels that read them 41.  A wavefront with 64 keys and
 // all 512 registers, one per SIMD, took as long as this one (1.39 ms at the large shape) and has half as many workgroups.
-// With attn_bias memory bounds the key-tile kernel: 16 x 4 heads, d 128, 512..2048 rows 890 MB (415 of zeros, 122 of dS, 306 fetched) in
-// 205 us = 4.3 TB/s; the call 364 -> 280 us, where dV, dQ storing dS and dK from it took 185 + 139 + 61.
-// The query-tile kernel moves dS once: 4.4 TB/s from memory at the large shape (0.64 ms), 0.35 of that from the cache.
+// With attn_bias the key-tile kernel at the slot 128 spills: 16 x 4 heads, d 128, 512..2048 rows 248 us, 193 before a block cleared what its
+// rows do not see of the bias (39 scratch instructions against 16, in every order of that code tried; none at the slot 64); the call
+// 368 -> 344 us, where dV, dQ storing dS and dK from it took 185 + 139 + 61.
+// The query-tile kernel moves dS once: at the large shape 3.8 GB fetched, 2.6 of them dS, in 0.65 ms = 5.8 TB/s.
 #pragma once
 #include "hstu_bwd_kernel.hip.h"
 #include "hstu_fwd_short_kernel.hip.h"
@@ -546,7 +547,8 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             }
             if (masked) {
                 // (what a row does not see -- hidden keys, padding, the next row -- may be anything and must not meet the products: 0 x NaN.
-                // A lane holds its row's bias, so the row's bit mask is at hand: 4 instructions a word, in masked blocks alone)
+                // A lane holds its row's bias, so the row's bit mask is at hand: 4 instructions a word, in masked blocks alone.  This side of
+                // next_bias(): behind it, where branches meet, the compiler would copy registers that the request still fills.)
                 const int seen = static_cast<int>(rows_see(x * 32) >> (8 * lh));
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
