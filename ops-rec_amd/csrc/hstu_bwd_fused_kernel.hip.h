@@ -24,6 +24,7 @@
 // 368 -> 344 us, where dV, dQ storing dS and dK from it took 185 + 139 + 61.
 // The query-tile kernel moves dS once: at the large shape 3.8 GB fetched, 2.6 of them dS, in 0.65 ms = 5.8 TB/s.
 #pragma once
+#include "hstu_bias_requests.h"
 #include "hstu_bwd_kernel.hip.h"
 #include "hstu_fwd_short_kernel.hip.h"
 #include "hstu_pinned_acc.hip.h"
@@ -253,23 +254,22 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     // attn_bias of the next step's block: lane (ln, lh) has row ln, keys 8 lh .. + 7 and 16 + 8 lh .. + 7 (past the row's end the next row's:
     // a step drops what the row does not see)
     u32x4_t bias[2] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
-    const uint32_t bias_pitch = static_cast<uint32_t>(a.max_k) * 2u;
-    const uint32_t bias_lane = (HAS_RAB && cw0 + 8 * lh < a.max_k) ? static_cast<uint32_t>(ln) * bias_pitch + (cw0 + 8 * lh) * 2u : kOutOfRange;
-    const uint8_t* bias_head = static_cast<const uint8_t*>(a.rab) + (HAS_RAB ? bias_plane_of(a, b, first_h) * 2 : 0);
-    int bias_left = n_iter, bias_x = x_first;
+    BiasRequests wanted;
+    wanted.plane = reinterpret_cast<uint64_t>(a.rab) + (HAS_RAB ? bias_plane_of(a, b, first_h) * 2 : 0);
+    wanted.pitch = static_cast<uint32_t>(a.max_k) * 2u;
+    wanted.size = static_cast<uint32_t>(a.max_q) * wanted.pitch;
+    wanted.x = wanted.first = x_first;
+    wanted.skip_from = x_skip_from;
+    wanted.skip_to = x_skip_to;
+    wanted.end = n_qsub;
+    wanted.left = n_iter;
+    wanted.set_lane(a.max_k, cw0, ln, lh);
     auto next_bias = [&]() {
-        const u32x4_t rsrc = make_rsrc_words(bias_head, static_cast<uint32_t>(a.max_q) * bias_pitch);
-        const uint32_t off = bias_lane + (bias_left > 0 ? static_cast<uint32_t>(bias_x * 32) * bias_pitch : kOutOfRange);
+        const u32x4_t rsrc = make_rsrc_words(reinterpret_cast<const uint8_t*>(wanted.plane), wanted.bytes());
+        const uint32_t off = wanted.offset();
         request_bias<0>(bias[0], rsrc, off);
         request_bias<32>(bias[1], rsrc, off);
-        --bias_left;
-        if (++bias_x == x_skip_from) {
-            bias_x = x_skip_to;
-        }
-        if (bias_x >= n_qsub) {
-            bias_x = x_first;
-            bias_head += static_cast<int64_t>(a.max_q) * bias_pitch;
-        }
+        wanted.advance();
     };
     // The product with a 0/1 matrix that moves a lane's pieces to its keys (see hstu_bwd_dkv_kernel): the element of k-slot (lh, e) of
     // product j that is 1 is e = ln - 16 j - 8 lh.  Eight registers for the whole sweep are not to be had: a block works it out.
