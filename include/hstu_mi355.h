@@ -210,9 +210,10 @@ typedef struct hstu_jagged_bwd_params {
 
 HSTU_API int hstu_jagged_bwd_workspace_size(const hstu_jagged_bwd_params* params, uint64_t* workspace_bytes);
 /* The workspace with which the call is fastest.  bf16 / fp16 calls without custom mask, head dims up to 256 in multiples of 8, attn_bias
- * (if any) in rows that start at multiples of four bytes: the kernel that produces grad_k and grad_v leaves dS in it, rounded to the input type, for the one that produces grad_q -- 2 KiB
- * per head and (32 query rows x 32 keys) block, blocks at or below the diagonal only where the mask is causal over equal offsets
- * without context rows; at most 4 GiB (or HSTU_MI355_BWD_WORKSPACE_MB), with as many heads per pair of launches as have room in it.
+ * (if any) in rows that start at multiples of four bytes: the kernel that produces grad_k and grad_v leaves dS in it, rounded to the
+ * input type, for the one that produces grad_q -- 2 KiB per head and (32 query rows x 32 keys) block, blocks at or below the diagonal
+ * only where the mask is causal over the same offsets and bounds without context rows; at most 4 GiB (or HSTU_MI355_BWD_WORKSPACE_MB),
+ * with as many heads per pair of launches as have room in it.
  * What hstu_jagged_bwd_workspace_size says is enough for the other orders; a caller may bring either, or anything between: the call takes
  * the fastest order that fits. */
 HSTU_API int hstu_jagged_bwd_best_workspace_size(const hstu_jagged_bwd_params* params, uint64_t* workspace_bytes);

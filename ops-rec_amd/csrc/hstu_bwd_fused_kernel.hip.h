@@ -32,7 +32,7 @@
 namespace hstu {
 
 // The dS workspace: 2 KiB tiles of 32 query rows x 32 keys, those of a (head, sequence, 32-row group) side by side in key order.
-// For a causal mask over equal query and key offsets without context rows (ds_tri) group g holds the tiles 0 .. g, otherwise all
+// For a causal mask over equal offsets and bounds of queries and keys without context rows (ds_tri) group g holds the tiles 0 .. g, otherwise all
 // ceil(max_k / 32).  Sequences are placed by their first row, 32 rows of slack each, so that the host knows the size without the
 // lengths: floor(q0 / 32) + b groups lie ahead of sequence b at most.
 // In a tile, row half h2 (16 rows) is 1 KiB: key k's 16 rows (32 bytes) at ((k ^ 4 h2) * 32): the key-tile kernel, which has 8 rows of

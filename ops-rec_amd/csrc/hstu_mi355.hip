@@ -911,8 +911,9 @@ static DsTiles ds_tiles(const hstu_jagged_fwd_params* f, int64_t cap)
 {
     DsTiles t;
     const int64_t n_blk = (f->max_seq_len_k + 31) / 32;
+    // (a sequence longer than a bound is cut at it: under two bounds it could keep more keys than rows, which see past the diagonal then)
     t.tri = f->mask_type == HSTU_MASK_TRIL && f->num_context == nullptr && f->seq_offset_k == f->seq_offset_q &&
-            f->total_k == f->total_q && f->max_seq_len_q <= f->max_seq_len_k;
+            f->total_k == f->total_q && f->max_seq_len_q == f->max_seq_len_k;
     const int64_t groups = f->total_q / 32 + (f->n_offsets - 1);
     t.head_tiles = t.tri ? (groups * (n_blk + 1) + 1) / 2 : groups * n_blk;
     const int64_t ratio = f->num_heads_q / f->num_heads_k;

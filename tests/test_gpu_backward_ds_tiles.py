@@ -151,3 +151,22 @@ def test_rows_and_keys_that_belong_to_no_tile(dim, monkeypatch):
         keep = torch.ones(a.shape[0], dtype=torch.bool, device=DEV)
         keep[first : first + 96] = False  # (the 32-key blocks that the row's 32-row block touches)
         assert torch.equal(a[keep], b[keep]) and torch.equal(a[:, 1], b[:, 1])
+
+
+@pytest.mark.parametrize("max_q,max_k", [(160, 260), (260, 160), (200, 200)])
+def test_sequences_longer_than_the_bounds(max_q, max_k, monkeypatch):
+    """Sequences are cut at either bound, and a causal mask is aligned to their ends: with fewer rows than keys kept, rows see past the
+    diagonal.  Rows and keys past the bounds are not written."""
+    w = make(batch=0, heads=2, dim=64, lo=0, hi=0, lengths=[250, 260, 90, 255], max_seq_len=260, seed=4)
+    w.seq_offset_k, w.max_seq_len, w.max_seq_len_k = w.seq_offset, max_q, max_k
+    grad_out = grad_for(w)
+    got = {}
+    for order in ("0", "3"):
+        helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", order)
+        got[order] = device_grads(w, grad_out)
+    for i, bound in enumerate((max_q, max_k, max_k)):
+        for b, n in enumerate(w.lengths):
+            first = int(w.seq_offset[b])
+            rows = slice(first, first + min(n, bound))
+            want = got["0"][i][rows].float()
+            torch.testing.assert_close(got["3"][i][rows].float(), want, atol=1e-2 * want.abs().max().item(), rtol=1e-2)

@@ -48,6 +48,8 @@ def test_tiles(dim):
     assert sizes(**dict(call, num_context=FAKE))[1] == tiles(below_diagonal=False)
     assert sizes(**dict(call, seq_offset_k=FAKE + 64))[1] == tiles(below_diagonal=False)
     assert sizes(**dict(call, max_seq_len_k=900))[1] == tiles(blocks=29, below_diagonal=False)  # (more query rows than keys in a sequence)
+    # a sequence of more than 900 rows keeps 900 of them and up to 1024 keys: rows see keys past the diagonal
+    assert sizes(**dict(call, max_seq_len_q=900))[1] == tiles(below_diagonal=False)
 
 
 def test_as_the_other_orders_elsewhere():
