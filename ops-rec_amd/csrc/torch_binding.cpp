@@ -252,7 +252,13 @@ Gradients backward(const Tensor& grad_in, const Call& c)
         p.grad_attn_bias = ptr(dbias);
         uint64_t ws_bytes = 0;
         if (hstu_jagged_bwd_best_workspace_size(&p, &ws_bytes) == HSTU_OK) {
-            const Tensor ws = empty_or_none(ws_bytes, q.device());  // (without one the library runs the launch order that needs none)
+            Tensor ws = empty_or_none(ws_bytes, q.device());
+            // no room: the workspace of the other launch orders where that is a smaller one, and none for the order that needs none
+            uint64_t less = 0;
+            if (!ws.defined() && hstu_jagged_bwd_workspace_size(&p, &less) == HSTU_OK && less < ws_bytes) {
+                ws_bytes = less;
+                ws = empty_or_none(ws_bytes, q.device());
+            }
             const int rc = hstu_jagged_bwd(&p, ptr(ws), ws.defined() ? ws_bytes : 0, stream_of(q));
             TORCH_CHECK(rc == HSTU_OK, "hstu_jagged_bwd failed (", rc, "): ", hstu_last_error());
             return {dq, dk, dv, dbias};

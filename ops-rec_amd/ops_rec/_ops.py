@@ -427,9 +427,7 @@ def _new_grad(like: torch.Tensor) -> torch.Tensor:
 
 
 def _new_workspace(n_bytes: int, device) -> Optional[torch.Tensor]:
-    """The workspace ``hstu_jagged_bwd`` asked for, or None when the device has no room for it: the library then
-    runs the launch order that needs none (everything recomputed where it is used), so a backward never fails for
-    want of scratch memory the reference's backward would not have needed."""
+    """A workspace for ``hstu_jagged_bwd``, or None when the device has no room for it."""
     if n_bytes == 0:
         return None
     try:
@@ -439,7 +437,14 @@ def _new_workspace(n_bytes: int, device) -> Optional[torch.Tensor]:
 
 
 def _launch_backward(p, ws_bytes: int, device) -> None:
+    """Without room for the workspace the library asked for, the one of the other launch orders where that is smaller, and none
+    for the order that needs none (everything recomputed where it is used): a backward never fails for want of scratch memory
+    the reference's backward would not have needed."""
     ws = _new_workspace(ws_bytes, device)
+    if ws is None and ws_bytes:
+        less = ctypes.c_uint64(0)
+        if _native.load().hstu_jagged_bwd_workspace_size(ctypes.byref(p), ctypes.byref(less)) == _native.HSTU_OK and less.value < ws_bytes:
+            ws = _new_workspace(less.value, device)
     stream = torch.cuda.current_stream(device).cuda_stream
     rc = _native.load().hstu_jagged_bwd(ctypes.byref(p), _ptr(ws), ws.numel() if ws is not None else 0, ctypes.c_void_p(stream))
     if rc != _native.HSTU_OK:

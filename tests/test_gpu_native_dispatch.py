@@ -122,6 +122,24 @@ def test_a_backward_whose_workspace_does_not_fit(monkeypatch):
     assert refused == 1 and all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, want))
 
 
+@pytest.mark.parametrize("python", [False, True], ids=["native", "python"])
+def test_a_backward_with_room_for_the_smaller_workspace(python, monkeypatch):
+    """Context rows, whole layouts: the dS of the three-launch order needs a few MiB less than the tiles, and is what the call takes
+    where those do not fit."""
+    w = workloads.make("oom", dtype=torch.bfloat16, device=DEV, seed=3, batch=4, heads=8, dim=128, lo=0, hi=0,
+                       lengths=[2052, 2052, 2016, 2006], max_seq_len=2052, num_context=4)  # fmt: skip
+    args = helpers.backward_args(w, torch.randn_like(w.q))
+    op = _ops.hstu_jagged_backward_delta if python else ops_rec.ascendc.attention.hstu_jagged_backward
+    call = lambda: op(*args)  # noqa: E731
+    tiles = helpers.allocated_beside(call)[1]
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "1")
+    want, plane = helpers.allocated_beside(call)
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", None)
+    assert plane + (4 << 20) <= tiles
+    got, refused = helpers.with_room_for(call, (plane + (2 << 20)) // (2 << 20) * (2 << 20), like=want)
+    assert refused == 1 and all((a is None and b is None) or torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("k", [1024, 1040])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_projection_backward_on_both_sides_of_the_rule_for_its_weight_gradient(k, dtype):
