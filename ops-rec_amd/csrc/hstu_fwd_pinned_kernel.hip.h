@@ -295,8 +295,13 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 3) void hstu_fwd_pinned_kernel(
             } else {
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
-                    s[2 * i + e] *= __builtin_amdgcn_rcpf(tt[e]);
+                    tt[e] = s[2 * i + e] * __builtin_amdgcn_rcpf(tt[e]);
                 }
+                // (rounded to fp32 here, as in the other forward kernels: left to itself the compiler takes the product and the rounding to fp16
+                // as one instruction in unmasked blocks, and the last bit of a row would depend on the kernel that its batch takes)
+                asm volatile("" : "+v"(tt[0]), "+v"(tt[1]));
+                s[2 * i] = tt[0];
+                s[2 * i + 1] = tt[1];
                 if constexpr (kMasked) {
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
