@@ -940,13 +940,17 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
 
 // Workgroups of the key-tile launch that do nothing but clear the attn_bias gradient: at the front of the grid, so that the zeros go out
 // beside the products from the start.  The fewer products a byte of the gradient comes with, the more of them (us of the backward with
-// 64 / 96 / 128): 16 x 4 heads, d 128, 512..2048 rows 287 / 290 / 296; 32 x 4 of
-// 256..1024 154 / 153 / 149; d 64 130 / - / 113; 64 x 4, d 64, 64..512 rows 82 / - / 68.  (Dealt over all workgroups ahead of their sweeps,
-// as the other orders have it, the zeros hold up every one of them: the dV launch alone takes 185 us at the first shape.)
-static int clear_workgroups(int64_t bytes, int64_t dmax, int cus)
+// 64 / 96 / 128, before the key-tile kernel cleared what rows do not see of the bias, which costs the first shape 50 us in each): 16 x 4
+// heads, d 128, 512..2048 rows 287 / 290 / 296; 32 x 4 of 256..1024 154 / 153 / 149; d 64 130 / - / 113; 64 x 4, d 64, 64..512 rows 82 / - /
+// 68.  (Dealt over all workgroups ahead of their sweeps, as the other orders have it, the zeros hold up every one of them: the dV launch
+// alone takes 185 us at the first shape.)
+// `groups`: the 32-row groups of all planes.  A wavefront takes about 2.5 us for a group however few its bytes are (the sequence's offsets,
+// one load after another), so small planes have a workgroup for every 16 of them: 512 x 1 heads, d 128, 64..100 rows 227 us with a workgroup per
+// MiB, 54 with this; 128 x 2 of 64..128 118 -> 32; 409 x 1, d 64, 158..204 90 -> 53; 64 x 2, d 256, 64..256 68 -> 48.
+static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus)
 {
     const int64_t most = dmax <= 64 ? cus / 2 : (dmax <= 128 ? 3 * cus / 8 : cus / 4);
-    return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, bytes >> 20) / 8 * 8));
+    return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, std::max(bytes >> 20, groups / 16)) / 8 * 8));
 }
 
 // Calls whose key-tile launch is a few workgroups that one sweep of all query rows (times query heads per K/V head) keeps busy long after
@@ -1492,6 +1496,7 @@ HSTU_API int hstu_jagged_bwd(const hstu_jagged_bwd_params* p, void* workspace, u
         // (rows of the gradient as whole lines from two query tiles per compute unit on: 16 x 4 heads of 512..2048 rows, query-tile kernel
         // 105 -> 79 us; a launch as long as one workgroup waits for the way through LDS: 2 x 4 of 2000..4000 rows, the call 269 -> 281 us)
         a.drab_lines = f->total_q / hstu::kBlockM * f->num_heads_q >= 2LL * cus ? 1 : 0;
+        const int64_t clear_groups = (f->n_offsets - 1) * f->num_heads_q * ((f->max_seq_len_q + 31) / 32);
         for (int first = 0; first < a.n_heads_q; first += static_cast<int>(tiles.heads)) {
             a.head_first = first;
             a.head_count = std::min(static_cast<int>(tiles.heads), a.n_heads_q - first);
@@ -1499,7 +1504,7 @@ HSTU_API int hstu_jagged_bwd(const hstu_jagged_bwd_params* p, void* workspace, u
             const int64_t kv_slots = static_cast<int64_t>(a.n_ktiles) * (a.pair_major ? 8 * ((pk + 7) / 8) : pk);
             const int64_t q_slots = static_cast<int64_t>(a.n_qtiles) * (a.pair_major ? 8 * ((pq + 7) / 8) : pq);
             a.drab_clear_bytes = drab_bytes;
-            a.clear_wgs = drab_bytes > 0 && first == 0 ? clear_workgroups(drab_bytes, std::max(f->head_dim_qk, f->head_dim_v), cus) : 0;
+            a.clear_wgs = drab_bytes > 0 && first == 0 ? clear_workgroups(drab_bytes, clear_groups, std::max(f->head_dim_qk, f->head_dim_v), cus) : 0;
             if (kv_slots + a.clear_wgs > 0x7fffffffLL || q_slots > 0x7fffffffLL) {
                 return fail(HSTU_ERR_INVALID, "grid out of range");
             }

@@ -102,6 +102,16 @@ def test_bias_gradient_written_by_the_line(max_seq_len, monkeypatch):
     against_recomputing(w, monkeypatch)
 
 
+@pytest.mark.parametrize("batch,heads", [(40, 1), (67, 2), (400, 2)])
+@pytest.mark.parametrize("dim", [64, 128, 256])
+def test_many_small_gradients_are_cleared(batch, heads, dim, monkeypatch):
+    """Clearing workgroups by the number of 32-row groups (at least 8, a multiple of 8, at most a share of the compute units): each group
+    is cleared once, whatever their number."""
+    w = make(batch=batch, heads=heads, dim=dim, lo=1, hi=100, max_seq_len=104, rab_std=0.5, seed=batch)
+    helpers.poison_workspace(monkeypatch)
+    against_recomputing(w, monkeypatch)
+
+
 @pytest.mark.parametrize("dim", [64, 128, 256])
 @pytest.mark.parametrize("mask_type", [0, 2], ids=["causal", "none"])
 @pytest.mark.parametrize("lq,lk", [([70, 200, 1, 96], [370, 333, 129, 96]), ([300, 129, 40], [65, 200, 0])], ids=["more_keys", "fewer_keys"])
