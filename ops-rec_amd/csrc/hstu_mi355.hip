@@ -953,6 +953,40 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
     return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, std::max(bytes >> 20, groups / 16)) / 8 * 8));
 }
 
+// The same for calls with attn_bias.  The key-tile kernel's step is longest there, most of all at the slot 128, where it spills, and a
+// workgroup has as many steps as its K/V head has query heads times row blocks: the order pays from the tiles on that keep the machine
+// busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute units,
+// whatever the group's size.
+// Measured on 125 shapes (device time in us, other order / dS handed over):
+//   slot 128, grouped: 32 x 8 on 2, 512 rows, 288 tiles 196 / 226; 16 x 8 on 2, 256..1024 (176 tiles) 230 / 304; 32 x 8 on 1, 1024 (272) 690 / 793;
+//     8 x 8 on 4, 1024..2048 (400, three quarters) 507 / 450; 32 x 8 on 4, 256..1024 (704) 328 / 296; 64 x 8 on 2, 256..1024 (704) 775 / 634
+//   slot 128, rows of one tile: 512 x 2, 100..128 rows 87 / 99; 256 x 8 on 4, 64..128 139 / 150; 512 x 4, 128 rows, 2048 tiles 209 / 197
+//   slot 128, a head each: 16 x 4, 300..500 rows, 230 tiles 54 / 58; 128 x 2, 256 rows, 640 tiles 59 / 62; 128 x 4, 200..300, 1256 tiles 150 / 138;
+//     8 x 4, 512..1024 108 / 102; 32 x 4, 256..1024 160 / 143
+//   slot 64, four query heads per K/V head and more: 16 x 8 on 2, 200..400 rows, 92 tiles 72 / 78; 32 x 8 on 1, 200..400 127 / 149; 64 x 8 on 2, 128..256,
+//     256 tiles 75 / 69; 4 x 8 on 1, 512..1024, 26 tiles 266 / 295; 16 x 8 on 1, 256..1024 324 / 288; two heads: 8 x 4 on 2, 200..400 45 / 42
+//   rows on a history, whose sweeps are short for their tiles: slot 128, 32 x 4, 64 rows on 1000 keys 83 / 69, 16 x 4, 200 on 1000 87 / 65, 16 x 8
+//     on 2, 256 on 1024 (272 tiles) 148 / 130, 4 x 8 on 2, 300 on 700 (48 tiles) 83 / 114; slot 64, 4 x 8 on 2, 300 on 700 81 / 72, 2 x 8 on 1, 100..200 on
+//     500 (8 tiles) 58 / 67; slot 256 120 / 118 and 94 / 105
+//   slot 256, as 64: 4 x 8 on 2, 1024..2048, 100 tiles 451 / 517; 16 x 8 on 2, 256..1024, 176 tiles 320 / 300; 32 x 8 on 1, 512..1024 833 / 637
+static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, int64_t tiles, int64_t cus)
+{
+    const int64_t batch = f->n_offsets - 1, ratio = f->num_heads_q / f->num_heads_k;
+    if (f->total_k >= 2 * f->total_q) {
+        return dmax > 64 && dmax <= 128 ? ratio > 1 && 2 * tiles < cus : ratio >= 8 && 8 * tiles <= cus;
+    }
+    if (dmax <= 64) {
+        return ratio >= 4 && ((f->total_q <= 400 * batch && 4 * tiles < 3 * cus) || (ratio >= 8 && 8 * tiles <= cus));
+    }
+    if (dmax > 128) {
+        return ratio >= 4 && 8 * tiles < 5 * cus;
+    }
+    if (f->total_q <= hstu::kBlockM * batch && tiles < 6 * cus) {
+        return true;
+    }
+    return ratio == 1 ? f->total_q < 600 * batch && 2 * tiles <= 5 * cus : 8 * tiles * f->total_q <= 9 * cus * batch * f->max_seq_len_q;
+}
+
 // Calls whose key-tile launch is a few workgroups that one sweep of all query rows (times query heads per K/V head) keeps busy long after
 // the machine has emptied: there the planes order, whose long launch has a workgroup per query tile and head, is the shorter one.
 // Grouped heads, K/V tiles of 128 keys (us, planes / dS handed over): 16 x 8 heads on 2, 256..1024 rows, d 128, 160 tiles 131 / 158, d 64
@@ -970,9 +1004,7 @@ static bool few_key_tiles(const hstu_jagged_fwd_params* f)
     const int64_t dmax = f->head_dim_qk > f->head_dim_v ? f->head_dim_qk : f->head_dim_v;
     const int64_t tiles = (f->total_k + 64 * batch) / 128 * f->num_heads_k;
     if (f->attn_bias != nullptr) {
-        // (its rows then go through two launches in every order: 16 x 8 on 2, 256..1024 rows, d 64 226 / 184; 3 x 2, 100..304 rows 32 / 28;
-        // 2 x 4 on 2, 60..136 rows, d 256 34 / 36)
-        return false;
+        return few_biased_key_tiles(f, dmax, tiles, cus);
     }
     if (f->num_heads_q > f->num_heads_k) {
         return 4 * tiles < 3LL * cus;

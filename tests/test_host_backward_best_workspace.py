@@ -75,3 +75,36 @@ def test_limits_and_switches(monkeypatch):
         assert size == best
     helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
     assert sizes(**dict(BATCH, n_offsets=3, total_q=500, total_k=500))[1] == tiles(rows=500, batch=2)
+
+
+BIASED = [  # heads, K/V heads, head dim, batch, rows, bound of rows, keys; whether the call takes the dS tiles
+    (8, 2, 128, 16, 640, 1024, 640, False),  # grouped heads: fewer (tiles x mean rows / longest rows) than 9/8 of the compute units
+    (8, 1, 128, 32, 1024, 1024, 1024, False),
+    (8, 4, 128, 32, 640, 1024, 640, True),
+    (8, 2, 128, 4, 300, 300, 700, False),  # on a history: fewer tiles than half of them
+    (8, 2, 128, 16, 256, 256, 1024, True),
+    (2, 2, 128, 512, 114, 128, 114, False),  # rows of one tile
+    (4, 4, 128, 512, 128, 128, 128, True),
+    (4, 4, 128, 16, 400, 500, 400, False),  # a head each: short rows
+    (4, 4, 128, 8, 768, 1024, 768, True),
+    (4, 4, 128, 128, 250, 300, 250, True),
+    (4, 4, 128, 32, 64, 64, 1000, True),
+    (8, 2, 64, 16, 300, 400, 300, False),
+    (8, 1, 64, 4, 768, 1024, 768, False),
+    (8, 1, 64, 16, 640, 1024, 640, True),
+    (4, 2, 64, 8, 300, 400, 300, True),
+    (8, 2, 256, 4, 1536, 2048, 1536, False),
+    (8, 2, 256, 16, 640, 1024, 640, True),
+    (4, 2, 256, 8, 768, 1024, 768, True),
+]
+
+
+@pytest.mark.parametrize("heads,heads_k,dim,batch,rows,max_rows,keys,taken", BIASED)
+def test_calls_with_a_bias(heads, heads_k, dim, batch, rows, max_rows, keys, taken):
+    """Where the orders without dS tiles were measured to be the faster ones (256 compute units), the call asks for their workspace."""
+    own = keys != rows
+    call = dict(n_offsets=batch + 1, num_heads_q=heads, num_heads_k=heads_k, head_dim_qk=dim, head_dim_v=dim, total_q=batch * rows,
+                total_k=batch * keys, max_seq_len_q=max_rows, max_seq_len_k=(keys if own else max_rows), seq_offset_k=FAKE + (64 if own else 0))  # fmt: skip
+    size, best = sizes(grad_attn_bias=FAKE, **call)
+    whole = tiles(rows=batch * rows, batch=batch, heads=heads, blocks=(call["max_seq_len_k"] + 31) // 32, below_diagonal=not own)
+    assert best == (whole if taken else size) and whole != size
