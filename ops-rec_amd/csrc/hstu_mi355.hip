@@ -945,12 +945,13 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
 // 68.  (Dealt over all workgroups ahead of their sweeps, as the other orders have it, the zeros hold up every one of them: the dV launch
 // alone takes 185 us at the first shape.)
 // `groups`: the 32-row groups of all planes.  A wavefront takes about 2.5 us for a group however few its bytes are (the sequence's offsets,
-// one load after another), so small planes have a workgroup for every 16 of them: 512 x 1 heads, d 128, 64..100 rows 227 us with a workgroup per
-// MiB, 54 with this; 128 x 2 of 64..128 118 -> 32; 409 x 1, d 64, 158..204 90 -> 53; 64 x 2, d 256, 64..256 68 -> 48.
+// one load after another), so small planes have a workgroup for every 8 of them, two per wavefront: 64 x 2 heads, d 64, 64..128 rows 59 us
+// with a workgroup per MiB, 23 with one for every 16 groups as well, 19.4 with one for 8; 32 x 4 of 40..200 78, 23.9, 23.0; 409 x 1 of 158..204
+// 90, 53, 53; d 128, 16 x 4, 200 rows on 1000 keys 65, 65, 60.
 static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus)
 {
     const int64_t most = dmax <= 64 ? cus / 2 : (dmax <= 128 ? 3 * cus / 8 : cus / 4);
-    return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, std::max(bytes >> 20, groups / 16)) / 8 * 8));
+    return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, std::max(bytes >> 20, groups / 8)) / 8 * 8));
 }
 
 // The same for calls with attn_bias.  The key-tile kernel's step is longest there, most of all at the slot 128, where it spills, and a
