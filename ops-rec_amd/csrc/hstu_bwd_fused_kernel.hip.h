@@ -491,6 +491,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             }
             HSTU_FENCE();
         });
+        acc_fence<kAccRegs>();
         // dS to the workspace: the two lanes of a key trade halves, 8 rows each
         {
             typedef __attribute__((ext_vector_type(2))) unsigned u2_t;
@@ -506,6 +507,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
                 __builtin_amdgcn_raw_buffer_store_b128(w, ds_rsrc, static_cast<int>((ds_lane ^ (128u * h2)) + 1024u * h2 + tile), 0, 0);
             }
         }
+        acc_fence<kAccRegs>();
         HSTU_FENCE();
         static_for<NCH>([&](auto ci) {
             constexpr int c = ci;
@@ -518,6 +520,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
 
     auto step = [&](const uint16_t* q_tile, int stage_o) {
         // this step's sub-tile has landed for everybody; the stage of the previous step is free
+        acc_fence<kAccRegs>();
         HSTU_FENCE();
         if constexpr (HAS_RAB) {
             asm volatile("s_waitcnt vmcnt(%2)" : "+v"(bias[0]), "+v"(bias[1]) : "n"(2 * LPW) : "memory");

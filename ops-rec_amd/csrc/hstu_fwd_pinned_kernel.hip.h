@@ -315,6 +315,7 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 3) void hstu_fwd_pinned_kernel(
             pk[i] = pack2<Tag>(s[2 * i], s[2 * i + 1]);
             asm volatile("" : "+v"(pk[i]));
         };
+        acc_fence<kAccRegs>();
         constexpr int kFirst = NCH >= 16 ? 2 : 1;  // (the last score product has to end first)
         auto parts_done = [](int g) constexpr { return g < kFirst ? 0 : ((g - kFirst + 1) * 16 + NCH - kFirst - 1) / (NCH - kFirst); };
         static_for<NCH>([&](auto ci) {

@@ -5,8 +5,10 @@
 // through vector registers (the source is compiled with the matrix instructions' results in vector registers, see _build.py).
 //
 // The compiler does not know what these registers hold.  It would use them for values of its own only when it is out of vector
-// registers; acc_fence() keeps any such value from living across it, and stands in every phase of the kernels.  A change to a
-// kernel that uses this header is checked by looking for accumulators outside assembly in what the compiler wrote.
+// registers; acc_fence() keeps any such value from living across it, and stands in every phase of the kernels.  Nor does it know what
+// the assembly here needs: that the vector unit leaves an operand of acc_mfma() alone for two instructions ahead of it, and that nobody
+// touches the registers of a load in assembly before its wait.  tests/test_host_pinned_registers.py looks for all three in what the
+// compiler makes of the kernels that use this header.
 #pragma once
 #include <utility>
 
