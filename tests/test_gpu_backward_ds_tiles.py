@@ -10,6 +10,7 @@ import torch
 import helpers
 from ops_rec import workloads
 from test_gpu_backward import DEV, check, device_grads, make
+from test_host_backward_best_workspace import tiles
 
 pytestmark = pytest.mark.gpu
 
@@ -19,6 +20,13 @@ def grad_for(w, seed=6):
     return torch.randn(w.q.shape[0], w.q.shape[1], w.v.shape[2], generator=g, device=DEV).to(w.q.dtype)
 
 
+def bytes_of_tiles(w):
+    args = helpers.backward_args(w, None)
+    max_q, max_k, offs_q, offs_k, context = args[7], args[8], args[10], args[11], args[12]
+    whole = w.mask_type != 0 or context is not None or offs_k is not offs_q or max_q != max_k
+    return tiles(rows=w.q.shape[0], batch=offs_q.numel() - 1, heads=w.q.shape[1], blocks=(max_k + 31) // 32, below_diagonal=not whole)
+
+
 def against_recomputing(w, monkeypatch):
     grad_out = grad_for(w)
     helpers.set_switch(monkeypatch, "HSTU_MI355_GENERIC_BACKWARD", "0")
@@ -26,7 +34,8 @@ def against_recomputing(w, monkeypatch):
     two = device_grads(w, grad_out)
     helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
     got, beside = helpers.allocated_beside(lambda: device_grads(w, grad_out))
-    assert beside >= 2048  # the tiles
+    # this order ran: the other ones' workspaces are of other sizes (beside the workspace: a few counts that backward_args makes)
+    assert 0 <= beside - bytes_of_tiles(w) < 2048
     # S is formed with its operands the other way round and dS is rounded before dQ's product, as before dK's: one rounding of the
     # input type in the terms of a sum
     tol = 1e-2 if w.q.dtype == torch.bfloat16 else 2e-3
