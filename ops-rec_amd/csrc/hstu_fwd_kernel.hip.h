@@ -1415,6 +1415,12 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             rows_only_from = (other_hi + 31) >> 5;
             rows_only_to = ctx_lo >> 5;
         }
+        // the sub-tiles ahead of this one are fully visible to every row of this wavefront
+        int full_tiles = lim_min >> 5;
+        if (any_hole) {
+            const int before_targets = hist_k > 0 ? hist_k >> 5 : 0;
+            full_tiles = full_tiles < before_targets ? full_tiles : before_targets;
+        }
         // (one scalar register: the d = 128 variants have none to spare)
         const uint32_t rows_only = static_cast<uint32_t>(uniform(rows_only_from | (rows_only_to << 16)));
         // per-lane bounds relative to the lane's first key of a sub-tile (key = c0 + 4*lh + kk)
@@ -1494,19 +1500,11 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 w[kRabWords - 1] = __builtin_amdgcn_raw_buffer_load_b32(rab_rsrc, static_cast<int>(off + 32u), 0, 0);
             }
         };
-        auto shift_rab = [&](int c0, uint32_t (&w)[kRabWords]) {
+        auto shift_rab = [&](uint32_t (&w)[kRabWords]) {
             const uint32_t shift = 8u * ((rab_ahead + 2u * static_cast<uint32_t>((wr0 + ln) * a.max_k)) & 2u);
 #pragma unroll
             for (int i = 0; i < kRabWords - 1; ++i) {
                 w[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], shift);
-            }
-            if (c0 + 32 > a.max_k) {
-                // (what lies behind the row, which may be anything, must not meet the products: 0 x NaN)
-#pragma unroll
-                for (int i = 0; i < kRabWords - 1; ++i) {
-                    const int left = a.max_k - (c0 + 16 * lh + 2 * i);
-                    w[i] = left >= 2 ? w[i] : (left == 1 ? w[i] & 0xffffu : 0u);
-                }
             }
         };
         // Requests the 16 bias (or mask) values of one 32-key sub-tile as 8 packed words; order_bias() must be
@@ -1575,6 +1573,32 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 w[3] = w[5];
                 w[4] = t2;
                 w[5] = t3;
+            }
+        };
+
+        // In a sub-tile that some row does not see whole: what a row does not see of its rab words -- hidden keys, padding, the next row -- may
+        // be anything and must not meet the routing products (0 x NaN).  16 x 8 heads of 1024..4096 rows, context and target rows 406 -> 410 us.
+        auto clear_rab = [&](int x, uint32_t (&w)[kRabWords]) {
+            const int c0 = x * 32;
+            if (x >= static_cast<int>(rows_only & 0xffffu) && x < static_cast<int>(rows_only >> 16)) {
+                const uint32_t keep = lim_lane > c0 ? 0xffffffffu : 0u;  // (context rows: whole or not at all)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    w[i] &= keep;
+                }
+                return;
+            }
+            auto keys_below = [&](int limit_lane) -> uint32_t {  // of the lane's 16 keys, those below a limit
+                int n = limit_lane - 12 * lh - c0;
+                n = n < 0 ? 0 : (n > 31 ? 31 : n);
+                return (1u << n) - 1u;
+            };
+            const int seen = static_cast<int>(keys_below(lim_lane) & ~(keys_below(hole_hi_lane) & ~keys_below(hole_lo_lane)));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 2 * i, 1));
+                const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 2 * i + 1, 1));
+                w[i] &= (hi << 16) | (lo & 0xffffu);
             }
         };
 
@@ -1960,8 +1984,13 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 }
                 if constexpr (HAS_RAB && !F8) {
                     // S^T(t+1) += rab^T, last so that the rab request has had the whole block to land
-                    if (!INTERIOR && !rab_words) {
-                        shift_rab(c0 + 32, rab_nxt);
+                    if constexpr (!INTERIOR) {
+                        if (!rab_words) {
+                            shift_rab(rab_nxt);
+                        }
+                        if (t + 1 >= full_tiles) {
+                            clear_rab(t + 1, rab_nxt);
+                        }
                     }
                     const u32x4_t r0 = {rab_nxt[0], rab_nxt[1], rab_nxt[2], rab_nxt[3]};
                     const u32x4_t r1 = {rab_nxt[4], rab_nxt[5], rab_nxt[6], rab_nxt[7]};
@@ -2026,17 +2055,13 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         __syncthreads();
         if (x_end > x_begin) {
             // interior steps of this wavefront: [x_begin + 1, t_interior).  Sub-tile t + 1 (t + 2 with rab) must exist,
-            // and sub-tile t must be fully visible: it ends at or before the smallest row limit and, when target
+            // and sub-tile t (t + 1 with rab, whose words a step does not clear) must be fully visible: it ends at or before the smallest row limit and, when target
             // rows carve holes, before the first target key.  The wavefronts of a workgroup run different numbers
             // of interior steps; every step of either kind ends in the same one barrier, so the counts match.
             int t_interior = nx_w - (HAS_RAB ? 2 : 1);
             {
-                int full_tiles = lim_min >> 5;
-                if (any_hole) {
-                    const int before_targets = hist_k > 0 ? hist_k >> 5 : 0;
-                    full_tiles = full_tiles < before_targets ? full_tiles : before_targets;
-                }
-                t_interior = t_interior < full_tiles ? t_interior : full_tiles;
+                const int last_full = full_tiles - ((HAS_RAB && !F8) ? 1 : 0);
+                t_interior = t_interior < last_full ? t_interior : last_full;
             }
             // (short sweeps stay on the general step: measured on MI355X, sweeps under about twenty steps gain nothing
             // from the second copy of the step and lose a little to fetching its instructions)
