@@ -889,9 +889,11 @@ static PairPlane pair_plane(const hstu_jagged_fwd_params* f)
     PairPlane pp;
     const int64_t batch = f->n_offsets - 1;
     const int64_t n_blk = (f->max_seq_len_k + 31) / 32;
+    // (under two bounds a sequence longer than either is cut to more rows than keys, or to rows that see past the diagonal: neither fits
+    // this form)
     pp.tri = f->mask_type == HSTU_MASK_TRIL && f->num_context == nullptr && f->seq_offset_k == f->seq_offset_q &&
-             f->total_k == f->total_q;
-    const int64_t groups = ((f->max_seq_len_q < f->max_seq_len_k ? f->max_seq_len_q : f->max_seq_len_k) + 31) / 32;
+             f->total_k == f->total_q && f->max_seq_len_q == f->max_seq_len_k;
+    const int64_t groups = (f->max_seq_len_q + 31) / 32;
     const int64_t pitch = hstu::pair_full_pitch_lines(f->max_seq_len_k);
     pp.head_lines = pp.tri ? ((f->total_q + 32 * batch) * (n_blk + 1) + 1) / 2 : f->total_q * pitch;
     pp.bytes = f->num_heads_q * pp.head_lines * 128;

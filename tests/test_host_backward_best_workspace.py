@@ -108,3 +108,29 @@ def test_calls_with_a_bias(heads, heads_k, dim, batch, rows, max_rows, keys, tak
     size, best = sizes(grad_attn_bias=FAKE, **call)
     whole = tiles(rows=batch * rows, batch=batch, heads=heads, blocks=(call["max_seq_len_k"] + 31) // 32, below_diagonal=not own)
     assert best == (whole if taken else size) and whole != size
+
+
+def pair_lines(groups):
+    """Lines of the pair plane that ``groups`` 32-row groups take up to the diagonal (row group g: g + 1 lines a row)."""
+    return 16 * groups * (groups + 1)
+
+
+@pytest.mark.parametrize("max_q,max_k", [(300, 300), (300, 160), (160, 300), (640, 64)])
+def test_the_planes_hold_sequences_that_are_cut(max_q, max_k, monkeypatch):
+    """Sequences longer than a bound are cut at it: whatever the bounds, the plane has room for what the kernels write (the last sequence's
+    lines end inside it), up to the diagonal only where rows and keys are cut alike."""
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "2")
+    heads, lengths = 2, [700, 650, 700]
+    call = dict(n_offsets=4, num_heads_q=heads, num_heads_k=heads, total_q=sum(lengths), total_k=sum(lengths), max_seq_len_q=max_q,
+                max_seq_len_k=max_k)  # fmt: skip
+    size = sizes(**call)[0]
+    blocks = (max_k + 31) // 32
+    if max_q == max_k:
+        assert size == heads * 128 * (((sum(lengths) + 32 * 3) * (blocks + 1) + 1) // 2)
+    else:
+        assert size == heads * 128 * sum(lengths) * (blocks | 1)
+    # the sequences' first lines as the kernels place them, and the end of the last one
+    first, ahead = sum(lengths[:-1]), 2
+    rows = min(lengths[-1], max_q)
+    end = (((first + 32 * ahead) * (blocks + 1) + 1) // 2 + pair_lines((rows + 31) // 32)) if max_q == max_k else (first + rows) * (blocks | 1)
+    assert end <= size // heads // 128
