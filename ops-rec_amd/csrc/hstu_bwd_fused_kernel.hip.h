@@ -60,12 +60,6 @@ __device__ __forceinline__ uint32_t ds_group_offset(const BwdArgs& a, int g)
     return ((u * (a.ds_tri ? u + 1u : 2u * (static_cast<uint32_t>(a.max_k + 31) >> 5))) >> 1) * kDsTileBytes;
 }
 
-// bits 0 .. n - 1
-__device__ __forceinline__ uint32_t bits_below(int n)
-{
-    return n <= 0 ? 0u : (n >= 32 ? 0xffffffffu : (1u << n) - 1u);
-}
-
 // In a masked block, whether element e of a lane (row 8 (e / 4) + e % 4 of the block, 4 more in the upper half-wave) is visible to the
 // lane's key, from the rows' bit masks over keys that the lanes 0 .. 31 hold: a row's mask is that of its half-wave's lanes.
 __device__ __forceinline__ bool row_sees(uint32_t visible, int e)
@@ -343,12 +337,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
 #define HSTU_FENCE() __builtin_amdgcn_sched_barrier(0)
 
     // (masked blocks) lane = row: its visible keys
-    auto rows_see = [&](int rq0) -> uint32_t {
-        int lim, hole_lo, hole_hi;
-        row_bounds(si, a.mask_type, a.target_group, rq0 + ln, lim, hole_lo, hole_hi);
-        lim = rq0 + ln < sq ? lim : 0;
-        return bits_below(lim - cw0) & ~(bits_below(hole_hi - cw0) & ~bits_below(hole_lo - cw0));
-    };
+    auto rows_see = [&](int rq0) -> uint32_t { return row_sees_keys(si, a.mask_type, a.target_group, rq0 + ln, cw0); };
 
     auto block = [&](auto masked, const uint16_t* q_tile, int rq0, const f32x16_t& s_first) {
         constexpr bool kMasked = decltype(masked)::value;
@@ -549,19 +538,9 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
                 }
             }
             if (masked) {
-                // (what a row does not see -- hidden keys, padding, the next row -- may be anything and must not meet the products: 0 x NaN.
-                // A lane holds its row's bias, so the row's bit mask is at hand: 4 instructions a word, in masked blocks alone.  This side of
-                // next_bias(): behind it, where branches meet, the compiler would copy registers that the request still fills.)
-                const int seen = static_cast<int>(rows_see(x * 32) >> (8 * lh));
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 16 * j + 2 * i, 1));
-                        const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 16 * j + 2 * i + 1, 1));
-                        bias[j][i] &= (hi << 16) | (lo & 0xffffu);
-                    }
-                }
+                // (A lane holds its row's bias, so the row's bit mask is at hand.  This side of next_bias(): behind it, where branches meet, the
+                // compiler would copy registers that the request still fills.)
+                clear_unseen(bias, static_cast<int>(rows_see(x * 32) >> (8 * lh)));
             }
             s = mfma32<Tag>(bias[0], route[0], s);
             s = mfma32<Tag>(bias[1], route[1], s);

@@ -238,6 +238,34 @@ __device__ __forceinline__ void row_bounds(const SeqInfo& s, int mask_type, int 
     }
 }
 
+// bits 0 .. n - 1
+__device__ __forceinline__ uint32_t bits_below(int n)
+{
+    return n <= 0 ? 0u : (n >= 32 ? 0xffffffffu : (1u << n) - 1u);
+}
+// which of the keys k0 .. k0 + 31 query row r sees
+__device__ __forceinline__ uint32_t row_sees_keys(const SeqInfo& s, int mask_type, int group, int r, int k0)
+{
+    int lim, hole_lo, hole_hi;
+    row_bounds(s, mask_type, group, r, lim, hole_lo, hole_hi);
+    lim = r < s.sq ? lim : 0;
+    return bits_below(lim - k0) & ~(bits_below(hole_hi - k0) & ~bits_below(hole_lo - k0));
+}
+// Clears what a row does not see of its 16-bit values, keys 0 .. 7 and 16 .. 23 of the bits in `seen`: hidden keys, padding and the next row
+// may be anything and must not meet the 0/1 products that move the values to their keys (0 x NaN).  4 instructions a word.
+__device__ __forceinline__ void clear_unseen(u32x4_t (&w)[2], int seen)
+{
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 16 * j + 2 * i, 1));
+            const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_sbfe(seen, 16 * j + 2 * i + 1, 1));
+            w[j][i] &= (hi << 16) | (lo & 0xffffu);
+        }
+    }
+}
+
 // The score algebra of the backward, per element, with X = alpha s, sig = sigmoid(X), t = exp(-X):
 //   P  = X sig scale                       = s * [alpha scale sig]
 //   dS = alpha scale dP sig (1 + X (1 - sig)) = dP * [alpha scale sig] * (1 + s * [alpha (1 - sig)])
@@ -1281,6 +1309,15 @@ __global__ __launch_bounds__(kDkvThreads, (MODE == 2 || MODE >= 4) ? bwd_dk_from
             f32x16_t mt16;  // custom mask tile, transposed by the matrix pipe
             if constexpr (HAS_RAB || HAS_MASK) {
                 if (vec8) {
+                    if (!full) {
+                        const int seen = static_cast<int>(row_sees_keys(si, a.mask_type, a.target_group, rq0 + ln, cw0) >> (8 * lh));
+                        if constexpr (HAS_RAB) {
+                            clear_unseen(ra, seen);
+                        }
+                        if constexpr (HAS_MASK) {
+                            clear_unseen(ma, seen);
+                        }
+                    }
                     if constexpr (HAS_RAB) {
                         s = mfma32<Tag>(ra[0], route[0], s);
                         s = mfma32<Tag>(ra[1], route[1], s);

@@ -32,19 +32,25 @@ def planes(max_len, lengths, heads, where, dtype=torch.bfloat16):
 
 @pytest.mark.parametrize("where", ["rows", "keys", "hidden"])
 @pytest.mark.parametrize("max_len", [298, 300, 301, 304, 320])
-@pytest.mark.parametrize("dim", [64, 128, 256])
-def test_bias_that_no_pair_reads_reaches_no_gradient(dim, max_len, where, monkeypatch):
-    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", "3")
+@pytest.mark.parametrize(
+    "dim,order,dtype",
+    [(dim, order, torch.bfloat16) for dim in (64, 128, 256) for order in ("0", "1", "2", "3")]
+    + [(320, None, torch.bfloat16), (60, None, torch.float16), (64, None, torch.float32)],
+    ids=str,
+)
+def test_bias_that_no_pair_reads_reaches_no_gradient(dim, order, dtype, max_len, where, monkeypatch):
+    helpers.set_switch(monkeypatch, "HSTU_MI355_BWD_HANDOFF", order)
     lengths, heads = [max_len - 7, max_len - 40, max_len, 97], 2
     gen = torch.Generator(device="cuda").manual_seed(0)
 
     def rand(*shape):
-        return (torch.randn(*shape, generator=gen, device="cuda") * 0.3).bfloat16()
+        return (torch.randn(*shape, generator=gen, device="cuda") * 0.3).to(dtype)
 
     rows = sum(lengths)
-    q, k, v, grad = (rand(rows, heads, dim) for _ in range(4))
+    q, k = (rand(rows, heads, dim) for _ in range(2))
+    v, grad = (rand(rows, heads, dim // 16 * 16) for _ in range(2))
     offsets = torch.tensor([0] + list(itertools.accumulate(lengths)), dtype=torch.int32, device="cuda")
-    clean, dirty = planes(max_len, lengths, heads, where)
+    clean, dirty = planes(max_len, lengths, heads, where, dtype)
 
     def run(bias):
         return torch.ops.ops_rec.hstu_jagged_backward.equal(
@@ -52,6 +58,24 @@ def test_bias_that_no_pair_reads_reaches_no_gradient(dim, max_len, where, monkey
         )[:4]
 
     for want, got in zip(run(clean), run(dirty)):
+        assert torch.equal(want, got)
+
+
+@pytest.mark.parametrize("where", ["rows", "keys"])
+@pytest.mark.parametrize("max_len", [298, 300, 301, 304])
+@pytest.mark.parametrize("biased", [False, True])
+def test_mask_values_past_a_sequence_reach_nothing(biased, max_len, where):
+    lengths, heads, dim = [max_len - 7, max_len - 40, max_len, 97], 2, 64
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v, grad = ((torch.randn(sum(lengths), heads, dim, generator=gen, device="cuda") * 0.3).bfloat16() for _ in range(4))
+    offsets = torch.tensor([0] + list(itertools.accumulate(lengths)), dtype=torch.int32, device="cuda")
+    bias = planes(max_len, lengths, heads, "rows")[0] if biased else None
+    results = []
+    for mask in planes(max_len, lengths, heads, where):
+        rest = (mask, bias, 3, max_len, 1.0 / max_len, offsets, None, None, 0, dim**-0.5)
+        out = torch.ops.ops_rec.hstu_jagged.equal(q, k, v, *rest)
+        results.append((out, *torch.ops.ops_rec.hstu_jagged_backward.equal(grad, q, k, v, *rest)[: 4 if biased else 3]))
+    for want, got in zip(*results):
         assert torch.equal(want, got)
 
 
