@@ -53,6 +53,7 @@ CASES = {
     "64-bit offsets": (dict(lengths=EDGES * 5, heads=2, dim=256, index_dtype=torch.int64), BF),
     "history": (dict(lengths=[130, 129, 256, 200] * 18, heads=2, dim=256, history=500), BF),
     "history, grouped": (dict(lengths=[130, 31, 256, 200] * 15, heads=4, heads_k=2, dim=256, history=450), FP),
+    "history, four tiles a pair": (dict(lengths=[400, 130, 500, 290] * 12, heads=2, dim=256, history=600), BF),
     "fewer keys than rows": (dict(lengths=[130, 129, 256, 200] * 18, heads=2, dim=256, history=-60), BF),
 }
 
