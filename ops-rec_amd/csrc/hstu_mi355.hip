@@ -447,18 +447,23 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
 }
 
 // The kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): 16-bit inputs without bias and custom mask, more slots than a launch
-// without a list takes.  At the slot 256:  It has no list that sorts the sequences, so it takes batches whose mean lengths are at least
-// half of the largest (a Zipf law of lengths up to 8192 with a mean of an eighth: 416 -> 761 us), and, where the sequences are long, only
-// those with little between them and pairs enough for all XCDs (6 x 2 heads, 3000..6000 rows: 209 -> 258 us; 32 x 2, 1000..4000 326 -> 340).
+// without a list takes.
+// At the slot 256: it has no list that sorts the sequences, so it takes batches whose mean lengths are at least half of the largest (a
+// Zipf law of lengths up to 8192 with a mean of an eighth: 416 -> 761 us), and, where the sequences are long, only those with little between
+// them and pairs enough for all XCDs (6 x 2 heads, 3000..6000 rows: 209 -> 258 us; 32 x 2, 1000..4000 326 -> 340).
 // *pair_major: the tiles of a pair side by side on one XCD, once the K / V rows are about what the last-level cache holds (24 x 8 heads
 // of 512..2048 rows, 244 MB: 272 us before, 261 level after level, 227 pair after pair; 12 x 8 of 2048 rows, 201 MB: 290, 224, 247), or on
 // keys that are mostly history, where a pair's tiles are equally long and nothing is lost at the end (30 x 8, 300 rows on 600 keys: 87, 76, 60).
 // Measured list -> this kernel, launches queued back to back: 200 x 4 of 65..128 rows 57.8 -> 36.5 us, 48 x 4 of 129..512 rows 55.3 -> 37.2,
 // 16 x 4 of 512..2048 rows 95.2 -> 90.8, 32 x 2 of the same 98.0 -> 98.7, 24 x 8 of 1024 rows 187 -> 143, 64 x 4 of 1000..4000 rows 1192 -> 1029.
+// Not on a history where the tiles that exist are at most one per compute unit (estimated from the rows: a bound just above a tile gives
+// every sequence a slot more): two workgroups would share one while others idle.  39 x 4, 82..165 rows on 660 keys (229 tiles) 34 -> 41 us,
+// 26 x 4, 100..300 on 600 (214) 33 -> 38, 18 x 4, 250..400 on 800 (218) 40 -> 44; 12 x 4, 700..1400 on 2100 (417) 117 -> 104; without a
+// history 37 x 4, 82..165 rows (217) 17.4 -> 17.2.
 // At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of two
 // tiles and more on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
-// keys (629 MB) 470 -> 335 us, 200 x 4, 200 rows 524 -> 367, 400 x 2, 400 rows on 800..1000 (369 MB) 269 -> 200, 24 x 8, 400 rows on 3072 (302 MB) 178 ->
-// 160, 100 x 8 over 4 K/V heads, 400 rows on 1500..3000 493 -> 465; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 147 -> 150, of one
+// keys (629 MB) 470 -> 335 us, 200 x 4, 200 rows 524 -> 367, 400 x 2, 400 rows on 800..1000 (369 MB) 269 -> 200, 24 x 8, 400 rows on 3072
+// (302 MB) 178 -> 160, 100 x 8 over 4 K/V heads, 400 rows on 1500..3000 493 -> 465 (131 x 8 over 4, 200..500 rows on 2000 1 to 2 % behind); below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 147 -> 150, of one
 // tile 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.
 const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool* pair_major)
 {
@@ -485,7 +490,11 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
         const bool shared_history = p->total_k >= 2 * p->total_q && p->max_seq_len_q > hstu::kBlockM;
         return shared_history && kv_bytes >= (288LL << 20) && slots >= 3LL * cus && switches().short_lists != 1 ? &pv[0] : nullptr;
     }
-    *pair_major = kv_bytes >= (224LL << 20) || p->total_k >= 2 * p->total_q;
+    const bool history = p->total_k >= 2 * p->total_q;
+    if (history && (p->total_q + 64 * batch) / hstu::kBlockM * p->num_heads_q <= cus) {
+        return nullptr;
+    }
+    *pair_major = kv_bytes >= (224LL << 20) || history;
     if (!*pair_major && p->max_seq_len_k > 2048 && (batch * p->num_heads_k < 24 || 4 * p->total_q < 3 * batch * p->max_seq_len_q)) {
         return nullptr;
     }

@@ -152,3 +152,9 @@ def test_batches_the_rule_leaves_to_the_lists():
     assert name(heads=4, dim=256, lo=200, hi=300, rab_std=0.2).find("_pinned") < 0
     assert name(heads=4, dim=256, lo=200, hi=300, max_seq_len=800).find("_pinned") < 0  # most slots would be empty
     assert name(heads=4, dim=256, lo=200, hi=300, batch=8).endswith("_direct")
+    for batch, taken in ((26, False), (60, True)):  # on a history, a tile per compute unit at most: 2 x 4 x 26 with rows of 100 .. 300
+        w = workloads.make("route", batch=batch, heads=4, dim=256, lo=0, hi=0, lengths=[100, 300] * (batch // 2), dtype=BF, device=DEV)
+        w.seq_offset_k = torch.arange(0, 601 * batch, 600, device=DEV)[: batch + 1].to(w.seq_offset.dtype)
+        w.max_seq_len_k = 600
+        w.k = w.v = torch.zeros(600 * batch, 4, 256, dtype=BF, device=DEV)
+        assert prepared(w).kernel_name().endswith("_pinned") == taken
