@@ -80,7 +80,7 @@ using hstu::Variant;
 //   HSTU_MI355_SPLIT=0             forward: never cut long items into parts, nor deal the keys of an fp32 row over wavefronts (the
 //                                  rows of a sequence are then the same bits whatever else is in the batch, where both take one kernel);
 //                                  =1: cut them also on sweeps that are short for it
-//   HSTU_MI355_SHORT=0 / 1         forward: never / whenever possible the kernel for short lists
+//   HSTU_MI355_SHORT=0 / 1         forward: the persistent kernel alone / whenever possible the kernel for short lists
 //   HSTU_MI355_GENERIC_BACKWARD=1  backward: the generic kernels also where tuned ones exist (for comparisons)
 //   HSTU_MI355_BWD_HANDOFF=0/1/2/3 backward: force the launch order (two launches / three / planes / dS tiles)
 //   HSTU_MI355_BWD_WORKSPACE_MB=n  backward: the largest workspace the library asks for
@@ -464,11 +464,11 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
 // tiles and more on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
 // keys (629 MB) 470 -> 335 us, 200 x 4, 200 rows 524 -> 367, 400 x 2, 400 rows on 800..1000 (369 MB) 269 -> 200, 24 x 8, 400 rows on 3072
 // (302 MB) 178 -> 160, 100 x 8 over 4 K/V heads, 400 rows on 1500..3000 493 -> 465 (131 x 8 over 4, 200..500 rows on 2000 1 to 2 % behind); below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 147 -> 150, of one
-// tile 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.
+// tile 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.  HSTU_MI355_SHORT=0 switches it off.
 const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool* pair_major)
 {
     if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || var->d_pad < 128 || var->d_pad > 256 || var->persistent_wgs_per_cu <= 0 ||
-        p->attn_bias != nullptr || p->mask != nullptr || p->mask_type == HSTU_MASK_CUSTOM) {
+        p->attn_bias != nullptr || p->mask != nullptr || p->mask_type == HSTU_MASK_CUSTOM || switches().short_lists == 0) {
         return nullptr;
     }
     int cus = 0;

@@ -140,6 +140,17 @@ def test_every_replay_of_a_captured_launch_is_the_eager_result():
         assert torch.equal(out, want)
 
 
+def test_the_switch_for_the_persistent_kernel(monkeypatch):
+    w = workloads.make("switch", batch=40, heads=4, dim=256, lo=200, hi=300, dtype=FP, device=DEV, seed=2)
+    p = prepared(w)
+    assert p.kernel_name().endswith("_pinned")
+    out = p.launch()
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", "0")
+    p = prepared(w)
+    assert not p.kernel_name().endswith("_pinned")
+    assert torch.equal(p.launch(), out)
+
+
 def test_batches_the_rule_leaves_to_the_lists():
     def name(**kw):
         w = workloads.make("route", batch=kw.pop("batch", 40), dtype=BF, device=DEV, seed=1, **kw)
