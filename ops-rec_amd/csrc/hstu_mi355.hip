@@ -446,6 +446,23 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
     return var->kernel_queues != nullptr && n_blocks >= 4 * resident;
 }
 
+// Whether the queues then take the items pair after pair, as hstu_fwd_kernel decides from the lengths (six items per resident workgroup, or
+// four where the sequences have at most seven tenths of the longest one's tiles on average), by an estimate of the tiles: all of them where the mean
+// length is within half a tile of the longest, else the mean length's and a half per sequence.
+bool queues_pair_after_pair(const Variant* var, const hstu_jagged_fwd_params* p)
+{
+    int64_t resident = 0;
+    if (!takes_queue_variant(var, p, &resident)) {
+        return false;
+    }
+    const int64_t batch = p->n_offsets - 1;
+    const int64_t most = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * batch;
+    const bool alike = batch * p->max_seq_len_q - p->total_q < hstu::kBlockM / 2 * batch;
+    const int64_t tiles = alike ? most : std::min(most, p->total_q / hstu::kBlockM + batch / 2);
+    const int64_t items = tiles * p->num_heads_q;
+    return (items >= 4 * resident && 10 * tiles <= 7 * most) || items >= 6 * resident;
+}
+
 // The kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): 16-bit inputs without bias and custom mask, more slots than a launch
 // without a list takes.
 // At the slot 256: it has no list that sorts the sequences, so it takes batches whose mean lengths are at least half of the largest (a
@@ -462,9 +479,14 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
 // history 37 x 4, 82..165 rows (217) 17.4 -> 17.2.
 // At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of two
 // tiles and more on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
-// keys (629 MB) 470 -> 335 us, 200 x 4, 200 rows 524 -> 367, 400 x 2, 400 rows on 800..1000 (369 MB) 269 -> 200, 24 x 8, 400 rows on 3072
-// (302 MB) 178 -> 160, 100 x 8 over 4 K/V heads, 400 rows on 1500..3000 493 -> 465 (131 x 8 over 4, 200..500 rows on 2000 1 to 2 % behind); below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 147 -> 150, of one
-// tile 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.  HSTU_MI355_SHORT=0 switches it off.
+// keys (629 MB) 456 -> 326 us, 200 x 4, 200 rows 518 -> 378, 400 x 2, 400 rows on 800..1000 (369 MB) 270 -> 194, 24 x 8, 400 rows on 3072
+// (302 MB) 171 -> 156, 64 x 8, 512 rows on 4000 797 -> 580; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 142 -> 142, of one tile
+// 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.  Lists that the queues take pair
+// after pair have the better order there already, and sorted: 131 x 8, 200..500 rows on 2000 461 -> 484, 100 x 8, 400 rows on 1500..3000 472 ->
+// 492, 200 x 8 over 4 850 -> 890, 165 x 4, d 96, 185..698 rows on 3624 523 -> 577 (120 of those, which they take level after level, 481 ->
+// 438; 100 x 8, 512 rows on 2500 529 -> 542 and 90 of those 694 -> 491).  Of long sweeps a few workgroups in a second round cost a whole one:
+// 22 x 4, 1100 rows on 7000 keys (792 slots) 374 -> 401, 24 (864) 413 -> 411, 31 (1116) 583 -> 515; up to 4096 keys 25 x 8, 400 rows
+// on 3072 (800) 187 -> 185, 49 x 8, 200 rows (784) 242 -> 200.  HSTU_MI355_SHORT=0 switches it off.
 const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool* pair_major)
 {
     if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || var->d_pad < 128 || var->d_pad > 256 || var->persistent_wgs_per_cu <= 0 ||
@@ -488,7 +510,11 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
     if (var->d_pad == 128) {
         *pair_major = true;
         const bool shared_history = p->total_k >= 2 * p->total_q && p->max_seq_len_q > hstu::kBlockM;
-        return shared_history && kv_bytes >= (288LL << 20) && slots >= 3LL * cus && switches().short_lists != 1 ? &pv[0] : nullptr;
+        if (!shared_history || kv_bytes < (288LL << 20) || slots < 3LL * cus || switches().short_lists == 1 ||
+            (p->max_seq_len_k > 4096 && 8 * slots < 27LL * cus)) {
+            return nullptr;
+        }
+        return short_variant(var, p) == nullptr && queues_pair_after_pair(var, p) ? nullptr : &pv[0];
     }
     const bool history = p->total_k >= 2 * p->total_q;
     if (history && (p->total_q + 64 * batch) / hstu::kBlockM * p->num_heads_q <= cus) {

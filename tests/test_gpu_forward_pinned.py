@@ -169,3 +169,27 @@ def test_batches_the_rule_leaves_to_the_lists():
         w.max_seq_len_k = 600
         w.k = w.v = torch.zeros(600 * batch, 4, 256, dtype=BF, device=DEV)
         assert prepared(w).kernel_name().endswith("_pinned") == taken
+
+
+@pytest.mark.parametrize(
+    "batch,heads,heads_k,rows,keys,kernel",
+    [
+        (200, 2, 2, (400, 400), 3072, "_pinned"),
+        (100, 8, 8, (400, 400), 2256, "_queues"),  # six items per resident workgroup: the queues take them pair after pair
+        (100, 8, 4, (400, 400), 3072, "_queues"),
+        (120, 4, 4, (185, 698), 3000, "_pinned"),  # uneven rows: pair after pair from four items on
+        (165, 4, 4, (185, 698), 3000, "_queues"),
+        (400, 2, 2, (400, 400), 1000, "_pinned"),  # as many items, but the kernel for short lists would take them
+        (22, 4, 4, (1100, 1100), 7000, "_split"),  # a few workgroups in a second round of long sweeps
+        (31, 4, 4, (1100, 1100), 7000, "_pinned"),
+    ],
+)
+def test_histories_at_the_slot_128_that_the_lists_order_better(batch, heads, heads_k, rows, keys, kernel):
+    lo, hi = rows
+    lengths = [lo + (hi - lo) * (2 * i + 1) // (2 * batch) for i in range(batch)]
+    q = torch.empty(sum(lengths), heads, 128, dtype=BF, device=DEV)
+    kv = torch.empty(keys * batch, heads_k, 128, dtype=BF, device=DEV)
+    offsets = torch.tensor([0] + lengths, device=DEV).cumsum(0).to(torch.int32)
+    offsets_k = torch.arange(0, keys * batch + 1, keys, device=DEV, dtype=torch.int32)
+    name = _ops.prepare_forward(q, kv, kv, None, None, 0, hi, keys, 1.0, offsets, offsets_k, None, None, 0, 1.0).kernel_name()
+    assert name.endswith(kernel), name
