@@ -1029,9 +1029,19 @@ static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, 
 // the machine has emptied: there the planes order, whose long launch has a workgroup per query tile and head, is the shorter one.
 // Grouped heads, K/V tiles of 128 keys (us, planes / dS handed over): 16 x 8 heads on 2, 256..1024 rows, d 128, 160 tiles 131 / 158, d 64
 // 111 / 124; 16 x 8 on 1, 1024 rows, 128 tiles 276 / 301; 4 x 8 on 2, 2048..4096 rows, 192 tiles 631 / 575; 32 x 8 on 2, 256..1024 rows, 320
-// tiles 234 / 185; 8 x 8 on 4, 1024 rows, 256 tiles 102 / 100 -- the line is at three quarters of the compute units.  One query head per
-// K/V head: only short rows at the slot 128, where the planes order has its 64-row query tiles: 2 x 1, 300 rows 22.5 / 25.4; 8 x 2, 200..300
-// rows, 40 tiles 22.6 / 24.9; 4 x 4, 300..700 rows, 70 tiles 39.6 / 38.5; 1 x 4, 1000 rows, 32 tiles 55.6 / 52.9.
+// tiles 234 / 185; 8 x 8 on 4, 1024 rows, 256 tiles 102 / 100 -- the line is at three quarters of the compute units.
+// Up to the slot 128 the other orders' query-tile launch of at most two workgroups per compute unit, all resident, holds on for longer
+// where the rows' last tiles are partly empty (those cost the key-tile kernel whole steps): 24 x 8 on 4, 200 rows (384 slots) 31.9 / 33.9, 32 x 8
+// (512) 34.0 / 36.2, 35 x 8 (560) 46.9 / 38.4; 30 x 8 on 4, 150 rows (480) 28.0 / 29.4, 34 x 8 (544) 39.7 / 31.4; d 64, 64 x 4 on 2, 200 rows (512) 27.4 / 29.2, 73 x
+// 4 (584) 33.8 / 30.7; whole tiles 23 x 8 on 4, 256 rows (368) 37.3 / 36.0; on a history 64 x 4 on 2, 200 rows on 400 keys (512) 58.4 / 51.3; one tile 48 x 8 on 4, 100 rows (384) 29.9 / 27.4 -- or, at the slot 128, where
+// rows of one tile meet keys of two, up to one per compute unit: 64 x 4 on 2, 100 rows on 160 keys (256) 23.2 / 27.9, 70 on 160 22.3 / 24.9, 80 x 4 (320)
+// 33.7 / 30.0; 100 on 400 (256) 41.2 / 40.1.
+// One query head per K/V head: only short rows at the slot 128, where the planes order has its 64-row query tiles -- up to one slot per
+// compute unit and fifteen sixteenths of it in key tiles: 16 x 4 of 100 rows 15.5 / 17.6, 15 x 4 of 116..168 17.6 / 20.8, 32 x 4 of 140 (204 tiles)
+// 18.3 / 20.0, 21 x 4 of 300 (236) 27.4 / 28.1, 8 x 4 of 400 28.1 / 29.4; 24 x 4 of 256 (240) 25.0 / 24.4, 32 x 4 of 256 (320) 27.0 / 26.1, 48 x 4 of 140 (384
+// slots) 25.0 / 22.6, 40 x 4 of 10..200 (320 slots) 25.3 / 22.5, 8 x 4 of 512 (144 tiles) 33.7 / 33.0, 5 x 4 of 700 42.8 / 41.2; on keys of twice the rows and more
+// the key tiles are many and their sweeps short: 16 x 4, 200 rows on 400 keys 29.0 / 25.1, 100 on 400 26.0 / 21.6.  And any such rows in at most 64 tiles:
+// 2 x 1, 300 rows 22.5 / 25.4; 8 x 2, 200..300 rows, 40 tiles 22.6 / 24.9; 4 x 4, 300..700 rows, 70 tiles 39.6 / 38.5; 1 x 4, 1000 rows, 32 tiles 55.6 / 52.9.
 static bool few_key_tiles(const hstu_jagged_fwd_params* f)
 {
     int cus = 0;
@@ -1044,10 +1054,20 @@ static bool few_key_tiles(const hstu_jagged_fwd_params* f)
     if (f->attn_bias != nullptr) {
         return few_biased_key_tiles(f, dmax, tiles, cus);
     }
+    const bool slot_128 = dmax > 64 && dmax <= 128, history = f->total_k >= 2 * f->total_q;
+    const int64_t q_slots = (f->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * batch * f->num_heads_q;
     if (f->num_heads_q > f->num_heads_k) {
-        return 4 * tiles < 3LL * cus;
+        const bool one_tile = f->total_q <= hstu::kBlockM * batch;
+        const bool part_empty = 8 * hstu::kBlockM * q_slots >= 9 * f->total_q * f->num_heads_q;
+        return 4 * tiles < 3LL * cus ||
+               (dmax <= 128 && !one_tile && part_empty && f->total_q <= 448 * batch && q_slots <= 2LL * cus && !history) ||
+               (slot_128 && one_tile && f->total_k > hstu::kBlockM * batch && 2 * f->total_k < 5 * f->total_q && q_slots <= cus);
     }
-    return dmax > 64 && dmax <= 128 && tiles <= 64 && f->total_q <= 512 * batch;
+    if (!slot_128) {
+        return false;
+    }
+    return (tiles <= 64 && f->total_q <= 512 * batch) ||
+           (16 * tiles < 15LL * cus && q_slots <= cus && f->total_q <= 448 * batch && !history);
 }
 
 // estimated microseconds of the three launch orders (see above)

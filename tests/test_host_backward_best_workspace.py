@@ -110,6 +110,41 @@ def test_calls_with_a_bias(heads, heads_k, dim, batch, rows, max_rows, keys, tak
     assert best == (whole if taken else size) and whole != size
 
 
+UNBIASED = [  # heads, K/V heads, head dim, batch, rows, bound of rows, keys; whether the call takes the dS tiles
+    (4, 4, 128, 16, 100, 100, 100, False),  # a head each at the slot 128: short rows in few tiles
+    (4, 4, 96, 15, 142, 168, 142, False),
+    (4, 4, 128, 32, 256, 256, 256, True),
+    (4, 4, 128, 48, 140, 140, 140, True),  # more than a slot per compute unit
+    (4, 4, 128, 40, 105, 200, 105, True),
+    (4, 4, 128, 8, 512, 512, 512, True),
+    (4, 4, 128, 16, 200, 200, 400, True),
+    (4, 4, 64, 16, 100, 100, 100, True),
+    (4, 4, 256, 16, 140, 140, 140, True),
+    (8, 4, 128, 32, 200, 200, 200, False),  # grouped heads: last tiles partly empty, up to two slots per compute unit
+    (8, 4, 128, 35, 200, 200, 200, True),
+    (8, 4, 128, 24, 256, 256, 256, True),
+    (8, 4, 128, 48, 100, 100, 100, True),
+    (4, 2, 64, 64, 200, 200, 200, False),
+    (4, 2, 128, 64, 200, 200, 400, True),
+    (4, 2, 256, 64, 200, 200, 200, True),
+    (4, 2, 128, 64, 100, 100, 160, False),  # rows of one tile on keys of two
+    (4, 2, 128, 80, 100, 100, 160, True),
+    (4, 2, 128, 64, 100, 100, 400, True),
+    (4, 2, 64, 64, 100, 100, 160, True),
+]
+
+
+@pytest.mark.parametrize("heads,heads_k,dim,batch,rows,max_rows,keys,taken", UNBIASED)
+def test_calls_without_a_bias(heads, heads_k, dim, batch, rows, max_rows, keys, taken):
+    """Where the orders without dS tiles were measured to be the faster ones (256 compute units), the call asks for their workspace."""
+    own = keys != rows
+    call = dict(n_offsets=batch + 1, num_heads_q=heads, num_heads_k=heads_k, head_dim_qk=dim, head_dim_v=dim, total_q=batch * rows,
+                total_k=batch * keys, max_seq_len_q=max_rows, max_seq_len_k=(keys if own else max_rows), seq_offset_k=FAKE + (64 if own else 0))  # fmt: skip
+    size, best = sizes(**call)
+    whole = tiles(rows=batch * rows, batch=batch, heads=heads, blocks=(call["max_seq_len_k"] + 31) // 32, below_diagonal=not own)
+    assert best == (whole if taken else size) and whole != size
+
+
 def pair_lines(groups):
     """Lines of the pair plane that ``groups`` 32-row groups take up to the diagonal (row group g: g + 1 lines a row)."""
     return 16 * groups * (groups + 1)
