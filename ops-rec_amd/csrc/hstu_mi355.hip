@@ -1007,17 +1007,30 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
 //     on 2, 256 on 1024 (272 tiles) 148 / 130, 4 x 8 on 2, 300 on 700 (48 tiles) 83 / 114; slot 64, 4 x 8 on 2, 300 on 700 81 / 72, 2 x 8 on 1, 100..200 on
 //     500 (8 tiles) 58 / 67; slot 256 120 / 118 and 94 / 105
 //   slot 256, as 64: 4 x 8 on 2, 1024..2048, 100 tiles 451 / 517; 16 x 8 on 2, 256..1024, 176 tiles 320 / 300; 32 x 8 on 1, 512..1024 833 / 637
-static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, int64_t tiles, int64_t cus)
+//   two heads at the slots 64 and 256, whose query-tile launch holds on up to one slot per compute unit: slot 64, 8 x 4 on 2, 112 rows 21.9 / 24.8,
+//     64 x 4 of 112 (256 slots) 25.7 / 27.7, 128 x 4 (512) 34.3 / 32.3, 32 x 4 of 200 (256) 33.9 / 35.5, 4 x 4 of 256 35.0 / 33.1; slot 256, 26 x 4 on 2, 200 rows (208
+//     slots) 50.3 / 54.8, 40 x 4 (320) 66.4 / 58.1, 13 x 4 of 464 88.1 / 90.5, 12 x 4 of 600 109 / 109, 6 x 4 of 1000 175 / 165
+//   slot 128, rows of one tile on a history: 64 x 4, 100 rows on 376 keys (256 slots) 59 / 63, 128 x 4 105 / 125, 32 x 4 44 / 39; 128 x 4, 64 rows on 1000 235 / 253,
+//     256 x 4 of 128 on 400 297 / 306; in pairs 32 x 4 on 2, 100 rows on 200 keys 33 / 38, on 376 45 / 43, 128 x 4 on 2 of the same 63 / 72 and 94 / 100, on 1000 290 / 272
+static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, int64_t tiles, int64_t cus, int64_t q_slots)
 {
     const int64_t batch = f->n_offsets - 1, ratio = f->num_heads_q / f->num_heads_k;
     if (f->total_k >= 2 * f->total_q) {
-        return dmax > 64 && dmax <= 128 ? ratio > 1 && 2 * tiles < cus : ratio >= 8 && 8 * tiles <= cus;
+        if (dmax <= 64 || dmax > 128) {
+            return ratio >= 8 && 8 * tiles <= cus;
+        }
+        const bool one_tile = f->total_q <= hstu::kBlockM * batch;
+        if (ratio == 1) {
+            return one_tile && q_slots >= cus;
+        }
+        return 2 * tiles < cus || (one_tile && (2 * f->total_k < 5 * f->total_q || (f->total_k < 4 * f->total_q && q_slots >= 2 * cus)));
     }
     if (dmax <= 64) {
-        return ratio >= 4 && ((f->total_q <= 400 * batch && 4 * tiles < 3 * cus) || (ratio >= 8 && 8 * tiles <= cus));
+        return (ratio >= 4 && ((f->total_q <= 400 * batch && 4 * tiles < 3 * cus) || (ratio >= 8 && 8 * tiles <= cus))) ||
+               (ratio >= 2 && f->total_q <= 224 * batch && q_slots <= cus);
     }
     if (dmax > 128) {
-        return ratio >= 4 && 8 * tiles < 5 * cus;
+        return (ratio >= 4 && 8 * tiles < 5 * cus) || (ratio >= 2 && f->total_q <= 512 * batch && q_slots <= cus);
     }
     if (f->total_q <= hstu::kBlockM * batch && tiles < 6 * cus) {
         return true;
@@ -1051,11 +1064,11 @@ static bool few_key_tiles(const hstu_jagged_fwd_params* f)
     const int64_t batch = f->n_offsets - 1;
     const int64_t dmax = f->head_dim_qk > f->head_dim_v ? f->head_dim_qk : f->head_dim_v;
     const int64_t tiles = (f->total_k + 64 * batch) / 128 * f->num_heads_k;
+    const int64_t q_slots = (f->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * batch * f->num_heads_q;
     if (f->attn_bias != nullptr) {
-        return few_biased_key_tiles(f, dmax, tiles, cus);
+        return few_biased_key_tiles(f, dmax, tiles, cus, q_slots);
     }
     const bool slot_128 = dmax > 64 && dmax <= 128, history = f->total_k >= 2 * f->total_q;
-    const int64_t q_slots = (f->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * batch * f->num_heads_q;
     if (f->num_heads_q > f->num_heads_k) {
         const bool one_tile = f->total_q <= hstu::kBlockM * batch;
         const bool part_empty = 8 * hstu::kBlockM * q_slots >= 9 * f->total_q * f->num_heads_q;

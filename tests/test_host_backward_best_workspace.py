@@ -96,6 +96,17 @@ BIASED = [  # heads, K/V heads, head dim, batch, rows, bound of rows, keys; whet
     (8, 2, 256, 4, 1536, 2048, 1536, False),
     (8, 2, 256, 16, 640, 1024, 640, True),
     (4, 2, 256, 8, 768, 1024, 768, True),
+    (4, 2, 64, 8, 112, 112, 112, False),  # in pairs: short rows in at most a slot per compute unit
+    (4, 2, 64, 128, 112, 112, 112, True),
+    (4, 2, 64, 4, 256, 256, 256, True),
+    (4, 2, 256, 26, 200, 200, 200, False),
+    (4, 2, 256, 40, 200, 200, 200, True),
+    (4, 2, 256, 6, 1000, 1000, 1000, True),
+    (4, 4, 128, 64, 100, 100, 376, False),  # rows of one tile on a history: a slot per compute unit and more
+    (4, 4, 128, 48, 100, 100, 376, True),
+    (4, 2, 128, 32, 100, 100, 200, False),
+    (4, 2, 128, 32, 100, 100, 376, True),
+    (4, 2, 128, 128, 100, 100, 376, False),
 ]
 
 
