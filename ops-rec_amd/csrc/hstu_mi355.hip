@@ -984,11 +984,12 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
 // `groups`: the 32-row groups of all planes.  A wavefront takes about 2.5 us for a group however few its bytes are (the sequence's offsets,
 // one load after another), so small planes have a workgroup for every 8 of them, two per wavefront: 64 x 2 heads, d 64, 64..128 rows 59 us
 // with a workgroup per MiB, 23 with one for every 16 groups as well, 19.4 with one for 8; 32 x 4 of 40..200 78, 23.9, 23.0; 409 x 1 of 158..204
-// 90, 53, 53; d 128, 16 x 4, 200 rows on 1000 keys 65, 65, 60.
+// 90, 53, 53; d 128, 16 x 4, 200 rows on 1000 keys 65, 65, 60.  (To the next multiple of 8, which keeps two groups per wavefront: 7 x 4 heads, d 64,
+// 101 rows, 112 groups, the call 21.4 us with 8 workgroups, 17.6 with 16.)
 static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus)
 {
     const int64_t most = dmax <= 64 ? cus / 2 : (dmax <= 128 ? 3 * cus / 8 : cus / 4);
-    return static_cast<int>(std::max<int64_t>(8, std::min<int64_t>(most, std::max(bytes >> 20, groups / 8)) / 8 * 8));
+    return static_cast<int>(std::min<int64_t>(most / 8, std::max<int64_t>(1, (std::max(bytes >> 20, groups / 8) + 7) / 8)) * 8);
 }
 
 // The same for calls with attn_bias.  The key-tile kernel's step is longest there, most of all at the slot 128, where it spills, and a
