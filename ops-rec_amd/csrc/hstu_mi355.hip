@@ -446,20 +446,26 @@ bool takes_queue_variant(const Variant* var, const hstu_jagged_fwd_params* p, in
     return var->kernel_queues != nullptr && n_blocks >= 4 * resident;
 }
 
-// Whether the queues then take the items pair after pair, as hstu_fwd_kernel decides from the lengths (six items per resident workgroup, or
-// four where the sequences have at most seven tenths of the longest one's tiles on average), by an estimate of the tiles: all of them where the mean
-// length is within half a tile of the longest, else the mean length's and a half per sequence.
+// The query tiles of all sequences, estimated without reading the lengths: the most there can be where the mean length is within half a tile
+// of the longest, else the mean length's and half a tile per sequence.
+int64_t estimated_tiles(const hstu_jagged_fwd_params* p)
+{
+    const int64_t batch = p->n_offsets - 1;
+    const int64_t most = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * batch;
+    const bool alike = batch * p->max_seq_len_q - p->total_q < hstu::kBlockM / 2 * batch;
+    return alike ? most : std::min(most, p->total_q / hstu::kBlockM + batch / 2);
+}
+
+// Whether the queues then take the items pair after pair, as hstu_fwd_kernel decides from the lengths: six items per resident workgroup, or
+// four where the sequences have at most seven tenths of the longest one's tiles on average.
 bool queues_pair_after_pair(const Variant* var, const hstu_jagged_fwd_params* p)
 {
     int64_t resident = 0;
     if (!takes_queue_variant(var, p, &resident)) {
         return false;
     }
-    const int64_t batch = p->n_offsets - 1;
-    const int64_t most = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * batch;
-    const bool alike = batch * p->max_seq_len_q - p->total_q < hstu::kBlockM / 2 * batch;
-    const int64_t tiles = alike ? most : std::min(most, p->total_q / hstu::kBlockM + batch / 2);
-    const int64_t items = tiles * p->num_heads_q;
+    const int64_t tiles = estimated_tiles(p), items = tiles * p->num_heads_q;
+    const int64_t most = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM * (p->n_offsets - 1);
     return (items >= 4 * resident && 10 * tiles <= 7 * most) || items >= 6 * resident;
 }
 
@@ -477,12 +483,20 @@ bool queues_pair_after_pair(const Variant* var, const hstu_jagged_fwd_params* p)
 // every sequence a slot more): two workgroups would share one while others idle.  39 x 4, 82..165 rows on 660 keys (229 tiles) 34 -> 41 us,
 // 26 x 4, 100..300 on 600 (214) 33 -> 38, 18 x 4, 250..400 on 800 (218) 40 -> 44; 12 x 4, 700..1400 on 2100 (417) 117 -> 104; without a
 // history 37 x 4, 82..165 rows (217) 17.4 -> 17.2.
-// At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of two
-// tiles and more on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
+// Long sweeps on a history come in few rounds: pairs are dealt to the XCDs, two workgroups per CU run at once, and a last round with few
+// of them takes 0.56 of a full one, where the list deals its tiles one per CU at 0.53 of it.  Up to four tiles per CU the estimates are
+// compared: 10 x 2 heads, 2000..3000 rows on 6000..8000 keys 366 us from the list, 517 here (72 slots per XCD, 64 of which run at once), 12 x 2 391, 518, 13 x 2
+// 551, 502, 17 x 2 616, 652, 20 x 2 732, 677, 22 x 2 782, 830, 28 x 2 1015, 868; 17 x 4 on 2, 700..1000 rows on 4000..5000 295, 345, 20 x 4 on 2 410, 355; 9 x 4,
+// 3500 rows on 8000 882, 896, 10 x 4 1027, 905; fewer than three pairs per XCD 3 x 4 of those 350, 393, 5 x 4 574, 617.
+// At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of more
+// than a tile on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
 // keys (629 MB) 456 -> 326 us, 200 x 4, 200 rows 518 -> 378, 400 x 2, 400 rows on 800..1000 (369 MB) 270 -> 194, 24 x 8, 400 rows on 3072
-// (302 MB) 171 -> 156, 64 x 8, 512 rows on 4000 797 -> 580; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 142 -> 142, of one tile
-// 400 x 2, 128 rows on 3000..6000 414 -> 423, and without history 64 x 4 of 1024..4096 rows 570 -> 604.  Lists that the queues take pair
-// after pair have the better order there already, and sorted: 131 x 8, 200..500 rows on 2000 461 -> 484, 100 x 8, 400 rows on 1500..3000 472 ->
+// (302 MB) 171 -> 156, 64 x 8, 512 rows on 4000 797 -> 580; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 142 -> 142, of uneven
+// lengths (a mean below five sevenths of the longest), which the lists sort, 134 x 2, d 96, 218..592 rows on 3112 (320 MB) 219 -> 236, 135 x 2,
+// 278..678 on 2584 (357) 214 -> 221, 80 x 4, d 96, 185..698 on 3300 (405) 290 -> 293, 180 x 2, 278..678 on 2584 (476) 344 -> 284; of one tile
+// 400 x 2, 128 rows on 3000..6000 414 -> 423, with half of the second tiles missing 111 x 8, 80..140 rows on 700 keys 79 -> 92, 68 x 8 on
+// 1800 120 -> 144, 111 x 8, 100..160 on 700 87 -> 92 (120..200 108 -> 94: the line is at a mean of nine eighths of a tile), and without
+// history 64 x 4 of 1024..4096 rows 570 -> 604.  Lists that the queues take pair after pair have the better order there already, and sorted: 131 x 8, 200..500 rows on 2000 461 -> 484, 100 x 8, 400 rows on 1500..3000 472 ->
 // 492, 200 x 8 over 4 850 -> 890, 165 x 4, d 96, 185..698 rows on 3624 523 -> 577 (120 of those, which they take level after level, 481 ->
 // 438; 100 x 8, 512 rows on 2500 529 -> 542 and 90 of those 694 -> 491).  Of long sweeps a few workgroups in a second round cost a whole one:
 // 22 x 4, 1100 rows on 7000 keys (792 slots) 374 -> 401, 24 (864) 413 -> 411, 31 (1116) 583 -> 515; up to 4096 keys 25 x 8, 400 rows
@@ -509,8 +523,9 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
     const hstu::ShortVariant* const pv = hstu::fwd_variants_pinned()[p->dtype == HSTU_DT_BF16 ? 0 : 1];
     if (var->d_pad == 128) {
         *pair_major = true;
-        const bool shared_history = p->total_k >= 2 * p->total_q && p->max_seq_len_q > hstu::kBlockM;
-        if (!shared_history || kv_bytes < (288LL << 20) || slots < 3LL * cus || switches().short_lists == 1 ||
+        const bool shared_history = p->total_k >= 2 * p->total_q && 8 * p->total_q >= 9 * hstu::kBlockM * batch;
+        const bool uneven = 7 * p->total_q < 5 * batch * p->max_seq_len_q;
+        if (!shared_history || kv_bytes < ((uneven ? 448LL : 288LL) << 20) || slots < 3LL * cus || switches().short_lists == 1 ||
             (p->max_seq_len_k > 4096 && 8 * slots < 27LL * cus)) {
             return nullptr;
         }
@@ -521,6 +536,14 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
         return nullptr;
     }
     *pair_major = kv_bytes >= (224LL << 20) || history;
+    if (history && p->max_seq_len_k > 2048) {
+        const int64_t pairs = batch * p->num_heads_k, items = estimated_tiles(p) * p->num_heads_q;
+        const int64_t per_xcd = (pairs + 7) / 8 * (slots / ((pairs + 7) / 8 * 8)), room = cus / 4, left = per_xcd % room;
+        const int64_t here = 100 * (per_xcd / room) + (left > 0 ? std::max<int64_t>(56, 100 * left / room) : 0);
+        if (pairs < 24 || (items <= 4LL * cus && 53 * ((items + cus - 1) / cus) < std::max<int64_t>(here, 100))) {
+            return nullptr;
+        }
+    }
     if (!*pair_major && p->max_seq_len_k > 2048 && (batch * p->num_heads_k < 24 || 4 * p->total_q < 3 * batch * p->max_seq_len_q)) {
         return nullptr;
     }
