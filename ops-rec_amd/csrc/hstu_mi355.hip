@@ -1023,6 +1023,8 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
 //   slot 128, grouped: 32 x 8 on 2, 512 rows, 288 tiles 196 / 226; 16 x 8 on 2, 256..1024 (176 tiles) 230 / 304; 32 x 8 on 1, 1024 (272) 690 / 793;
 //     8 x 8 on 4, 1024..2048 (400, three quarters) 507 / 450; 32 x 8 on 4, 256..1024 (704) 328 / 296; 64 x 8 on 2, 256..1024 (704) 775 / 634
 //   slot 128, rows of one tile: 512 x 2, 100..128 rows 87 / 99; 256 x 8 on 4, 64..128 139 / 150; 512 x 4, 128 rows, 2048 tiles 209 / 197
+//   slot 128, short uneven rows, a head each: 234 x 4, 58..214 rows, 1460 tiles 118 / 126; 128 x 4 69 / 74; 180 x 4, 20..250 91 / 97; 128 x 4, 100..300 103 / 106;
+//     400 x 4, 58..214, 2500 tiles 239 / 224; rows alike 180 x 4, 140 rows 96 / 91; 100 x 4 of 160 60 / 55
 //   slot 128, a head each: 16 x 4, 300..500 rows, 230 tiles 54 / 58; 128 x 2, 256 rows, 640 tiles 59 / 62; 128 x 4, 200..300, 1256 tiles 150 / 138;
 //     8 x 4, 512..1024 108 / 102; 32 x 4, 256..1024 160 / 143
 //   slot 64, four query heads per K/V head and more: 16 x 8 on 2, 200..400 rows, 92 tiles 72 / 78; 32 x 8 on 1, 200..400 127 / 149; 64 x 8 on 2, 128..256,
@@ -1034,6 +1036,8 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
 //   two heads at the slots 64 and 256, whose query-tile launch holds on up to one slot per compute unit: slot 64, 8 x 4 on 2, 112 rows 21.9 / 24.8,
 //     64 x 4 of 112 (256 slots) 25.7 / 27.7, 128 x 4 (512) 34.3 / 32.3, 32 x 4 of 200 (256) 33.9 / 35.5, 4 x 4 of 256 35.0 / 33.1; slot 256, 26 x 4 on 2, 200 rows (208
 //     slots) 50.3 / 54.8, 40 x 4 (320) 66.4 / 58.1, 13 x 4 of 464 88.1 / 90.5, 12 x 4 of 600 109 / 109, 6 x 4 of 1000 175 / 165
+//   slot 256, a head each, one short tile: the key tiles and the clearing workgroups are more than the machine holds at once, one per CU: 52 x 4, 64
+//     rows (208 slots) 24.5 / 29.2, 64 x 4 25.9 / 30.3, 48 x 4 (192) 24.4 / 22.3; 40 x 4 of 128 rows 36.7 / 32.3
 //   slot 128, rows of one tile on a history: 64 x 4, 100 rows on 376 keys (256 slots) 59 / 63, 128 x 4 105 / 125, 32 x 4 44 / 39; 128 x 4, 64 rows on 1000 235 / 253,
 //     256 x 4 of 128 on 400 297 / 306; in pairs 32 x 4 on 2, 100 rows on 200 keys 33 / 38, on 376 45 / 43, 128 x 4 on 2 of the same 63 / 72 and 94 / 100, on 1000 290 / 272
 static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, int64_t tiles, int64_t cus, int64_t q_slots)
@@ -1054,9 +1058,13 @@ static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, 
                (ratio >= 2 && f->total_q <= 224 * batch && q_slots <= cus);
     }
     if (dmax > 128) {
+        if (ratio == 1) {
+            return f->total_q <= 80 * batch && 4 * q_slots > 3 * cus && q_slots <= cus;
+        }
         return (ratio >= 4 && 8 * tiles < 5 * cus) || (ratio >= 2 && f->total_q <= 512 * batch && q_slots <= cus);
     }
-    if (f->total_q <= hstu::kBlockM * batch && tiles < 6 * cus) {
+    const bool short_uneven = ratio == 1 && f->total_q <= 200 * batch && 5 * f->total_q <= 4 * batch * f->max_seq_len_q;
+    if ((f->total_q <= hstu::kBlockM * batch || short_uneven) && tiles < 6 * cus) {
         return true;
     }
     return ratio == 1 ? f->total_q < 600 * batch && 2 * tiles <= 5 * cus : 8 * tiles * f->total_q <= 9 * cus * batch * f->max_seq_len_q;

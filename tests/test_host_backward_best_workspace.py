@@ -107,6 +107,12 @@ BIASED = [  # heads, K/V heads, head dim, batch, rows, bound of rows, keys; whet
     (4, 2, 128, 32, 100, 100, 200, False),
     (4, 2, 128, 32, 100, 100, 376, True),
     (4, 2, 128, 128, 100, 100, 376, False),
+    (4, 4, 128, 234, 136, 216, 136, False),  # short uneven rows
+    (4, 4, 128, 400, 136, 216, 136, True),
+    (4, 4, 128, 180, 140, 144, 140, True),
+    (4, 4, 256, 56, 64, 64, 64, False),  # short single tiles of nearly all compute units, beside the clearing workgroups
+    (4, 4, 256, 48, 64, 64, 64, True),
+    (4, 4, 256, 40, 128, 128, 128, True),
 ]
 
 
