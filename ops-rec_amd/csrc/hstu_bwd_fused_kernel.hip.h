@@ -19,9 +19,11 @@
 // 2.0 + 0.9 ms of the kernels that recompute.  Ordinary ones the vector unit and the longest workgroup: 32 x 4 heads, d 128, 256..1024
 // rows 62 + 21 us, where the query-tile kernel with dS and P took 61 and the kernels that read them 41.  A wavefront with 64 keys and
 // all 512 registers, one per SIMD, took as long as this one (1.39 ms at the large shape) and has half as many workgroups.
-// With attn_bias the key-tile kernel at the slot 128 spills: 16 x 4 heads, d 128, 512..2048 rows 248 us, 193 before a block cleared what its
-// rows do not see of the bias (39 scratch instructions against 16, in every order of that code tried; none at the slot 64); the call
-// 368 -> 344 us, where dV, dQ storing dS and dK from it took 185 + 139 + 61.
+// With attn_bias the key-tile kernel at the slot 128 spills: 16 x 4 heads, d 128, 512..2048 rows 245 us, 193 before a block cleared what its
+// rows do not see of the bias (39 scratch instructions against 16, in every order of that code tried; none at the slot 64).  Four of the
+// eight K fragments are read back from scratch between the products of S, and a wait for such a load, whose count is in order, is one for
+// everything asked for before it: the bias and the tiles that this step has just requested for the next two.  The call 385 -> 350 us, where
+// dV, dQ storing dS and dK from it took 185 + 139 + 61.
 // The query-tile kernel moves dS once: at the large shape 3.8 GB fetched, 2.6 of them dS, in 0.65 ms = 5.8 TB/s.
 #pragma once
 #include "hstu_bias_requests.h"

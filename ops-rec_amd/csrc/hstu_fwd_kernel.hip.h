@@ -2055,8 +2055,8 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         __syncthreads();
         if (x_end > x_begin) {
             // interior steps of this wavefront: [x_begin + 1, t_interior).  Sub-tile t + 1 (t + 2 with rab) must exist,
-            // and sub-tile t (t + 1 with rab, whose words a step does not clear) must be fully visible: it ends at or before the smallest row limit and, when target
-            // rows carve holes, before the first target key.  The wavefronts of a workgroup run different numbers
+            // and sub-tile t (t + 1 with rab, whose words a step does not clear) must be fully visible: it ends at or before the
+            // smallest row limit and, when target rows carve holes, before the first target key.  The wavefronts of a workgroup run different numbers
             // of interior steps; every step of either kind ends in the same one barrier, so the counts match.
             int t_interior = nx_w - (HAS_RAB ? 2 : 1);
             {

@@ -30,7 +30,8 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 3) void hstu_fwd_pinned_kernel(
     constexpr int LPW = SUB_BYTES / 4096;       // 1 KiB load instructions per sub-tile and wavefront
     constexpr int KSTEPS = D / 16, MTILES = D / 32, NCH = 2 * MTILES;
     constexpr int KS = 3, VS = D == 256 ? 2 : 3;               // ring slots
-    constexpr int kOpen = VS == 2 ? LPW : 2 * LPW;                  // what may be under way when a step starts: behind V(t - 1), VS - 1 steps ago, and K(t), two steps ago
+    // what may be under way when a step starts: behind V(t - 1), VS - 1 steps ago, and K(t), two steps ago
+    constexpr int kOpen = VS == 2 ? LPW : 2 * LPW;
     constexpr int kAccRegs = MTILES * 16;
     constexpr uint32_t kPastEnd = 0x40000000u;
     constexpr int kV0 = 0, kK0 = VS * SUB_BYTES;

@@ -5,7 +5,8 @@
 namespace hstu {
 namespace {
 #define HSTU_BWD_FUSED(tag, tagname, D) \
-    {"hstu_bwd_" tagname "_d" #D "_fused", hstu_bwd_kv_fused_kernel<tag, D>, hstu_bwd_kv_fused_kernel<tag, D, true>, hstu_bwd_dq_from_ds_kernel<tag, D, false>, hstu_bwd_dq_from_ds_kernel<tag, D, true>}
+    {"hstu_bwd_" tagname "_d" #D "_fused", hstu_bwd_kv_fused_kernel<tag, D>, hstu_bwd_kv_fused_kernel<tag, D, true>, \
+     hstu_bwd_dq_from_ds_kernel<tag, D, false>, hstu_bwd_dq_from_ds_kernel<tag, D, true>}
 const BwdFusedVariant kFused[2][3] = {
     {HSTU_BWD_FUSED(bf16_tag, "bf16", 64), HSTU_BWD_FUSED(bf16_tag, "bf16", 128), HSTU_BWD_FUSED(bf16_tag, "bf16", 256)},
     {HSTU_BWD_FUSED(f16_tag, "f16", 64), HSTU_BWD_FUSED(f16_tag, "f16", 128), HSTU_BWD_FUSED(f16_tag, "f16", 256)}};

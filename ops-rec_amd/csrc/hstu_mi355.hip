@@ -483,24 +483,24 @@ bool queues_pair_after_pair(const Variant* var, const hstu_jagged_fwd_params* p)
 // every sequence a slot more): two workgroups would share one while others idle.  39 x 4, 82..165 rows on 660 keys (229 tiles) 34 -> 41 us,
 // 26 x 4, 100..300 on 600 (214) 33 -> 38, 18 x 4, 250..400 on 800 (218) 40 -> 44; 12 x 4, 700..1400 on 2100 (417) 117 -> 104; without a
 // history 37 x 4, 82..165 rows (217) 17.4 -> 17.2.
-// Long sweeps on a history come in few rounds: pairs are dealt to the XCDs, two workgroups per CU run at once, and a last round with few
-// of them takes 0.56 of a full one, where the list deals its tiles one per CU at 0.53 of it.  Up to four tiles per CU the estimates are
-// compared: 10 x 2 heads, 2000..3000 rows on 6000..8000 keys 366 us from the list, 517 here (72 slots per XCD, 64 of which run at once), 12 x 2 391, 518, 13 x 2
-// 551, 502, 17 x 2 616, 652, 20 x 2 732, 677, 22 x 2 782, 830, 28 x 2 1015, 868; 17 x 4 on 2, 700..1000 rows on 4000..5000 295, 345, 20 x 4 on 2 410, 355; 9 x 4,
-// 3500 rows on 8000 882, 896, 10 x 4 1027, 905; fewer than three pairs per XCD 3 x 4 of those 350, 393, 5 x 4 574, 617.
-// At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of more
-// than a tile on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072
-// keys (629 MB) 456 -> 326 us, 200 x 4, 200 rows 518 -> 378, 400 x 2, 400 rows on 800..1000 (369 MB) 270 -> 194, 24 x 8, 400 rows on 3072
-// (302 MB) 171 -> 156, 64 x 8, 512 rows on 4000 797 -> 580; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 142 -> 142, of uneven
-// lengths (a mean below five sevenths of the longest), which the lists sort, 134 x 2, d 96, 218..592 rows on 3112 (320 MB) 219 -> 236, 135 x 2,
-// 278..678 on 2584 (357) 214 -> 221, 80 x 4, d 96, 185..698 on 3300 (405) 290 -> 293, 180 x 2, 278..678 on 2584 (476) 344 -> 284; of one tile
-// 400 x 2, 128 rows on 3000..6000 414 -> 423, with half of the second tiles missing 111 x 8, 80..140 rows on 700 keys 79 -> 92, 68 x 8 on
-// 1800 120 -> 144, 111 x 8, 100..160 on 700 87 -> 92 (120..200 108 -> 94: the line is at a mean of nine eighths of a tile), and without
-// history 64 x 4 of 1024..4096 rows 570 -> 604.  Lists that the queues take pair after pair have the better order there already, and sorted: 131 x 8, 200..500 rows on 2000 461 -> 484, 100 x 8, 400 rows on 1500..3000 472 ->
-// 492, 200 x 8 over 4 850 -> 890, 165 x 4, d 96, 185..698 rows on 3624 523 -> 577 (120 of those, which they take level after level, 481 ->
-// 438; 100 x 8, 512 rows on 2500 529 -> 542 and 90 of those 694 -> 491).  Of long sweeps a few workgroups in a second round cost a whole one:
-// 22 x 4, 1100 rows on 7000 keys (792 slots) 374 -> 401, 24 (864) 413 -> 411, 31 (1116) 583 -> 515; up to 4096 keys 25 x 8, 400 rows
-// on 3072 (800) 187 -> 185, 49 x 8, 200 rows (784) 242 -> 200.  HSTU_MI355_SHORT=0 switches it off.
+// Long sweeps on a history come in few rounds: pairs are dealt to the XCDs, two workgroups per CU run at once, and a last round with few of them
+// takes 0.56 of a full one, where the list deals its tiles one per CU at 0.53 of it.  Up to four tiles per CU the estimates are compared: 10 x 2
+// heads, 2000..3000 rows on 6000..8000 keys 366 us from the list, 517 here (72 slots per XCD, 64 of which run at once), 12 x 2 391, 518, 13 x 2 551,
+// 502, 17 x 2 616, 652, 20 x 2 732, 677, 22 x 2 782, 830, 28 x 2 1015, 868; 17 x 4 on 2, 700..1000 rows on 4000..5000 295, 345, 20 x 4 on 2 410, 355;
+// 9 x 4, 3500 rows on 8000 882, 896, 10 x 4 1027, 905; fewer than three pairs per XCD 3 x 4 of those 350, 393, 5 x 4 574, 617.
+// At the slot 128 the other kernels are level or better on most calls; it takes those where the order of the slots decides, rows of more than a tile
+// on a history of which the caches do not hold the K / V rows, three slots per CU and more: 200 x 2 heads, 400 rows on 3072 keys (629 MB) 456 -> 326
+// us, 200 x 4, 200 rows 518 -> 378, 400 x 2, 400 rows on 800..1000 (369 MB) 270 -> 194, 24 x 8, 400 rows on 3072 (302 MB) 171 -> 156, 64 x 8, 512
+// rows on 4000 797 -> 580; below that size 100 x 2, 400 rows on 1500..3000 (238 MB) 142 -> 142, of uneven lengths (a mean below five sevenths of the
+// longest), which the lists sort, 134 x 2, d 96, 218..592 rows on 3112 (320 MB) 219 -> 236, 135 x 2, 278..678 on 2584 (357) 214 -> 221, 80 x 4, d 96,
+// 185..698 on 3300 (405) 290 -> 293, 180 x 2, 278..678 on 2584 (476) 344 -> 284; of one tile 400 x 2, 128 rows on 3000..6000 414 -> 423, with half of
+// the second tiles missing 111 x 8, 80..140 rows on 700 keys 79 -> 92, 68 x 8 on 1800 120 -> 144, 111 x 8, 100..160 on 700 87 -> 92 (120..200 108 ->
+// 94: the line is at a mean of nine eighths of a tile), and without history 64 x 4 of 1024..4096 rows 570 -> 604.  Lists that the queues take pair
+// after pair have the better order there already, and sorted: 131 x 8, 200..500 rows on 2000 461 -> 484, 100 x 8, 400 rows on 1500..3000 472 -> 492,
+// 200 x 8 over 4 850 -> 890, 165 x 4, d 96, 185..698 rows on 3624 523 -> 577 (120 of those, which they take level after level, 481 -> 438; 100 x 8,
+// 512 rows on 2500 529 -> 542 and 90 of those 694 -> 491).  Of long sweeps a few workgroups in a second round cost a whole one: 22 x 4, 1100 rows on
+// 7000 keys (792 slots) 374 -> 401, 24 (864) 413 -> 411, 31 (1116) 583 -> 515; up to 4096 keys 25 x 8, 400 rows on 3072 (800) 187 -> 185, 49 x 8, 200
+// rows (784) 242 -> 200.  HSTU_MI355_SHORT=0 switches it off.
 const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool* pair_major)
 {
     if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || var->d_pad < 128 || var->d_pad > 256 || var->persistent_wgs_per_cu <= 0 ||
@@ -991,8 +991,8 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
     // (attn_bias: rows that start at multiples of four bytes, which 16-byte loads and stores need)
     const bool bias_ok = f->attn_bias == nullptr || (reinterpret_cast<uintptr_t>(f->attn_bias) % 4 == 0 && f->max_seq_len_k % 2 == 0 &&
                                                      reinterpret_cast<uintptr_t>(p->grad_attn_bias) % 4 == 0);
-    if ((f->dtype != HSTU_DT_BF16 && f->dtype != HSTU_DT_FP16) || !bias_ok || f->mask_type == HSTU_MASK_CUSTOM || dmax > 256 || f->head_dim_qk % 8 != 0 || f->head_dim_v % 8 != 0 || is_generic_bwd(var) ||
-        var->dq_ds_p == nullptr) {
+    if ((f->dtype != HSTU_DT_BF16 && f->dtype != HSTU_DT_FP16) || !bias_ok || f->mask_type == HSTU_MASK_CUSTOM || dmax > 256 ||
+        f->head_dim_qk % 8 != 0 || f->head_dim_v % 8 != 0 || is_generic_bwd(var) || var->dq_ds_p == nullptr) {
         return nullptr;
     }
     return &hstu::bwd_variants_fused()[f->dtype == HSTU_DT_BF16 ? 0 : 1][dmax <= 64 ? 0 : (dmax <= 128 ? 1 : 2)];
@@ -1004,42 +1004,44 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
 // heads, d 128, 512..2048 rows 287 / 290 / 296; 32 x 4 of 256..1024 154 / 153 / 149; d 64 130 / - / 113; 64 x 4, d 64, 64..512 rows 82 / - /
 // 68.  (Dealt over all workgroups ahead of their sweeps, as the other orders have it, the zeros hold up every one of them: the dV launch
 // alone takes 185 us at the first shape.)
-// `groups`: the 32-row groups of all planes.  A wavefront takes about 2.5 us for a group however few its bytes are (the sequence's offsets,
-// one load after another), so small planes have a workgroup for every 8 of them, two per wavefront: 64 x 2 heads, d 64, 64..128 rows 59 us
-// with a workgroup per MiB, 23 with one for every 16 groups as well, 19.4 with one for 8; 32 x 4 of 40..200 78, 23.9, 23.0; 409 x 1 of 158..204
-// 90, 53, 53; d 128, 16 x 4, 200 rows on 1000 keys 65, 65, 60.  (To the next multiple of 8, which keeps two groups per wavefront: 7 x 4 heads, d 64,
-// 101 rows, 112 groups, the call 21.4 us with 8 workgroups, 17.6 with 16.)
+// `groups`: the 32-row groups of all planes.  A wavefront takes about 2.5 us for a group however few its bytes are (the sequence's offsets, one load
+// after another), so small planes have a workgroup for every 8 of them, two per wavefront: 64 x 2 heads, d 64, 64..128 rows 59 us with a workgroup
+// per MiB, 23 with one for every 16 groups as well, 19.4 with one for 8; 32 x 4 of 40..200 78, 23.9, 23.0; 409 x 1 of 158..204 90, 53, 53; d 128, 16
+// x 4, 200 rows on 1000 keys 65, 65, 60.  (To the next multiple of 8, which keeps two groups per wavefront: 7 x 4 heads, d 64, 101 rows, 112 groups,
+// the call 21.4 us with 8 workgroups, 17.6 with 16.)
 static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus)
 {
     const int64_t most = dmax <= 64 ? cus / 2 : (dmax <= 128 ? 3 * cus / 8 : cus / 4);
     return static_cast<int>(std::min<int64_t>(most / 8, std::max<int64_t>(1, (std::max(bytes >> 20, groups / 8) + 7) / 8)) * 8);
 }
 
-// The same for calls with attn_bias.  The key-tile kernel's step is longest there, most of all at the slot 128, where it spills, and a
-// workgroup has as many steps as its K/V head has query heads times row blocks: the order pays from the tiles on that keep the machine
-// busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute units,
-// whatever the group's size.
-// Measured on 125 shapes (device time in us, other order / dS handed over):
+// Calls with attn_bias that keep the orders without dS tiles (see few_key_tiles).  The key-tile kernel's step is longest there, most of all at the
+// slot 128, where it spills, and a workgroup has as many steps as its K/V head has query heads times row blocks: the order pays from the tiles on
+// that keep the machine busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute
+// units, whatever the group's size.
+// Measured on 125 shapes, and 300 more for short rows, pairs of heads and histories (device time in us, other order / dS handed over):
 //   slot 128, grouped: 32 x 8 on 2, 512 rows, 288 tiles 196 / 226; 16 x 8 on 2, 256..1024 (176 tiles) 230 / 304; 32 x 8 on 1, 1024 (272) 690 / 793;
 //     8 x 8 on 4, 1024..2048 (400, three quarters) 507 / 450; 32 x 8 on 4, 256..1024 (704) 328 / 296; 64 x 8 on 2, 256..1024 (704) 775 / 634
 //   slot 128, rows of one tile: 512 x 2, 100..128 rows 87 / 99; 256 x 8 on 4, 64..128 139 / 150; 512 x 4, 128 rows, 2048 tiles 209 / 197
-//   slot 128, short uneven rows, a head each: 234 x 4, 58..214 rows, 1460 tiles 118 / 126; 128 x 4 69 / 74; 180 x 4, 20..250 91 / 97; 128 x 4, 100..300 103 / 106;
-//     400 x 4, 58..214, 2500 tiles 239 / 224; rows alike 180 x 4, 140 rows 96 / 91; 100 x 4 of 160 60 / 55
+//   slot 128, short uneven rows, a head each: 234 x 4, 58..214 rows, 1460 tiles 118 / 126; 128 x 4 69 / 74; 180 x 4, 20..250 91 / 97; 128 x 4,
+//     100..300 103 / 106; 400 x 4, 58..214, 2500 tiles 239 / 224; rows alike 180 x 4, 140 rows 96 / 91; 100 x 4 of 160 60 / 55
 //   slot 128, a head each: 16 x 4, 300..500 rows, 230 tiles 54 / 58; 128 x 2, 256 rows, 640 tiles 59 / 62; 128 x 4, 200..300, 1256 tiles 150 / 138;
 //     8 x 4, 512..1024 108 / 102; 32 x 4, 256..1024 160 / 143
-//   slot 64, four query heads per K/V head and more: 16 x 8 on 2, 200..400 rows, 92 tiles 72 / 78; 32 x 8 on 1, 200..400 127 / 149; 64 x 8 on 2, 128..256,
-//     256 tiles 75 / 69; 4 x 8 on 1, 512..1024, 26 tiles 266 / 295; 16 x 8 on 1, 256..1024 324 / 288; two heads: 8 x 4 on 2, 200..400 45 / 42
+//   slot 64, four query heads per K/V head and more: 16 x 8 on 2, 200..400 rows, 92 tiles 72 / 78; 32 x 8 on 1, 200..400 127 / 149; 64 x 8 on 2,
+//     128..256, 256 tiles 75 / 69; 4 x 8 on 1, 512..1024, 26 tiles 266 / 295; 16 x 8 on 1, 256..1024 324 / 288; two heads: 8 x 4 on 2, 200..400 45 /
+//     42
 //   rows on a history, whose sweeps are short for their tiles: slot 128, 32 x 4, 64 rows on 1000 keys 83 / 69, 16 x 4, 200 on 1000 87 / 65, 16 x 8
-//     on 2, 256 on 1024 (272 tiles) 148 / 130, 4 x 8 on 2, 300 on 700 (48 tiles) 83 / 114; slot 64, 4 x 8 on 2, 300 on 700 81 / 72, 2 x 8 on 1, 100..200 on
-//     500 (8 tiles) 58 / 67; slot 256 120 / 118 and 94 / 105
+//     on 2, 256 on 1024 (272 tiles) 148 / 130, 4 x 8 on 2, 300 on 700 (48 tiles) 83 / 114; slot 64, 4 x 8 on 2, 300 on 700 81 / 72, 2 x 8 on 1,
+//     100..200 on 500 (8 tiles) 58 / 67; slot 256 120 / 118 and 94 / 105
 //   slot 256, as 64: 4 x 8 on 2, 1024..2048, 100 tiles 451 / 517; 16 x 8 on 2, 256..1024, 176 tiles 320 / 300; 32 x 8 on 1, 512..1024 833 / 637
 //   two heads at the slots 64 and 256, whose query-tile launch holds on up to one slot per compute unit: slot 64, 8 x 4 on 2, 112 rows 21.9 / 24.8,
-//     64 x 4 of 112 (256 slots) 25.7 / 27.7, 128 x 4 (512) 34.3 / 32.3, 32 x 4 of 200 (256) 33.9 / 35.5, 4 x 4 of 256 35.0 / 33.1; slot 256, 26 x 4 on 2, 200 rows (208
-//     slots) 50.3 / 54.8, 40 x 4 (320) 66.4 / 58.1, 13 x 4 of 464 88.1 / 90.5, 12 x 4 of 600 109 / 109, 6 x 4 of 1000 175 / 165
-//   slot 256, a head each, one short tile: the key tiles and the clearing workgroups are more than the machine holds at once, one per CU: 52 x 4, 64
-//     rows (208 slots) 24.5 / 29.2, 64 x 4 25.9 / 30.3, 48 x 4 (192) 24.4 / 22.3; 40 x 4 of 128 rows 36.7 / 32.3
-//   slot 128, rows of one tile on a history: 64 x 4, 100 rows on 376 keys (256 slots) 59 / 63, 128 x 4 105 / 125, 32 x 4 44 / 39; 128 x 4, 64 rows on 1000 235 / 253,
-//     256 x 4 of 128 on 400 297 / 306; in pairs 32 x 4 on 2, 100 rows on 200 keys 33 / 38, on 376 45 / 43, 128 x 4 on 2 of the same 63 / 72 and 94 / 100, on 1000 290 / 272
+//     64 x 4 of 112 (256 slots) 25.7 / 27.7, 128 x 4 (512) 34.3 / 32.3, 32 x 4 of 200 (256) 33.9 / 35.5, 4 x 4 of 256 35.0 / 33.1; slot 256, 26 x 4
+//     on 2, 200 rows (208 slots) 50.3 / 54.8, 40 x 4 (320) 66.4 / 58.1, 13 x 4 of 464 88.1 / 90.5, 12 x 4 of 600 109 / 109, 6 x 4 of 1000 175 / 165
+//   slot 256, a head each, one short tile: the key tiles and the clearing workgroups are more than the machine holds at once, one per CU: 52 x 4,
+//     64 rows (208 slots) 24.5 / 29.2, 64 x 4 25.9 / 30.3, 48 x 4 (192) 24.4 / 22.3; 40 x 4 of 128 rows 36.7 / 32.3
+//   slot 128, rows of one tile on a history: 64 x 4, 100 rows on 376 keys (256 slots) 59 / 63, 128 x 4 105 / 125, 32 x 4 44 / 39; 128 x 4, 64 rows
+//     on 1000 235 / 253, 256 x 4 of 128 on 400 297 / 306; in pairs 32 x 4 on 2, 100 rows on 200 keys 33 / 38, on 376 45 / 43, 128 x 4 on 2 of the
+//     same 63 / 72 and 94 / 100, on 1000 290 / 272
 static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, int64_t tiles, int64_t cus, int64_t q_slots)
 {
     const int64_t batch = f->n_offsets - 1, ratio = f->num_heads_q / f->num_heads_k;
@@ -1072,21 +1074,22 @@ static bool few_biased_key_tiles(const hstu_jagged_fwd_params* f, int64_t dmax, 
 
 // Calls whose key-tile launch is a few workgroups that one sweep of all query rows (times query heads per K/V head) keeps busy long after
 // the machine has emptied: there the planes order, whose long launch has a workgroup per query tile and head, is the shorter one.
-// Grouped heads, K/V tiles of 128 keys (us, planes / dS handed over): 16 x 8 heads on 2, 256..1024 rows, d 128, 160 tiles 131 / 158, d 64
-// 111 / 124; 16 x 8 on 1, 1024 rows, 128 tiles 276 / 301; 4 x 8 on 2, 2048..4096 rows, 192 tiles 631 / 575; 32 x 8 on 2, 256..1024 rows, 320
-// tiles 234 / 185; 8 x 8 on 4, 1024 rows, 256 tiles 102 / 100 -- the line is at three quarters of the compute units.
-// Up to the slot 128 the other orders' query-tile launch of at most two workgroups per compute unit, all resident, holds on for longer
-// where the rows' last tiles are partly empty (those cost the key-tile kernel whole steps): 24 x 8 on 4, 200 rows (384 slots) 31.9 / 33.9, 32 x 8
-// (512) 34.0 / 36.2, 35 x 8 (560) 46.9 / 38.4; 30 x 8 on 4, 150 rows (480) 28.0 / 29.4, 34 x 8 (544) 39.7 / 31.4; d 64, 64 x 4 on 2, 200 rows (512) 27.4 / 29.2, 73 x
-// 4 (584) 33.8 / 30.7; whole tiles 23 x 8 on 4, 256 rows (368) 37.3 / 36.0; on a history 64 x 4 on 2, 200 rows on 400 keys (512) 58.4 / 51.3; one tile 48 x 8 on 4, 100 rows (384) 29.9 / 27.4 -- or, at the slot 128, where
-// rows of one tile meet keys of two, up to one per compute unit: 64 x 4 on 2, 100 rows on 160 keys (256) 23.2 / 27.9, 70 on 160 22.3 / 24.9, 80 x 4 (320)
-// 33.7 / 30.0; 100 on 400 (256) 41.2 / 40.1.
-// One query head per K/V head: only short rows at the slot 128, where the planes order has its 64-row query tiles -- up to one slot per
-// compute unit and fifteen sixteenths of it in key tiles: 16 x 4 of 100 rows 15.5 / 17.6, 15 x 4 of 116..168 17.6 / 20.8, 32 x 4 of 140 (204 tiles)
-// 18.3 / 20.0, 21 x 4 of 300 (236) 27.4 / 28.1, 8 x 4 of 400 28.1 / 29.4; 24 x 4 of 256 (240) 25.0 / 24.4, 32 x 4 of 256 (320) 27.0 / 26.1, 48 x 4 of 140 (384
-// slots) 25.0 / 22.6, 40 x 4 of 10..200 (320 slots) 25.3 / 22.5, 8 x 4 of 512 (144 tiles) 33.7 / 33.0, 5 x 4 of 700 42.8 / 41.2; on keys of twice the rows and more
-// the key tiles are many and their sweeps short: 16 x 4, 200 rows on 400 keys 29.0 / 25.1, 100 on 400 26.0 / 21.6.  And any such rows in at most 64 tiles:
-// 2 x 1, 300 rows 22.5 / 25.4; 8 x 2, 200..300 rows, 40 tiles 22.6 / 24.9; 4 x 4, 300..700 rows, 70 tiles 39.6 / 38.5; 1 x 4, 1000 rows, 32 tiles 55.6 / 52.9.
+// Grouped heads, K/V tiles of 128 keys (us, planes / dS handed over): 16 x 8 heads on 2, 256..1024 rows, d 128, 160 tiles 131 / 158, d 64 111 / 124;
+// 16 x 8 on 1, 1024 rows, 128 tiles 276 / 301; 4 x 8 on 2, 2048..4096 rows, 192 tiles 631 / 575; 32 x 8 on 2, 256..1024 rows, 320 tiles 234 / 185; 8
+// x 8 on 4, 1024 rows, 256 tiles 102 / 100 -- the line is at three quarters of the compute units.
+// Up to the slot 128 the other orders' query-tile launch of at most two workgroups per compute unit, all resident, holds on for longer where the
+// rows' last tiles are partly empty (those cost the key-tile kernel whole steps): 24 x 8 on 4, 200 rows (384 slots) 31.9 / 33.9, 32 x 8 (512) 34.0 /
+// 36.2, 35 x 8 (560) 46.9 / 38.4; 30 x 8 on 4, 150 rows (480) 28.0 / 29.4, 34 x 8 (544) 39.7 / 31.4; d 64, 64 x 4 on 2, 200 rows (512) 27.4 / 29.2,
+// 73 x 4 (584) 33.8 / 30.7; whole tiles 23 x 8 on 4, 256 rows (368) 37.3 / 36.0; on a history 64 x 4 on 2, 200 rows on 400 keys (512) 58.4 / 51.3;
+// one tile 48 x 8 on 4, 100 rows (384) 29.9 / 27.4 -- or, at the slot 128, where rows of one tile meet keys of two, up to one per compute unit: 64 x
+// 4 on 2, 100 rows on 160 keys (256) 23.2 / 27.9, 70 on 160 22.3 / 24.9, 80 x 4 (320) 33.7 / 30.0; 100 on 400 (256) 41.2 / 40.1.
+// One query head per K/V head: only short rows at the slot 128, where the planes order has its 64-row query tiles -- up to one slot per compute unit
+// and fifteen sixteenths of it in key tiles: 16 x 4 of 100 rows 15.5 / 17.6, 15 x 4 of 116..168 17.6 / 20.8, 32 x 4 of 140 (204 tiles) 18.3 / 20.0,
+// 21 x 4 of 300 (236) 27.4 / 28.1, 8 x 4 of 400 28.1 / 29.4; 24 x 4 of 256 (240) 25.0 / 24.4, 32 x 4 of 256 (320) 27.0 / 26.1, 48 x 4 of 140 (384
+// slots) 25.0 / 22.6, 40 x 4 of 10..200 (320 slots) 25.3 / 22.5, 8 x 4 of 512 (144 tiles) 33.7 / 33.0, 5 x 4 of 700 42.8 / 41.2; on keys of twice the
+// rows and more the key tiles are many and their sweeps short: 16 x 4, 200 rows on 400 keys 29.0 / 25.1, 100 on 400 26.0 / 21.6.  And any such rows
+// in at most 64 tiles: 2 x 1, 300 rows 22.5 / 25.4; 8 x 2, 200..300 rows, 40 tiles 22.6 / 24.9; 4 x 4, 300..700 rows, 70 tiles 39.6 / 38.5; 1 x 4,
+// 1000 rows, 32 tiles 55.6 / 52.9.
 static bool few_key_tiles(const hstu_jagged_fwd_params* f)
 {
     int cus = 0;
@@ -1252,9 +1255,10 @@ static BwdPlan plan_bwd(const hstu_jagged_bwd_params* p, const BwdVariant* var)
 
 // The tiles of the order that hands dS alone over, for a call that takes it when it has `room` bytes of workspace: none (heads == 0) where
 // another order is the faster one or is asked for.  5 products and 4 bytes of traffic per pair beside the operands, where the planes
-// order has 5 and 8: measured on 66 shapes (us, best other order -> this one) 32 x 4 heads of 256..1024 rows, d 128 100 -> 79, 16 x 4 of
+// order has 5 and 8: measured on 66 shapes without attn_bias (us, best other order -> this one) 32 x 4 heads of 256..1024 rows, d 128 100 -> 79, 16 x 4 of
 // 512..2048 210 -> 126, 8 x 8 of 4096..8000 2909 -> 2005, 32 x 8 of 1024 rows, d 64 244 -> 195, 16 x 4 of 501 rows and 1000 keys, d 64 62 -> 44,
-// 32 x 4 of 256..1024, d 256 191 -> 135, 256 x 4 of 40..200 88 -> 69; behind on few_key_tiles() only.
+// 32 x 4 of 256..1024, d 256 191 -> 135, 256 x 4 of 40..200 88 -> 69.  Where it is behind: few_key_tiles(), and few_biased_key_tiles() with an
+// attn_bias, whose key-tile kernel is slower.
 static DsTiles fused_plan(const hstu_jagged_bwd_params* p, const BwdVariant* var, int64_t room)
 {
     const hstu_jagged_fwd_params* f = &p->fwd;
