@@ -1484,9 +1484,9 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         // Requests the rab values of keys c0 + 16 lh .. + 15 of this lane's row, 8 packed words in memory order (what the routing MFMAs above
         // take as their B operands).  A row may start on any even address: the words asked for are the aligned ones that hold the values,
         // nine of them where some rows start in the middle of a word (!rab_words), and shift_rab() brings those into place.
-        // The words at the two ends of a plane may hold a neighbour's value, or two bytes in front of or behind the tensor; shift_rab() drops
-        // both.  16 x 4 heads of 512..2048 rows, d 128: max_seq_len_k 2049 143 -> 77 us and 2050 138 -> 72 (one value at a time before), 2052
-        // 67.4 -> 65.8 (8 bytes at a time), 2048 64 -> 61 (no branch left in the straight-line step).
+        // The words at the two ends of a plane may hold a neighbour's value, or two bytes in front of or behind the tensor; shift_rab() and
+        // clear_rab() drop both.  16 x 4 heads of 512..2048 rows, d 128: max_seq_len_k 2049 143 -> 74 us and 2050 141 -> 70 (one value at a time before), 2052
+        // 71.6 -> 69.3 (8 bytes at a time), 2048 60.3 -> 60.3.
         auto load_rab = [&](int c0, uint32_t (&w)[kRabWords], bool words) {
             const uint32_t off = rab_off + static_cast<uint32_t>(c0) * 2u;
             const U32Quad t0 = __builtin_bit_cast(U32Quad, __builtin_amdgcn_raw_buffer_load_b128(rab_rsrc, static_cast<int>(off), 0, 0));

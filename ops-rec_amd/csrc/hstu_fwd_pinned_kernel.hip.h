@@ -67,8 +67,8 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 3) void hstu_fwd_pinned_kernel(
         slot.r = rem - slot.level * ratio;
         // The workgroups of an XCD go to its four shader engines in turn, whether or not they find work: with a multiple of four slots a pair
         // would meet the same engines at every level, and those of a level that few sequences have would stand idle -- so the levels move on
-        // by one place per pair.  146 x 8 heads, 200..400 rows on 900 keys 229 -> 197 us, 291 x 4 on 2, 65..131 on 1767 209 -> 162; other counts
-        // of slots per pair level.
+        // by one place per pair.  d 128, 175 x 4 heads, 300..400 rows on 1500 keys 236 -> 212 us; d 256, 146 x 8, 200..400 on 900 469 -> 409;
+        // other counts of slots per pair level.
         if ((per_pair & 3) == 0) {
             slot.level += turn - div_small(turn, n_levels) * n_levels;
             slot.level -= slot.level >= n_levels ? n_levels : 0;
