@@ -218,6 +218,11 @@ struct InLinearSiluArgs {
     int k;
     int split_end[3];  // first column after the user, value and query parts
     int xcd_groups;    // 1: tiles dealt so that all n tiles of an m tile run on one XCD (grid padded to 8 m tiles)
+    // kernel with the weights in registers: groups of consecutive 32-row tiles, a workgroup each per 256 columns; the first
+    // longer_groups of them have group_tiles + 1 tiles, the others group_tiles (at least one)
+    int row_groups;
+    int group_tiles;
+    int longer_groups;
 };
 
 // element-wise stage of in_linear_silu's backward (in_linear_silu_bwd_kernel.hip.h)

@@ -8,6 +8,7 @@
 #include "hstu_error.h"
 #include "in_linear_silu_bwd_kernel.hip.h"
 #include "in_linear_silu_kernel.hip.h"
+#include "in_linear_silu_rows_kernel.h"
 #include "in_linear_silu_wgrad_kernel.hip.h"
 
 namespace {
@@ -35,6 +36,45 @@ const IlsVariant kVariants[2][4] = {
      ILS_VARIANT(f16_tag, "f16", 2, 256)},
 };
 
+// groups of rows of the kernel with the weights in registers: one workgroup per CU in all
+int rows_groups(const in_linear_silu_params* p)
+{
+    int cus = 0;
+    if (hstu::compute_units(&cus) != HSTU_OK) {
+        cus = 256;  // (a size asked for where there is no device)
+    }
+    const int64_t tiles = (p->m + hstu::kIlsRowsTile - 1) / hstu::kIlsRowsTile;
+    const int64_t cols = (p->n + hstu::kIlsRowsCols - 1) / hstu::kIlsRowsCols;
+    const int64_t groups = cus / cols > 1 ? cus / cols : 1;
+    return static_cast<int>(groups < tiles ? groups : tiles);
+}
+
+// The kernel with the weights in registers, where it is taken: k of 129 to 512 (the registers hold no more; at k = 128 the kernels
+// are level, 20480 x 4096 66.2 against 65.3 us: both write at 5 TB/s), at least six 32-row tiles per workgroup to pay for the weights on their
+// way in (us, bf16, this kernel against the other: 4 tiles 2048 x 512 16.6 / 16.4, 1024 x 256 12.8 / 12.0; 6 tiles 1536 x 384 18.5 /
+// 18.9, 1536 x 192 15.5 / 15.7; 8 tiles 2048 x 512 24.7 / 27.5, 4096 x 256 19.4 / 20.2; 20 tiles 2048 x 512 52.6 / 70.3; 131072 rows,
+// 128 tiles, 373 / 472), and splits that begin at 128-byte lines: elsewhere neighbouring wavefronts write parts of a line
+// (100000 rows of 240 -> 960 147 / 132, of 272 -> 1088 with 40000 rows 70 / 65).
+const hstu::IlsRowsVariant* select_rows(const in_linear_silu_params* p)
+{
+    if (p->k <= 128 || p->k > 512 || p->m > 0x7fffffff - hstu::kIlsRowsTile) {
+        return nullptr;
+    }
+    for (int i = 0; i < 4; ++i) {
+        if (p->split[i] % 64 != 0) {
+            return nullptr;
+        }
+    }
+    if (p->m / hstu::kIlsRowsTile < 6 * static_cast<int64_t>(rows_groups(p))) {
+        return nullptr;
+    }
+    const hstu::IlsRowsVariant* v = hstu::ils_rows_variants(p->dtype == HSTU_DT_BF16);
+    while (p->k > 16 * v->steps) {
+        ++v;
+    }
+    return v;
+}
+
 const IlsVariant* select(const in_linear_silu_params* p)
 {
     int ring;
@@ -61,6 +101,10 @@ bool xcd_groups(const in_linear_silu_params* p)
 // workgroups of a launch: m tiles (rounded up to whole groups of one per XCD in the grouped order) times n tiles
 int64_t grid_size(const in_linear_silu_params* p)
 {
+    if (select_rows(p) != nullptr) {  // (the kernel deals places to the XCDs in equal runs)
+        const int64_t places = rows_groups(p) * ((p->n + hstu::kIlsRowsCols - 1) / hstu::kIlsRowsCols);
+        return (places + hstu::kIlsXcds - 1) / hstu::kIlsXcds * hstu::kIlsXcds;
+    }
     const int tile_n = select(p)->tile_n;
     int64_t tiles_m = (p->m + hstu::kIlsTileM - 1) / hstu::kIlsTileM;
     const int64_t tiles_n = (p->n + tile_n - 1) / tile_n;
@@ -394,7 +438,11 @@ HSTU_API int in_linear_silu_bwd_dmixed(const in_linear_silu_bwd_params* p, void*
 
 HSTU_API const char* in_linear_silu_fwd_kernel_name(const in_linear_silu_params* params)
 {
-    return validate(params) == HSTU_OK ? select(params)->name : nullptr;
+    if (validate(params) != HSTU_OK) {
+        return nullptr;
+    }
+    const hstu::IlsRowsVariant* rows = select_rows(params);
+    return rows != nullptr ? rows->name : select(params)->name;
 }
 
 HSTU_API int in_linear_silu_fwd(const in_linear_silu_params* p, void* stream)
@@ -403,7 +451,6 @@ HSTU_API int in_linear_silu_fwd(const in_linear_silu_params* p, void* stream)
     if (rc != HSTU_OK) {
         return rc;
     }
-    const IlsVariant* v = select(p);
     InLinearSiluArgs a;
     a.x = p->x;
     a.weight = p->weight;
@@ -420,12 +467,20 @@ HSTU_API int in_linear_silu_fwd(const in_linear_silu_params* p, void* stream)
     a.split_end[1] = a.split_end[0] + static_cast<int>(p->split[1]);
     a.split_end[2] = a.split_end[1] + static_cast<int>(p->split[2]);
     a.xcd_groups = xcd_groups(p) ? 1 : 0;
-    const int64_t tiles = grid_size(p);
-    hipLaunchKernelGGL(v->kernel, dim3(static_cast<unsigned>(tiles)), dim3(hstu::kIlsThreads), 0,
-                       static_cast<hipStream_t>(stream), a);
+    a.row_groups = a.group_tiles = a.longer_groups = 0;
+    const hstu::IlsRowsVariant* rows = select_rows(p);
+    if (rows != nullptr) {
+        const int row_tiles = static_cast<int>((p->m + hstu::kIlsRowsTile - 1) / hstu::kIlsRowsTile);
+        a.row_groups = rows_groups(p);
+        a.group_tiles = row_tiles / a.row_groups;
+        a.longer_groups = row_tiles % a.row_groups;
+    }
+    const unsigned grid = static_cast<unsigned>(grid_size(p));
+    hipLaunchKernelGGL(rows != nullptr ? rows->kernel : select(p)->kernel, dim3(grid),
+                       dim3(rows != nullptr ? hstu::kIlsRowsThreads : hstu::kIlsThreads), 0, static_cast<hipStream_t>(stream), a);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
-        return hstu::set_error(HSTU_ERR_RUNTIME, "launch of %s failed: %s", v->name, hipGetErrorString(err));
+        return hstu::set_error(HSTU_ERR_RUNTIME, "launch of %s failed: %s", in_linear_silu_fwd_kernel_name(p), hipGetErrorString(err));
     }
     return HSTU_OK;
 }

@@ -20,6 +20,7 @@ SOURCES = [
     "hstu_mi355.hip",
     "ln_mul_mi355.hip",
     "in_linear_silu_mi355.hip",
+    "in_linear_silu_kernels_rows.hip",
     "hstu_kernels_fwd_bf16.hip",
     "hstu_kernels_fwd_f16.hip",
     "hstu_kernels_fwd_f8.hip",
@@ -31,9 +32,14 @@ SOURCES = [
     "hstu_kernels_fwd_pinned.hip",
 ]
 # These kernels name the accumulator registers they keep their sums in (hstu_pinned_acc.hip.h); every other matrix result belongs in
-# vector registers, where the compiler would otherwise keep it in accumulators as well and copy each element out.
+# vector registers, where the compiler would otherwise keep it in accumulators as well and copy each element out.  So it does in
+# the kernel that keeps its weights there.
 _VGPR_FORM = ("-mllvm", "-amdgpu-mfma-vgpr-form=1")
-SOURCE_FLAGS = {"hstu_kernels_bwd_fused.hip": _VGPR_FORM, "hstu_kernels_fwd_pinned.hip": _VGPR_FORM}
+SOURCE_FLAGS = {
+    "hstu_kernels_bwd_fused.hip": _VGPR_FORM,
+    "hstu_kernels_fwd_pinned.hip": _VGPR_FORM,
+    "in_linear_silu_kernels_rows.hip": _VGPR_FORM,
+}
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",

@@ -115,6 +115,31 @@ def test_edges_and_long_k(m, n, k, split):
     check(x, w, bias, split)
 
 
+@pytest.mark.parametrize("m,n,k,split,variant", [
+    (768, 16384, 512, [4096] * 4, "rows512"),                      # six whole tiles for each of the four row groups
+    (801, 16384, 512, [4096, 64, 8128, 4096], "rows512"),          # one row in the last tile; groups of 7, 7, 6, 6 tiles
+    (799, 16000, 400, [4032, 3968, 4032, 3968], "rows512"),        # k = 25 of 32 steps; half of the last column block exists
+    (900, 16128, 336, [4032] * 4, "rows384"),
+    (1000, 16384, 256, [4096] * 4, "rows256"),
+    (777, 16128, 144, [64, 8000, 64, 8000], "rows256"),            # k = 9 of 16 steps
+    (6500, 2112, 176, [576, 512, 512, 512], "rows256"),            # 28 row groups of nine column blocks, the last of 64 columns
+])  # fmt: skip
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_weights_in_registers(m, n, k, split, variant, dtype):
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(dtype)
+    w = (torch.randn(n, k, generator=g) / k**0.5).to(dtype)
+    bias = torch.randn(n, generator=g)
+    p = _native.new_in_linear_silu_params()
+    p.x, p.weight, p.bias = 0x1000, 0x2000, 0x3000  # never dereferenced
+    p.user, p.value, p.query, p.key, p.linear_output = 0x4000, 0x5000, 0x6000, 0x7000, 0x8000
+    p.m, p.n, p.k, p.dtype = m, n, k, _native.DT_BF16 if dtype == torch.bfloat16 else _native.DT_FP16
+    for i in range(4):
+        p.split[i] = split[i]
+    assert _native.load().in_linear_silu_fwd_kernel_name(ctypes.byref(p)).decode().endswith(variant)
+    check(x, w, bias, split)
+
+
 def test_every_output_column_names_its_weight_row():
     # one-hot x rows and weight[j, i] = (j % 64) + i / 16 (exact in fp16): each output element tells which weight row,
     # which k and which split made it; covers the permuted placement of weight rows in LDS and the split boundaries
