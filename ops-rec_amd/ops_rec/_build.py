@@ -32,14 +32,11 @@ SOURCES = [
     "hstu_kernels_fwd_pinned.hip",
 ]
 # These kernels name the accumulator registers they keep their sums in (hstu_pinned_acc.hip.h); every other matrix result belongs in
-# vector registers, where the compiler would otherwise keep it in accumulators as well and copy each element out.  So it does in
-# the kernel that keeps its weights there.
+# vector registers, where the compiler would otherwise keep it in accumulators as well and copy each element out.
 _VGPR_FORM = ("-mllvm", "-amdgpu-mfma-vgpr-form=1")
-SOURCE_FLAGS = {
-    "hstu_kernels_bwd_fused.hip": _VGPR_FORM,
-    "hstu_kernels_fwd_pinned.hip": _VGPR_FORM,
-    "in_linear_silu_kernels_rows.hip": _VGPR_FORM,
-}
+SOURCE_FLAGS = {"hstu_kernels_bwd_fused.hip": _VGPR_FORM, "hstu_kernels_fwd_pinned.hip": _VGPR_FORM}
+# The same where it is operands that stay in accumulators (the compiler knows of those: none is named).
+OPERAND_SOURCE_FLAGS = {"in_linear_silu_kernels_rows.hip": _VGPR_FORM}
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -93,7 +90,8 @@ def build(verbose: bool = False, jobs: int | None = None, extra_flags: tuple = (
         objects = [os.path.join(obj_dir, os.path.splitext(s)[0] + ".o") for s in SOURCES]
         with ThreadPoolExecutor(max_workers=jobs) as pool:
             jobs_done = [
-                pool.submit(_run, [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(s, ()), *extra_flags, "-c", os.path.join(CSRC, s), "-o", o], verbose)
+                pool.submit(_run, [hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(s, OPERAND_SOURCE_FLAGS.get(s, ())), *extra_flags, "-c",
+                                   os.path.join(CSRC, s), "-o", o], verbose)
                 for s, o in zip(SOURCES, objects)
             ]
             for j in jobs_done:
