@@ -19,11 +19,12 @@
 // 2.0 + 0.9 ms of the kernels that recompute.  Ordinary ones the vector unit and the longest workgroup: 32 x 4 heads, d 128, 256..1024
 // rows 62 + 21 us, where the query-tile kernel with dS and P took 61 and the kernels that read them 41.  A wavefront with 64 keys and
 // all 512 registers, one per SIMD, took as long as this one (1.39 ms at the large shape) and has half as many workgroups.
-// With attn_bias the key-tile kernel at the slot 128 spills: 16 x 4 heads, d 128, 512..2048 rows 245 us, 193 before a block cleared what its
-// rows do not see of the bias (39 scratch instructions against 16, in every order of that code tried; none at the slot 64).  Four of the
-// eight K fragments are read back from scratch between the products of S, and a wait for such a load, whose count is in order, is one for
-// everything asked for before it: the bias and the tiles that this step has just requested for the next two.  The call 385 -> 350 us, where
-// dV, dQ storing dS and dK from it took 185 + 139 + 61.
+// With attn_bias a step also clears what its rows do not see and moves the bias to its keys, and the registers are what it is built around: a loop of
+// steps with a mask and one of steps without (under one loop the compiler keeps the scores of the block with a mask, 16 registers, through the one
+// without), offsets of the transposed reads worked out where they are used (8 registers).  With both in one loop the slot 128 kept four of the eight K
+// fragments in scratch memory, and a wait for such a load, whose count is in order, is one for everything asked for before it, the bias and the tiles of
+// the next two steps: 16 x 4 heads, d 128, 512..2048 rows 245 us, now 177, the training call 415 -> 340.  (Slots 64 and 256, which did not spill: 0.98 ..
+// 1.00 of the time.  Without a bias the unrolled loop of both is the faster one by 1 to 3 %.)
 // The query-tile kernel moves dS once: at the large shape 3.8 GB fetched, 2.6 of them dS, in 0.65 ms = 5.8 TB/s.
 #pragma once
 #include "hstu_bias_requests.h"
@@ -122,6 +123,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     __shared__ __attribute__((aligned(1024))) uint16_t s_ring[3 * kStageElems];
     __shared__ __attribute__((aligned(1024))) uint16_t s_v[4 * T::ELEMS];  // V rows, a sub-tile per wavefront
     constexpr uint32_t kPastEnd = 0x40000000u;
+    constexpr bool kTwoLoops = HAS_RAB;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -324,10 +326,24 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     auto read_n = [&](const uint16_t* tile, int first_off, int js) -> u32x4_t {
         return *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint8_t*>(tile) + (first_off ^ (js * 32)));
     };
+    uint32_t t_off[2] = {0, 0};  // (kTwoLoops) bytes from the ring's first stage
     auto read_t = [&](const uint16_t* tile, int c) -> u32x4_t {
         const int j2 = c / MTILES, mt = c % MTILES;
-        const u32x2_t lo = lds_read_tr16_b64(tile + t_lane_off[mt][0] + 16 * j2 * D);
-        const u32x2_t hi = lds_read_tr16_b64(tile + t_lane_off[mt][1] + 16 * j2 * D);
+        u32x2_t lo, hi;
+        if constexpr (kTwoLoops) {
+            // (the output tile's bits flipped where it is read: offsets worked out ahead are registers that are not to be had)
+            uint32_t o[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                asm volatile("v_xor_b32 %0, %2, %1" : "=v"(o[i]) : "v"(t_off[i]), "n"(64 * mt));
+                o[i] += 32u * j2 * D;
+            }
+            lo = lds_read_tr16_b64(reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(tile) + o[0]));
+            hi = lds_read_tr16_b64(reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(tile) + o[1]));
+        } else {
+            lo = lds_read_tr16_b64(tile + t_lane_off[mt][0] + 16 * j2 * D);
+            hi = lds_read_tr16_b64(tile + t_lane_off[mt][1] + 16 * j2 * D);
+        }
         const u32x4_t r = {lo[0], lo[1], hi[0], hi[1]};
         return r;
     };
@@ -335,6 +351,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
         const u32x4_t r = {w[4 * j2], w[4 * j2 + 1], w[4 * j2 + 2], w[4 * j2 + 3]};
         return r;
     };
+    int cur_stage = 0;  // (kTwoLoops) the current step's
     const uint32_t ds_lane = static_cast<uint32_t>(ln * 32 + lh * 16);
 #define HSTU_FENCE() __builtin_amdgcn_sched_barrier(0)
 
@@ -365,6 +382,14 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
         }
         int n_off = n_first_off;
         asm volatile("" : "+v"(n_off));  // (not to be worked out ahead of the sweep)
+        if constexpr (kTwoLoops) {
+            const uint32_t at = static_cast<uint32_t>(cur_stage) * (kStageElems * 2u);
+            t_off[0] = 2u * t_lane_off[0][0] + at;
+            t_off[1] = 2u * t_lane_off[0][1] + at;
+            asm volatile("" : "+v"(t_off[0]), "+v"(t_off[1]));
+            n_off += static_cast<int>(at);
+            asm volatile("" : "+v"(n_off));
+        }
         int v_off = wave * T::ELEMS * 2 + n_first_off;
         asm volatile("" : "+v"(v_off));
         auto fetch = [&](int k) {  // operand of slot k
@@ -509,7 +534,8 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
         });
     };
 
-    auto step = [&](const uint16_t* q_tile, int stage_o) {
+    auto step = [&](auto kind, const uint16_t* q_tile, int stage_o) {
+        constexpr int kKind = decltype(kind)::value;  // 0: masked or not by the sub-tile; 1: no block of it masked; 2: all
         // this step's sub-tile has landed for everybody; the stage of the previous step is free
         acc_fence<kAccRegs>();
         HSTU_FENCE();
@@ -526,7 +552,7 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
             s[i] = 0.f;
         }
         const int x = cur_x;
-        const bool masked = x < full_from || x >= full_to;
+        const bool masked = kKind == 2 || (kKind == 0 && (x < full_from || x >= full_to));
         if constexpr (HAS_RAB) {
             // the matrix pipe transposes the bias into the scores' accumulators; its registers take the next block's at once
             int word = one_word;
@@ -567,17 +593,34 @@ __global__ __launch_bounds__(kDkvThreads, bwd_kv_fused_wgs_per_cu(D)) void hstu_
     };
 
     if (n_iter > 0) {
+        [[maybe_unused]] constexpr std::integral_constant<int, 0> any{};
         int it = 0;
-        while (true) {  // (step it reads stage it mod 3 and has stage (it + 2) mod 3 filled)
-            step(s_ring, 2);
+        if constexpr (kTwoLoops) {
+            auto next = [&]() {
+                cur_stage = cur_stage == 2 ? 0 : cur_stage + 1;
+                ++it;
+            };
+            while (it < n_iter) {
+                while (it < n_iter && cur_x >= full_from && cur_x < full_to) {
+                    step(std::integral_constant<int, 1>{}, s_ring, cur_stage == 0 ? 2 : cur_stage - 1);
+                    next();
+                }
+                while (it < n_iter && (cur_x < full_from || cur_x >= full_to)) {
+                    step(std::integral_constant<int, 2>{}, s_ring, cur_stage == 0 ? 2 : cur_stage - 1);
+                    next();
+                }
+            }
+        }
+        while (!kTwoLoops) {  // (step it reads stage it mod 3 and has stage (it + 2) mod 3 filled)
+            step(any, s_ring, 2);
             if (++it >= n_iter) {
                 break;
             }
-            step(s_ring + kStageElems, 0);
+            step(any, s_ring + kStageElems, 0);
             if (++it >= n_iter) {
                 break;
             }
-            step(s_ring + 2 * kStageElems, 1);
+            step(any, s_ring + 2 * kStageElems, 1);
             if (++it >= n_iter) {
                 break;
             }

@@ -231,10 +231,8 @@ __device__ __forceinline__ void row_bounds(const SeqInfo& s, int mask_type, int 
     lim = lim < 0 ? 0 : (lim > s.sk ? s.sk : lim);
     if (s.n_tgt > 0 && group > 0) {
         const int ti = r - (s.sq - s.n_tgt);
-        if (ti >= 0) {
-            hole_lo = s.hist_k;
-            hole_hi = s.hist_k + (ti / group) * group;
-        }
+        hole_lo = s.hist_k;
+        hole_hi = s.hist_k + (ti > 0 ? ti : 0) / group * group;  // (empty ahead of the target rows)
     }
 }
 

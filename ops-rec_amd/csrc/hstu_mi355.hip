@@ -1000,7 +1000,7 @@ static const hstu::BwdFusedVariant* fused_variant(const hstu_jagged_bwd_params* 
 
 // Workgroups of the key-tile launch that do nothing but clear the attn_bias gradient: at the front of the grid, so that the zeros go out
 // beside the products from the start.  The fewer products a byte of the gradient comes with, the more of them (us of the backward with
-// 64 / 96 / 128, before the key-tile kernel cleared what rows do not see of the bias, which costs the first shape 50 us in each): 16 x 4
+// 64 / 96 / 128, of an earlier key-tile kernel): 16 x 4
 // heads, d 128, 512..2048 rows 287 / 290 / 296; 32 x 4 of 256..1024 154 / 153 / 149; d 64 130 / - / 113; 64 x 4, d 64, 64..512 rows 82 / - /
 // 68.  (Dealt over all workgroups ahead of their sweeps, as the other orders have it, the zeros hold up every one of them: the dV launch
 // alone takes 185 us at the first shape.)
@@ -1015,11 +1015,12 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
     return static_cast<int>(std::min<int64_t>(most / 8, std::max<int64_t>(1, (std::max(bytes >> 20, groups / 8) + 7) / 8)) * 8);
 }
 
-// Calls with attn_bias that keep the orders without dS tiles (see few_key_tiles).  The key-tile kernel's step is longest there, most of all at the
-// slot 128, where it spills, and a workgroup has as many steps as its K/V head has query heads times row blocks: the order pays from the tiles on
+// Calls with attn_bias that keep the orders without dS tiles (see few_key_tiles).  The key-tile kernel's step is longest there, and a workgroup has as many steps as its K/V head has query heads times row blocks: the order pays from the tiles on
 // that keep the machine busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute
 // units, whatever the group's size.
-// Measured on 125 shapes, and 300 more for short rows, pairs of heads and histories (device time in us, other order / dS handed over):
+// Measured on 125 shapes, and 300 more for short rows, pairs of heads and histories (device time in us, other order / dS handed over), at the slot 128
+// with a key-tile kernel that spilled and took 245 us where it now takes 177: the lines below leave it no call that is slower, and some that would
+// now be faster (forward included, 16 x 4, 300..500 rows 79 / 66, 234 x 4, 58..216 164 / 149, 64 x 4, 100 on 376 keys 79 / 75, 32 x 8 on 1, 1024 841 / 668):
 //   slot 128, grouped: 32 x 8 on 2, 512 rows, 288 tiles 196 / 226; 16 x 8 on 2, 256..1024 (176 tiles) 230 / 304; 32 x 8 on 1, 1024 (272) 690 / 793;
 //     8 x 8 on 4, 1024..2048 (400, three quarters) 507 / 450; 32 x 8 on 4, 256..1024 (704) 328 / 296; 64 x 8 on 2, 256..1024 (704) 775 / 634
 //   slot 128, rows of one tile: 512 x 2, 100..128 rows 87 / 99; 256 x 8 on 4, 64..128 139 / 150; 512 x 4, 128 rows, 2048 tiles 209 / 197
