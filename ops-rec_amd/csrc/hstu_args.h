@@ -95,6 +95,7 @@ struct FwdArgs {
     uint64_t launch_id;      // split variant: the launch's number, 1 .. 2^48 - 1, above the counts of its arrival counters
     float* ws;           // split variant: room for ws_parts partial outputs of kBlockM x D floats each (may be null)
     uint32_t ws_parts;
+    int slot_parts;      // split and paged variants without a list: parts that every item is cut into, 1 .. kMaxParts
     // paged variant: the first (key count - num_target) key rows of a sequence live in pages of kv_cache
     // [num_pages, 2 (K, V), page_size, n_heads_k, d]; k / v then hold the rows of ALL query tokens, of which the last
     // num_target of each sequence are its remaining keys

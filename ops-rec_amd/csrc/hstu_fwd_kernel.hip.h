@@ -412,7 +412,8 @@ struct U32Quad {
 // multiple of 8 so that a pair's tiles meet on one XCD, levels in list order so that the longest items start first; slots
 // past the end of their sequence leave at once.  That spares every workgroup the histogram, the list and the hand-over of
 // its item through LDS, 1.5 .. 4 us ahead of its first request.  (A variant of its own: as a branch of the plain one it cost
-// that 1 us.)
+// that 1 us.)  With SPLIT every item is cut into the same number of parts (FwdArgs::slot_parts), a workgroup each: for items
+// whose sweeps are about equally long, a few query rows on a history.
 template <typename Tag, typename OutTag, int D, bool HAS_RAB, bool HAS_MASK, bool QUEUES = false, bool SPLIT = false,
           bool PAGED = false, bool DIRECT = false>
 __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hstu_fwd_kernel(const FwdArgs a)
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     static_assert(!F8 || !(HAS_RAB || HAS_MASK) || !SPLIT, "fp8 with rab / custom mask: whole items only");
     static_assert(!F8 || D >= 64, "fp8 rows are at least 64 bytes");
     static_assert(!(QUEUES && SPLIT), "one list policy per variant");
-    static_assert(!DIRECT || !(QUEUES || SPLIT || PAGED), "no list, no list policy");
+    static_assert(!DIRECT || !QUEUES, "no list, no queues");
     static_assert(!PAGED || (SPLIT && !F8), "the paged variant builds on the split variant, 16-bit inputs");
     constexpr int CPR = D * ES / 16;             // 16-byte chunks per row
     constexpr int EPC16 = 16 / ES;               // elements per 16-byte chunk
@@ -474,9 +475,9 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     // K/V head, q0 lo/hi, q1 lo/hi, k0 lo/hi, k1 lo/hi, context count, target count])
     // and, with SPLIT, the part word, the arrival counter and the first partial buffer
     __shared__ uint32_t s_next[!QUEUES ? 2 : 1][20];
-    __shared__ uint8_t s_parts[SPLIT ? kMaxLevels + 2 : 1];         // parts per item of each level
-    __shared__ uint32_t s_split_first[SPLIT ? kMaxLevels + 2 : 1];  // first arrival counter of each split level
-    __shared__ uint32_t s_ws_first[SPLIT ? kMaxLevels + 2 : 1];     // first partial buffer of each split level
+    __shared__ uint8_t s_parts[SPLIT ? kListLevels : 1];         // parts per item of each level
+    __shared__ uint32_t s_split_first[SPLIT ? kListLevels : 1];  // first arrival counter of each split level
+    __shared__ uint32_t s_ws_first[SPLIT ? kListLevels : 1];     // first partial buffer of each split level
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1084,15 +1085,28 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         int64_t q0, q1, k0, k1;
         int n_ctx = 0;
         int n_tgt = 0;
+        int part = 0, n_parts = 1, split_item = 0, split_buffer = 0;  // (split items) their arrival counter and first partial output
         if constexpr (DIRECT) {
-            const int pairs_pad = (a.n_batch * a.n_heads_k + 7) & ~7;
-            const int per_level = pairs_pad * a.head_ratio;
+            const int pairs = a.n_batch * a.n_heads_k;
+            const int pairs_pad = (pairs + 7) & ~7;
+            if constexpr (SPLIT) {
+                n_parts = a.slot_parts;
+            }
+            const int per_level = pairs_pad * a.head_ratio * n_parts;
             const int lvl = static_cast<int>(blockIdx.x) / per_level;
             const int rest = static_cast<int>(blockIdx.x) - lvl * per_level;
-            const int in_group = rest / pairs_pad;
-            const int pair = rest - in_group * pairs_pad;
-            if (pair >= a.n_batch * a.n_heads_k) {
+            const int group = rest / pairs_pad;
+            const int pair = rest - group * pairs_pad;
+            if (pair >= pairs) {
                 break;
+            }
+            const int in_group = SPLIT ? group / n_parts : group;
+            part = group - in_group * n_parts;
+            if constexpr (SPLIT) {
+                split_item = (lvl * a.head_ratio + in_group) * pairs + pair;
+                split_buffer = split_item * n_parts;
+            } else {
+                part = 0;
             }
             qt = tile_of_level(lvl);
             b = pair / a.n_heads_k;
@@ -1209,12 +1223,14 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         }
         const int sub_shift = a.page_shift - 5;  // sub-tiles per page, as a shift
         const int last_pid = static_cast<int>(a.num_pages - 1);
+        // (The low word of the entry alone, whatever its type, and clamped where it is used, a step on: a branch on the type, or the clamp
+        // here, makes the step wait for the load it has just sent.  With that and the requests without lane masks below 32 x 4 heads, d 128,
+        // 64..96 rows on 3072 keys 50 -> 47 us, on 4096 65 -> 63; 44.5 and 57.5 with the rows in order.)
         auto page_of = [&](int x) -> int {
             int idx = page_first + (x >> sub_shift);
             idx = idx < page_hi ? idx : page_hi;
-            int pid = static_cast<int>(load_index_uniform(a.page_ids, idx, a.idx64));
-            pid = pid < last_pid ? pid : last_pid;
-            return pid < 0 ? 0 : pid;
+            typedef const __attribute__((address_space(4))) int* cint_t;
+            return *(cint_t)(reinterpret_cast<uintptr_t>(a.page_ids) + (static_cast<uint64_t>(static_cast<uint32_t>(idx)) << (2 + a.idx64)));
         };
 
         // ---- buffer descriptors sized to this sequence / head ----
@@ -1266,12 +1282,12 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         // the part of them this entry of the list stands for
         int x_begin = 0;
         int x_end = n_sub;
-        int part = 0;
-        int n_parts = 1;
         if constexpr (SPLIT) {
-            const uint32_t part_word = s_next[round & 1][15];
-            part = uniform(static_cast<int>(part_word & 0xffu));
-            n_parts = uniform(static_cast<int>(part_word >> 8));
+            if constexpr (kStaticList) {
+                const uint32_t part_word = s_next[round & 1][15];
+                part = uniform(static_cast<int>(part_word & 0xffu));
+                n_parts = uniform(static_cast<int>(part_word >> 8));
+            }
             if (n_parts > 1) {
                 const int len = ((n_sub + n_parts - 1) / n_parts + 3) & ~3;
                 x_begin = part * len;
@@ -1285,6 +1301,8 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         // come from the page, the others from the new rows; a request past the end moves nothing.
         auto request_paged = [&](uint16_t* dst, const __amdgpu_buffer_rsrc_t new_rsrc, const uint32_t (&src)[LPW], int x,
                                  int pid, int kv) {
+            pid = pid < last_pid ? pid : last_pid;
+            pid = pid < 0 ? 0 : pid;
             const bool live = x < x_end;
             const int bnd = live ? n_cached - x * 32 : 0;
             const int rows_c = bnd < 0 ? 0 : (bnd > 32 ? 32 : bnd);
@@ -1295,6 +1313,13 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             // offset of sub-tile row 0 among the new rows (negative, as a wrapped unsigned, while bnd > 0: the
             // lanes that use it have rows >= bnd, which brings the sum back into range)
             const uint32_t new_base = live ? static_cast<uint32_t>(x * 32 - n_cached) * k_stride : kPastEnd;
+            if (bnd >= 32) {  // (nearly all of them: no lane masks)
+#pragma unroll
+                for (int i = 0; i < LPW; ++i) {
+                    load_to_lds_b128(page_rsrc, dst + (wave * LPW + i) * 512, src[i]);
+                }
+                return;
+            }
 #pragma unroll
             for (int i = 0; i < LPW; ++i) {
                 if (ld_row[i] < bnd) {
@@ -2117,13 +2142,17 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 constexpr int kDeviceScope = 1 | 16;  // cache policy bits sc0 | sc1 of gfx94x / gfx950 buffer accesses
                 constexpr int kQuads = MTILES * 4;                       // 16-byte pieces of a lane's accumulators
                 constexpr uint32_t kPartBytes = kBlockM * D * 4u;        // one partial output
-                const int ws_index = uniform(static_cast<int>(s_next[round & 1][17]));
+                if constexpr (kStaticList) {
+                    split_item = uniform(static_cast<int>(s_next[round & 1][16]));
+                    split_buffer = uniform(static_cast<int>(s_next[round & 1][17]));
+                }
                 const __amdgpu_buffer_rsrc_t ws_rsrc =
-                    make_rsrc(reinterpret_cast<const uint8_t*>(a.ws) + static_cast<int64_t>(ws_index) * kPartBytes,
+                    make_rsrc(reinterpret_cast<const uint8_t*>(a.ws) + static_cast<int64_t>(split_buffer) * kPartBytes,
                               static_cast<uint32_t>(n_parts) * kPartBytes);
                 // piece q of (wavefront, lane) sits at ((wave * kQuads + q) * 64 + lane) * 16 bytes: each store
                 // instruction writes 1 KiB in a row
-                const uint32_t lane_off = static_cast<uint32_t>(wave * kQuads * 64 + lane) * 16u;
+                // (rows past the end of the sequence are not handed over: 96 rows are three quarters of a tile)
+                const uint32_t lane_off = wr0 + ln < sq ? static_cast<uint32_t>(wave * kQuads * 64 + lane) * 16u : kOutOfRange;
                 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 #pragma unroll
                 for (int q = 0; q < kQuads; ++q) {
@@ -2137,7 +2166,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
                 }
                 __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();  // every wavefront's stores have completed
-                uint64_t* const arrived = reinterpret_cast<uint64_t*>(a.counters + kSplitCounterBase) + s_next[round & 1][16];
+                uint64_t* const arrived = reinterpret_cast<uint64_t*>(a.counters + kSplitCounterBase) + split_item;
                 if (tid == 0) {
                     const uint64_t none = a.launch_id << 16;  // no part has arrived in this launch
                     uint64_t seen = __hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -558,9 +558,36 @@ const hstu::ShortVariant* pinned_variant(const Variant* var, const hstu_jagged_f
 constexpr uint64_t kMaxWorkspaceBytes = 128ull << 20;
 constexpr uint64_t kCounterBytes = hstu::kCounterBlockBytes;  // head of the workspace of the variants that pull from counters
 uint64_t split_part_bytes(const Variant* var) { return static_cast<uint64_t>(hstu::kBlockM) * var->d_pad * sizeof(float); }
+// Parts that a split or paged launch without a list cuts every item into (1: paged, whole items), 0 where it takes the list: items whose
+// sweeps are about equally long -- one query tile, or at least as many keys behind the rows as there are rows, no context rows -- and that are
+// all resident at once, in as many parts of eight steps and more as the machine holds.  Measured with parts of at least 8, 12, 16 and 24 steps
+// (us): 16 x 4 heads, paged, 64..96 rows on 512 keys 21.9 / 25.2 / 25.2 / 25.3, on 1024 26.8 / 28.4 / 28.5 / 37.3, on 2048 36.0 / 32.9 / 32.3 / 40.8; 4
+// x 4 on 1536 25.6 / 27.0 / 27.5 / 32.3; 32 x 4 from 1024 keys on level.
+// List -> slots, with page ids that a step does not wait for (us, d 128, 64..96 rows): paged 32 x 4 on 512 keys 30.5 -> 23.1, on 2048..4096 61.0 -> 52.0, 16 x
+// 4 on 2048 50.7 -> 35.7, 64 x 4 on 4096 126 -> 116; 32 x 4, 80 rows on 3000 keys 53.4 -> 42.1 (4.7 TB/s), 16 x 4, 200 on 3000 51.8 -> 42.6, d 64, 32 x
+// 4 on 3000 43.1 -> 30.2.  The slot 256, whose items were not cut before: paged 4 x 4 on 4096 186 -> 46, 32 x 4 196 -> 120, 64 x 4 (no room for
+// parts) 236 -> 212; 16 x 4, 80 rows on 2128 71 -> 42, 2 x 4, d 192, 500 on 3000..4000 117 -> 45.  No call of 110 was slower.
+int slot_parts(const Variant* var, const hstu_jagged_fwd_params* p, bool paged, int64_t resident, int64_t room)
+{
+    if ((paged ? var->kernel_paged_direct : var->kernel_split_direct) == nullptr || p->num_context != nullptr) {
+        return 0;
+    }
+    const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
+    if (n_qtiles > 1 && 2 * p->max_seq_len_q > p->max_seq_len_k) {
+        return 0;
+    }
+    const int64_t items = n_qtiles * (p->n_offsets - 1) * p->num_heads_q;
+    if (items > resident) {
+        return 0;
+    }
+    const int64_t steps = (p->max_seq_len_k + 31) / 32;
+    const int64_t parts = std::min({resident / items, room / items, steps / 8, int64_t{8}});
+    return static_cast<int>(parts >= 2 ? parts : (paged ? 1 : 0));
+}
+
 bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p, int64_t* resident_out, bool paged = false)
 {
-    if (var->persistent_wgs_per_cu <= 0 || var->kernel_split == nullptr) {
+    if (var->persistent_wgs_per_cu <= 0 || (var->kernel_split == nullptr && (paged ? var->kernel_paged : var->kernel_split_direct) == nullptr)) {
         return false;
     }
     // HSTU_MI355_SPLIT=0 turns splitting off: the rows of a sequence then come out bit for bit the same whatever
@@ -581,6 +608,10 @@ bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p,
     // (items of at most 16 sub-tiles: parts of 8, the kernel's shortest, do not earn back what a part costs --
     // 8 x 4 sequences of 512 rows: 23.0 us split, 20.7 us not)
     if (n_blocks >= 2 * resident || p->max_seq_len_k <= 16 * 32) {
+        return false;
+    }
+    // (The slot 256 has no list with split items, and up to 1024 keys its rows keep the bits that the kernel with pinned sums gives them.)
+    if (var->kernel_split == nullptr && !paged && (p->max_seq_len_k <= 1024 || slot_parts(var, p, false, resident, resident) == 0)) {
         return false;
     }
     // A launch without a list (which the paged variant does not have) needs no building of a list, no hand-over of parts through memory
@@ -1974,6 +2005,13 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         if (paged != nullptr) {
             kernel = var->kernel_paged;  // (splits when it was given room above, otherwise not; the caller checked the block)
             a.counters = static_cast<unsigned int*>(workspace);
+        }
+        if (kernel == var->kernel_split || paged != nullptr) {
+            a.slot_parts = slot_parts(var, p, paged != nullptr, hstu::split_grid(resident), a.ws != nullptr ? a.ws_parts : 0);
+            if (a.slot_parts > 0) {
+                kernel = paged != nullptr ? var->kernel_paged_direct : var->kernel_split_direct;
+                n_blocks = direct_slots(p) * a.slot_parts;
+            }
         }
         if (a.counters == nullptr && takes_direct_list(var, p, static_cast<int64_t>(cus) * wgs_per_cu(var, p))) {
             kernel = var->kernel_direct;

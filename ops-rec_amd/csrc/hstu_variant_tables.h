@@ -40,6 +40,27 @@ constexpr auto paged_kernel() -> void (*)(const FwdArgs)
     }
 }
 
+// the same without a list
+template <typename Tag, typename OutTag, int D, bool RAB, bool MASK>
+constexpr auto split_direct_kernel() -> void (*)(const FwdArgs)
+{
+    if constexpr ((D == 64 || D == 128 || (D == 256 && !elem_traits<Tag>::kF8)) && !RAB && !MASK) {
+        return hstu_fwd_kernel<Tag, OutTag, D, RAB, MASK, false, true, false, true>;
+    } else {
+        return nullptr;
+    }
+}
+
+template <typename Tag, typename OutTag, int D, bool RAB, bool MASK>
+constexpr auto paged_direct_kernel() -> void (*)(const FwdArgs)
+{
+    if constexpr ((D == 64 || D == 128 || D == 256) && !RAB && !MASK) {
+        return hstu_fwd_kernel<Tag, OutTag, D, RAB, MASK, false, true, true, true>;
+    } else {
+        return nullptr;
+    }
+}
+
 }  // namespace hstu
 
 #define HSTU_VARIANT(tag, tagname, D, RAB, MASK)                                              \
@@ -51,7 +72,9 @@ constexpr auto paged_kernel() -> void (*)(const FwdArgs)
      hstu::split_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(),                                      \
      hstu::paged_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(), D, 256, hstu::fwd_wgs_per_cu(D, RAB, MASK),  \
      hstu::hstu_fwd_kernel<hstu::tag, hstu::tag, D, RAB, MASK, false, false, false, true>,          \
-     "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_direct"}
+     "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_direct",                               \
+     hstu::split_direct_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(),                               \
+     hstu::paged_direct_kernel<hstu::tag, hstu::tag, D, RAB, MASK>()}
 #define HSTU_DIMS(tag, tagname, RAB, MASK)                                                           \
     {HSTU_VARIANT(tag, tagname, 32, RAB, MASK), HSTU_VARIANT(tag, tagname, 64, RAB, MASK), \
      HSTU_VARIANT(tag, tagname, 128, RAB, MASK), HSTU_VARIANT(tag, tagname, 256, RAB, MASK)}

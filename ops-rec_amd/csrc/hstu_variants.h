@@ -22,6 +22,8 @@ struct Variant {
     int persistent_wgs_per_cu;  // > 0: persistent kernel, this many workgroups per CU; 0: one workgroup per tile
     void (*kernel_direct)(const FwdArgs);  // the persistent kernel without a list, a workgroup per slot, for the shortest lists
     const char* name_direct;
+    void (*kernel_split_direct)(const FwdArgs);  // the split variant without a list, all items cut alike; may be nullptr
+    void (*kernel_paged_direct)(const FwdArgs);  // the paged one likewise; may be nullptr
 };
 
 // the forward kernel for short work lists (hstu_fwd_short_kernel.hip.h): one workgroup of `threads` per
