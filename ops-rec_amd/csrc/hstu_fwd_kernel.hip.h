@@ -785,13 +785,23 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         k_src[i] = (kc * EPC16 < a.d_qk) ? static_cast<uint32_t>(r) * k_stride + kc * 16u : kOutOfRange;
         v_src[i] = (vc * EPC16 < a.d_v) ? static_cast<uint32_t>(r) * v_stride + vc * 16u : kOutOfRange;
     }
-    // LDS read offsets relative to a sub-tile, in bytes.  In the bias variants each goes through empty assembly once per time step (kFreshOffsets):
-    // what the slots add to it is then worked out where it is read, as the constant part of the address.  Left alone, the compiler keeps the sums for
-    // all four slots in registers, 36 of them at the slot 128, where the bias variants then had 29 values per item in scratch memory.  They have
-    // none now: one wave of items, which pays the reads of the start of an item in full, gains most.  Measured, us: 64 x 4 heads of 300..600 keys
-    // 57.1 -> 50.6, 16 x 4 of 512..2048 67.1 -> 62.2, 16 x 8 of 1024..4096 406 -> 400; at the slot 64, 128 x 4 of 100..300 29.8 -> 25.6, else level.
-    // Not the slot 256, whose slots take more than the 64 KB that the constant part reaches (107.3 -> 108.5), nor without a bias, where nothing is in scratch (level).
+    // LDS read offsets relative to a sub-tile (in elements; fp8 and kFreshOffsets: in bytes).  In the bias variants each goes through empty assembly
+    // once per time step (kFreshOffsets): what the slots add to it is then worked out where it is read, as the constant part of the address.  Left
+    // alone, the compiler keeps the sums for all four slots in registers, 36 of them at the slot 128, where the bias variants then had 29 values per
+    // item in scratch memory.  They have none now: one wave of items, which pays the reads of the start of an item in full, gains most.  Measured, us:
+    // 64 x 4 heads of 300..600 keys 57.1 -> 50.6, 16 x 4 of 512..2048 67.1 -> 62.2, 16 x 8 of 1024..4096 406 -> 400; at the slot 64, 128 x 4 of 100..300
+    // 29.8 -> 25.6, else level.  Not the slot 256, whose slots take more than the 64 KB that the constant part reaches (107.3 -> 108.5), nor without a
+    // bias, where nothing is in scratch (level).  Those keep offsets in elements too: in bytes the launches without a list of the slot 256 took 1.5 to 3 %
+    // longer (3 x 4 heads on 2, d 192, 321..451 keys 20.2 -> 20.9; with a bias, 4 x 4 on 2, d 256, 312..520 keys 24.9 -> 25.5).
     constexpr bool kFreshOffsets = HAS_RAB && !F8 && D <= 128;
+    constexpr int kOffsetUnit = kFreshOffsets ? 2 : 1;
+    auto at_offset = [](const uint16_t* tile, int off) {
+        if constexpr (F8 || kFreshOffsets) {
+            return reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(tile) + off);
+        } else {
+            return tile + off;
+        }
+    };
     constexpr int KREADS = F8 ? KSTEPS / 2 : KSTEPS;  // fp8: one 16-byte read feeds two MFMA steps
     int k_lane_off[KREADS];
     int v_lane_off[MTILES];
@@ -814,13 +824,13 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     } else {
 #pragma unroll
         for (int js = 0; js < KREADS; ++js) {
-            k_lane_off[js] = (ln * D + k_chunk_swizzle<D>(ln, 2 * js + lh) * 8) * 2;
+            k_lane_off[js] = (ln * D + k_chunk_swizzle<D>(ln, 2 * js + lh) * 8) * kOffsetUnit;
         }
         const int vr0 = 4 * lh + ((lane & 15) >> 2);
 #pragma unroll
         for (int mt = 0; mt < MTILES; ++mt) {
             const int col = 32 * mt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-            v_lane_off[mt] = (vr0 * D + v_chunk_swizzle<D>(vr0, col >> 3) * 8 + (col & 7)) * 2;
+            v_lane_off[mt] = (vr0 * D + v_chunk_swizzle<D>(vr0, col >> 3) * 8 + (col & 7)) * kOffsetUnit;
         }
     }
     float c_exp = a.c_exp;
@@ -1776,13 +1786,13 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             //     to the packed P^T, and only in the steps whose sub-tile is not fully visible.
             // K operand read r (16-bit inputs: MFMA step r; fp8: steps 2r and 2r+1) and V^T operand of chunk c
             auto read_k = [&](int r) -> u32x4_t {
-                return *reinterpret_cast<const u32x4_t*>(reinterpret_cast<const uint8_t*>(kt) + k_lane_off[r]);
+                return *reinterpret_cast<const u32x4_t*>(at_offset(kt, k_lane_off[r]));
             };
             // chunk c of the PV block = key half c % 2 of output tile c / 2: two consecutive MFMAs accumulate into the
             // same registers
             auto read_v = [&](int c) -> u32x4_t {
                 const int j2 = c % 2, mt = c / 2;
-                const uint16_t* p = reinterpret_cast<const uint16_t*>(reinterpret_cast<const uint8_t*>(vt) + v_lane_off[mt]) + 16 * j2 * D;
+                const uint16_t* p = at_offset(vt, v_lane_off[mt]) + 16 * j2 * D;
                 const u32x2_t lo = lds_read_tr16_b64(p);
                 const u32x2_t hi = lds_read_tr16_b64(p + 8 * D);
                 const u32x4_t r = {lo[0], lo[1], hi[0], hi[1]};
