@@ -1239,14 +1239,25 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         }
         const int sub_shift = a.page_shift - 5;  // sub-tiles per page, as a shift
         const int last_pid = static_cast<int>(a.num_pages - 1);
-        // (The low word of the entry alone, whatever its type, and clamped where it is used, a step on: a branch on the type, or the clamp
-        // here, makes the step wait for the load it has just sent.  With that and the requests without lane masks below 32 x 4 heads, d 128,
-        // 64..96 rows on 3072 keys 50 -> 47 us, on 4096 65 -> 63; 44.5 and 57.5 with the rows in order.)
+        auto clamp_page = [&](int pid) -> int {
+            pid = pid < last_pid ? pid : last_pid;
+            return pid < 0 ? 0 : pid;
+        };
+        // (kPageLate: the low word of the entry alone, whatever its type, and clamped where it is used, a step on: a branch on the type, or the clamp
+        // here, makes the step wait for the load it has just sent.  With that and the requests without lane masks below, without a list 32 x 4 heads, d
+        // 128, 64..96 rows on 3072 keys 50 -> 47 us, on 4096 65 -> 63; 44.5 and 57.5 with the rows in order.  With a list, 64..96 rows: d 256, 100 x 4 on
+        // 1500..2500 keys 239 -> 214, 75 x 4 on 2000..4000 350 -> 309, 300 x 4 on 100..300 133 -> 127; d 128, 150 x 4 on 2000..4000 283 -> 272; but d 64,
+        // 291 x 2 on 73 24.8 -> 25.8 and 600 x 4 on 100..300 83.8 -> 85.1 (200 x 4 on 1500..2500 154 -> 152).)
+        constexpr bool kPageLate = DIRECT || D > 64;
         auto page_of = [&](int x) -> int {
             int idx = page_first + (x >> sub_shift);
             idx = idx < page_hi ? idx : page_hi;
-            typedef const __attribute__((address_space(4))) int* cint_t;
-            return *(cint_t)(reinterpret_cast<uintptr_t>(a.page_ids) + (static_cast<uint64_t>(static_cast<uint32_t>(idx)) << (2 + a.idx64)));
+            if constexpr (kPageLate) {
+                typedef const __attribute__((address_space(4))) int* cint_t;
+                return *(cint_t)(reinterpret_cast<uintptr_t>(a.page_ids) + (static_cast<uint64_t>(static_cast<uint32_t>(idx)) << (2 + a.idx64)));
+            } else {
+                return clamp_page(static_cast<int>(load_index_uniform(a.page_ids, idx, a.idx64)));
+            }
         };
 
         // ---- buffer descriptors sized to this sequence / head ----
@@ -1317,8 +1328,9 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         // come from the page, the others from the new rows; a request past the end moves nothing.
         auto request_paged = [&](uint16_t* dst, const __amdgpu_buffer_rsrc_t new_rsrc, const uint32_t (&src)[LPW], int x,
                                  int pid, int kv) {
-            pid = pid < last_pid ? pid : last_pid;
-            pid = pid < 0 ? 0 : pid;
+            if constexpr (kPageLate) {
+                pid = clamp_page(pid);
+            }
             const bool live = x < x_end;
             const int bnd = live ? n_cached - x * 32 : 0;
             const int rows_c = bnd < 0 ? 0 : (bnd > 32 ? 32 : bnd);
@@ -1329,7 +1341,7 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
             // offset of sub-tile row 0 among the new rows (negative, as a wrapped unsigned, while bnd > 0: the
             // lanes that use it have rows >= bnd, which brings the sum back into range)
             const uint32_t new_base = live ? static_cast<uint32_t>(x * 32 - n_cached) * k_stride : kPastEnd;
-            if (bnd >= 32) {  // (nearly all of them: no lane masks)
+            if (kPageLate && bnd >= 32) {  // (nearly all of them: no lane masks)
 #pragma unroll
                 for (int i = 0; i < LPW; ++i) {
                     load_to_lds_b128(page_rsrc, dst + (wave * LPW + i) * 512, src[i]);
