@@ -413,7 +413,8 @@ struct U32Quad {
 // past the end of their sequence leave at once.  That spares every workgroup the histogram, the list and the hand-over of
 // its item through LDS, 1.5 .. 4 us ahead of its first request.  (A variant of its own: as a branch of the plain one it cost
 // that 1 us.)  With SPLIT every item is cut into the same number of parts (FwdArgs::slot_parts), a workgroup each: for items
-// whose sweeps are about equally long, a few query rows on a history.
+// whose sweeps are about equally long, a few query rows on a history.  There it is (part, pair) that is padded to a multiple of 8: what meets on an
+// XCD is the tiles that read the same keys, and one pair alone has work for all eight.
 template <typename Tag, typename OutTag, int D, bool HAS_RAB, bool HAS_MASK, bool QUEUES = false, bool SPLIT = false,
           bool PAGED = false, bool DIRECT = false>
 __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hstu_fwd_kernel(const FwdArgs a)
@@ -1104,25 +1105,23 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
         int part = 0, n_parts = 1, split_item = 0, split_buffer = 0;  // (split items) their arrival counter and first partial output
         if constexpr (DIRECT) {
             const int pairs = a.n_batch * a.n_heads_k;
-            const int pairs_pad = (pairs + 7) & ~7;
             if constexpr (SPLIT) {
                 n_parts = a.slot_parts;
             }
-            const int per_level = pairs_pad * a.head_ratio * n_parts;
+            const int pairs_pad = (pairs * n_parts + 7) & ~7;  // (split: every part of every pair)
+            const int per_level = pairs_pad * a.head_ratio;
             const int lvl = static_cast<int>(blockIdx.x) / per_level;
             const int rest = static_cast<int>(blockIdx.x) - lvl * per_level;
-            const int group = rest / pairs_pad;
-            const int pair = rest - group * pairs_pad;
-            if (pair >= pairs) {
+            const int in_group = rest / pairs_pad;
+            int pair = rest - in_group * pairs_pad;
+            if (pair >= pairs * n_parts) {
                 break;
             }
-            const int in_group = SPLIT ? group / n_parts : group;
-            part = group - in_group * n_parts;
             if constexpr (SPLIT) {
+                part = pair / pairs;
+                pair -= part * pairs;
                 split_item = (lvl * a.head_ratio + in_group) * pairs + pair;
                 split_buffer = split_item * n_parts;
-            } else {
-                part = 0;
             }
             qt = tile_of_level(lvl);
             b = pair / a.n_heads_k;

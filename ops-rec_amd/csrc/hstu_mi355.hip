@@ -405,10 +405,10 @@ int wgs_per_cu(const Variant* var, const hstu_jagged_fwd_params* p)
 }
 
 // slots of a launch without a list: pairs padded to a multiple of 8 (hstu_fwd_kernel.hip.h)
-int64_t direct_slots(const hstu_jagged_fwd_params* p)
+int64_t direct_slots(const hstu_jagged_fwd_params* p, int64_t parts = 1)
 {
     const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
-    const int64_t pairs_pad = ((p->n_offsets - 1) * p->num_heads_k + 7) & ~int64_t{7};
+    const int64_t pairs_pad = ((p->n_offsets - 1) * p->num_heads_k * parts + 7) & ~int64_t{7};
     return n_qtiles * pairs_pad * (p->num_heads_q / p->num_heads_k);
 }
 
@@ -566,7 +566,9 @@ uint64_t split_part_bytes(const Variant* var) { return static_cast<uint64_t>(hst
 // List -> slots, with page ids that a step does not wait for (us, d 128, 64..96 rows): paged 32 x 4 on 512 keys 30.5 -> 23.1, on 2048..4096 61.0 -> 52.0, 16 x
 // 4 on 2048 50.7 -> 35.7, 64 x 4 on 4096 126 -> 116; 32 x 4, 80 rows on 3000 keys 53.4 -> 42.1 (4.7 TB/s), 16 x 4, 200 on 3000 51.8 -> 42.6, d 64, 32 x
 // 4 on 3000 43.1 -> 30.2.  The slot 256, whose items were not cut before: paged 4 x 4 on 4096 186 -> 46, 32 x 4 196 -> 120, 64 x 4 (no room for
-// parts) 236 -> 212; 16 x 4, 80 rows on 2128 71 -> 42, 2 x 4, d 192, 500 on 3000..4000 117 -> 45.  No call of 110 was slower.
+// parts) 236 -> 212; 16 x 4, 80 rows on 2128 71 -> 42, 2 x 4, d 192, 500 on 3000..4000 117 -> 45.
+// (Part, pair) slots dealt to the XCDs, against pairs dealt: 25 x 1, 298 rows on 3266..6294 keys 53.3 -> 39.6 (48.1 with the list: one XCD had 72 of its
+// 64 workgroups' room asked for), 2 x 4 on 2, d 64, 500 on 5000..6000 30.7 -> 24.3; 33 x 1, 100..200 on 3000..6000 37.2 -> 39.1 (list 49.0).
 int slot_parts(const Variant* var, const hstu_jagged_fwd_params* p, bool paged, int64_t resident, int64_t room)
 {
     if ((paged ? var->kernel_paged_direct : var->kernel_split_direct) == nullptr || p->num_context != nullptr) {
@@ -576,12 +578,15 @@ int slot_parts(const Variant* var, const hstu_jagged_fwd_params* p, bool paged, 
     if (n_qtiles > 1 && 2 * p->max_seq_len_q > p->max_seq_len_k) {
         return 0;
     }
-    const int64_t items = n_qtiles * (p->n_offsets - 1) * p->num_heads_q;
-    if (items > resident) {
+    // ((part, pair) slots go over the XCDs in turn, a workgroup per query tile and query head of the pair each: what fits on the fullest XCD)
+    const int64_t pairs = (p->n_offsets - 1) * p->num_heads_k;
+    const int64_t tiles = n_qtiles * (p->num_heads_q / p->num_heads_k);
+    const int64_t slots = resident / 8 / tiles * 8;
+    if (pairs > slots) {
         return 0;
     }
     const int64_t steps = (p->max_seq_len_k + 31) / 32;
-    const int64_t parts = std::min({resident / items, room / items, steps / 8, int64_t{8}});
+    const int64_t parts = std::min({slots / pairs, room / (pairs * tiles), steps / 8, int64_t{8}});
     return static_cast<int>(parts >= 2 ? parts : (paged ? 1 : 0));
 }
 
@@ -2010,7 +2015,7 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
             a.slot_parts = slot_parts(var, p, paged != nullptr, hstu::split_grid(resident), a.ws != nullptr ? a.ws_parts : 0);
             if (a.slot_parts > 0) {
                 kernel = paged != nullptr ? var->kernel_paged_direct : var->kernel_split_direct;
-                n_blocks = direct_slots(p) * a.slot_parts;
+                n_blocks = direct_slots(p, a.slot_parts);
             }
         }
         if (a.counters == nullptr && takes_direct_list(var, p, static_cast<int64_t>(cus) * wgs_per_cu(var, p))) {

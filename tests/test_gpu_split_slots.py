@@ -31,6 +31,8 @@ CASES = {  # rows and keys of each sequence
     "slot 256": (dict(heads=2, dim=256), [1, 128, 77], [2500, 4000, 2049], FP),
     "slot 256, odd dims": (dict(heads=4, heads_k=1, dim=200, dim_v=144), [200, 129, 256], [2500, 2100, 2300], BF),
     "64-bit offsets": (dict(heads=2, dim=128, index_dtype=torch.int64), [64, 100, 12], [2500, 2100, 2300], BF),
+    "one pair": (dict(heads=1, dim=128), [200], [4000], BF),
+    "slots not in eights": (dict(heads=5, dim=128), [128, 100, 1, 128, 127], [5000, 3000, 2049, 100, 4100], FP),
     "no mask": (dict(heads=2, dim=64), [64, 100, 12], [2500, 2100, 2300], BF),
 }
 
