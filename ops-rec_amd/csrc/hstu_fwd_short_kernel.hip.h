@@ -17,6 +17,11 @@
 //   * slot -> workgroup so that all tiles that read the K / V rows of one (sequence, K/V head) run on one XCD
 //     (workgroup i runs on XCD i mod 8) and find those rows in that XCD's L2.
 //
+// At the head-dim slot 64 a sub-tile is 4 KiB: four wavefronts bring its K rows and four its V rows, 80 registers let three workgroups share a
+// CU.  What it gains there is mostly the start (no list, two trips to memory): bf16, us, the persistent kernel's variants -> this one, 16 x 4 heads of
+// 128 rows 8.3 -> 6.1, 64 x 4 of 500 30.1 -> 19.6, 32 x 4 of 1024 41.0 -> 28.7; sides of the rule: hstu_mi355.hip.  Steps of 64 keys (half the
+// barriers, 100 registers, two workgroups per CU) took longer on all but 20 of 220 shapes: 64 x 4 of 500 24.5, 16 x 4 of 501 rows on 1000 18.0 -> 19.0.
+//
 // It pays twice the LDS operand traffic per product (an A operand of 1 KiB feeds a 16-row MFMA instead of a 32-row
 // one), which is why long lists stay on the persistent kernel.  Same arithmetic per element as that kernel:
 // p = s / (1 + exp2(-alpha log2e s)) rounded to the input type, alpha * silu_scale applied once to the fp32 output,
@@ -34,7 +39,7 @@ namespace hstu {
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
 
 constexpr int kShortWaveM = 16;     // query rows per wavefront
-constexpr int kShortWavesPerSimd = 4;  // two workgroups per CU
+constexpr int short_waves_per_simd(int d) { return d == 64 ? 6 : 4; }  // three workgroups per CU at the slot 64, two at 128
 
 template <typename Tag>
 __device__ __forceinline__ f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c);
@@ -57,7 +62,10 @@ __device__ __forceinline__ f32x4_t mfma16<f16_tag>(u32x4_t a, u32x4_t b, f32x4_t
 template <int D>
 __device__ __forceinline__ int v16_chunk_swizzle(int row, int chunk)
 {
-    static_assert(D == 128, "built for the head-dim slot 128");
+    static_assert(D == 128 || D == 64, "built for the head-dim slots 64 and 128");
+    if constexpr (D == 64) {
+        return chunk ^ (((row >> 1) & 3) << 1);  // (two rows per 256 bytes: the 32-byte pieces XOR-ed with the pair of rows)
+    }
     return chunk ^ (((row & 3) << 2) | (((row >> 2) & 1) << 1));
 }
 
@@ -131,18 +139,19 @@ __device__ __forceinline__ void rab_wait(u32x2_t& lo, u32x2_t& hi)
 }
 
 template <typename Tag, int D, bool HAS_RAB = false>
-__global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_short_kernel(const FwdArgs a)
+__global__ __launch_bounds__(kShortThreads, short_waves_per_simd(D)) void hstu_fwd_short_kernel(const FwdArgs a)
 {
-    static_assert(D == 128, "built for the head-dim slot 128");
     constexpr int SUB_ELEMS = 32 * D;       // one 32-key sub-tile, in 16-bit units
     constexpr int CPR = D / 8;              // 16-byte chunks per row
     constexpr int KSTEPS = D / 32;          // MFMA steps over the head dim (QK product)
     constexpr int MTILES = D / 16;          // 16-wide output tiles over the head dim (PV product)
-    constexpr int SUB_KIB = 32 * D * 2 / 1024;  // 1 KiB load instructions per sub-tile: one per wavefront
-    static_assert(SUB_KIB == kShortThreads / 64, "one load instruction per wavefront and sub-tile");
-    // vmcnt(4): the tile requests of two steps may be open; with a bias the two bias requests of a step come on top
-    // (steps t - 1 and t: five pairs since the tile requests of sub-tile t + 1)
-    constexpr int kWaitTiles = ((HAS_RAB ? 10 : 4) & 15) | (7 << 4) | (15 << 8);
+    constexpr int SUB_KIB = 32 * D * 2 / 1024;  // 1 KiB load instructions per sub-tile
+    // load instructions per wavefront and step: one of K and one of V, or (slot 64) wavefronts 0 .. 3 bring K and 4 .. 7 V
+    constexpr int kRequests = 2 * SUB_KIB / (kShortThreads / 64);
+    static_assert(kRequests * (kShortThreads / 64) == 2 * SUB_KIB && (kRequests == 1 || kRequests == 2), "dealt evenly");
+    // the tile requests of two steps may be open; with a bias the two bias requests of a step come on top (of steps t - 2, t - 1 and t
+    // since the tile requests of sub-tile t + 1)
+    constexpr int kWaitTiles = ((HAS_RAB ? 2 * kRequests + 6 : 2 * kRequests) & 15) | (7 << 4) | (15 << 8);
     constexpr uint32_t kPastEnd = 0x40000000u;
 
     // four slots each for K and V sub-tiles (sub-tile x in slot x mod 4); separate arrays so that the compiler can
@@ -260,8 +269,9 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
         // K / V sub-tile streaming: the load instruction of this wavefront fills LDS bytes [wave * 1024, + 1024) of a
         // slot; the per-lane source offset is fixed, only the base moves
         uint32_t k_src, v_src;
+        const int kv_wave = kRequests == 2 ? wave : wave & (SUB_KIB - 1);  // the wavefront's KiB of a sub-tile
         {
-            const int piece = wave * 64 + lane;  // 16-byte piece within the sub-tile
+            const int piece = kv_wave * 64 + lane;  // 16-byte piece within the sub-tile
             const int r = piece / CPR;
             const int pc = piece % CPR;
             const int kc = k_chunk_swizzle<D>(r, pc);  // XOR swizzles are their own inverse
@@ -269,6 +279,11 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
             k_src = (kc * 8 < a.d_qk) ? static_cast<uint32_t>(r) * k_stride + kc * 16u : kOutOfRange;
             v_src = (vc * 8 < a.d_v) ? static_cast<uint32_t>(r) * v_stride + vc * 16u : kOutOfRange;
         }
+        // (kRequests == 1) the tensor that this wavefront brings
+        const bool brings_k = kRequests == 2 || wave < SUB_KIB;
+        const u32x4_t kv_rsrc = brings_k ? k_rsrc : v_rsrc;
+        const uint32_t kv_src = brings_k ? k_src : v_src;
+        const uint32_t kv_stride = brings_k ? k_stride : v_stride;
         auto k_slot = [&](auto ic) -> uint16_t* {
             constexpr int I = decltype(ic)::value & 3;
             if constexpr (I == 0) {
@@ -296,8 +311,13 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
         // requests past the last sub-tile move nothing but keep the number of requests per step constant
         auto request = [&](auto ic, int x) {
             const uint32_t past = (x < n_sub) ? 0u : kPastEnd;
-            request_to_lds_b128(k_rsrc, lds_address(k_slot(ic)) + wave * 1024u, k_src + static_cast<uint32_t>(x * 32) * k_stride + past);
-            request_to_lds_b128(v_rsrc, lds_address(v_slot(ic)) + wave * 1024u, v_src + static_cast<uint32_t>(x * 32) * v_stride + past);
+            if constexpr (kRequests == 2) {
+                request_to_lds_b128(k_rsrc, lds_address(k_slot(ic)) + wave * 1024u, k_src + static_cast<uint32_t>(x * 32) * k_stride + past);
+                request_to_lds_b128(v_rsrc, lds_address(v_slot(ic)) + wave * 1024u, v_src + static_cast<uint32_t>(x * 32) * v_stride + past);
+            } else {
+                request_to_lds_b128(kv_rsrc, (brings_k ? lds_address(k_slot(ic)) : lds_address(v_slot(ic))) + kv_wave * 1024u,
+                                    kv_src + static_cast<uint32_t>(x * 32) * kv_stride + past);
+            }
         };
         typedef std::integral_constant<int, 0> ic0_t;
         typedef std::integral_constant<int, 1> ic1_t;
@@ -408,11 +428,11 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
                     s1 = mfma16<Tag>(kb, qf[js], s1);
                 }
                 if constexpr (HAS_RAB) {
-                    // the bias of this sub-tile is in: asked for two steps ago, and since then the tile requests and the
+                    // the bias of this sub-tile is in: asked for two steps ago, and since then the tile requests and the two
                     // bias requests of one step and the tile requests of this one have gone out
                     u32x2_t& lo = (S & 1) ? rab_lo1 : rab_lo0;
                     u32x2_t& hi = (S & 1) ? rab_hi1 : rab_hi0;
-                    rab_wait<6>(lo, hi);
+                    rab_wait<2 * kRequests + 2>(lo, hi);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         s0[e] += (e & 1) ? hi_to_float<Tag>(lo[e >> 1]) : lo_to_float<Tag>(lo[e >> 1]);
@@ -508,7 +528,7 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
             // slots) and everybody is done reading before anybody writes a slot
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
-            // the wavefront's 16 rows pass through 4 KiB of LDS of its own (16-byte chunks XOR-ed with the row) and
+            // the wavefront's 16 rows pass through 4 (2) KiB of LDS of its own (16-byte chunks XOR-ed with the row) and
             // leave 16 bytes per lane, whole lines per instruction
             uint16_t* const slot_of_wave = (wave & 3) == 0 ? s_k0 : ((wave & 3) == 1 ? s_k1 : ((wave & 3) == 2 ? s_k2 : s_k3));
             uint16_t* const stage = slot_of_wave + (wave >> 2) * (16 * D);
@@ -517,7 +537,7 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
                 u32x2_t w;
                 w[0] = pack2<Tag>(o_acc[mt][0] * c_out, o_acc[mt][1] * c_out);
                 w[1] = pack2<Tag>(o_acc[mt][2] * c_out, o_acc[mt][3] * c_out);
-                const int chunk = (2 * mt + (g_e >> 1)) ^ n_e;
+                const int chunk = (2 * mt + (g_e >> 1)) ^ (n_e & (CPR - 1));
                 *reinterpret_cast<u32x2_t*>(stage + n_e * D + chunk * 8 + 4 * (g_e & 1)) = w;
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -530,7 +550,7 @@ __global__ __launch_bounds__(kShortThreads, kShortWavesPerSimd) void hstu_fwd_sh
 #pragma unroll
             for (int i = 0; i < kShortWaveM / RPI; ++i) {
                 const int r = i * RPI + rr;
-                const u32x4_t piece = *reinterpret_cast<const u32x4_t*>(stage + r * D + (cc ^ r) * 8);
+                const u32x4_t piece = *reinterpret_cast<const u32x4_t*>(stage + r * D + (cc ^ (r & (CPR - 1))) * 8);
                 const uint32_t off = (cc * 8 < a.d_v) ? static_cast<uint32_t>(wr0 + r) * o_stride + cc * 16u : kOutOfRange;
                 __builtin_amdgcn_raw_buffer_store_b128(piece, o_rsrc, static_cast<int>(off), 0, kNonTemporal);
             }

@@ -1,4 +1,4 @@
-// kernels for short work lists / short rows (16-bit inputs, head-dim slot 128, no custom mask): the forward (with and
+// kernels for short work lists / short rows (16-bit inputs, head-dim slots 64 and 128, no custom mask): the forward (with and
 // without attn_bias), the forward and the backward for batches of tiny sequences, the backward for sequences of few query
 // rows, and the backward's query-tile kernel (no bias)
 #include "hstu_bwd_dq_short_kernel.hip.h"
@@ -11,14 +11,14 @@
 
 namespace hstu {
 namespace {
-const ShortVariant kTable[4] = {
-    {"hstu_fwd_bf16_d128_short", hstu_fwd_short_kernel<bf16_tag, 128>},
-    {"hstu_fwd_f16_d128_short", hstu_fwd_short_kernel<f16_tag, 128>},
-    {"hstu_fwd_bf16_d128_rab_short", hstu_fwd_short_kernel<bf16_tag, 128, true>},
-    {"hstu_fwd_f16_d128_rab_short", hstu_fwd_short_kernel<f16_tag, 128, true>},
+#define HSTU_SHORT(tag, tagname, D) {"hstu_fwd_" tagname "_d" #D "_short", hstu_fwd_short_kernel<tag, D>}
+#define HSTU_SHORT_RAB(tag, tagname, D) {"hstu_fwd_" tagname "_d" #D "_rab_short", hstu_fwd_short_kernel<tag, D, true>}
+const ShortVariant kTable[2][4] = {
+    {HSTU_SHORT(bf16_tag, "bf16", 64), HSTU_SHORT(f16_tag, "f16", 64), HSTU_SHORT_RAB(bf16_tag, "bf16", 64), HSTU_SHORT_RAB(f16_tag, "f16", 64)},
+    {HSTU_SHORT(bf16_tag, "bf16", 128), HSTU_SHORT(f16_tag, "f16", 128), HSTU_SHORT_RAB(bf16_tag, "bf16", 128), HSTU_SHORT_RAB(f16_tag, "f16", 128)},
 };
 }
-const ShortVariant* fwd_variants_short() { return kTable; }
+const ShortVariant (*fwd_variants_short())[4] { return kTable; }
 
 namespace {
 #define HSTU_TINY(tag, tagname, D, R) {"hstu_fwd_" tagname "_d" #D "_tiny" #R, hstu_fwd_tiny_kernel<tag, D, R>}

@@ -325,15 +325,40 @@ const hstu::ShortVariant* one_item_variant(const Variant* var, const hstu_jagged
     return few_rows_variant(var, p);
 }
 
-// The kernel for short work lists (hstu_fwd_short_kernel.hip.h) takes 16-bit inputs at the head-dim slot 128 without
-// bias or custom mask.  It is the faster one while the list -- at most n_blocks entries -- is a few items per
+// The kernel for short work lists at the head-dim slot 64, where three workgroups share a compute unit.  Its steps are no shorter than the
+// persistent kernel's (0.43 us per 32 keys alone on a compute unit, 0.3 there), but it begins 4 to 5 us sooner.  Measured, us, the
+// other variants -> this kernel, without a bias:
+//   up to 1024 keys most of 250 shapes faster, 1.02 to 1.5 x: 32 x 4 heads of 60..200 rows 9.0 -> 7.1, 16 x 4 of 501 rows 14.4 -> 11.1, 64 x 4 of 500
+//   30.1 -> 19.6, 32 x 4 of 1024 41.0 -> 28.7, 256..1024 26.9 -> 25.7, 256 x 4 of 256..512 74 -> 54, 501 rows on 1000 16 x 4 20.0 -> 18.2, 64 x 4
+//   56 -> 44; but where few slots have many keys each, the split list shares the keys out: 4 x 4 of 100..300 rows on 700 keys (48 slots) 14.8 -> 13.4,
+//   on 1000 15.0 -> 17.5, 1 x 4 of 70 on 1000 12.9 -> 17.2 (64 slots are past that: 16 x 4 of 70 on 1000 17.6 -> 17.4);
+//   longer keys go either way: 16 x 4 of 2048 60 -> 51, 512..2048 39 -> 46, 16 x 4 of 501 on 1200..1400 24.1 -> 23.2, 16 x 4 of 1024..4096 97 -> 122.
+// With an attn_bias, whose rows it reads 32 bytes at a time: 256 x 4 of 60..200 39 -> 28, 64 x 4 of 250 13.8 -> 13.5, 1024 x 2 of 100..250 86 -> 77
+// (4096 slots), but 1000 x 4 of 100..256 (8000) 167 -> 180; up to a slot per compute unit on 512 keys, 16 x 4 of 500 16.4 -> 13.0; with two it is even (32 x 4 of 256..512 17.1 -> 18.3, of 500 18.2 -> 16.1), and
+// longer rows lose (16 x 4 of 256..1024 23.7 -> 29.4).
+bool short_at_slot_64(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus)
+{
+    if (p->attn_bias != nullptr) {
+        return (p->max_seq_len_k <= 256 && n_blocks <= 16 * cus) || (p->max_seq_len_k <= 512 && n_blocks <= cus);
+    }
+    // Not over more K / V rows than the caches hold, which the queues keep to one XCD pair by pair (512 x 4 of 1024 481 -> 579, 256..1024, 335 MB, even,
+    // 512 x 4 of 500 on 1000 340 -> 410; 256 x 4 of 1024, 268 MB, 243 -> 236), nor where most slots of the grid are empty (128 x 8 of 8..1000, 233 on
+    // average, 3.4 slots to an item 65 -> 66; 64 x 4 of 8..1024, 1.9 to an item 39 -> 33).
+    const int64_t kv_bytes = p->total_k * p->num_heads_k * (p->head_dim_qk + p->head_dim_v) * 2;
+    const int64_t items = (p->total_q + 64 * (p->n_offsets - 1)) * p->num_heads_q / hstu::kBlockM;  // (by the mean length)
+    const bool history = p->total_k >= 2 * p->total_q;
+    return p->max_seq_len_k <= (history && n_blocks < 64 ? 704 : 1024) && kv_bytes <= (256LL << 20) && n_blocks <= 3 * items;
+}
+
+// The kernel for short work lists (hstu_fwd_short_kernel.hip.h) takes 16-bit inputs at the head-dim slots 64 (rule above) and 128
+// without custom mask.  It is the faster one while the list -- at most n_blocks entries -- is a few items per
 // workgroup the persistent kernel would keep resident: there a launch lasts as long as its longest item, which the
 // short kernel's narrower wavefronts finish in about half the time; on longer lists the persistent kernel's
 // steady-state rate wins.  HSTU_MI355_SHORT in the environment overrides the rule: 0 = never, 1 = whenever the
 // kernel can take the call.
 const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool have_counters = true)
 {
-    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || p->mask_type == HSTU_MASK_CUSTOM || var->d_pad != 128 ||
+    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || p->mask_type == HSTU_MASK_CUSTOM || (var->d_pad != 64 && var->d_pad != 128) ||
         var->persistent_wgs_per_cu <= 0 || var->kernel_queues == nullptr) {
         return nullptr;
     }
@@ -347,7 +372,7 @@ const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fw
                  p->max_seq_len_q * p->max_seq_len_k * 2 >= (1LL << 32))) {
         return nullptr;
     }
-    const hstu::ShortVariant* const sv = &hstu::fwd_variants_short()[(bias ? 2 : 0) + (p->dtype == HSTU_DT_BF16 ? 0 : 1)];
+    const hstu::ShortVariant* const sv = &hstu::fwd_variants_short()[var->d_pad == 64 ? 0 : 1][(bias ? 2 : 0) + (p->dtype == HSTU_DT_BF16 ? 0 : 1)];
     const int forced = switches().short_lists;
     if (forced == 0) {
         return nullptr;
@@ -368,6 +393,9 @@ const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fw
     const int64_t resident = static_cast<int64_t>(cus) * var->persistent_wgs_per_cu;
     const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
     const int64_t n_blocks = n_qtiles * (p->n_offsets - 1) * p->num_heads_q;
+    if (var->d_pad == 64) {
+        return short_at_slot_64(p, n_blocks, cus) ? sv : nullptr;
+    }
     if (bias) {
         // with an attn_bias: keys up to 1024 and at most one slot per resident workgroup -- 8 x 4 of 1024 36.6 -> 27.6 us,
         // 16 x 4 lengths 512..1024 45.0 -> 38.4; two slots per workgroup are even (32 x 4 lengths 256..1024, 64 x 4 of 512)
