@@ -336,21 +336,40 @@ const hstu::ShortVariant* one_item_variant(const Variant* var, const hstu_jagged
 // With an attn_bias, whose rows it reads 32 bytes at a time: 256 x 4 of 60..200 39 -> 28, 64 x 4 of 250 13.8 -> 13.5, 1024 x 2 of 100..250 86 -> 77
 // (4096 slots), but 1000 x 4 of 100..256 (8000) 167 -> 180; up to a slot per compute unit on 512 keys, 16 x 4 of 500 16.4 -> 13.0; with two it is even (32 x 4 of 256..512 17.1 -> 18.3, of 500 18.2 -> 16.1), and
 // longer rows lose (16 x 4 of 256..1024 23.7 -> 29.4).
+//
+// Without a bias, not over more K / V rows than the caches hold, which the queues keep to one XCD pair by pair (512 x 4 of 1024 481 -> 579, 256..1024,
+// 335 MB, even, 512 x 4 of 500 on 1000 340 -> 410; 256 x 4 of 1024, 268 MB, 243 -> 236), nor where most slots of the grid are empty (128 x 8 of 8..1000,
+// 233 on average, 3.4 slots to an item 65 -> 66; 64 x 4 of 8..1024, 1.9 to an item 39 -> 33).
+bool short_fits_caches(const hstu_jagged_fwd_params* p, int64_t n_blocks)
+{
+    const int64_t kv_bytes = p->total_k * p->num_heads_k * (p->head_dim_qk + p->head_dim_v) * 2;
+    const int64_t items = (p->total_q + 64 * (p->n_offsets - 1)) * p->num_heads_q / hstu::kBlockM;  // (by the mean length)
+    return kv_bytes <= (256LL << 20) && n_blocks <= 3 * items;
+}
 bool short_at_slot_64(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus)
 {
     if (p->attn_bias != nullptr) {
         return (p->max_seq_len_k <= 256 && n_blocks <= 16 * cus) || (p->max_seq_len_k <= 512 && n_blocks <= cus);
     }
-    // Not over more K / V rows than the caches hold, which the queues keep to one XCD pair by pair (512 x 4 of 1024 481 -> 579, 256..1024, 335 MB, even,
-    // 512 x 4 of 500 on 1000 340 -> 410; 256 x 4 of 1024, 268 MB, 243 -> 236), nor where most slots of the grid are empty (128 x 8 of 8..1000, 233 on
-    // average, 3.4 slots to an item 65 -> 66; 64 x 4 of 8..1024, 1.9 to an item 39 -> 33).
-    const int64_t kv_bytes = p->total_k * p->num_heads_k * (p->head_dim_qk + p->head_dim_v) * 2;
-    const int64_t items = (p->total_q + 64 * (p->n_offsets - 1)) * p->num_heads_q / hstu::kBlockM;  // (by the mean length)
     const bool history = p->total_k >= 2 * p->total_q;
-    return p->max_seq_len_k <= (history && n_blocks < 64 ? 704 : 1024) && kv_bytes <= (256LL << 20) && n_blocks <= 3 * items;
+    return p->max_seq_len_k <= (history && n_blocks < 64 ? 704 : 1024) && short_fits_caches(p, n_blocks);
+}
+// At the slot 32 the kernel of the slot 64 has half its products for nothing and still begins sooner.  Measured, us, as above: up to 512 keys 64 x 4 of
+// 128 7.7 -> 6.3, 16 x 4 of 500 13.1 -> 11.1, 256 x 4 of 256..512 69 -> 51, 512 x 4 of 60..200 54 -> 32; up to 704 in few rounds 16 x 4 of 501 on 700
+// 15.3 -> 13.6; but with four slots per compute unit, which the other kernel has resident at once, 64 x 4 of 500
+// 18.2 -> 18.4 and 64 x 8 of 250 15.6 -> 15.8; longer keys 16 x 4 of 70 on 1000 17.2 -> 17.5, 64 x 4 of 501 on 1000 36.5 -> 38.6, 256 x 4 of 256..1024
+// 106 -> 115.  With a bias: 64 x 4 of 250 (512 slots) 14.1 -> 13.3, 256 x 4 of 250 40.6 -> 45.3, 64 x 8 of 250 (1024) 21 -> 25; 16 x 4 of 500 (256)
+// 17.6 -> 12.9, 16 x 4 of 256..1024 26 -> 29.
+bool short_at_slot_32(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus)
+{
+    if (p->attn_bias != nullptr) {
+        return (p->max_seq_len_k <= 256 && n_blocks <= 2 * cus) || (p->max_seq_len_k <= 512 && n_blocks <= cus);
+    }
+    const bool four_resident = n_blocks > 3 * cus && n_blocks <= 4 * cus && p->max_seq_len_k > 128;
+    return p->max_seq_len_k <= (n_blocks <= 3 * cus ? 704 : 512) && !four_resident && short_fits_caches(p, n_blocks);
 }
 
-// The kernel for short work lists (hstu_fwd_short_kernel.hip.h) takes 16-bit inputs at the head-dim slots 64 (rule above) and 128
+// The kernel for short work lists (hstu_fwd_short_kernel.hip.h) takes 16-bit inputs at the head-dim slots 32, 64 (rules above) and 128
 // without custom mask.  It is the faster one while the list -- at most n_blocks entries -- is a few items per
 // workgroup the persistent kernel would keep resident: there a launch lasts as long as its longest item, which the
 // short kernel's narrower wavefronts finish in about half the time; on longer lists the persistent kernel's
@@ -358,7 +377,7 @@ bool short_at_slot_64(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus
 // kernel can take the call.
 const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fwd_params* p, bool have_counters = true)
 {
-    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || p->mask_type == HSTU_MASK_CUSTOM || (var->d_pad != 64 && var->d_pad != 128) ||
+    if ((p->dtype != HSTU_DT_BF16 && p->dtype != HSTU_DT_FP16) || p->mask_type == HSTU_MASK_CUSTOM || var->d_pad > 128 ||
         var->persistent_wgs_per_cu <= 0 || var->kernel_queues == nullptr) {
         return nullptr;
     }
@@ -372,7 +391,7 @@ const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fw
                  p->max_seq_len_q * p->max_seq_len_k * 2 >= (1LL << 32))) {
         return nullptr;
     }
-    const hstu::ShortVariant* const sv = &hstu::fwd_variants_short()[var->d_pad == 64 ? 0 : 1][(bias ? 2 : 0) + (p->dtype == HSTU_DT_BF16 ? 0 : 1)];
+    const hstu::ShortVariant* const sv = &hstu::fwd_variants_short()[var->d_pad <= 64 ? 0 : 1][(bias ? 2 : 0) + (p->dtype == HSTU_DT_BF16 ? 0 : 1)];
     const int forced = switches().short_lists;
     if (forced == 0) {
         return nullptr;
@@ -393,8 +412,8 @@ const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fw
     const int64_t resident = static_cast<int64_t>(cus) * var->persistent_wgs_per_cu;
     const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
     const int64_t n_blocks = n_qtiles * (p->n_offsets - 1) * p->num_heads_q;
-    if (var->d_pad == 64) {
-        return short_at_slot_64(p, n_blocks, cus) ? sv : nullptr;
+    if (var->d_pad <= 64) {
+        return (var->d_pad == 64 ? short_at_slot_64(p, n_blocks, cus) : short_at_slot_32(p, n_blocks, cus)) ? sv : nullptr;
     }
     if (bias) {
         // with an attn_bias: keys up to 1024 and at most one slot per resident workgroup -- 8 x 4 of 1024 36.6 -> 27.6 us,

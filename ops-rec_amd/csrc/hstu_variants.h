@@ -86,7 +86,7 @@ const Variant (*fwd_variants_f8())[2][2][3];
 const Variant (*fwd_variants_f32())[2][4];
 // forward, 16-bit inputs with head dims in (256, 512], q/k head dim a multiple of 8: [bf16, fp16][rab][custom mask]
 const Variant (*fwd_variants_wide())[2][2];
-// forward for short work lists, 16-bit inputs at the head-dim slots 64 and 128 without custom mask: [slot][bf16, fp16, bf16
+// forward for short work lists, 16-bit inputs at the head-dim slots 64 (32 too) and 128 without custom mask: [slot][bf16, fp16, bf16
 // with attn_bias, fp16 with attn_bias]
 const ShortVariant (*fwd_variants_short())[4];
 // the forward kernel with pinned accumulators (hstu_fwd_pinned_kernel.hip.h): [bf16, f16][slots 128, 256]

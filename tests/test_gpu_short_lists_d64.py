@@ -1,4 +1,4 @@
-"""The forward kernel for short work lists at the head-dim slot 64 (three workgroups of eight 16-row wavefronts per compute unit; four of
+"""The forward kernel for short work lists at the head-dim slots 64 and 32 (three workgroups of eight 16-row wavefronts per compute unit; four of
 the wavefronts bring K and four V), forced with HSTU_MI355_SHORT=1, against the CPU oracle: tile and sub-tile edges, padded head dims, masks,
 grouped heads, keys of their own, outputs on addresses that take no 16-byte stores, with and without attn_bias."""
 
@@ -29,6 +29,8 @@ CASES = {
     "context, targets, groups": dict(heads=2, lengths=[20, 400, 131, 260], num_context=5, max_target=17, target_group_size=3),
     "grouped heads": dict(heads=4, heads_k=2, lengths=[200, 129, 30, 1]),
     "padded head dims": dict(heads=2, dim=48, dim_v=48, lengths=[260, 100, 33]),
+    "slot 32": dict(heads=4, heads_k=2, dim=32, lengths=[260, 100, 33, 128], num_context=3, max_target=9, target_group_size=2),
+    "dims of 16": dict(heads=2, dim=16, lengths=[129, 300, 32, 1]),
     "64-key edges": dict(heads=2, lengths=[63, 64, 65, 191, 192, 193]),
     "narrow v": dict(heads=2, dim=64, dim_v=16, lengths=[260, 100, 33]),
     "odd pitch of the bias": dict(heads=2, lengths=[300, 150], max_seq_len=308),
@@ -79,15 +81,18 @@ def test_keys_of_their_own_and_rows_past_the_last(rows, keys, monkeypatch):
     torch.testing.assert_close(got[:-5].double(), ref, atol=1e-2, rtol=1e-2)
 
 
-@pytest.mark.parametrize("batch,rows,keys,bias,short", [
+@pytest.mark.parametrize("batch,rows,keys,bias,short,dim", [(*c, 64) for c in (
     (32, 1024, 1024, False, True), (32, 1024, 1025, False, False), (3, 300, 704, False, True), (3, 300, 708, False, False),
     (64, 300, 708, False, True), (256, 1024, 1024, False, True), (257, 1024, 1024, False, False), (2, 66, 66, False, True),
     (4, 512, 512, True, True), (4, 516, 516, True, False), (64, 256, 256, True, True), (64, 260, 260, True, False),
-], ids=str)  # fmt: skip
-def test_the_rule(batch, rows, keys, bias, short):
+)] + [(*c, 32) for c in (
+    (16, 500, 704, False, True), (16, 500, 705, False, False), (64, 500, 500, False, False), (80, 500, 512, False, True), (80, 500, 513, False, False),
+    (64, 256, 256, True, True), (65, 256, 256, True, False), (16, 512, 512, True, True), (17, 512, 512, True, False), (16, 516, 516, True, False),
+)], ids=str)  # fmt: skip
+def test_the_rule(batch, rows, keys, bias, short, dim):
     """Which calls of 4 heads take the kernel by themselves: bounds on keys, K / V bytes, slots; 256 compute units."""
-    q = torch.empty(batch * rows, 4, 64, dtype=torch.bfloat16, device=DEV)
-    k = torch.empty(batch * keys, 4, 64, dtype=torch.bfloat16, device=DEV)
+    q = torch.empty(batch * rows, 4, dim, dtype=torch.bfloat16, device=DEV)
+    k = torch.empty(batch * keys, 4, dim, dtype=torch.bfloat16, device=DEV)
     offs, offs_k = ((torch.arange(batch + 1, dtype=torch.int32) * n).to(DEV) for n in (rows, keys))
     rab = torch.empty(batch, 4, rows, keys, dtype=torch.bfloat16, device=DEV) if bias else None
     p = _ops.prepare_forward(q, k, k, None, rab, 0, rows, keys, 1.0 / keys, offs, offs_k, None, None, 0, 0.125)
