@@ -50,10 +50,10 @@ INFINITY_CACHE_BYTES = 256 << 20  # MI355X memory-side cache; a working set belo
 # the forward kernel's source at the time).  A figure whose hash no longer matches the source in the tree is stale
 # and is reported as null.
 MEASURED_TRAFFIC = {
-    "C2": (99_100_000, "profiles/hstu_fwd_bf16_d128_C2_trace_and_counters.md", "7cf633f94624baac"),
-    "C3": (308_500_000, "profiles/hstu_fwd_bf16_d128_rab_C3_trace_and_counters.md", "6ae93d101a7a9d44"),
-    "C4": (1_506_800_000, "profiles/hstu_fwd_bf16_d128_rab_C4_trace_and_counters.md", "6ae93d101a7a9d44"),
-    "C5": (844_800_000, "profiles/hstu_fwd_f8e4m3_d128_C5_trace_and_counters.md", "6ae93d101a7a9d44"),
+    "C2": (99_100_000, "profiles/hstu_fwd_bf16_d128_C2_trace_and_counters.md", "604ccafbb82b3aae"),
+    "C3": (284_100_000, "profiles/hstu_fwd_bf16_d128_rab_C3_trace_and_counters.md", "6c73dd4252c513e9"),
+    "C4": (1_470_300_000, "profiles/hstu_fwd_bf16_d128_rab_C4_trace_and_counters.md", "6c73dd4252c513e9"),
+    "C5": (847_400_000, "profiles/hstu_fwd_f8e4m3_d128_C5_trace_and_counters.md", "6c73dd4252c513e9"),
 }
 _CSRC = os.path.join(_ROOT, "ops-rec_amd", "csrc")
 KERNEL_SOURCE = os.path.join(_CSRC, "hstu_fwd_kernel.hip.h")  # the persistent kernel (and the helpers the others share)
