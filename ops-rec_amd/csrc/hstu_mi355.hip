@@ -2047,22 +2047,24 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         const uint64_t part_bytes = split_part_bytes(var);
         if (usable_workspace(workspace, workspace_bytes, kCounterBytes + 2 * part_bytes) &&
             may_take_split_variant(var, p, nullptr, paged != nullptr)) {
-            kernel = var->kernel_split;
-            a.counters = static_cast<unsigned int*>(workspace);
-            a.ws = reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes);
             const uint64_t parts = (workspace_bytes - kCounterBytes) / part_bytes;
             a.ws_parts = static_cast<uint32_t>(parts < 0x7fffffffull ? parts : 0x7fffffffull);
-            n_blocks = hstu::split_grid(resident);  // the list may have more entries than items: all resident workgroups take part
         }
-        if (paged != nullptr) {
-            kernel = var->kernel_paged;  // (splits when it was given room above, otherwise not; the caller checked the block)
-            a.counters = static_cast<unsigned int*>(workspace);
+        // (the slot 256 has no list with split items: room that is too little to cut every item leaves it with the launches that need none)
+        void (*const listed)(const hstu::FwdArgs) = paged != nullptr ? var->kernel_paged : var->kernel_split;
+        if (a.ws_parts > 0 || paged != nullptr) {
+            a.slot_parts = slot_parts(var, p, paged != nullptr, hstu::split_grid(resident), a.ws_parts);
         }
-        if (kernel == var->kernel_split || paged != nullptr) {
-            a.slot_parts = slot_parts(var, p, paged != nullptr, hstu::split_grid(resident), a.ws != nullptr ? a.ws_parts : 0);
+        if (a.slot_parts > 0 || ((a.ws_parts > 0 || paged != nullptr) && listed != nullptr)) {
+            a.counters = static_cast<unsigned int*>(workspace);  // (paged: the caller checked the block)
+            a.ws = a.ws_parts > 0 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes) : nullptr;
             if (a.slot_parts > 0) {
                 kernel = paged != nullptr ? var->kernel_paged_direct : var->kernel_split_direct;
                 n_blocks = direct_slots(p, a.slot_parts);
+            } else {
+                kernel = listed;  // (the paged one splits when it was given room, otherwise not)
+                // a list with parts may have more entries than items: all resident workgroups take part
+                n_blocks = a.ws_parts > 0 ? hstu::split_grid(resident) : n_blocks;
             }
         }
         if (a.counters == nullptr && takes_direct_list(var, p, static_cast<int64_t>(cus) * wgs_per_cu(var, p))) {
