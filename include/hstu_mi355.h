@@ -138,7 +138,10 @@ typedef struct hstu_jagged_fwd_params {
  * each has a workspace (and an output) of its own.  The library keeps no device state between calls.
  * A caller that passes less than asked for, or nothing, gets the same results from the fixed schedule.  Because a
  * split changes the order of the fp32 sums, the last bit of an output element may then depend on what else is in
- * the batch; HSTU_MI355_SPLIT=0 in the environment turns the split off.  The same holds for fp32 inputs, whose kernel
+ * the batch; HSTU_MI355_SPLIT=0 in the environment turns the split off.  The same holds for the kernels for short
+ * lists and short sequences, which a 16-bit batch of few or short sequences takes and which add in an order of their
+ * own: HSTU_MI355_SPLIT=0 keeps sequences of more than 64 rows at head dims up to 64 on one order, and with
+ * HSTU_MI355_SHORT=0 beside it every 16-bit call is.  And it holds for fp32 inputs, whose kernel
  * needs no workspace: it deals the keys of a row over as many wavefronts as it takes to fill the machine, which
  * depends on the batch, the heads and max_seq_len; with HSTU_MI355_SPLIT=0 one wavefront takes them all. */
 HSTU_API int hstu_jagged_fwd_workspace_size(const hstu_jagged_fwd_params* params, uint64_t* workspace_bytes);

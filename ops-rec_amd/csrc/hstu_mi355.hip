@@ -77,8 +77,10 @@ using hstu::Variant;
 // Process-wide switches.  They are read from the environment once, at the first call that looks at one, and again
 // only when hstu_reload_switches() is called (a test that changes the environment calls it); a launch reads no
 // environment variable.  A value of -1 means "not set: the library's own rule applies".
-//   HSTU_MI355_SPLIT=0             forward: never cut long items into parts, nor deal the keys of an fp32 row over wavefronts (the
-//                                  rows of a sequence are then the same bits whatever else is in the batch, where both take one kernel);
+//   HSTU_MI355_SPLIT=0             forward: never cut long items into parts, nor deal the keys of an fp32 row over wavefronts, nor take
+//                                  the kernel for short lists at the slots 32 and 64 by its rule; the rows of a sequence are then the same bits
+//                                  whatever else is in the batch, where both take one kernel (above 64 rows in 16 bits at the slots 32 and 64
+//                                  always; elsewhere in 16 bits with HSTU_MI355_SHORT=0 beside it);
 //                                  =1: cut them also on sweeps that are short for it
 //   HSTU_MI355_SHORT=0 / 1         forward: the persistent kernel alone / whenever possible the kernel for short lists
 //   HSTU_MI355_GENERIC_BACKWARD=1  backward: the generic kernels also where tuned ones exist (for comparisons)
@@ -399,6 +401,11 @@ const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fw
     if (forced == 1) {
         return sv;
     }
+    // (it adds in another order than the persistent kernel: at the slots 32 and 64 HSTU_MI355_SPLIT=0 keeps to the latter, so that a row's bits
+    // do not depend on how long the list is)
+    if (var->d_pad <= 64 && switches().split == 0) {
+        return nullptr;
+    }
     int cus = 0;
     if (compute_units(&cus) != HSTU_OK) {
         return nullptr;
@@ -642,8 +649,8 @@ bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p,
     if (var->persistent_wgs_per_cu <= 0 || (var->kernel_split == nullptr && (paged ? var->kernel_paged : var->kernel_split_direct) == nullptr)) {
         return false;
     }
-    // HSTU_MI355_SPLIT=0 turns splitting off: the rows of a sequence then come out bit for bit the same whatever
-    // else is in the batch (a split changes the order of the fp32 sums)
+    // HSTU_MI355_SPLIT=0 turns splitting off: where the batch does not decide the kernel either (HSTU_MI355_SHORT=0), the rows of a
+    // sequence then come out bit for bit the same whatever else is in it (a split changes the order of the fp32 sums)
     if (switches().split == 0) {
         return false;
     }
