@@ -348,10 +348,22 @@ bool short_fits_caches(const hstu_jagged_fwd_params* p, int64_t n_blocks)
     const int64_t items = (p->total_q + 64 * (p->n_offsets - 1)) * p->num_heads_q / hstu::kBlockM;  // (by the mean length)
     return kv_bytes <= (256LL << 20) && n_blocks <= 3 * items;
 }
+// Rows that neither fill 128-byte lines nor divide them (48 elements): the heads of a position share lines, and heads of one sequence run on different
+// XCDs, so that a line comes in twice and more for every tile that is swept, where the queues fetch the rows of a pair about once.  On lists that the
+// queues take (four slots per workgroup they keep resident), with a K/V head per query head, us, queues -> this kernel, d 48: 175 x 8 heads of 943 rows 310
+// -> 424, 299 x 4 of 728 171 -> 224, 164 x 8 of 49..795 105 -> 127, 356 x 8 of 311 142 -> 153, 52 x 8 of 941 (3328 slots) 113 -> 127, 391 rows on
+// 391..782 433 x 4 174 -> 238; the other way 289 x 2 of 373..746 80 -> 72, 236 x 4 of 438 86 -> 87, up to 256 keys 541 x 8 of 118..237 122 -> 105, a head
+// alone 933 x 1 of 510 89 -> 62, two query heads per K/V head 164 x 8 on 4 of 346..692 136 -> 109, below four slots all of 40 draws; d 64, whole lines, 113 x
+// 8 of 472..944 146 -> 125.
+bool straddles_lines(int64_t dim) { return 128 % (2 * dim) != 0 && 2 * dim % 128 != 0; }
 bool short_at_slot_64(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus)
 {
     if (p->attn_bias != nullptr) {
         return (p->max_seq_len_k <= 256 && n_blocks <= 16 * cus) || (p->max_seq_len_k <= 512 && n_blocks <= cus);
+    }
+    if (p->num_heads_k > 1 && p->num_heads_k == p->num_heads_q && (straddles_lines(p->head_dim_qk) || straddles_lines(p->head_dim_v)) &&
+        p->max_seq_len_k > 256 && n_blocks >= 12 * cus) {
+        return false;
     }
     const bool history = p->total_k >= 2 * p->total_q;
     return p->max_seq_len_k <= (history && n_blocks < 64 ? 704 : 1024) && short_fits_caches(p, n_blocks);
@@ -362,10 +374,17 @@ bool short_at_slot_64(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus
 // 18.2 -> 18.4 and 64 x 8 of 250 15.6 -> 15.8; longer keys 16 x 4 of 70 on 1000 17.2 -> 17.5, 64 x 4 of 501 on 1000 36.5 -> 38.6, 256 x 4 of 256..1024
 // 106 -> 115.  With a bias: 64 x 4 of 250 (512 slots) 14.1 -> 13.3, 256 x 4 of 250 40.6 -> 45.3, 64 x 8 of 250 (1024) 21 -> 25; 16 x 4 of 500 (256)
 // 17.6 -> 12.9, 16 x 4 of 256..1024 26 -> 29.
+// Long lists (17 slots per workgroup that the queues keep resident, and more) of more than 256 keys go to the queues, for the lines that heads share
+// as at the slot 64: d 16 1963 x 8 of 24..399 375 -> 409, 1376 x 4 of 112..449 204 -> 214, 1661 x 8 of 64..258 221 -> 232, d 32 995 x 8 of 19..306 148 -> 153,
+// 1131 x 8 on 4 of 256..513 411 -> 422; shorter lists d 32 515 x 8 of 222..444 (16.1) 169 -> 162, 2048 x 2 of 31..502 (16) 146 -> 140, d 16 351 x 8
+// of 99..396 (11) 85 -> 83, though 357 x 8 of 26..419 81 -> 84; up to 256 keys d 32 2048 x 8 of 108 187 -> 148.
 bool short_at_slot_32(const hstu_jagged_fwd_params* p, int64_t n_blocks, int cus)
 {
     if (p->attn_bias != nullptr) {
         return (p->max_seq_len_k <= 256 && n_blocks <= 2 * cus) || (p->max_seq_len_k <= 512 && n_blocks <= cus);
+    }
+    if (p->max_seq_len_k > 256 && n_blocks >= 68 * cus) {
+        return false;
     }
     const bool four_resident = n_blocks > 3 * cus && n_blocks <= 4 * cus && p->max_seq_len_k > 128;
     return p->max_seq_len_k <= (n_blocks <= 3 * cus ? 704 : 512) && !four_resident && short_fits_caches(p, n_blocks);
