@@ -36,25 +36,40 @@ const IlsVariant kVariants[2][4] = {
      ILS_VARIANT(f16_tag, "f16", 2, 256)},
 };
 
+int compute_units_or_256()  // (a size asked for where there is no device)
+{
+    int cus = 0;
+    return hstu::compute_units(&cus) == HSTU_OK ? cus : 256;
+}
+
 // groups of rows of the kernel with the weights in registers: one workgroup per CU in all
 int rows_groups(const in_linear_silu_params* p)
 {
-    int cus = 0;
-    if (hstu::compute_units(&cus) != HSTU_OK) {
-        cus = 256;  // (a size asked for where there is no device)
-    }
+    const int cus = compute_units_or_256();
     const int64_t tiles = (p->m + hstu::kIlsRowsTile - 1) / hstu::kIlsRowsTile;
     const int64_t cols = (p->n + hstu::kIlsRowsCols - 1) / hstu::kIlsRowsCols;
     const int64_t groups = cus / cols > 1 ? cus / cols : 1;
     return static_cast<int>(groups < tiles ? groups : tiles);
 }
 
-// The kernel with the weights in registers, where it is taken: k of 129 to 512 (the registers hold no more; at k = 128 the kernels
-// are level, 20480 x 4096 66.2 against 65.3 us: both write at 5 TB/s), at least six 32-row tiles per workgroup to pay for the weights on their
-// way in (us, bf16, this kernel against the other: 4 tiles 2048 x 512 16.6 / 16.4, 1024 x 256 12.8 / 12.0; 6 tiles 1536 x 384 18.5 /
-// 18.9, 1536 x 192 15.5 / 15.7; 8 tiles 2048 x 512 24.7 / 27.5, 4096 x 256 19.4 / 20.2; 20 tiles 2048 x 512 52.6 / 70.3; 131072 rows,
-// 128 tiles, 373 / 472), and splits that begin at 128-byte lines: elsewhere neighbouring wavefronts write parts of a line
-// (100000 rows of 240 -> 960 147 / 132, of 272 -> 1088 with 40000 rows 70 / 65).
+// The kernel with the weights in registers, where it is taken (us, bf16, the other kernel -> this one; 1600 calls with k of 144 to 512 and n up to
+// 32768 measured on both):
+//   k of 129 to 512: the registers hold no more, and at k = 128 the kernels are level, 20480 x 4096 65.3 -> 66.2: both write at 5 TB/s;
+//   splits that begin at 128-byte lines: elsewhere neighbouring wavefronts write parts of a line (100000 rows of 240 -> 960 132 -> 147, 40000
+//     of 272 -> 1088 65 -> 70);
+//   six 32-row tiles per workgroup at least, to pay for the weights on their way in: 4 tiles 2048 x 512 16.4 -> 16.6, 1024 x 256 12.0 -> 12.8; 6 tiles
+//     1536 x 384 18.9 -> 18.5, 1536 x 192 15.7 -> 15.5; 8 tiles 2048 x 512 27.5 -> 24.7, 4096 x 256 20.2 -> 19.4; 20 tiles 2048 x 512 70.3 -> 52.6;
+//     131072 rows, 128 tiles, 472 -> 373;
+//   past 24 blocks of columns, where few groups of rows are left, leave compute units idle and bring in all of the weights each, 20 tiles: below that
+//     7680 x 384, 2064 rows 24.3 -> 26.6, 7680 x 320, 3122 rows 29.7 -> 33.7, 8192 x 512, 1791 rows 27.1 -> 29.2, 13824 x 288, 1444 rows 26.1 -> 28.6,
+//     22528 x 512, 474 rows 22.3 -> 26.2, at 13 to 14 tiles 22528 x 352, 17920 x 320, 11264 x 352 0.86 to 0.88 x, others up to 1.2 x; from 20 tiles on
+//     442 of 468 calls faster, up to 1.53 x (23552 x 256, 30 tiles, 0.91 x, 24576 x 192, 4201 rows, 86.7 -> 103.5).  Still six where the last of the
+//     other kernel's k steps of 32 is half empty (20800 x 400, 637 rows 30.2 -> 25.8, 10304 x 368, 2155 rows 41.0 -> 31.0; 8704 x 272, 1744 rows
+//     21.8 -> 23.5), and where 64 blocks and more leave no compute unit idle, which goes either way: 16384 x 256, 903 rows 1.12 x, 1000 rows
+//     level, 16384 x 512, 801 rows 28.2 -> 29.1, 768 rows, exactly one round of the other kernel, 22.7 -> 27.4;
+//   up to k = 160, of which the instance for 256 spends 16 steps, less than eight tiles, a round and a bit of the other kernel: 2304 x 144, 5911 rows 1.10
+//     x, 16128 x 144, 777 rows 17.6 -> 16.5; more tiles 576 x 144, 130972 rows 65.3 -> 79.7, 1920 x 160, 49364 rows 76.9 -> 81.9, 6912 x 144, 20951 rows
+//     level (k = 176: 1408 x 176, 30462 rows 40.2 -> 39.6).
 const hstu::IlsRowsVariant* select_rows(const in_linear_silu_params* p)
 {
     if (p->k <= 128 || p->k > 512 || p->m > 0x7fffffff - hstu::kIlsRowsTile) {
@@ -65,7 +80,9 @@ const hstu::IlsRowsVariant* select_rows(const in_linear_silu_params* p)
             return nullptr;
         }
     }
-    if (p->m / hstu::kIlsRowsTile < 6 * static_cast<int64_t>(rows_groups(p))) {
+    const int64_t tiles = p->m / hstu::kIlsRowsTile, groups = rows_groups(p), cols = (p->n + hstu::kIlsRowsCols - 1) / hstu::kIlsRowsCols;
+    const bool six_pay = cols <= 24 || p->k % 32 != 0 || (cols >= 64 && cols * groups == compute_units_or_256());
+    if (tiles < (six_pay ? 6 : 20) * groups || (p->k <= 160 && tiles >= 8 * groups)) {
         return nullptr;
     }
     const hstu::IlsRowsVariant* v = hstu::ils_rows_variants(p->dtype == HSTU_DT_BF16);
