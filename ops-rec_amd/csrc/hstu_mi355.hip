@@ -327,6 +327,14 @@ const hstu::ShortVariant* one_item_variant(const Variant* var, const hstu_jagged
     return few_rows_variant(var, p);
 }
 
+// slots of a launch without a list: pairs padded to a multiple of 8 (hstu_fwd_kernel.hip.h)
+int64_t direct_slots(const hstu_jagged_fwd_params* p, int64_t parts = 1)
+{
+    const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
+    const int64_t pairs_pad = ((p->n_offsets - 1) * p->num_heads_k * parts + 7) & ~int64_t{7};
+    return n_qtiles * pairs_pad * (p->num_heads_q / p->num_heads_k);
+}
+
 // The kernel for short work lists at the head-dim slot 64, where three workgroups share a compute unit.  Its steps are no shorter than the
 // persistent kernel's (0.43 us per 32 keys alone on a compute unit, 0.3 there), but it begins 4 to 5 us sooner.  Measured, us, the
 // other variants -> this kernel, without a bias:
@@ -412,6 +420,9 @@ const hstu::ShortVariant* short_variant(const Variant* var, const hstu_jagged_fw
                  p->max_seq_len_q * p->max_seq_len_k * 2 >= (1LL << 32))) {
         return nullptr;
     }
+    if (direct_slots(p) > (1LL << 22)) {  // (the kernel's divisions of a slot's number; the lists hold the items alone)
+        return nullptr;
+    }
     const hstu::ShortVariant* const sv = &hstu::fwd_variants_short()[var->d_pad <= 64 ? 0 : 1][(bias ? 2 : 0) + (p->dtype == HSTU_DT_BF16 ? 0 : 1)];
     const int forced = switches().short_lists;
     if (forced == 0) {
@@ -475,14 +486,6 @@ int wgs_per_cu(const Variant* var, const hstu_jagged_fwd_params* p)
         return 2;
     }
     return var->persistent_wgs_per_cu;
-}
-
-// slots of a launch without a list: pairs padded to a multiple of 8 (hstu_fwd_kernel.hip.h)
-int64_t direct_slots(const hstu_jagged_fwd_params* p, int64_t parts = 1)
-{
-    const int64_t n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM;
-    const int64_t pairs_pad = ((p->n_offsets - 1) * p->num_heads_k * parts + 7) & ~int64_t{7};
-    return n_qtiles * pairs_pad * (p->num_heads_q / p->num_heads_k);
 }
 
 // Whether a plain launch does without a list, a workgroup per slot: when every slot is resident at once, and, up to the head-dim
@@ -2035,17 +2038,12 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
     if (const hstu::ShortVariant* const sv =
             (paged == nullptr) ? short_variant(var, p, usable_workspace(workspace, workspace_bytes, kCounterBytes)) : nullptr) {
         // one workgroup per (query tile, K/V pair padded to a multiple of 8, query head of the pair) slot
-        const int64_t pairs_pad = (static_cast<int64_t>(a.n_batch) * a.n_heads_k + 7) & ~static_cast<int64_t>(7);
-        const int64_t slots = static_cast<int64_t>(a.n_qtiles) * pairs_pad * a.head_ratio;
-        if (slots > (1LL << 22)) {
-            return fail(HSTU_ERR_INVALID, "grid of %lld workgroups is out of range", (long long)slots);
-        }
 #ifdef HSTU_TIMELINE
         if (const char* const t = getenv("HSTU_TIMELINE_BUFFER")) {
             a.counters = reinterpret_cast<unsigned int*>(strtoull(t, nullptr, 0));  // development builds: where the workgroups leave their time stamps
         }
 #endif
-        hipLaunchKernelGGL(sv->kernel, dim3(static_cast<unsigned>(slots)), dim3(hstu::kShortThreads), 0,
+        hipLaunchKernelGGL(sv->kernel, dim3(static_cast<unsigned>(direct_slots(p))), dim3(hstu::kShortThreads), 0,
                            static_cast<hipStream_t>(stream), a);
         const hipError_t err_short = hipGetLastError();
         if (err_short != hipSuccess) {
