@@ -280,6 +280,8 @@ HSTU_API int hstu_version(void);
 /* name of the kernel variant hstu_jagged_fwd would launch for `params` (for profiles and logs),
  * or NULL after an error.  The string is static. */
 HSTU_API const char* hstu_jagged_fwd_kernel_name(const hstu_jagged_fwd_params* params);
+/* the same for hstu_paged_fwd, given the workspace hstu_paged_fwd_workspace_size asks for */
+HSTU_API const char* hstu_paged_fwd_kernel_name(const hstu_paged_fwd_params* params);
 
 #ifdef __cplusplus
 }

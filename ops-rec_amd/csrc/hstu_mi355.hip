@@ -721,6 +721,13 @@ uint64_t split_workspace_bytes(const Variant* var, const hstu_jagged_fwd_params*
     return bytes < kMaxWorkspaceBytes ? bytes : kMaxWorkspaceBytes;
 }
 
+// room for partial outputs in what a launch asks for
+int64_t asked_parts(const Variant* var, const hstu_jagged_fwd_params* p, bool paged = false)
+{
+    const uint64_t bytes = split_workspace_bytes(var, p, paged);
+    return bytes > kCounterBytes ? static_cast<int64_t>((bytes - kCounterBytes) / split_part_bytes(var)) : 0;
+}
+
 // what a forward launch described by p asks of its caller: the counter block when the list may be long enough for
 // the variant with per-XCD queues, the counter block and room for partial outputs when it may be short enough to
 // split items, nothing for the lists in between (fixed schedule, no device counters)
@@ -1923,9 +1930,31 @@ HSTU_API const char* hstu_jagged_fwd_kernel_name(const hstu_jagged_fwd_params* p
         return v->name_queues;
     }
     if (may_take_split_variant(v, params, nullptr)) {
-        return v->name_split;
+        return slot_parts(v, params, false, hstu::split_grid(resident), asked_parts(v, params)) > 0 ? v->name_split_direct : v->name_split;
     }
     return takes_direct_list(v, params, resident) ? v->name_direct : v->name;
+}
+
+HSTU_API const char* hstu_paged_fwd_kernel_name(const hstu_paged_fwd_params* params)
+{
+    hstu_jagged_fwd_params g;
+    uint64_t region = 0;
+    if (validate_paged(params, &g, &region) != HSTU_OK) {
+        return nullptr;
+    }
+    const Variant* v = select(&g);
+    if (v == nullptr) {
+        return nullptr;
+    }
+    if (v->kernel_paged == nullptr) {
+        return hstu_jagged_fwd_kernel_name(&g);  // (on gathered rows)
+    }
+    int cus = 0;
+    if (compute_units(&cus) != HSTU_OK) {
+        return v->name_paged;
+    }
+    const int64_t resident = static_cast<int64_t>(cus) * wgs_per_cu(v, &g);
+    return slot_parts(v, &g, true, hstu::split_grid(resident), asked_parts(v, &g, true)) > 0 ? v->name_paged_direct : v->name_paged;
 }
 
 }  // extern "C"
@@ -2052,6 +2081,7 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         return HSTU_OK;
     }
     void (*kernel)(const hstu::FwdArgs) = var->kernel;
+    const char* name = var->name;
     if (var->persistent_wgs_per_cu > 0) {
         // persistent kernel: a fixed number of workgroups pulls the (at most n_blocks) work items
         int cus = 0;
@@ -2065,6 +2095,7 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         const bool have_counters = usable_workspace(workspace, workspace_bytes, kCounterBytes);
         if (have_counters && takes_queue_variant(var, p, &resident)) {
             kernel = var->kernel_queues;
+            name = var->name_queues;
             a.counters = static_cast<unsigned int*>(workspace);
         }
         n_blocks = n_blocks < resident ? n_blocks : resident;
@@ -2084,8 +2115,10 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
             a.ws = a.ws_parts > 0 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + kCounterBytes) : nullptr;
             if (a.slot_parts > 0) {
                 kernel = paged != nullptr ? var->kernel_paged_direct : var->kernel_split_direct;
+                name = paged != nullptr ? var->name_paged_direct : var->name_split_direct;
                 n_blocks = direct_slots(p, a.slot_parts);
             } else {
+                name = paged != nullptr ? var->name_paged : var->name_split;
                 kernel = listed;  // (the paged one splits when it was given room, otherwise not)
                 // a list with parts may have more entries than items: all resident workgroups take part
                 n_blocks = a.ws_parts > 0 ? hstu::split_grid(resident) : n_blocks;
@@ -2093,6 +2126,7 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
         }
         if (a.counters == nullptr && takes_direct_list(var, p, static_cast<int64_t>(cus) * wgs_per_cu(var, p))) {
             kernel = var->kernel_direct;
+            name = var->name_direct;
             n_blocks = direct_slots(p);
         }
         if (kernel == var->kernel_queues) {
@@ -2122,7 +2156,7 @@ int launch_forward(const hstu_jagged_fwd_params* p, const hstu_paged_fwd_params*
                        static_cast<hipStream_t>(stream), a);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) {
-        return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", var->name, hipGetErrorString(err));
+        return fail(HSTU_ERR_RUNTIME, "launch of %s failed: %s", name, hipGetErrorString(err));
     }
     return HSTU_OK;
 }

@@ -22,7 +22,8 @@ constexpr auto queues_kernel() -> void (*)(const FwdArgs)
 template <typename Tag, typename OutTag, int D, bool RAB, bool MASK>
 constexpr auto split_kernel() -> void (*)(const FwdArgs)
 {
-    // (at the slot 256 split items were measured level with the plain list: -12 .. +16 % over ten shapes)
+    // (at the slot 256 a list with split items was measured level with the plain list, -12 .. +16 % over ten shapes; items cut alike without a list
+    // are a gain there: split_direct_kernel below)
     if constexpr (D == 64 || D == 128) {
         return hstu_fwd_kernel<Tag, OutTag, D, RAB, MASK, false, true>;
     } else {
@@ -74,7 +75,10 @@ constexpr auto paged_direct_kernel() -> void (*)(const FwdArgs)
      hstu::hstu_fwd_kernel<hstu::tag, hstu::tag, D, RAB, MASK, false, false, false, true>,          \
      "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_direct",                               \
      hstu::split_direct_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(),                               \
-     hstu::paged_direct_kernel<hstu::tag, hstu::tag, D, RAB, MASK>()}
+     hstu::paged_direct_kernel<hstu::tag, hstu::tag, D, RAB, MASK>(),                              \
+     "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_slots_split",                         \
+     "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_paged",                               \
+     "hstu_fwd_" tagname "_d" #D "_rab" #RAB "_mask" #MASK "_slots_paged"}
 #define HSTU_DIMS(tag, tagname, RAB, MASK)                                                           \
     {HSTU_VARIANT(tag, tagname, 32, RAB, MASK), HSTU_VARIANT(tag, tagname, 64, RAB, MASK), \
      HSTU_VARIANT(tag, tagname, 128, RAB, MASK), HSTU_VARIANT(tag, tagname, 256, RAB, MASK)}

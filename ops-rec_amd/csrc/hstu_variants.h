@@ -7,8 +7,8 @@
 
 namespace hstu {
 
-// the persistent kernel's variants (hstu_variant_tables.h): with split items for the head-dim slots 64 and 128, with paged keys for
-// 64, 128 and 256 (nullptr elsewhere)
+// the persistent kernel's variants (hstu_variant_tables.h): with split items from a list for the head-dim slots 64 and 128, without one and
+// with paged keys for 64, 128 and 256 (nullptr elsewhere)
 struct Variant {
     const char* name;
     const char* name_queues;
@@ -24,6 +24,9 @@ struct Variant {
     const char* name_direct;
     void (*kernel_split_direct)(const FwdArgs);  // the split variant without a list, all items cut alike; may be nullptr
     void (*kernel_paged_direct)(const FwdArgs);  // the paged one likewise; may be nullptr
+    const char* name_split_direct;
+    const char* name_paged;
+    const char* name_paged_direct;
 };
 
 // the forward kernel for short work lists (hstu_fwd_short_kernel.hip.h): one workgroup of `threads` per

@@ -30,6 +30,7 @@ EXPORTED_SYMBOLS = (
     "hstu_jagged_bwd",
     "hstu_paged_fwd_workspace_size",
     "hstu_paged_fwd",
+    "hstu_paged_fwd_kernel_name",
     "ln_mul_fwd",
     "ln_mul_fwd_kernel_name",
     "in_linear_silu_fwd",
@@ -244,6 +245,8 @@ def load() -> ctypes.CDLL:
     lib.hstu_paged_fwd_workspace_size.argtypes = [ctypes.POINTER(PagedParams), ctypes.POINTER(ctypes.c_uint64)]
     lib.hstu_paged_fwd.restype = ctypes.c_int
     lib.hstu_paged_fwd.argtypes = [ctypes.POINTER(PagedParams), ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p]
+    lib.hstu_paged_fwd_kernel_name.restype = ctypes.c_char_p
+    lib.hstu_paged_fwd_kernel_name.argtypes = [ctypes.POINTER(PagedParams)]
     lib.ln_mul_fwd.restype = ctypes.c_int
     lib.ln_mul_fwd.argtypes = [ctypes.POINTER(LnMulParams), ctypes.c_void_p]
     lib.ln_mul_fwd_kernel_name.restype = ctypes.c_char_p
