@@ -14,13 +14,13 @@ pytestmark = pytest.mark.gpu
 BF, F8 = torch.bfloat16, torch.float8_e4m3fn
 
 
-def params(batch, heads, heads_k, dim, rows, keys, dtype=BF, dim_v=None, context=False, bias=False):
+def params(batch, heads, heads_k, dim, rows, keys, dtype=BF, dim_v=None, context=False, bias=False, mean=None):
     p = _native.new_params()
     p.q, p.k, p.v, p.out, p.seq_offset_q, p.seq_offset_k = (0x100000 * i for i in range(1, 7))  # never dereferenced
     p.dtype = _native.DT_FP8_E4M3 if dtype == F8 else _native.DT_BF16
     p.out_dtype = _native.DT_BF16
     p.n_offsets, p.num_heads_q, p.num_heads_k, p.head_dim_qk, p.head_dim_v = batch + 1, heads, heads_k, dim, dim_v or dim
-    p.max_seq_len_q, p.max_seq_len_k, p.total_q, p.total_k = rows, keys, batch * rows, batch * keys
+    p.max_seq_len_q, p.max_seq_len_k, p.total_q, p.total_k = rows, keys, batch * (mean or rows), batch * keys
     p.alpha, p.silu_scale = 0.125, 1.0
     p.num_context = 0x800000 if context else None
     p.attn_bias = 0x900000 if bias else None
@@ -94,6 +94,35 @@ def test_rows_on_a_history(args, kw, ending, monkeypatch):
 def test_paged(args, kw, ending, monkeypatch):
     helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", "0")
     name = name_of(params(*args, **kw), paged=True)
+    assert name.endswith(ending), name
+
+
+@pytest.mark.parametrize(
+    "args,mean,paged,ending",
+    [
+        # uneven rows at the slot 128: two parts of each slot, or those that a list makes of the tiles that the mean length tells of
+        ((22, 2, 1, 128, 429, 6254), 241, False, "_maskfalse_split"),  # 176 slots, 104 tiles: 4.9 parts spare 58 steps of 196
+        ((22, 2, 1, 128, 429, 2080), 241, False, "_slots_split"),  # 19.2 of 65
+        ((22, 2, 1, 128, 429, 6254), 414, False, "_maskfalse_split"),  # 176 tiles, 2.9 parts: 30.6
+        ((50, 2, 2, 128, 200, 3000), 150, False, "_slots_split"),  # 200 slots, 167 tiles: 16.3 steps of 94, two rounds either way
+        ((50, 2, 2, 128, 200, 3700), 150, False, "_maskfalse_split"),  # 20.2 of 116
+        # at the slot 64 from 25 steps on, or ten and a round less
+        ((82, 2, 2, 64, 166, 2560), 110, False, "_maskfalse_split"),  # 328 slots, 223 tiles
+        ((82, 2, 2, 64, 166, 1500), 110, False, "_slots_split"),  # two rounds instead of three, but 9.9 steps
+        # whole items of paged calls: two parts of each tile, or a round less
+        ((68, 2, 1, 128, 222, 3600), 130, True, "_maskfalse_paged"),
+        ((68, 2, 1, 128, 222, 3600), 215, True, "_slots_paged"),
+        ((363, 1, 1, 64, 149, 5400), 99, True, "_maskfalse_paged"),  # 462 tiles: two rounds instead of three
+        ((363, 1, 1, 64, 149, 5400), 140, True, "_slots_paged"),
+        ((52, 1, 1, 256, 400, 3000), 100, True, "_slots_paged"),  # no rule at the slot 256
+        ((4, 2, 2, 128, 100, 6000), 20, False, "_slots_split"),  # one tile
+    ],
+    ids=str,
+)
+def test_uneven_rows(args, mean, paged, ending, monkeypatch):
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SPLIT", "1")
+    helpers.set_switch(monkeypatch, "HSTU_MI355_SHORT", "0")
+    name = name_of(params(*args, mean=mean), paged=paged)
     assert name.endswith(ending), name
 
 
