@@ -46,7 +46,7 @@ constexpr int kQueueCounterBytes = 1024;   // of which the work counters of the 
 // grid of a launch that may split is what bounds them: at most this many workgroups (split_grid).
 constexpr int kMaxSplitItems = 1024;
 constexpr int64_t split_grid(int64_t resident) { return resident < kMaxSplitItems ? resident : kMaxSplitItems; }
-// (on the 256 CUs of an MI355X that is every resident workgroup of the variants that split, the slots 64 and 128)
+// (on the 256 CUs of an MI355X that is every resident workgroup of the variants that split: the slots 64 and 128, and 256 with one per CU)
 static_assert(split_grid(256 * fwd_wgs_per_cu(64, false, false)) == 256 * 3 && split_grid(256 * fwd_wgs_per_cu(128, false, false)) == 256 * 2,
               "no resident workgroup is left out");
 static_assert(split_grid(int64_t{2048} * 3) == kMaxSplitItems, "and no launch has more items to split than there are counters");

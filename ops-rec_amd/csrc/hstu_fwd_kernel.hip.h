@@ -789,10 +789,11 @@ __global__ __launch_bounds__(256, fwd_wgs_per_cu(D, HAS_RAB, HAS_MASK)) void hst
     // LDS read offsets relative to a sub-tile (in elements; fp8 and kFreshOffsets: in bytes).  In the bias variants each goes through empty assembly
     // once per time step (kFreshOffsets): what the slots add to it is then worked out where it is read, as the constant part of the address.  Left
     // alone, the compiler keeps the sums for all four slots in registers, 36 of them at the slot 128, where the bias variants then had 29 values per
-    // item in scratch memory.  They have none now: one wave of items, which pays the reads of the start of an item in full, gains most.  Measured, us:
+    // item in scratch memory.  Those with a bias alone have none now (with a custom mask beside it the lists of the slot 128 keep 64 to 80 bytes per lane
+    // there, the launch without a list none): one wave of items, which pays the reads of the start of an item in full, gains most.  Measured, us:
     // 64 x 4 heads of 300..600 keys 57.1 -> 50.6, 16 x 4 of 512..2048 67.1 -> 62.2, 16 x 8 of 1024..4096 406 -> 400; at the slot 64, 128 x 4 of 100..300
     // 29.8 -> 25.6, else level.  Not the slot 256, whose slots take more than the 64 KB that the constant part reaches (107.3 -> 108.5), nor without a
-    // bias, where nothing is in scratch (level).  Those keep offsets in elements too: in bytes the launches without a list of the slot 256 took 1.5 to 3 %
+    // bias, where nothing is in scratch but 12 bytes of the paged lists and 76 to 96 of the lists with a custom mask at the slot 128 (level).  Those keep offsets in elements too: in bytes the launches without a list of the slot 256 took 1.5 to 3 %
     // longer (3 x 4 heads on 2, d 192, 321..451 keys 20.2 -> 20.9; with a bias, 4 x 4 on 2, d 256, 312..520 keys 24.9 -> 25.5).
     constexpr bool kFreshOffsets = HAS_RAB && !F8 && D <= 128;
     constexpr int kOffsetUnit = kFreshOffsets ? 2 : 1;

@@ -344,8 +344,9 @@ int64_t direct_slots(const hstu_jagged_fwd_params* p, int64_t parts = 1)
 //   on 1000 15.0 -> 17.5, 1 x 4 of 70 on 1000 12.9 -> 17.2 (64 slots are past that: 16 x 4 of 70 on 1000 17.6 -> 17.4);
 //   longer keys go either way: 16 x 4 of 2048 60 -> 51, 512..2048 39 -> 46, 16 x 4 of 501 on 1200..1400 24.1 -> 23.2, 16 x 4 of 1024..4096 97 -> 122.
 // With an attn_bias, whose rows it reads 32 bytes at a time: 256 x 4 of 60..200 39 -> 28, 64 x 4 of 250 13.8 -> 13.5, 1024 x 2 of 100..250 86 -> 77
-// (4096 slots), but 1000 x 4 of 100..256 (8000) 167 -> 180; up to a slot per compute unit on 512 keys, 16 x 4 of 500 16.4 -> 13.0; with two it is even (32 x 4 of 256..512 17.1 -> 18.3, of 500 18.2 -> 16.1), and
-// longer rows lose (16 x 4 of 256..1024 23.7 -> 29.4).
+// (4096 slots), but 1000 x 4 of 100..256 (8000) 167 -> 180; up to a slot per compute unit on
+// 512 keys, 16 x 4 of 500 16.4 -> 13.0; with two it is even (32 x 4 of 256..512 17.1 -> 18.3, of 500 18.2 -> 16.1), and longer rows lose (16 x 4 of
+// 256..1024 23.7 -> 29.4).
 //
 // Without a bias, not over more K / V rows than the caches hold, which the queues keep to one XCD pair by pair (512 x 4 of 1024 481 -> 579, 256..1024,
 // 335 MB, even, 512 x 4 of 500 on 1000 340 -> 410; 256 x 4 of 1024, 268 MB, 243 -> 236), nor where most slots of the grid are empty (128 x 8 of 8..1000,
@@ -721,9 +722,10 @@ bool may_take_split_variant(const Variant* var, const hstu_jagged_fwd_params* p,
     if (var->kernel_split == nullptr && !paged && (p->max_seq_len_k <= 1024 || slot_parts(var, p, false, resident, resident) == 0)) {
         return false;
     }
-    // A launch without a list (which the paged variant does not have) needs no building of a list, no hand-over of parts through memory
-    // and no counters: on short sweeps that outweighs what idle compute units could add, unless there is next to nothing to do or a
-    // tile is much longer than the others.  Measured, split -> without a list: up to 1024 keys -- slot 64, 16 x 4 heads, 501 rows on 1000
+    // A launch of whole items without a list (paged launches choose in slot_parts) needs no building of a list, no hand-over of parts through
+    // memory and no counters: on short sweeps that outweighs what idle compute units could add, unless there is next to nothing to do or a
+    // tile is much longer than the others.  Measured, parts from a list -> whole items without one (parts in slots, which rows on a history take
+    // instead of the list, build none either: these lines are from before them): up to 1024 keys -- slot 64, 16 x 4 heads, 501 rows on 1000
     // 30.6 -> 22.3 us, 8 x 4 of 512..1000 22.0 -> 18.9, slot 128 with a bias 26.6 <- 34.1; up to 2048 keys, the rows at most half of them --
     // slot 64, 16 x 4, 200 rows on 1500 34.5 -> 25.2, slot 128 37.9 -> 33.3.  It loses below 64 slots (1 x 2 of 2000 24.4 -> 30.3), with a bias
     // on longer keys (slot 64, 4 x 4 of 1000..2000 30.5 -> 34.2), on longer causal rows (slot 128, 1 x 8 of 2000 36.4 -> 38.9; slot 64 mixed),
@@ -1160,8 +1162,8 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
     return static_cast<int>(std::min<int64_t>(most / 8, std::max<int64_t>(1, (std::max(bytes >> 20, groups / 8) + 7) / 8)) * 8);
 }
 
-// Calls with attn_bias that keep the orders without dS tiles (see few_key_tiles).  The key-tile kernel's step is longest there, and a workgroup has as many steps as its K/V head has query heads times row blocks: the order pays from the tiles on
-// that keep the machine busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute
+// Calls with attn_bias that keep the orders without dS tiles (see few_key_tiles).  The key-tile kernel's step is longest there, and a workgroup has as
+// many steps as its K/V head has query heads times row blocks: the order pays from the tiles on that keep the machine busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute
 // units, whatever the group's size.
 // Measured on 125 shapes, and 300 more for short rows, pairs of heads and histories (device time in us, other order / dS handed over), at the slot 128
 // with a key-tile kernel that spilled and took 245 us where it now takes 177: the lines below leave it no call that is slower, and some that would

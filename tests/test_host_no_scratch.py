@@ -1,5 +1,6 @@
-"""Kernels whose waits count the requests under way: nothing of theirs may go through scratch memory, whose accesses count too.  Looked for in
-what the compiler reports of them under the build's own flags."""
+"""Kernels whose waits count the requests under way, with every register spoken for: nothing of theirs goes through scratch memory, whose accesses
+would count among the requests and turn each wait into one for the next tile as well.  Looked for in what the compiler reports of them under the
+build's own flags."""
 
 import os
 import re
