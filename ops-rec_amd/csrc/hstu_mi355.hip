@@ -636,18 +636,18 @@ constexpr uint64_t kMaxWorkspaceBytes = 128ull << 20;
 constexpr uint64_t kCounterBytes = hstu::kCounterBlockBytes;  // head of the workspace of the variants that pull from counters
 uint64_t split_part_bytes(const Variant* var) { return static_cast<uint64_t>(hstu::kBlockM) * var->d_pad * sizeof(float); }
 // Whether a list is the faster one for items of several query tiles all the same, at the slots that have one with parts.  Slots are there for tiles that are
-// not, too: with rows of uneven lengths a list has fewer entries, cuts them further where the room for the slots' last parts falls between two whole
-// numbers, and deals them one per compute unit before it deals a second.  It is taken where its parts spare the longest sweep 20 steps (25 at the slot
-// 64) and more, or where it needs a round of one entry per compute unit less and spares ten.  Measured, 1400 calls of several tiles, us, list -> slots:
+// not, too: with rows of uneven lengths a list has fewer entries, cuts them further, and deals them one per compute unit before it deals a second.  It
+// is taken against up to three parts where it has room for one more and those spare the longest sweep 20 steps (25 at the slot 64) and more, or
+// where it needs a round of one entry per compute unit less and spares ten.  Measured, 1400 calls of several tiles, us, list -> slots:
 // 62 x 1, fp8, d 64, 95..574 rows on 1611..6444 keys 59 -> 85, 22 x 2 on 1, d 128, 53..429 on 1563..6254 54 -> 76, 152 x 1, d 64, 26..158 on 2473..4946 50 ->
 // 65, 17 x 2 on 1, fp8, d 128, 272..544 on 3143..6287 51 -> 67; paged 90 x 1, d 64, 88..264 on 5843 69 -> 97, 17 x 4, d 128, 155..466 on 3173 75 -> 101; a
 // round less 40 x 4, d 64, 112..150 on 853..3412 (20 steps) 43 -> 49, whole paged items 363 x 1, d 64, 49..149 on 2632..5265 141 -> 164, 80 x 2, d 64, 161..484
 // on 5113 139 -> 169.  The other way 34 x 4, d 64, 126..168 on 1298..5192 60 -> 57, paged 125 x 1, d 64, 330..440 on 2070..4141 1.06 x; of
-// the 990 calls that the rule leaves on the slots 12 are slower there by more than 3 %, of the 450 that it sends to the list 280.
+// the 1050 calls that the rule leaves on the slots 16 are slower there by more than 3 %, of the 390 that it sends to the list 270, and 60 faster.
 bool list_beats_slots(const Variant* var, const hstu_jagged_fwd_params* p, int64_t resident, int64_t room, int64_t parts)
 {
     const int64_t batch = p->n_offsets - 1, n_qtiles = (p->max_seq_len_q + hstu::kBlockM - 1) / hstu::kBlockM, slots = n_qtiles * batch * p->num_heads_q;
-    if (n_qtiles == 1 || var->d_pad > 128) {
+    if (n_qtiles == 1 || var->d_pad > 128 || parts > 3) {
         return false;
     }
     const bool alike = batch * p->max_seq_len_q - p->total_q < 16 * batch;
@@ -657,7 +657,8 @@ bool list_beats_slots(const Variant* var, const hstu_jagged_fwd_params* p, int64
     const double spared = steps * (1.0 / parts - 1.0 / listed);
     const double cus = static_cast<double>(resident) / var->persistent_wgs_per_cu;
     const bool round_less = std::ceil(items * parts / cus) < std::ceil(slots * parts / cus);
-    return ((parts > 1 || listed >= 2.0) && spared >= (var->d_pad == 64 ? 25.0 : 20.0)) || (round_less && spared >= 10.0 && (var->d_pad == 64 || parts == 1));
+    return (listed >= parts + 1 && spared >= (var->d_pad == 64 ? 25.0 : 20.0)) ||
+           (round_less && spared >= 10.0 && (parts == 1 || (parts == 2 && var->d_pad == 64)));
 }
 
 // Parts that a split or paged launch without a list cuts every item into (1: paged, whole items), 0 where it takes the list: items whose

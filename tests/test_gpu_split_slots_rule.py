@@ -103,7 +103,8 @@ def test_paged(args, kw, ending, monkeypatch):
         # uneven rows at the slot 128: two parts of each slot, or those that a list makes of the tiles that the mean length tells of
         ((22, 2, 1, 128, 429, 6254), 241, False, "_maskfalse_split"),  # 176 slots, 104 tiles: 4.9 parts spare 58 steps of 196
         ((22, 2, 1, 128, 429, 2080), 241, False, "_slots_split"),  # 19.2 of 65
-        ((22, 2, 1, 128, 429, 6254), 414, False, "_maskfalse_split"),  # 176 tiles, 2.9 parts: 30.6
+        ((22, 2, 1, 128, 429, 6254), 414, False, "_slots_split"),  # 176 tiles: no room for a third part of each
+        ((10, 4, 4, 128, 300, 7000), 80, False, "_slots_split"),  # four parts of each slot
         ((50, 2, 2, 128, 200, 3000), 150, False, "_slots_split"),  # 200 slots, 167 tiles: 16.3 steps of 94, two rounds either way
         ((50, 2, 2, 128, 200, 3700), 150, False, "_maskfalse_split"),  # 20.2 of 116
         # at the slot 64 from 25 steps on, or ten and a round less
