@@ -1164,8 +1164,8 @@ static int clear_workgroups(int64_t bytes, int64_t groups, int64_t dmax, int cus
 }
 
 // Calls with attn_bias that keep the orders without dS tiles (see few_key_tiles).  The key-tile kernel's step is longest there, and a workgroup has as
-// many steps as its K/V head has query heads times row blocks: the order pays from the tiles on that keep the machine busy for longer than the longest of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute
-// units, whatever the group's size.
+// many steps as its K/V head has query heads times row blocks: the order pays from the tiles on that keep the machine busy for longer than the longest
+// of them, which for grouped heads is (tiles x mean rows / longest rows) against the compute units, whatever the group's size.
 // Measured on 125 shapes, and 300 more for short rows, pairs of heads and histories (device time in us, other order / dS handed over), at the slot 128
 // with a key-tile kernel that spilled and took 245 us where it now takes 177: the lines below leave it no call that is slower, and some that would
 // now be faster (forward included, 16 x 4, 300..500 rows 79 / 66, 234 x 4, 58..216 164 / 149, 64 x 4, 100 on 376 keys 79 / 75, 32 x 8 on 1, 1024 841 / 668):
